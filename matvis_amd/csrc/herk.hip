@@ -120,7 +120,8 @@ __device__ inline int active_slices_wave(int ktiles, int ntiles,
     const uint64_t o = __shfl_xor(key, off, 64);
     key = o < key ? o : key;
   }
-  return lo + (int)(key & 63);
+  // every lane holds the least key: a scalar, so that what depends on it is
+  return lo + __builtin_amdgcn_readfirstlane((int)(key & 63));
 }
 
 // Columns of each segment: the device count never exceeds the host bound the
@@ -157,6 +158,100 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// 16 bytes from global memory per lane straight into LDS: lane l's bytes
+// land at byte 16 l of the wave-uniform destination `lds`.
+__device__ __forceinline__ void copy16_to_lds(const uint32_t *src,
+                                              uint32_t *lds) {
+  __builtin_amdgcn_global_load_lds(src, lds, 16, 0, 0);
+}
+// Wait until this wave's global loads, LDS copies included, have landed.
+__device__ __forceinline__ void wait_global_loads() {
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), other counters unchecked
+}
+
+// ------------------------------------------------------------ panel groups
+
+// The upper triangle of the n x n grid of P-row panels is cut into groups of
+// at most four panel pairs (i, j), i <= j, that touch at most four panels: a
+// workgroup stages the group's panels and each of its four waves computes one
+// pair.  Every pair is in exactly one group and only the last group of a run
+// of diagonal pairs holds fewer than four, where square tiles of 2 x 2 pairs
+// leave a wave idle on every diagonal tile and two on every tile of a
+// half-empty last column (11 panels: 17 groups instead of 21 tiles).
+//   Off the diagonal: blocks I < J of two panels, all four pairs.
+//   n even, diagonal: the pairs (2I, 2I), (2I, 2I + 1), (2I + 1, 2I + 1) of
+//     I = 0, 1, ... in sequence, four a group (at most four adjacent panels).
+//   n odd, last panel L = n - 1: per block (2I, 2I), (2I, 2I + 1), (2I, L),
+//     (2I + 1, L); then the pairs (2I + 1, 2I + 1) and (L, L), four a group.
+__host__ __device__ inline int panel_groups(int n) {
+  const int h = n / 2;
+  const int off = h * (h - 1) / 2;
+  return (n & 1) ? off + h + icdiv(h + 1, 4) : off + icdiv(3 * h, 4);
+}
+
+// Row-major index of pair (i, j), i <= j, in the upper triangle of n panels.
+__host__ __device__ inline int pair_index(int i, int j, int n) {
+  return i * n - i * (i - 1) / 2 + (j - i);
+}
+
+// What wave w of group g does: it stages panel `load` into slot w (none if
+// negative) and computes the pair of panels (i, j), held in slots si and sj
+// (none if i is negative).
+struct WavePair {
+  int load, i, j, si, sj;
+};
+__host__ __device__ inline WavePair group_wave(int g, int n, int w) {
+  const int h = n / 2;
+  const int off = h * (h - 1) / 2;
+  WavePair p;
+  if (g < off) {
+    int I = 0, t = g;
+    while (t >= h - 1 - I) {
+      t -= h - 1 - I;
+      ++I;
+    }
+    const int J = I + 1 + t;
+    p.si = w >> 1;
+    p.sj = 2 + (w & 1);
+    p.i = 2 * I + p.si;
+    p.j = 2 * J + (w & 1);
+    p.load = w < 2 ? 2 * I + w : 2 * J + w - 2;
+    return p;
+  }
+  g -= off;
+  if (n & 1) {
+    const int L = n - 1;
+    if (g < h) {
+      // slots: 0 = 2g, 1 = 2g + 1, 2 = L
+      p.load = w < 2 ? 2 * g + w : (w == 2 ? L : -1);
+      p.si = w == 3 ? 1 : 0;
+      p.sj = w < 2 ? w : 2;
+      p.i = 2 * g + p.si;
+      p.j = w < 2 ? 2 * g + w : L;
+      return p;
+    }
+    const int e = 4 * (g - h) + w;  // (2e + 1, 2e + 1), the last one (L, L)
+    p.load = e < h ? 2 * e + 1 : (e == h ? L : -1);
+    p.i = p.j = p.load;
+    p.si = p.sj = w;
+    return p;
+  }
+  // pair s of the sequence: block s / 3, entry s % 3
+  const int s0 = 4 * g, s = s0 + w;
+  const int first = 2 * (s0 / 3) + (s0 % 3 == 2);  // row panel of pair s0
+  p.load = first + w < n ? first + w : -1;
+  if (s >= 3 * h) {
+    p.i = p.j = -1;
+    p.si = p.sj = 0;
+    return p;
+  }
+  p.i = 2 * (s / 3) + (s % 3 == 2);
+  p.j = 2 * (s / 3) + (s % 3 != 0);
+  p.si = p.i - first;
+  p.sj = p.j - first;
+  return p;
+}
+
 // ------------------------------------------------------------ plain forms
 
 template <typename T> struct PlainMfma;
@@ -167,156 +262,261 @@ template <> struct PlainMfma<double> {
   __device__ static acc op(double a, double b, acc c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
-  __device__ static int row(int g, int r) { return g + 4 * r; }
+  static constexpr int kRowStep = 4;
+  __device__ static int row(int g, int r) { return g + kRowStep * r; }
 };
 template <> struct PlainMfma<float> {
   typedef v4f acc;
   __device__ static acc op(float a, float b, acc c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
-  __device__ static int row(int g, int r) { return 4 * g + r; }
+  static constexpr int kRowStep = 1;
+  __device__ static int row(int g, int r) { return 4 * g + kRowStep * r; }
 };
 
-constexpr int kPT = 64;  // tile side, complex rows
+constexpr int kPT = 64;  // side the accumulator of the plain forms is padded to
 constexpr int kPK = 16;  // complex columns per LDS stage (one K tile)
-constexpr int kPRow = kPK + 1;  // LDS row length (one element of padding)
 
-// 256 threads = 4 waves in a 2x2 arrangement, each wave a 32x32 sub-tile made
-// of 2x2 blocks of 16x16.  One 16x16x4 MFMA consumes two complex columns:
-// lane l supplies k-slot g = l / 16 -> column g / 2, part g % 2 (re / im).
-// One (slice, tile) item of a plain HERK: the slice's K tiles staged through
-// two LDS stages (As for the tile's rows, Bs for its columns; separate
-// __shared__ arrays of the calling kernel, which the compiler aligns for
-// 16-byte LDS reads), the partial tile written to `part`.
+// Bytes of a panel row in LDS (one K tile) and the 16-byte chunks it has.
+template <typename T> constexpr int kPRowBytes = kPK * 2 * (int)sizeof(T);
+
+// Where column c of row r of a panel sits in LDS: rows are not padded; the
+// row's 16-byte chunks are permuted by an XOR with bits of the row, so that
+// the 16 rows (times the columns of a lane group) one operand read touches
+// fall in distinct banks: 16 chunks of one complex128 against r % 16, 8
+// chunks of two complex64 against (r / 2) % 8 (rows 2q and 2q + 1 are the two
+// halves of the 64 banks).
+template <typename T> __device__ __forceinline__ int plain_swz(int r) {
+  return sizeof(T) == 8 ? (r & 15) : ((r >> 1) & 7);
+}
+template <typename T> __device__ __forceinline__ int plain_pos(int r, int c) {
+  const int b = c * 2 * (int)sizeof(T);  // byte within the row
+  return r * kPRowBytes<T> + (((b >> 4) ^ plain_swz<T>(r)) << 4) + (b & 15);
+}
+
+// One K tile of a group's four panels; the two stages of a kernel are
+// separate __shared__ objects (see the split forms' stages).
+template <typename T, int P> struct alignas(16) PlainStage {
+  char x[4][P * kPRowBytes<T>];
+};
+
+// One plain HERK instance as the kernels read it.
+template <typename T> struct PlainProblem {
+  const cplx<T> *z;
+  int64_t ldz, seg_stride;
+  cplx<T> *part;
+  int m, n, ngroups, npairs;  // rows, panels, groups, panel pairs
+  int wide;  // rows are 16-byte aligned and offsets fit 32-bit 16-byte units
+};
+
+// Whether the 16-byte copies apply: every row and segment starts on 16 bytes
+// and a row's offset fits 32 bits of 16-byte units.
 template <typename T>
-__device__ __forceinline__ void plain_item(
-    const cplx<T> *__restrict__ z, int m, int64_t ldz, int64_t seg_stride,
-    int64_t seg_len, int64_t kt_per_seg, int nb, int ntiles, int ktiles,
-    int ns, int slice, int tile, cplx<T> *__restrict__ part,
-    cplx<T> (&As)[2][kPT * kPRow], cplx<T> (&Bs)[2][kPT * kPRow]) {
+__host__ __device__ inline int plain_wide(const PlainProblem<T> &Q, int nseg) {
+  constexpr int per = 16 / (2 * (int)sizeof(T));  // columns in 16 bytes
+  return (uintptr_t)Q.z % 16 == 0 && Q.ldz % per == 0 &&
+         (nseg == 1 || Q.seg_stride % per == 0) &&
+         (int64_t)Q.m * Q.ldz / per < ((int64_t)1 << 32);
+}
+
+// The P x P panel pairs of one (slice, group) item, each wave its own pair as
+// (P / 16)^2 blocks of 16x16.
+//
+// Three real products a complex one, conj(a + ib)(c + id):
+//   T1 = a c, T2 = b d, T3 = (a - b)(c + d): Re = T1 + T2, Im = T3 - T1 + T2,
+// one 16x16x4 MFMA each per 4 complex columns (lane group g = l / 16 supplies
+// column g), where the four products of the plain formula take four MFMAs:
+// the matrix cores bind this kernel, and the sums and differences are one
+// VALU instruction an operand.  The accumulators' chains are half as long as
+// four products' (K / 4 MFMAs, not K / 2), which offsets the third term of
+// Im.  FP32 chains are cut further: two accumulator sets over alternate
+// columns at P = 32 (kSets), half as many K tiles a slice (form_cmax).
+// Errors |dV| / |V| (2-norms) of four products -> these: complex64 against
+// FP64, incoherent Z 0.9-2.8e-7 -> 0.8-2.3e-7, nearly coherent Z (phases
+// within 0.3 rad) 1.9-6.3e-8 -> 1.9-5.4e-8, a whole time of the 350-antenna
+// sky 8.4e-7 -> 3.8e-7; complex128 against extended precision, incoherent
+// 2.0-2.8e-16 -> 1.9-2.9e-16, nearly coherent 0.8-1.5e-16 -> 0.9-1.8e-16,
+// the whole time 9.9e-15 (its phases) in both.  The diagonal is exactly real.
+//
+// Measured, m = 700 (350 antennas, polarized): FP64, 29.9k sources up, 2.47
+// -> 1.48 ms; FP32, 59.7k sources, 2.71 -> 1.51 ms: 80% of the rate of
+// three products at the peak (78.6 and 157 TFLOP/s), from 63% and 58% of four
+// products'.  Square tiles, copies through registers with a mask on every
+// element and half of each operand read thrown away made the difference.
+//
+// Copies go straight from global memory into the other LDS stage
+// (global_load_lds: 16 bytes a lane where rows are 16-byte aligned, else 4),
+// each wave one panel, while the current K tile is computed; the last K tile
+// of a segment that is not whole goes through registers with a column mask.
+// Rows past m are read as row m - 1: they reach output rows and columns past
+// m only.
+template <typename T, int P>
+__device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
+                                           int64_t seg_len, int slice,
+                                           int group, int ns, int ktiles,
+                                           int kps, PlainStage<T, P> &L0,
+                                           PlainStage<T, P> &L1) {
   typedef typename PlainMfma<T>::acc acc_t;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wr = wave >> 1, wc = wave & 1;
-  const int lrow = tid >> 2, lcol = (tid & 3) * 4;
+  typedef T vec2 __attribute__((ext_vector_type(2)));
+  constexpr int RB = kPRowBytes<T>, CH = RB / 16;  // row bytes, chunks a row
+  constexpr int NB = P / 16;                       // 16-row blocks a panel
+  constexpr int NI = P * RB / 1024;                // 1 KB copies a panel
+  // the wave's index in a scalar register: what it does is uniform over it
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
   const int g = lane >> 4, rl = lane & 15;
-  const bool im_part = g & 1;
-  int bi, bj;
-  tile_coords(tile, nb, bi, bj);
-  const bool diag = bi == bj;
-  // sub-tiles below the diagonal or wholly in the row padding do no MFMA
-  const bool active = !(diag && wr > wc) && bi * kPT + wr * 32 < m &&
-                      bj * kPT + wc * 32 < m;
-  const int64_t kt0 = (int64_t)slice * ktiles / ns;
-  const int64_t kt1 = (int64_t)(slice + 1) * ktiles / ns;
-  const int64_t grow_a = (int64_t)bi * kPT + lrow;
-  const int64_t grow_b = (int64_t)bj * kPT + lrow;
+  const WavePair wp = group_wave(group, Q.n, wave);
+  const int kt0 = (int)((int64_t)slice * ktiles / ns);
+  const int kt1 = (int)((int64_t)(slice + 1) * ktiles / ns);
 
-  acc_t acc_re[2][2], acc_im[2][2];
+  // this lane's part of copy u: row u 1024 / RB + lane / CH of the panel,
+  // LDS chunk lane % CH, i.e. logical chunk (lane % CH) ^ swz(row)
+  uint32_t off[NI];
+  const int prow0 = wp.load * P;
+  if (wp.load >= 0 && Q.wide) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      acc_re[i][j] = acc_t{};
-      acc_im[i][j] = acc_t{};
-    }
-
-  cplx<T> ra[4], rb[4];
-  auto gload = [&](int64_t kt, int64_t grow, cplx<T> *r) {
-    const int64_t sg = kt / kt_per_seg;
-    const int64_t c0 = (kt % kt_per_seg) * kPK + lcol;
-    const cplx<T> *src = z + grow * ldz + sg * seg_stride + c0;
-    const bool row_ok = grow < m;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      r[q] = (row_ok && c0 + q < seg_len) ? src[q] : cplx<T>{(T)0, (T)0};
-  };
-  auto lstore = [&](cplx<T> *dst, const cplx<T> *r) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) dst[lrow * kPRow + lcol + q] = r[q];
-  };
-
-  if (kt0 < kt1) {
-    gload(kt0, grow_a, ra);
-    lstore(As[0], ra);
-    if (!diag) {
-      gload(kt0, grow_b, rb);
-      lstore(Bs[0], rb);
+    for (int u = 0; u < NI; ++u) {
+      const int r = u * (1024 / RB) + lane / CH;
+      const int gr = prow0 + r < Q.m ? prow0 + r : Q.m - 1;
+      const int c = (lane % CH) ^ plain_swz<T>(r);
+      off[u] = (uint32_t)((int64_t)gr * Q.ldz * (2 * (int)sizeof(T)) / 16) + c;
     }
   }
-  lds_barrier();
-
-  for (int64_t kt = kt0; kt < kt1; ++kt) {
-    const int buf = (int)((kt - kt0) & 1);
-    const bool has_next = kt + 1 < kt1;
-    if (has_next) {
-      gload(kt + 1, grow_a, ra);
-      if (!diag) gload(kt + 1, grow_b, rb);
-    }
-    const cplx<T> *Ab = As[buf];
-    const cplx<T> *Bb = diag ? As[buf] : Bs[buf];
-    if (active) {
+  int sg = kt0 / (kps > 0 ? kps : 1), kc = kt0 - sg * kps;
+  auto copy = [&](PlainStage<T, P> &D) {
+    const int64_t c0 = (int64_t)kc * kPK;
+    if (wp.load >= 0) {
+      const cplx<T> *src = Q.z + sg * Q.seg_stride + c0;
+      if (c0 + kPK <= seg_len) {
+        if (Q.wide) {
 #pragma unroll
-      for (int ks = 0; ks < kPK / 2; ++ks) {
-        const int col = 2 * ks + (g >> 1);
-        T a[2], bre[2], bim[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          cplx<T> v = Ab[(wr * 32 + i * 16 + rl) * kPRow + col];
-          a[i] = im_part ? v.im : v.re;
-        }
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          cplx<T> v = Bb[(wc * 32 + j * 16 + rl) * kPRow + col];
-          bre[j] = im_part ? v.im : v.re;
-          bim[j] = im_part ? -v.re : v.im;
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            acc_re[i][j] = PlainMfma<T>::op(a[i], bre[j], acc_re[i][j]);
-            acc_im[i][j] = PlainMfma<T>::op(a[i], bim[j], acc_im[i][j]);
+          for (int u = 0; u < NI; ++u)
+            copy16_to_lds(
+                (const uint32_t *)((const char *)src + ((uint64_t)off[u] << 4)),
+                (uint32_t *)&D.x[wave][u * 1024]);
+        } else {
+#pragma unroll 1
+          for (int u = 0; u < 4 * NI; ++u) {
+            const int b = u * 256 + lane * 4, r = b / RB, x = b % RB;
+            const int gr = prow0 + r < Q.m ? prow0 + r : Q.m - 1;
+            const char *row = (const char *)(src + (int64_t)gr * Q.ldz);
+            __builtin_amdgcn_global_load_lds(
+                (const uint32_t *)(row + (((x >> 4) ^ plain_swz<T>(r)) << 4) +
+                                   (x & 15)),
+                (uint32_t *)&D.x[wave][u * 256], 4, 0, 0);
           }
+        }
+      } else {
+        const int valid = (int)(seg_len - c0);  // 1 .. kPK - 1 columns
+#pragma unroll 1
+        for (int e = lane; e < P * kPK; e += 64) {
+          const int r = e / kPK, c = e % kPK;
+          const int gr = prow0 + r < Q.m ? prow0 + r : Q.m - 1;
+          const cplx<T> v = src[(int64_t)gr * Q.ldz + (c < valid ? c : 0)];
+          *(vec2 *)&D.x[wave][plain_pos<T>(r, c)] =
+              c < valid ? vec2{v.re, v.im} : vec2{(T)0, (T)0};
+        }
       }
     }
-    if (has_next) {
-      lstore(As[buf ^ 1], ra);
-      if (!diag) lstore(Bs[buf ^ 1], rb);
+    if (++kc == kps) {
+      kc = 0;
+      ++sg;
     }
-    lds_barrier();
-  }
+  };
 
+  constexpr int kSets = sizeof(T) == 4 && P == 32 ? 2 : 1;
+  acc_t t1[kSets][NB][NB], t2[kSets][NB][NB], t3[kSets][NB][NB];
+#pragma unroll
+  for (int q = 0; q < kSets; ++q)
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        t1[q][i][j] = t2[q][i][j] = t3[q][i][j] = acc_t{};
+
+  auto compute = [&](const PlainStage<T, P> &D) {
+    const char *A = D.x[wp.si], *B = D.x[wp.sj];
+#pragma unroll
+    for (int ks = 0; ks < kPK / 4; ++ks) {
+      const int pos = plain_pos<T>(rl, 4 * ks + g);
+      vec2 a[NB], b[NB];
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        a[i] = *(const vec2 *)&A[i * 16 * RB + pos];
+        b[i] = *(const vec2 *)&B[i * 16 * RB + pos];
+      }
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+          constexpr int S = kSets - 1;
+          acc_t &x = t1[ks & S][i][j], &y = t2[ks & S][i][j],
+                &z = t3[ks & S][i][j];
+          x = PlainMfma<T>::op(a[i][0], b[j][0], x);
+          y = PlainMfma<T>::op(a[i][1], b[j][1], y);
+          z = PlainMfma<T>::op(a[i][0] - a[i][1], b[j][0] + b[j][1], z);
+        }
+      // operand reads stay in their step: hoisted over the unrolled steps
+      // they would spill (the other wave of the SIMD covers their latency)
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // one K tile computed from stage C while the next is copied into N
+  auto step = [&](PlainStage<T, P> &C, PlainStage<T, P> &N, int kt) {
+    if (kt + 1 < kt1) copy(N);
+    if (wp.i >= 0) compute(C);
+    wait_global_loads();  // this wave's copies into N
+    lds_barrier();
+  };
+
+  if (kt0 < kt1) copy(L0);
+  wait_global_loads();
+  lds_barrier();
+  for (int kt = kt0; kt < kt1; kt += 2) {
+    step(L0, L1, kt);
+    if (kt + 1 < kt1) step(L1, L0, kt + 1);
+  }
+  // every wave is past the last barrier: LDS is free for the next item
+
+  if (wp.i < 0) return;
   // 16x16 accumulator: lane l = 16 g + rl, register r -> row
   // PlainMfma<T>::row(g, r), column rl
-  cplx<T> *out = part + ((int64_t)slice * ntiles + tile) * kPT * kPT;
+  // (the base is opaque so that the store addresses are formed here)
+  cplx<T> *out = Q.part +
+                 ((int64_t)slice * Q.npairs + pair_index(wp.i, wp.j, Q.n)) * P * P;
+  int obase = PlainMfma<T>::row(g, 0) * P + rl;
+  asm volatile("" : "+v"(obase));
+  out += obase;
+  constexpr int rstep = PlainMfma<T>::kRowStep * P;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < NB; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = wr * 32 + i * 16 + PlainMfma<T>::row(g, r);
-        const int col = wc * 32 + j * 16 + rl;
-        out[row * kPT + col] = cplx<T>{acc_re[i][j][r], acc_im[i][j][r]};
+        T x = t1[0][i][j][r], y = t2[0][i][j][r], w = t3[0][i][j][r];
+        if constexpr (kSets == 2) {
+          x += t1[1][i][j][r];
+          y += t2[1][i][j][r];
+          w += t3[1][i][j][r];
+        }
+        out[i * 16 * P + r * rstep + j * 16] =
+            cplx<T>{x + y, (w - x) + y};
       }
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void herk_plain_kernel(
-    const cplx<T> *__restrict__ z, int m, int64_t ldz, int nseg,
-    int64_t seg_stride, int64_t seg_len_host,
-    const int32_t *__restrict__ seg_len_dev, int nb, int ntiles,
-    SliceCfg cfg, cplx<T> *__restrict__ part) {
-  __shared__ cplx<T> As[2][kPT * kPRow];
-  __shared__ cplx<T> Bs[2][kPT * kPRow];
+template <typename T, int P>
+__global__ __launch_bounds__(256, 2) void herk_plain_kernel(
+    PlainProblem<T> Q, int nseg, int64_t seg_len_host,
+    const int32_t *__restrict__ seg_len_dev, SliceCfg cfg) {
+  __shared__ PlainStage<T, P> L0, L1;
   const int64_t seg_len = seg_columns(seg_len_host, seg_len_dev);
-  const int64_t kt_per_seg = cdiv(seg_len, (int64_t)kPK);
-  const int ktiles = (int)(kt_per_seg * nseg);
-  const int ns = active_slices_wave(ktiles, ntiles, cfg);
-  for_items((int64_t)ntiles * ns, [&](int64_t it) {
-    plain_item<T>(z, m, ldz, seg_stride, seg_len, kt_per_seg, nb, ntiles,
-                  ktiles, ns, (int)(it / ntiles), (int)(it % ntiles), part,
-                  As, Bs);
+  const int kps = (int)cdiv(seg_len, (int64_t)kPK);  // K tiles per segment
+  const int ktiles = kps * nseg;
+  const int ns = active_slices_wave(ktiles, Q.ngroups, cfg);
+  for_items((int64_t)Q.ngroups * ns, [&](int64_t it) {
+    plain_item<T, P>(Q, seg_len, (int)(it / Q.ngroups), (int)(it % Q.ngroups), ns,
+                     ktiles, kps, L0, L1);
   });
 }
 
@@ -404,7 +604,8 @@ struct SplitProblem {
   cplx<double> *vacc;
   int64_t ldv;
   double scale;
-  int m, nseg, nb, ntiles, accumulate;
+  int m, nseg, nb, ntiles, accumulate;  // ntiles: partial tiles a slice
+  int ngroups;  // work items a slice (tiles, or groups of panel pairs)
 };
 
 // Block shape of the split kernels for a tile side: 128 -> 256 threads as
@@ -422,17 +623,6 @@ template <int TILE> struct SplitShape {
 __device__ __forceinline__ int swz(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
 __device__ __forceinline__ int lds_word(int r, int w) {
   return r * kSK + (((w >> 2) ^ swz(r)) << 2);
-}
-
-// 16 bytes from global memory per lane straight into LDS: lane l's bytes
-// land at byte 16 l of the wave-uniform destination `lds`.
-__device__ __forceinline__ void copy16_to_lds(const uint32_t *src,
-                                              uint32_t *lds) {
-  __builtin_amdgcn_global_load_lds(src, lds, 16, 0, 0);
-}
-// Wait until this wave's global loads, LDS copies included, have landed.
-__device__ __forceinline__ void wait_global_loads() {
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), other counters unchecked
 }
 
 // One K-tile stage: the A rows (xa) and B rows (xb) of every term.  The two
@@ -722,16 +912,18 @@ struct GroupPlan {
   int32_t *tile_off;  // [nprob + 1]
 };
 
-// Single block: every problem's internal descriptor (tile grid, partial
+// Single block: every problem's internal descriptor (tile or, with `panels`,
+// panel grid of side ts, partial
 // areas carved from `parts` in problem order: cap x ntiles x ts^2 partial
 // elements of part_bytes each, then, with row_norms, cap x ntiles x ts FP64
 // row norms), its slice count (enough slices that no chain exceeds cmax K
 // tiles, at most its capacity: a function of the problem alone) and the
 // prefix offsets.
 __global__ __launch_bounds__(256) void herk_group_plan_kernel(
-    const mv_herk_problem *__restrict__ pub, int nprob, int ts, int kc,
-    int cmax, int part_bytes, int row_norms, SplitProblem *__restrict__ probs,
-    char *__restrict__ parts, GroupPlan plan) {
+    const mv_herk_problem *__restrict__ pub, int nprob, int ts, int panels,
+    int kc, int cmax, int part_bytes, int row_norms,
+    SplitProblem *__restrict__ probs, char *__restrict__ parts,
+    GroupPlan plan) {
   for (int p = threadIdx.x; p < nprob; p += blockDim.x) {
     const mv_herk_problem &q = pub[p];
     SplitProblem P;
@@ -748,6 +940,7 @@ __global__ __launch_bounds__(256) void herk_group_plan_kernel(
     P.accumulate = q.accumulate;
     P.nb = icdiv(q.m, ts);
     P.ntiles = P.nb * (P.nb + 1) / 2;
+    P.ngroups = panels ? panel_groups(P.nb) : P.ntiles;
     P.part = nullptr;
     P.dpart = nullptr;
     probs[p] = P;
@@ -771,7 +964,7 @@ __global__ __launch_bounds__(256) void herk_group_plan_kernel(
       if (row_norms) bytes += cap * P.ntiles * (int64_t)ts * 8;
       plan.item_off[p] = items;
       plan.tile_off[p] = tiles;
-      items += (int64_t)P.ntiles * plan.ns[p];
+      items += (int64_t)P.ngroups * plan.ns[p];
       tiles += P.ntiles;
     }
     plan.item_off[nprob] = items;
@@ -814,23 +1007,30 @@ __global__ __launch_bounds__(SplitShape<TILE>::kThreads,
 
 // Grouped plain HERK: the items of all problems, as the grouped split
 // kernel; each problem's Z is its term pointer 0.
-template <typename T>
-__global__ __launch_bounds__(256) void herk_plain_grouped_kernel(
+template <typename T, int P>
+__global__ __launch_bounds__(256, 2) void herk_plain_grouped_kernel(
     const SplitProblem *__restrict__ probs, int nprob, GroupPlan plan) {
-  __shared__ cplx<T> As[2][kPT * kPRow];
-  __shared__ cplx<T> Bs[2][kPT * kPRow];
+  __shared__ PlainStage<T, P> L0, L1;
   const int64_t items = plan.item_off[nprob];
   for_items(items, [&](int64_t it) {
     const int p = find_segment(plan.item_off, nprob, it);
-    const SplitProblem P = probs[p];
+    const SplitProblem &S = probs[p];
+    PlainProblem<T> Q;
+    Q.z = (const cplx<T> *)S.t[0];
+    Q.ldz = S.ldz;
+    Q.seg_stride = S.seg_stride;
+    const int64_t seg_len = seg_columns(S.seg_len_host, S.seg_len_dev);
+    Q.part = (cplx<T> *)S.part;
+    Q.m = S.m;
+    Q.n = S.nb;
+    Q.ngroups = S.ngroups;
+    Q.npairs = S.ntiles;
+    Q.wide = plain_wide(Q, S.nseg);
     const int ns = plan.ns[p];
     const int64_t local = it - plan.item_off[p];
-    const int64_t seg_len = seg_columns(P.seg_len_host, P.seg_len_dev);
-    const int64_t kt_per_seg = cdiv(seg_len, (int64_t)kPK);
-    plain_item<T>((const cplx<T> *)P.t[0], P.m, P.ldz, P.seg_stride, seg_len,
-                  kt_per_seg, P.nb, P.ntiles, (int)(kt_per_seg * P.nseg), ns,
-                  (int)(local / P.ntiles), (int)(local % P.ntiles),
-                  (cplx<T> *)P.part, As, Bs);
+    const int kps = (int)cdiv(seg_len, (int64_t)kPK);
+    plain_item<T, P>(Q, seg_len, (int)(local / Q.ngroups), (int)(local % Q.ngroups), ns,
+                     kps * S.nseg, kps, L0, L1);
   });
 }
 
@@ -938,6 +1138,8 @@ __device__ __forceinline__ void reduce_elems_t(
       vr = d;
       vi = 0.0;
     }
+  } else if (bi == bj && r == c + h) {
+    vi -= vi;  // the diagonal is real: 0, or NaN where it is not finite
   }
   cplx<double> *dst =
       vacc + ((int64_t)bi * ts + r) * ldv + (int64_t)bj * ts + c + h;
@@ -965,18 +1167,19 @@ __device__ __forceinline__ void reduce_elems(
                               ns, scale, vacc, ldv, accumulate);
 }
 
-// Blocks of 256 threads (128 element groups), per tile.
+// Blocks of 256 threads (128 element groups), per tile (looped past the
+// grid's 65535).
 template <typename TP> dim3 reduce_grid(int ts, int64_t ntiles) {
   return dim3((unsigned)cdiv((int64_t)ts * ts,
                              (int64_t)128 * kReduceEpt<TP>),
-              (unsigned)ntiles);
+              (unsigned)(ntiles < 65535 ? ntiles : 65535));
 }
 
 // grid reduce_grid<TP>(ts, ntiles); the slice count is found once per block
 template <typename TP>
 __global__ __launch_bounds__(256) void herk_reduce_kernel(
     const cplx<TP> *__restrict__ part, const double *__restrict__ dpart,
-    int ntiles, int nb, int ts, int m, int64_t seg_len_host,
+    int ntiles, int ngroups, int nb, int ts, int m, int64_t seg_len_host,
     const int32_t *__restrict__ seg_len_dev, int nseg, int kc, SliceCfg cfg,
     double scale, cplx<double> *__restrict__ vacc, int64_t ldv,
     int accumulate) {
@@ -984,15 +1187,16 @@ __global__ __launch_bounds__(256) void herk_reduce_kernel(
   if (threadIdx.x < 64) {
     const int64_t seg_len = seg_columns(seg_len_host, seg_len_dev);
     const int ktiles = (int)(cdiv(seg_len, (int64_t)kc) * nseg);
-    const int ns = active_slices_wave(ktiles, ntiles, cfg);
+    const int ns = active_slices_wave(ktiles, ngroups, cfg);
     if (threadIdx.x == 0) ns_shared = ns;
   }
   __syncthreads();
   int h;
   const int64_t e = reduce_group<TP>(h);
   if (e >= (int64_t)ts * ts) return;
-  reduce_elems(part, dpart, ntiles, nb, ts, m, (int)blockIdx.y, e, h,
-               ns_shared, scale, vacc, ldv, accumulate);
+  for (int tile = blockIdx.y; tile < ntiles; tile += gridDim.y)
+    reduce_elems(part, dpart, ntiles, nb, ts, m, tile, e, h, ns_shared, scale,
+                 vacc, ldv, accumulate);
 }
 
 // Grouped reduce: blockIdx.y runs over the tiles of all problems (prefix
@@ -1006,12 +1210,14 @@ __global__ __launch_bounds__(256) void herk_group_reduce_kernel(
   if (e >= (int64_t)ts * ts) return;
   // the grid covers the tiles of the problems' largest shapes (a graph
   // replayed with smaller ones keeps it); tiles past this plan's total idle
-  if ((int32_t)blockIdx.y >= plan.tile_off[nprob]) return;
-  const int p = find_segment(plan.tile_off, nprob, (int32_t)blockIdx.y);
-  const SplitProblem &P = probs[p];
-  reduce_elems((const cplx<TP> *)P.part, P.dpart, P.ntiles, P.nb, ts, P.m,
-               (int)blockIdx.y - plan.tile_off[p], e, h, plan.ns[p], P.scale,
-               P.vacc, P.ldv, P.accumulate);
+  const int32_t total = plan.tile_off[nprob];
+  for (int32_t t = blockIdx.y; t < total; t += gridDim.y) {
+    const int p = find_segment(plan.tile_off, nprob, t);
+    const SplitProblem &P = probs[p];
+    reduce_elems((const cplx<TP> *)P.part, P.dpart, P.ntiles, P.nb, ts, P.m,
+                 (int)(t - plan.tile_off[p]), e, h, plan.ns[p], P.scale,
+                 P.vacc, P.ldv, P.accumulate);
+  }
 }
 
 __global__ __launch_bounds__(256) void vacc_sum_kernel(
@@ -1074,7 +1280,7 @@ int split_maxord(int nterms, int nprod) {
 int form_cmax(int form) {
   switch (form) {
     case MV_FORM_C128: return 1 << 30;  // FP64 accumulation: no limit
-    case MV_FORM_C64: return 256;
+    case MV_FORM_C64: return 128;
     default: return 192;
   }
 }
@@ -1102,11 +1308,20 @@ template <class K> int kernel_slots(K kernel, int block = 256) {
   return slots;
 }
 
+// ts: side of the partial tiles (plain: of the panels), nb of them a side,
+// ntiles partial tiles and ngroups work items a slice
 struct HerkPlan {
-  int ts, nb, ntiles, kc;
+  int ts, nb, ntiles, ngroups, kc;
   SliceCfg cfg;
   int grid;
 };
+
+// Panel side of the plain forms for row count m (of the largest problem in a
+// grouped launch): 32 for complex128, whose 64-row panels' accumulators would
+// not fit the registers.
+int panel_side(int form, int m) {
+  return form == MV_FORM_C64 && m > 128 ? 64 : 32;
+}
 
 }  // namespace
 }  // namespace mv
@@ -1153,12 +1368,14 @@ extern "C" int mv_herk_max_slices(int form, int m, int64_t kmax) {
 }
 
 namespace {
-// The kernel instantiation for (form, nterms, maxord) as a type-erased
-// pointer for occupancy queries.
-const void *herk_kernel(int form, int nterms, int maxord) {
+// The kernel instantiation for (form, nterms, maxord, panel side) as a
+// type-erased pointer for occupancy queries.
+const void *herk_kernel(int form, int nterms, int maxord, int panel) {
   switch (form) {
-    case MV_FORM_C128: return (const void *)&herk_plain_kernel<double>;
-    case MV_FORM_C64: return (const void *)&herk_plain_kernel<float>;
+    case MV_FORM_C128: return (const void *)&herk_plain_kernel<double, 32>;
+    case MV_FORM_C64:
+      return panel == 64 ? (const void *)&herk_plain_kernel<float, 64>
+                         : (const void *)&herk_plain_kernel<float, 32>;
     default: break;
   }
   const bool f16 = form == MV_FORM_SPLIT_F16;
@@ -1187,15 +1404,16 @@ const void *grouped_kernel_t(bool f16, int nterms, int maxord) {
 
 int plan_herk(int form, int nterms, int maxord, int m, int nslices,
               HerkPlan &p) {
-  p.ts = mv_herk_tile(form);
+  const bool plain = form == MV_FORM_C128 || form == MV_FORM_C64;
+  p.ts = plain ? panel_side(form, m) : kST;
   p.nb = (int)cdiv((int64_t)m, (int64_t)p.ts);
   p.ntiles = p.nb * (p.nb + 1) / 2;
-  p.kc = p.ts == kPT ? kPK : kSK;
-  const int slots = kernel_slots(herk_kernel(form, nterms, maxord));
+  p.ngroups = plain ? panel_groups(p.nb) : p.ntiles;
+  p.kc = plain ? kPK : kSK;
+  const int slots = kernel_slots(herk_kernel(form, nterms, maxord, p.ts));
   if (slots <= 0) return -1;
-  p.cfg = SliceCfg{nslices, slots, form_cmax(form),
-                   form == MV_FORM_C128 || form == MV_FORM_C64 ? 2 : 4};
-  const int64_t items = (int64_t)p.ntiles * nslices;
+  p.cfg = SliceCfg{nslices, slots, form_cmax(form), plain ? 2 : 4};
+  const int64_t items = (int64_t)p.ngroups * nslices;
   p.grid = (int)(items < slots ? items : slots);
   return 0;
 }
@@ -1212,11 +1430,52 @@ extern "C" int mv_herk_slices(int form, int nterms, int nprod, int m,
   if (plan_herk(form, nterms, maxord, m, nslices, p))
     return MV_ERR_HIP;
   const int ktiles = (int)(cdiv(seg_len, (int64_t)p.kc) * nseg);
-  return active_slices(ktiles, p.ntiles, p.cfg);
+  return active_slices(ktiles, p.ngroups, p.cfg);
 }
 
 namespace {
 constexpr int kPhaseCompute = 1, kPhaseReduce = 2;
+
+struct PlainLaunch {
+  const void *z;
+  int m;
+  int64_t ldz;
+  int nseg;
+  int64_t seg_stride, seg_len;
+  const int32_t *seg_len_dev;
+  double scale;
+  double *vacc;
+  int64_t ldv;
+  int accumulate;
+  void *workspace;
+  int phases;
+  hipStream_t st;
+};
+
+template <typename T, int P>
+int plain_run(const HerkPlan &p, const PlainLaunch &L) {
+  PlainProblem<T> Q;
+  Q.z = (const cplx<T> *)L.z;
+  Q.ldz = L.ldz;
+  Q.seg_stride = L.seg_stride;
+  Q.part = (cplx<T> *)L.workspace;
+  Q.m = L.m;
+  Q.n = p.nb;
+  Q.ngroups = p.ngroups;
+  Q.npairs = p.ntiles;
+  Q.wide = plain_wide(Q, L.nseg);
+  if (L.phases & kPhaseCompute) {
+    herk_plain_kernel<T, P>
+        <<<p.grid, 256, 0, L.st>>>(Q, L.nseg, L.seg_len, L.seg_len_dev, p.cfg);
+    if (int e = check_launch("mv_herk/plain")) return e;
+  }
+  if (!(L.phases & kPhaseReduce)) return MV_OK;
+  herk_reduce_kernel<T><<<reduce_grid<T>(p.ts, p.ntiles), 256, 0, L.st>>>(
+      (const cplx<T> *)L.workspace, nullptr, p.ntiles, p.ngroups, p.nb, p.ts,
+      L.m, L.seg_len, L.seg_len_dev, L.nseg, p.kc, p.cfg, L.scale,
+      (cplx<double> *)L.vacc, L.ldv, L.accumulate);
+  return check_launch("mv_herk/reduce");
+}
 
 // Validation shared by every phase, then the compute kernel (partial tiles
 // into the workspace) and/or the reduce kernel (workspace into Vacc).
@@ -1264,35 +1523,12 @@ int herk_run(int phases, int form, int nterms, int nprod, const void *z0,
     return MV_ERR_HIP;
   }
   hipStream_t st = as_stream(stream);
-  if (form == MV_FORM_C128) {
-    if (phases & kPhaseCompute) {
-      herk_plain_kernel<double><<<p.grid, 256, 0, st>>>(
-          (const cplx<double> *)z0, m, ldz, nseg, seg_stride, seg_len,
-          seg_len_dev, p.nb, p.ntiles, p.cfg, (cplx<double> *)workspace);
-      if (int e = check_launch("mv_herk/plain64")) return e;
-    }
-    if (!(phases & kPhaseReduce)) return MV_OK;
-    herk_reduce_kernel<double>
-        <<<reduce_grid<double>(ts, ntiles), 256, 0, st>>>(
-        (const cplx<double> *)workspace, nullptr, p.ntiles, p.nb, ts, m,
-        seg_len, seg_len_dev, nseg, p.kc, p.cfg, scale, (cplx<double> *)vacc,
-        ldv, accumulate);
-    return check_launch("mv_herk/reduce");
-  }
-  if (form == MV_FORM_C64) {
-    if (phases & kPhaseCompute) {
-      herk_plain_kernel<float><<<p.grid, 256, 0, st>>>(
-          (const cplx<float> *)z0, m, ldz, nseg, seg_stride, seg_len,
-          seg_len_dev, p.nb, p.ntiles, p.cfg, (cplx<float> *)workspace);
-      if (int e = check_launch("mv_herk/plain32")) return e;
-    }
-    if (!(phases & kPhaseReduce)) return MV_OK;
-    herk_reduce_kernel<float>
-        <<<reduce_grid<float>(ts, ntiles), 256, 0, st>>>(
-        (const cplx<float> *)workspace, nullptr, p.ntiles, p.nb, ts, m,
-        seg_len, seg_len_dev, nseg, p.kc, p.cfg, scale, (cplx<double> *)vacc,
-        ldv, accumulate);
-    return check_launch("mv_herk/reduce");
+  if (plain) {
+    const PlainLaunch L = {z0,      m,      ldz,  nseg, seg_stride, seg_len,
+                           seg_len_dev, scale, vacc, ldv,  accumulate,
+                           workspace, phases, st};
+    if (form == MV_FORM_C128) return plain_run<double, 32>(p, L);
+    return p.ts == 64 ? plain_run<float, 64>(p, L) : plain_run<float, 32>(p, L);
   }
   MV_REQUIRE(z1 && (nterms < 3 || z2), "mv_herk: missing term arrays");
   MV_REQUIRE(((uintptr_t)z0 | (uintptr_t)z1 | (uintptr_t)(z2 ? z2 : z0)) %
@@ -1322,6 +1558,7 @@ int herk_run(int phases, int form, int nterms, int nprod, const void *z0,
   P.nseg = nseg;
   P.nb = p.nb;
   P.ntiles = p.ntiles;
+  P.ngroups = p.ngroups;
   P.accumulate = accumulate;
 #define MV_SPLIT_LAUNCH(NT, MO, F)                                           \
   herk_split_kernel<NT, MO, F, kST><<<p.grid, 256, 0, st>>>(P, p.cfg)
@@ -1341,9 +1578,9 @@ int herk_run(int phases, int form, int nterms, int nprod, const void *z0,
 #undef MV_SPLIT_LAUNCH
   if (!(phases & kPhaseReduce)) return MV_OK;
   herk_reduce_kernel<float><<<reduce_grid<float>(ts, ntiles), 256, 0, st>>>(
-      (const cplx<float> *)workspace, dpart, p.ntiles, p.nb, ts, m, seg_len,
-      seg_len_dev, nseg, p.kc, p.cfg, scale, (cplx<double> *)vacc, ldv,
-      accumulate);
+      (const cplx<float> *)workspace, dpart, p.ntiles, p.ngroups, p.nb, ts, m,
+      seg_len, seg_len_dev, nseg, p.kc, p.cfg, scale, (cplx<double> *)vacc,
+      ldv, accumulate);
   return check_launch("mv_herk/reduce");
 }
 
@@ -1524,8 +1761,10 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
   MV_REQUIRE(problems_host && problems_dev && workspace && nprob >= 1,
              "mv_herk_grouped: null pointer or no problems");
   int64_t total_tiles = 0, max_items = 0;
+  int max_m = 0;
   for (int i = 0; i < nprob; ++i) {
     const mv_herk_problem &q = problems_host[i];
+    max_m = q.m > max_m ? q.m : max_m;
     MV_REQUIRE(q.m >= 1 && q.nseg >= 1 && q.seg_len >= 0 &&
                    q.nslices >= 1 && q.kchain >= 0,
                "mv_herk_grouped: problem %d: bad sizes m=%d nseg=%d "
@@ -1565,11 +1804,13 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
              "mv_herk_grouped: workspace too small (%zu < %lld)", ws_bytes,
              (long long)g.total);
   const bool f16 = form == MV_FORM_SPLIT_F16;
+  const int side = split ? tile : panel_side(form, max_m);
   const void *kernel =
       split ? grouped_kernel(tile, f16, nterms, maxord)
-            : (form == MV_FORM_C128
-                   ? (const void *)&herk_plain_grouped_kernel<double>
-                   : (const void *)&herk_plain_grouped_kernel<float>);
+      : form == MV_FORM_C128
+          ? (const void *)&herk_plain_grouped_kernel<double, 32>
+      : side == 64 ? (const void *)&herk_plain_grouped_kernel<float, 64>
+                   : (const void *)&herk_plain_grouped_kernel<float, 32>;
   const int threads = !split ? 256
                       : tile == 64 ? SplitShape<64>::kThreads
                                    : SplitShape<kST>::kThreads;
@@ -1586,27 +1827,36 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
   // slices of a problem: split forms bound the FP32 chain (form_cmax);
   // plain forms take slices of 64 K tiles (1024 columns) for parallelism
   herk_group_plan_kernel<<<1, 256, 0, st>>>(
-      problems_dev, nprob, tile, split ? kSK : kPK,
+      problems_dev, nprob, side, split ? 0 : 1, split ? kSK : kPK,
       split ? form_cmax(form) : 64, part_bytes(form), split ? 1 : 0, probs,
       ws + g.parts, plan);
   if (int e = check_launch("mv_herk_grouped/plan")) return e;
   const int grid = (int)(max_items < slots ? max_items : slots);
   if (!split) {
-    if (form == MV_FORM_C128) {
-      herk_plain_grouped_kernel<double><<<grid, 256, 0, st>>>(probs, nprob,
-                                                              plan);
-      if (int e = check_launch("mv_herk_grouped/plain")) return e;
-      herk_group_reduce_kernel<double>
-          <<<reduce_grid<double>(tile, total_tiles), 256, 0, st>>>(
-              probs, nprob, tile, plan);
-    } else {
-      herk_plain_grouped_kernel<float><<<grid, 256, 0, st>>>(probs, nprob,
-                                                             plan);
-      if (int e = check_launch("mv_herk_grouped/plain")) return e;
-      herk_group_reduce_kernel<float>
-          <<<reduce_grid<float>(tile, total_tiles), 256, 0, st>>>(
-              probs, nprob, tile, plan);
+    // the reduce runs over panel pairs, of which there are more than tiles
+    int64_t pairs = 0;
+    for (int i = 0; i < nprob; ++i) {
+      const int64_t n = cdiv((int64_t)problems_host[i].m, (int64_t)side);
+      pairs += n * (n + 1) / 2;
     }
+    if (form == MV_FORM_C128)
+      herk_plain_grouped_kernel<double, 32><<<grid, 256, 0, st>>>(probs, nprob,
+                                                                  plan);
+    else if (side == 64)
+      herk_plain_grouped_kernel<float, 64><<<grid, 256, 0, st>>>(probs, nprob,
+                                                                 plan);
+    else
+      herk_plain_grouped_kernel<float, 32><<<grid, 256, 0, st>>>(probs, nprob,
+                                                                 plan);
+    if (int e = check_launch("mv_herk_grouped/plain")) return e;
+    if (form == MV_FORM_C128)
+      herk_group_reduce_kernel<double>
+          <<<reduce_grid<double>(side, pairs), 256, 0, st>>>(probs, nprob,
+                                                             side, plan);
+    else
+      herk_group_reduce_kernel<float>
+          <<<reduce_grid<float>(side, pairs), 256, 0, st>>>(probs, nprob, side,
+                                                            plan);
     return check_launch("mv_herk_grouped/reduce");
   }
 #define MV_GROUP_LAUNCH(NT, MO, F, T)                                        \

@@ -173,6 +173,9 @@ inline void emu_global_load_lds(const void *src, void *dst, unsigned size) {
 #define __builtin_amdgcn_global_load_lds(src, dst, size, off, aux) \
   emu_global_load_lds(src, (char *)(dst) + (off), size)
 #define __builtin_amdgcn_s_waitcnt(imm) ((void)0)
+#define __builtin_amdgcn_sched_barrier(mask) ((void)0)
+// the sources take it of wave-uniform values only
+#define __builtin_amdgcn_readfirstlane(x) (x)
 #define __builtin_amdgcn_s_setprio(p) ((void)0)
 inline int __popcll(unsigned long long x) { return __builtin_popcountll(x); }
 // blocks run one at a time here; the atomic keeps the same contract anyway

@@ -304,6 +304,24 @@ def test_herk_plain_vs_numpy(m, k, form):
     assert err < (1e-13 if form == FORM_C128 else 2e-6), err
 
 
+@pytest.mark.parametrize("form", [FORM_C128, FORM_C64])
+@pytest.mark.parametrize("m", [31, 32, 33, 96, 97, 128, 129, 192, 193, 257,
+                               320, 321, 385, 577])
+def test_herk_plain_panel_edges(m, form):
+    """Every panel grouping from 1 to 19 panels (odd and even counts, partly
+    filled last panels), rows of an odd length (no 16-byte rows in
+    complex64), two segments that end inside a K tile."""
+    dtype = np.complex128 if form == FORM_C128 else np.complex64
+    seg, n = 55, 53
+    z = _herk_case(m, 2 * seg + 1, dtype, seed=m)
+    h, v = _run_herk(form, [_dev(z)], m, 2 * seg + 1, 2, seg, n, nslices=4)
+    zv = np.concatenate([z[:, :n], z[:, seg:seg + n]], 1).astype(np.complex128)
+    want = zv.conj() @ zv.T
+    d = np.sqrt(np.diag(want).real)
+    err = (np.abs(_vis_full(h, v, m) - want) / (d[:, None] * d[None])).max()
+    assert err < (1e-13 if form == FORM_C128 else 2e-6), err
+
+
 def test_herk_segments_and_device_length():
     m, seg, n = 70, 48, 37
     z = _herk_case(m, 2 * seg, np.complex128, seed=9)
