@@ -1,11 +1,12 @@
 // (d) V = conj(Z) Z^T as a Hermitian rank-k update on MFMA tiles.
 //
-// Only tiles (bi, bj) with bi <= bj of the upper triangle are computed, and
-// inside them only the 64x64 (split) / 32x32 (plain) wave sub-tiles that hold
-// elements (r, c) with r <= c < m; the accumulator is defined on r <= c.
+// Rows are cut into panels (64 rows; 32 in complex128) and only the panel
+// pairs (i, j) with i <= j of the upper triangle are computed, in groups of
+// four pairs a workgroup (one pair a wave); the accumulator is defined on
+// r <= c.
 //
 // K (the source axis, times nax) is cut into slices.  A work item is one
-// (tile, slice) pair; it writes its partial tile to the workspace, and a
+// (group, slice); its waves write their partial pairs to the workspace, and a
 // reduce kernel sums the slices in FP64 in a fixed order, so results are
 // deterministic.  The number of active slices is chosen on the device from
 // the device-side column count (sources above the horizon are only known
@@ -44,18 +45,6 @@ __device__ __forceinline__ void tile_coords(int t, int nb, int &bi, int &bj) {
   }
   bi = i;
   bj = i + t;
-}
-
-// A 64 x 64 wave sub-tile (wr, wc) of tile (bi, bj), tile side ts, that the
-// split kernels leave idle: below the diagonal of a diagonal tile, or
-// starting at or past row or column m.  Idle sub-tiles get no MFMAs and no
-// partials, and the reduce skips them: their accumulator elements lie below
-// the diagonal or past m, which the accumulator's contract leaves as scratch.
-// (Plain tiles are one 64-wide sub-tile that always starts below m.)
-__host__ __device__ inline bool subtile_idle(int bi, int bj, int wr, int wc,
-                                             int ts, int m) {
-  return (bi == bj && wr > wc) || bi * ts + wr * 64 >= m ||
-         bj * ts + wc * 64 >= m;
 }
 
 struct SliceCfg {
@@ -197,8 +186,13 @@ __host__ __device__ inline int pair_index(int i, int j, int n) {
 // What wave w of group g does: it stages panel `load` into slot w (none if
 // negative) and computes the pair of panels (i, j), held in slots si and sj
 // (none if i is negative).
+// norm: the slot of a panel whose row norms (the split forms' exact diagonal)
+// the group sums as its w-th, -1 if none.  Each panel's are summed once, by a
+// group that stages it: the work would otherwise gather in the last groups.
+// Blocks I, I + 1 off the diagonal take the odd panel of I; the even panels
+// and the last odd one stay with the group of their diagonal pair.
 struct WavePair {
-  int load, i, j, si, sj;
+  int load, i, j, si, sj, norm;
 };
 __host__ __device__ inline WavePair group_wave(int g, int n, int w) {
   const int h = n / 2;
@@ -216,6 +210,7 @@ __host__ __device__ inline WavePair group_wave(int g, int n, int w) {
     p.i = 2 * I + p.si;
     p.j = 2 * J + (w & 1);
     p.load = w < 2 ? 2 * I + w : 2 * J + w - 2;
+    p.norm = w == 1 && J == I + 1 ? 1 : -1;
     return p;
   }
   g -= off;
@@ -228,12 +223,14 @@ __host__ __device__ inline WavePair group_wave(int g, int n, int w) {
       p.sj = w < 2 ? w : 2;
       p.i = 2 * g + p.si;
       p.j = w < 2 ? 2 * g + w : L;
+      p.norm = w == 0 ? 0 : -1;
       return p;
     }
     const int e = 4 * (g - h) + w;  // (2e + 1, 2e + 1), the last one (L, L)
     p.load = e < h ? 2 * e + 1 : (e == h ? L : -1);
     p.i = p.j = p.load;
     p.si = p.sj = w;
+    p.norm = e == h - 1 || e == h ? w : -1;
     return p;
   }
   // pair s of the sequence: block s / 3, entry s % 3
@@ -241,7 +238,7 @@ __host__ __device__ inline WavePair group_wave(int g, int n, int w) {
   const int first = 2 * (s0 / 3) + (s0 % 3 == 2);  // row panel of pair s0
   p.load = first + w < n ? first + w : -1;
   if (s >= 3 * h) {
-    p.i = p.j = -1;
+    p.i = p.j = p.norm = -1;
     p.si = p.sj = 0;
     return p;
   }
@@ -249,6 +246,7 @@ __host__ __device__ inline WavePair group_wave(int g, int n, int w) {
   p.j = 2 * (s / 3) + (s % 3 != 0);
   p.si = p.i - first;
   p.sj = p.j - first;
+  p.norm = p.i == p.j && (s % 3 == 0 || s == 3 * h - 1) ? p.si : -1;
   return p;
 }
 
@@ -563,19 +561,18 @@ template <bool F16> __device__ __forceinline__ float hi_half(uint32_t w) {
     return __builtin_bit_cast(float, w & 0xffff0000u);
 }
 
-// sum over the 8 complex values a thread stages of |t0 + t1 (+ t2)|^2, in
-// FP64 (two bf16 terms add exactly in FP32; three round once at 2^-24): the
-// sum of the squares of all 16 summed components, whichever column each
-// 16-bit half of a word belongs to
+// sum over 4 columns of |t0 + t1 (+ t2)|^2, in FP64 (two bf16 terms add
+// exactly in FP32; three round once at 2^-24): the sum of the squares of all
+// 8 summed components, whichever column each 16-bit half of a word belongs to
 template <int NT, bool F16>
-__device__ __forceinline__ double row_norm2(const u32x4 (*r)[2]) {
+__device__ __forceinline__ double row_norm2(const u32x4 *r) {
   double s = 0.0;
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
+  for (int q = 0; q < 4; ++q) {
     float re = 0.0f, im = 0.0f;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const uint32_t w = r[t][q >> 2][q & 3];
+      const uint32_t w = r[t][q];
       re += lo_half<F16>(w);
       im += hi_half<F16>(w);
     }
@@ -585,15 +582,14 @@ __device__ __forceinline__ double row_norm2(const u32x4 (*r)[2]) {
 }
 
 // One HERK instance of a split form as the kernels read it.  `part` holds
-// `nslices` x ntiles partial tiles of TILE x TILE complex<float>, `dpart`
-// the FP64 row norms of the diagonal tiles (nslices x ntiles x TILE).
+// `nslices` x ntiles partial panel pairs of 64 x 64 complex<float>, `dpart`
+// the FP64 row norms of the panels (nslices x nb x 64).
 //
 // Split terms are stored K-tile-major: K tile q (columns 16 q .. 16 q + 15
 // of the concatenated segments, seg_stride a multiple of 16) is `ldz` rows
 // of 16 words, row r at word (q ldz + r) 16.  The rows one copy
 // instruction reads (16 consecutive rows of one K tile) are 1 KB of
-// contiguous memory and a workgroup's panel of a K tile is one run of
-// 128 x 64 bytes, where a row-major layout puts every row's 64 bytes on its
+// contiguous memory and a panel of a K tile is one run of 64 x 64 bytes, where a row-major layout puts every row's 64 bytes on its
 // own page.
 struct SplitProblem {
   const uint32_t *t[3];
@@ -604,17 +600,14 @@ struct SplitProblem {
   cplx<double> *vacc;
   int64_t ldv;
   double scale;
-  int m, nseg, nb, ntiles, accumulate;  // ntiles: partial tiles a slice
-  int ngroups;  // work items a slice (tiles, or groups of panel pairs)
+  // nb panels, ntiles = nb (nb + 1) / 2 partial pairs a slice
+  int m, nseg, nb, ntiles, accumulate;
+  int ngroups;  // work items a slice (panel groups, or pairs)
 };
 
-// Block shape of the split kernels for a tile side: 128 -> 256 threads as
-// 2x2 waves of 64x64; 64 -> one wave of 64x64.  Each thread stages PAIRS
-// (row, half-row) pieces of 8 words of each operand panel per K tile.
-template <int TILE> struct SplitShape {
-  static constexpr int kThreads = TILE == 128 ? 256 : 64;
-  static constexpr int kPairs = TILE * 2 / kThreads;
-};
+// Workgroups of the split kernels: four waves on a panel group (a launch's
+// large problems), or one wave on one panel pair (small ones, tile 64).
+constexpr int kSP = 64;  // rows of a panel
 
 // LDS position of word w (a multiple of 4) of row r in a K-tile panel of
 // 16 words a row: the row's 16-byte chunk c is stored at chunk c ^ swz(r),
@@ -625,12 +618,11 @@ __device__ __forceinline__ int lds_word(int r, int w) {
   return r * kSK + (((w >> 2) ^ swz(r)) << 2);
 }
 
-// One K-tile stage: the A rows (xa) and B rows (xb) of every term.  The two
-// stages of a kernel are separate __shared__ objects, so that the compiler
-// sees that loads in flight into one do not alias reads from the other.
-template <int NT, int TILE> struct alignas(16) SplitStage {
-  uint32_t xa[NT][TILE * kSK];
-  uint32_t xb[NT][TILE * kSK];
+// One K-tile stage: every term of the group's panels.  The two stages of a
+// kernel are separate __shared__ objects, so that the compiler sees that
+// loads in flight into one do not alias reads from the other.
+template <int NT, int WAVES> struct alignas(16) SplitStage {
+  uint32_t x[WAVES == 4 ? 4 : 2][NT][kSP * kSK];
 };
 
 // [x lanes 0-31 | y lanes 0-31] and [x lanes 32-63 | y lanes 32-63] of each
@@ -650,7 +642,7 @@ __device__ __forceinline__ u32x4 halves_hi(u32x4 x, u32x4 y) {
   return r;
 }
 
-// Waves compute 64x64 sub-tiles as 2x2 blocks of 32x32x16 MFMA, whose
+// A wave computes its 64x64 panel pair as 2x2 blocks of 32x32x16 MFMA, whose
 // K = 16 reals are 8 from lanes 0-31 and 8 from lanes 32-63.
 //
 // Term products are grouped so that small ones share an instruction with a
@@ -666,126 +658,170 @@ __device__ __forceinline__ u32x4 halves_hi(u32x4 x, u32x4 y) {
 // The imaginary-part operand Y = (im, -re) of a B fragment is formed in
 // registers.
 //
-// K tiles go through two LDS stages.  Each wave copies its share of the next
-// tile's rows straight from global memory into the other stage
+// K tiles go through two LDS stages.  Each wave copies its panel of the next
+// tile straight from global memory into the other stage
 // (global_load_lds_dwordx4: 16 bytes a lane, lane l to byte 16 l of a 1 KB
 // run of 16 rows), then computes the current tile; one barrier per K tile
 // publishes the copy and frees the stage just read.  Rows past m are read as
 // row m - 1: they only reach output rows and columns past m, which nothing
-// reads.  For a diagonal tile the threads also sum |t0 + t1 (+ t2)|^2 of the
-// staged rows in FP64 (the exact diagonal).
-template <int NT, int MAXORD, bool F16, int TILE>
+// reads.  All threads of a group that has panels' row norms to sum add
+// |t0 + t1 (+ t2)|^2 of those panels' staged rows in FP64 (the exact
+// diagonal), a quarter of a row each.
+//
+// Measured at m = 700, 2 x 59.7k columns, 2 terms, 3 products: on panel
+// groups instead of square 128-row tiles (17 items a slice, not 21; 68 panel
+// copies, not 72) and with the row norms spread over the groups, 20
+// frequencies of the 350-antenna sky take 16.2 ms (17.6), 16 of 128
+// antennas, unpolarized, 1.08 ms (1.21); three terms on a chunked sky 6.6 ms
+// (7.3).  Norms left with their diagonal pairs: 16.4, 1.09, 7.25 ms.  Taking
+// parts out of that 680 us launch: copies and barriers alone 283 us, no
+// copies 478, neither copies nor norms 465, no norms 635; it ran 1.30M cycles
+// at 2.0 GHz, 56% of them MFMA-busy.
+template <int NT, int MAXORD, bool F16, int WAVES>
 __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
-                                           int tile, int ns, int ktiles,
-                                           int kps, int64_t seg_len,
-                                           SplitStage<NT, TILE> &L0,
-                                           SplitStage<NT, TILE> &L1) {
-  typedef SplitShape<TILE> S;
-  constexpr int kWaves = S::kThreads / 64;
-  constexpr int kRuns = TILE / 16 / kWaves;  // 16-row runs a wave copies
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wr = TILE == 128 ? wave >> 1 : 0, wc = TILE == 128 ? wave & 1 : 0;
+                                           int group, int ns, int ktiles,
+                                           int kps,
+                                           SplitStage<NT, WAVES> &L0,
+                                           SplitStage<NT, WAVES> &L1) {
+  typedef SplitStage<NT, WAVES> Stage;
+  constexpr int kRuns = kSP / 16;  // 16-row runs of a panel
+  // the wave's index in a scalar register: what it does is uniform over it
+  const int wave =
+      WAVES == 4 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
+  const int lane = threadIdx.x & 63;
   const int lr = lane & 31, lh = lane >> 5;
-  int bi, bj;
-  tile_coords(tile, P.nb, bi, bj);
-  const bool diag = bi == bj;
-  const bool active = !subtile_idle(bi, bj, wr, wc, TILE, P.m);
+  WavePair wp;
+  int second = -1;  // one wave stages its pair's other panel too
+  if constexpr (WAVES == 4) {
+    wp = group_wave(group, P.nb, wave);
+  } else {
+    tile_coords(group, P.nb, wp.i, wp.j);
+    wp.load = wp.i;
+    wp.si = 0;
+    wp.sj = wp.i == wp.j ? 0 : 1;
+    wp.norm = wp.i == wp.j ? 0 : -1;
+    if (wp.i != wp.j) second = wp.j;
+  }
   const int kt0 = (int)((int64_t)slice * ktiles / ns);
   const int kt1 = (int)((int64_t)(slice + 1) * ktiles / ns);
-  // copy lanes: run g = wave * kRuns + u covers rows 16 g .. 16 g + 15;
-  // lane l fills LDS chunk l % 4 of row 16 g + l / 4, i.e. logical chunk
+  // copy lanes: run u covers rows 16 u .. 16 u + 15 of the panel; lane l
+  // fills LDS chunk l % 4 of row 16 u + l / 4, i.e. logical chunk
   // (l % 4) ^ swz(row) of that row
-  int64_t coff_a[kRuns], coff_b[kRuns];
+  uint32_t coff[WAVES == 4 ? 1 : 2][kRuns];
 #pragma unroll
-  for (int u = 0; u < kRuns; ++u) {
-    const int r = (wave * kRuns + u) * 16 + (lane >> 2);
-    const int c = (lane & 3) ^ swz(r);
-    const int ra = bi * TILE + r, rb = bj * TILE + r;
-    const int ga = ra < P.m ? ra : P.m - 1, gb = rb < P.m ? rb : P.m - 1;
-    coff_a[u] = (int64_t)ga * kSK + 4 * c;
-    coff_b[u] = (int64_t)gb * kSK + 4 * c;
-  }
-  // diagonal sums: piece pi covers half lw of row lrow (8 words)
-  int lrow[S::kPairs], lw[S::kPairs];
-  double dsum[S::kPairs];
+  for (int q = 0; q < (WAVES == 4 ? 1 : 2); ++q)
 #pragma unroll
-  for (int p = 0; p < S::kPairs; ++p) {
-    const int pi = tid + p * S::kThreads, l = pi & 63;
-    lrow[p] = (pi >> 6) * 32 + 16 * (l >> 5) + (l & 15);
-    lw[p] = ((l >> 4) & 1) * 8;
-    dsum[p] = 0.0;
-  }
-
-  v16f acc_re[2][2], acc_im[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      acc_re[i][j] = v16f{};
-      acc_im[i][j] = v16f{};
+    for (int u = 0; u < kRuns; ++u) {
+      const int r = u * 16 + (lane >> 2);
+      const int row = (q ? second : wp.load) * kSP + r;
+      const int c = (lane & 3) ^ swz(r);
+      coff[q][u] = (uint32_t)((row < P.m ? row : P.m - 1) * kSK + 4 * c);
     }
+  // the panels whose row norms this group sums (slots, -1: none)
+  int dslot[WAVES];
+  double dsum[WAVES];
+  bool any_diag = false;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    const WavePair q = WAVES == 4 ? group_wave(group, P.nb, w) : wp;
+    dslot[w] = q.norm;
+    any_diag = any_diag || dslot[w] >= 0;
+    dsum[w] = 0.0;
+  }
+  double dsum1[4] = {0.0, 0.0, 0.0, 0.0};  // the one wave's
+
+  // Three terms keep their two small products in accumulators of their own
+  // (set 1): only one product a column step rounds at the size of the sum.
+  // (One workgroup a CU fits by LDS, which leaves the registers for it.)
+  constexpr int kSets = NT == 3 ? 2 : 1;
+  v16f acc_re[kSets][2][2], acc_im[kSets][2][2];
+#pragma unroll
+  for (int q = 0; q < kSets; ++q)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        acc_re[q][i][j] = v16f{};
+        acc_im[q][i][j] = v16f{};
+      }
 
   // position of the K tile to copy next: segment sg, tile kc within it;
   // whole K tiles: columns [seg_len, round_up(seg_len, 16)) of every
   // segment are zero by contract
   int sg = kt0 / (kps > 0 ? kps : 1), kc = kt0 - sg * kps;
   const int64_t seg_tiles = P.seg_stride / kSK;
-  auto copy = [&](SplitStage<NT, TILE> &D) {
+  auto copy = [&](Stage &D) {
     const int64_t k0 = (sg * seg_tiles + kc) * P.ldz * kSK;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int u = 0; u < kRuns; ++u) {
-        const int run = (wave * kRuns + u) * 16 * kSK;
-        copy16_to_lds(P.t[t] + k0 + coff_a[u], &D.xa[t][run]);
-        if (!diag) copy16_to_lds(P.t[t] + k0 + coff_b[u], &D.xb[t][run]);
+        if (WAVES == 1 || wp.load >= 0)
+          copy16_to_lds(P.t[t] + k0 + coff[0][u],
+                        &D.x[wave][t][u * 16 * kSK]);
+        if (WAVES == 1 && second >= 0)
+          copy16_to_lds(P.t[t] + k0 + coff[WAVES == 1][u],
+                        &D.x[1][t][u * 16 * kSK]);
       }
     if (++kc == kps) {
       kc = 0;
       ++sg;
     }
   };
-  auto diag_sums = [&](const SplitStage<NT, TILE> &D) {
+  // thread t: quarter t % 4 (4 columns) of row t / 4, and with one wave the
+  // rows 16, 32, 48 further on
+  auto diag_sums = [&](const Stage &D) {
 #pragma unroll
-    for (int p = 0; p < S::kPairs; ++p) {
-      u32x4 r[NT][2];
+    for (int w = 0; w < WAVES; ++w) {
+      if (dslot[w] < 0) continue;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        r[t][0] = *(const u32x4 *)&D.xa[t][lds_word(lrow[p], lw[p])];
-        r[t][1] = *(const u32x4 *)&D.xa[t][lds_word(lrow[p], lw[p] + 4)];
+      for (int q = 0; q < 4 / WAVES; ++q) {
+        const int row = q * 16 + ((int)threadIdx.x >> 2);
+        u32x4 r[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          r[t] = *(const u32x4 *)&D.x[dslot[w]][t][lds_word(row, (lane & 3) * 4)];
+        if constexpr (WAVES == 4) dsum[w] += row_norm2<NT, F16>(r);
+        else dsum1[q] += row_norm2<NT, F16>(r);
       }
-      dsum[p] += row_norm2<NT, F16>(r);
     }
   };
   // the MFMAs of one K tile from stage D
-  auto compute = [&](const SplitStage<NT, TILE> &D) {
-    const uint32_t(*Ax)[TILE * kSK] = D.xa;
-    const uint32_t(*Bx)[TILE * kSK] = diag ? D.xa : D.xb;
+  auto compute = [&](const Stage &D) {
+    const uint32_t(*Ax)[kSP * kSK] = D.x[wp.si];
+    const uint32_t(*Bx)[kSP * kSK] = D.x[wp.sj];
     // lane half lh reads term t_lh at word offset w_lh of its row
     auto ld_a = [&](int t0, int t1, int w0, int w1, u32x4 (&a)[2]) {
       const uint32_t *base = Ax[lh ? t1 : t0];
       const int w = lh ? w1 : w0;
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        a[i] = *(const u32x4 *)&base[lds_word(wr * 64 + i * 32 + lr, w)];
+        a[i] = *(const u32x4 *)&base[lds_word(i * 32 + lr, w)];
     };
     auto ld_b = [&](int t0, int t1, int w0, int w1, u32x4 (&b)[2]) {
       const uint32_t *base = Bx[lh ? t1 : t0];
       const int w = lh ? w1 : w0;
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        b[j] = *(const u32x4 *)&base[lds_word(wc * 64 + j * 32 + lr, w)];
+        b[j] = *(const u32x4 *)&base[lds_word(j * 32 + lr, w)];
     };
-    auto mma = [&](const u32x4 (&a)[2], const u32x4 (&b)[2]) {
+    auto mma_into = [&](const u32x4 (&a)[2], const u32x4 (&b)[2],
+                        v16f (&re)[2][2], v16f (&im)[2][2]) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const u32x4 y = swap_negate4(b[j]);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-          acc_re[i][j] = SplitMfma<F16>::op(a[i], b[j], acc_re[i][j]);
-          acc_im[i][j] = SplitMfma<F16>::op(a[i], y, acc_im[i][j]);
+          re[i][j] = SplitMfma<F16>::op(a[i], b[j], re[i][j]);
+          im[i][j] = SplitMfma<F16>::op(a[i], y, im[i][j]);
         }
       }
+    };
+    auto mma = [&](const u32x4 (&a)[2], const u32x4 (&b)[2]) {
+      mma_into(a, b, acc_re[0], acc_im[0]);
+    };
+    auto mma_small = [&](const u32x4 (&a)[2], const u32x4 (&b)[2]) {
+      mma_into(a, b, acc_re[kSets - 1], acc_im[kSets - 1]);
     };
     u32x4 a[2], b[2];
     if constexpr (NT == 2 && MAXORD == 1) {
@@ -823,18 +859,20 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
         ld_b(0, 1, 4 * q, 4 * q, b);
         mma(a, b);
         ld_b(1, 0, 4 * q, 4 * q, b);
-        mma(a, b);
+        mma_small(a, b);
         ld_a(0, 2, 4 * q, 4 * q, a);
         ld_b(2, 0, 4 * q, 4 * q, b);
-        mma(a, b);
+        mma_small(a, b);
+        // operand reads stay in their step: hoisted they would spill
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
   // one K tile computed from stage C while the next is copied into N
-  auto step = [&](SplitStage<NT, TILE> &C, SplitStage<NT, TILE> &N, int kt) {
+  auto step = [&](Stage &C, Stage &N, int kt) {
     if (kt + 1 < kt1) copy(N);
-    if (diag) diag_sums(C);
-    if (active) {
+    if (any_diag) diag_sums(C);
+    if (WAVES == 1 || wp.i >= 0) {
       // issue priority to waves in their MFMA phase over waves copying or
       // waiting at the barrier
       __builtin_amdgcn_s_setprio(1);
@@ -853,23 +891,35 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
     if (kt + 1 < kt1) step(L1, L0, kt + 1);
   }
   // every wave is past the last barrier: LDS is free for the next item
-  if (diag) {
-    // two threads share each row: lanes l and l ^ 16 of one wave
+  if (any_diag) {
+    // the four threads of a row are lanes 4 q .. 4 q + 3
+    auto store = [&](int panel, int row, double s) {
+      s += __shfl_xor(s, 1, 64);
+      s += __shfl_xor(s, 2, 64);
+      if ((lane & 3) == 0)
+        P.dpart[((int64_t)slice * P.nb + panel) * kSP + row] = s;
+    };
+    if constexpr (WAVES == 4) {
 #pragma unroll
-    for (int p = 0; p < S::kPairs; ++p) {
-      const double s = dsum[p] + __shfl_xor(dsum[p], 16, 64);
-      if (lw[p] == 0)
-        P.dpart[((int64_t)slice * P.ntiles + tile) * TILE + lrow[p]] = s;
+      for (int w = 0; w < WAVES; ++w)
+        if (dslot[w] >= 0)
+          store(group_wave(group, P.nb, dslot[w]).load,
+                (int)threadIdx.x >> 2, dsum[w]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) store(wp.i, q * 16 + (lane >> 2), dsum1[q]);
     }
   }
 
-  if (!active) return;  // an idle sub-tile has no partials
+  if (WAVES == 4 && wp.i < 0) return;  // no pair, no partials
   // 32x32 accumulator layout: lane l, register r ->
   //   row 8*(r/4) + 4*(l/32) + r%4, col l%32.
   // The thread's base offset is opaque to the optimizer so that the store
   // addresses are formed here rather than kept live across the K loop.
-  cplx<float> *out = P.part + ((int64_t)slice * P.ntiles + tile) * TILE * TILE;
-  int obase = (wr * 64 + 4 * lh) * TILE + wc * 64 + lr;
+  cplx<float> *out =
+      P.part + ((int64_t)slice * P.ntiles + pair_index(wp.i, wp.j, P.nb)) *
+                   kSP * kSP;
+  int obase = 4 * lh * kSP + lr;
   asm volatile("" : "+v"(obase));
   out += obase;
 #pragma unroll
@@ -879,26 +929,29 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = i * 32 + 8 * (r >> 2) + (r & 3);
-        out[row * TILE + j * 32] =
-            cplx<float>{acc_re[i][j][r], acc_im[i][j][r]};
+        float re = acc_re[0][i][j][r], im = acc_im[0][i][j][r];
+        if constexpr (kSets == 2) {
+          re += acc_re[1][i][j][r];
+          im += acc_im[1][i][j][r];
+        }
+        out[row * kSP + j * 32] = cplx<float>{re, im};
       }
 }
 
 // One split HERK: K tiles and the slice count from the device column count,
-// items (tile, slice) swept per XCD.
-template <int NT, int MAXORD, bool F16, int TILE>
-__global__ __launch_bounds__(SplitShape<TILE>::kThreads,
-                             TILE == 128 ? 2 : 8) void herk_split_kernel(
+// items (group, slice) swept per XCD.
+template <int NT, int MAXORD, bool F16>
+__global__ __launch_bounds__(256, NT == 2 ? 2 : 1) void herk_split_kernel(
     SplitProblem P, SliceCfg cfg) {
-  __shared__ SplitStage<NT, TILE> L0, L1;
+  __shared__ SplitStage<NT, 4> L0, L1;
   const int64_t seg_len = seg_columns(P.seg_len_host, P.seg_len_dev);
   const int kps = (int)cdiv(seg_len, (int64_t)kSK);  // K tiles per segment
   const int ktiles = kps * P.nseg;
-  const int ns = active_slices_wave(ktiles, P.ntiles, cfg);
-  for_items((int64_t)P.ntiles * ns, [&](int64_t it) {
-    split_item<NT, MAXORD, F16, TILE>(P, (int)(it / P.ntiles),
-                                      (int)(it % P.ntiles), ns, ktiles, kps,
-                                      seg_len, L0, L1);
+  const int ns = active_slices_wave(ktiles, P.ngroups, cfg);
+  for_items((int64_t)P.ngroups * ns, [&](int64_t it) {
+    split_item<NT, MAXORD, F16, 4>(P, (int)(it / P.ngroups),
+                                   (int)(it % P.ngroups), ns, ktiles, kps, L0,
+                                   L1);
   });
 }
 
@@ -961,7 +1014,7 @@ __global__ __launch_bounds__(256) void herk_group_plan_kernel(
       P.part = (cplx<float> *)(parts + bytes);
       bytes += cap * P.ntiles * (int64_t)ts * ts * part_bytes;
       P.dpart = row_norms ? (double *)(parts + bytes) : nullptr;
-      if (row_norms) bytes += cap * P.ntiles * (int64_t)ts * 8;
+      if (row_norms) bytes += cap * P.nb * (int64_t)ts * 8;
       plan.item_off[p] = items;
       plan.tile_off[p] = tiles;
       items += (int64_t)P.ngroups * plan.ns[p];
@@ -986,11 +1039,11 @@ __device__ __forceinline__ int find_segment(const T *off, int n, T x) {
 
 // All problems' items in one persistent launch, problem-major then
 // slice-major, swept per XCD as in the single-problem kernel.
-template <int NT, int MAXORD, bool F16, int TILE>
-__global__ __launch_bounds__(SplitShape<TILE>::kThreads,
-                             TILE == 128 ? 2 : 8) void herk_split_grouped_kernel(
+template <int NT, int MAXORD, bool F16, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, NT == 2 ? 2 : 1) void
+herk_split_grouped_kernel(
     const SplitProblem *__restrict__ probs, int nprob, GroupPlan plan) {
-  __shared__ SplitStage<NT, TILE> L0, L1;
+  __shared__ SplitStage<NT, WAVES> L0, L1;
   const int64_t items = plan.item_off[nprob];
   for_items(items, [&](int64_t it) {
     const int p = find_segment(plan.item_off, nprob, it);
@@ -999,9 +1052,9 @@ __global__ __launch_bounds__(SplitShape<TILE>::kThreads,
     const int64_t local = it - plan.item_off[p];
     const int64_t seg_len = seg_columns(P.seg_len_host, P.seg_len_dev);
     const int kps = (int)cdiv(seg_len, (int64_t)kSK);
-    split_item<NT, MAXORD, F16, TILE>(P, (int)(local / P.ntiles),
-                                      (int)(local % P.ntiles), ns,
-                                      kps * P.nseg, kps, seg_len, L0, L1);
+    split_item<NT, MAXORD, F16, WAVES>(P, (int)(local / P.ngroups),
+                                       (int)(local % P.ngroups), ns,
+                                       kps * P.nseg, kps, L0, L1);
   });
 }
 
@@ -1062,24 +1115,21 @@ __device__ __forceinline__ int64_t reduce_group(int &half) {
 template <typename TP, bool DTILE>
 __device__ __forceinline__ void reduce_elems_t(
     const cplx<TP> *__restrict__ part, const double *__restrict__ dpart,
-    int ntiles, int bi, int bj, int ts, int m, int tile, int64_t e, int h,
+    int ntiles, int nb, int bi, int bj, int ts, int tile, int64_t e, int h,
     int ns, double scale, cplx<double> *__restrict__ vacc, int64_t ldv,
     int accumulate) {
   constexpr int E = kReduceEpt<TP>;
   static_assert(E == 2, "lane half h stores element h of its group");
   const int64_t tsz = (int64_t)ts * ts;
   const int64_t r = e / ts, c = e % ts;
-  // the group's E adjacent columns share a sub-tile (E divides 64); both
-  // lane halves of a group leave together
-  if (subtile_idle(bi, bj, (int)(r >> 6), (int)(c >> 6), ts, m)) return;
   const cplx<TP> *src = part + (int64_t)tile * tsz + e;
   const int64_t step = (int64_t)ntiles * tsz;
   // diagonal tiles (DTILE) also sum the row norms of the group's row, in the
   // same loop (every lane of the tile, so no lane runs extra rounds of
   // dependent loads after it)
   constexpr bool dtile = DTILE;
-  const double *dp = dtile ? dpart + (int64_t)tile * ts + r : nullptr;
-  const int64_t dstep = (int64_t)ntiles * ts;
+  const double *dp = dtile ? dpart + (int64_t)bi * ts + r : nullptr;
+  const int64_t dstep = (int64_t)nb * ts;
   double re[E][4], im[E][4], dn[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -1154,16 +1204,16 @@ __device__ __forceinline__ void reduce_elems_t(
 template <typename TP>
 __device__ __forceinline__ void reduce_elems(
     const cplx<TP> *__restrict__ part, const double *__restrict__ dpart,
-    int ntiles, int nb, int ts, int m, int tile, int64_t e, int h, int ns,
+    int ntiles, int nb, int ts, int tile, int64_t e, int h, int ns,
     double scale, cplx<double> *__restrict__ vacc, int64_t ldv,
     int accumulate) {
   int bi, bj;
   tile_coords(tile, nb, bi, bj);
   if (dpart && bi == bj)  // uniform over the block: one tile a block
-    reduce_elems_t<TP, true>(part, dpart, ntiles, bi, bj, ts, m, tile, e, h,
+    reduce_elems_t<TP, true>(part, dpart, ntiles, nb, bi, bj, ts, tile, e, h,
                              ns, scale, vacc, ldv, accumulate);
   else
-    reduce_elems_t<TP, false>(part, dpart, ntiles, bi, bj, ts, m, tile, e, h,
+    reduce_elems_t<TP, false>(part, dpart, ntiles, nb, bi, bj, ts, tile, e, h,
                               ns, scale, vacc, ldv, accumulate);
 }
 
@@ -1179,7 +1229,7 @@ template <typename TP> dim3 reduce_grid(int ts, int64_t ntiles) {
 template <typename TP>
 __global__ __launch_bounds__(256) void herk_reduce_kernel(
     const cplx<TP> *__restrict__ part, const double *__restrict__ dpart,
-    int ntiles, int ngroups, int nb, int ts, int m, int64_t seg_len_host,
+    int ntiles, int ngroups, int nb, int ts, int64_t seg_len_host,
     const int32_t *__restrict__ seg_len_dev, int nseg, int kc, SliceCfg cfg,
     double scale, cplx<double> *__restrict__ vacc, int64_t ldv,
     int accumulate) {
@@ -1195,7 +1245,7 @@ __global__ __launch_bounds__(256) void herk_reduce_kernel(
   const int64_t e = reduce_group<TP>(h);
   if (e >= (int64_t)ts * ts) return;
   for (int tile = blockIdx.y; tile < ntiles; tile += gridDim.y)
-    reduce_elems(part, dpart, ntiles, nb, ts, m, tile, e, h, ns_shared, scale,
+    reduce_elems(part, dpart, ntiles, nb, ts, tile, e, h, ns_shared, scale,
                  vacc, ldv, accumulate);
 }
 
@@ -1214,7 +1264,7 @@ __global__ __launch_bounds__(256) void herk_group_reduce_kernel(
   for (int32_t t = blockIdx.y; t < total; t += gridDim.y) {
     const int p = find_segment(plan.tile_off, nprob, t);
     const SplitProblem &P = probs[p];
-    reduce_elems((const cplx<TP> *)P.part, P.dpart, P.ntiles, P.nb, ts, P.m,
+    reduce_elems((const cplx<TP> *)P.part, P.dpart, P.ntiles, P.nb, ts,
                  (int)(t - plan.tile_off[p]), e, h, plan.ns[p], P.scale,
                  P.vacc, P.ldv, P.accumulate);
   }
@@ -1380,35 +1430,36 @@ const void *herk_kernel(int form, int nterms, int maxord, int panel) {
   }
   const bool f16 = form == MV_FORM_SPLIT_F16;
   if (nterms == 2 && maxord == 1)
-    return f16 ? (const void *)&herk_split_kernel<2, 1, true, kST>
-               : (const void *)&herk_split_kernel<2, 1, false, kST>;
+    return f16 ? (const void *)&herk_split_kernel<2, 1, true>
+               : (const void *)&herk_split_kernel<2, 1, false>;
   if (nterms == 2)
-    return f16 ? (const void *)&herk_split_kernel<2, 2, true, kST>
-               : (const void *)&herk_split_kernel<2, 2, false, kST>;
-  return f16 ? (const void *)&herk_split_kernel<3, 2, true, kST>
-             : (const void *)&herk_split_kernel<3, 2, false, kST>;
+    return f16 ? (const void *)&herk_split_kernel<2, 2, true>
+               : (const void *)&herk_split_kernel<2, 2, false>;
+  return f16 ? (const void *)&herk_split_kernel<3, 2, true>
+             : (const void *)&herk_split_kernel<3, 2, false>;
 }
 
-// The grouped kernel instantiation for (form, nterms, maxord, tile).
-template <int TILE>
+// The grouped kernel instantiation for (form, nterms, maxord), `WAVES`
+// waves a workgroup.
+template <int WAVES>
 const void *grouped_kernel_t(bool f16, int nterms, int maxord) {
   if (nterms == 2 && maxord == 1)
-    return f16 ? (const void *)&herk_split_grouped_kernel<2, 1, true, TILE>
-               : (const void *)&herk_split_grouped_kernel<2, 1, false, TILE>;
+    return f16 ? (const void *)&herk_split_grouped_kernel<2, 1, true, WAVES>
+               : (const void *)&herk_split_grouped_kernel<2, 1, false, WAVES>;
   if (nterms == 2)
-    return f16 ? (const void *)&herk_split_grouped_kernel<2, 2, true, TILE>
-               : (const void *)&herk_split_grouped_kernel<2, 2, false, TILE>;
-  return f16 ? (const void *)&herk_split_grouped_kernel<3, 2, true, TILE>
-             : (const void *)&herk_split_grouped_kernel<3, 2, false, TILE>;
+    return f16 ? (const void *)&herk_split_grouped_kernel<2, 2, true, WAVES>
+               : (const void *)&herk_split_grouped_kernel<2, 2, false, WAVES>;
+  return f16 ? (const void *)&herk_split_grouped_kernel<3, 2, true, WAVES>
+             : (const void *)&herk_split_grouped_kernel<3, 2, false, WAVES>;
 }
 
 int plan_herk(int form, int nterms, int maxord, int m, int nslices,
               HerkPlan &p) {
   const bool plain = form == MV_FORM_C128 || form == MV_FORM_C64;
-  p.ts = plain ? panel_side(form, m) : kST;
+  p.ts = plain ? panel_side(form, m) : kSP;
   p.nb = (int)cdiv((int64_t)m, (int64_t)p.ts);
   p.ntiles = p.nb * (p.nb + 1) / 2;
-  p.ngroups = plain ? panel_groups(p.nb) : p.ntiles;
+  p.ngroups = panel_groups(p.nb);
   p.kc = plain ? kPK : kSK;
   const int slots = kernel_slots(herk_kernel(form, nterms, maxord, p.ts));
   if (slots <= 0) return -1;
@@ -1472,7 +1523,7 @@ int plain_run(const HerkPlan &p, const PlainLaunch &L) {
   if (!(L.phases & kPhaseReduce)) return MV_OK;
   herk_reduce_kernel<T><<<reduce_grid<T>(p.ts, p.ntiles), 256, 0, L.st>>>(
       (const cplx<T> *)L.workspace, nullptr, p.ntiles, p.ngroups, p.nb, p.ts,
-      L.m, L.seg_len, L.seg_len_dev, L.nseg, p.kc, p.cfg, L.scale,
+      L.seg_len, L.seg_len_dev, L.nseg, p.kc, p.cfg, L.scale,
       (cplx<double> *)L.vacc, L.ldv, L.accumulate);
   return check_launch("mv_herk/reduce");
 }
@@ -1561,7 +1612,7 @@ int herk_run(int phases, int form, int nterms, int nprod, const void *z0,
   P.ngroups = p.ngroups;
   P.accumulate = accumulate;
 #define MV_SPLIT_LAUNCH(NT, MO, F)                                           \
-  herk_split_kernel<NT, MO, F, kST><<<p.grid, 256, 0, st>>>(P, p.cfg)
+  herk_split_kernel<NT, MO, F><<<p.grid, 256, 0, st>>>(P, p.cfg)
   if (phases & kPhaseCompute) {
     if (nterms == 2 && maxord == 1) {
       if (f16) MV_SPLIT_LAUNCH(2, 1, true);
@@ -1577,8 +1628,8 @@ int herk_run(int phases, int form, int nterms, int nprod, const void *z0,
   }
 #undef MV_SPLIT_LAUNCH
   if (!(phases & kPhaseReduce)) return MV_OK;
-  herk_reduce_kernel<float><<<reduce_grid<float>(ts, ntiles), 256, 0, st>>>(
-      (const cplx<float> *)workspace, dpart, p.ntiles, p.ngroups, p.nb, ts, m,
+  herk_reduce_kernel<float><<<reduce_grid<float>(p.ts, p.ntiles), 256, 0, st>>>(
+      (const cplx<float> *)workspace, dpart, p.ntiles, p.ngroups, p.nb, p.ts,
       seg_len, seg_len_dev, nseg, p.kc, p.cfg, scale, (cplx<double> *)vacc,
       ldv, accumulate);
   return check_launch("mv_herk/reduce");
@@ -1720,8 +1771,8 @@ GroupLayout group_layout(int form, int ts, const mv_herk_problem *q,
 }
 
 const void *grouped_kernel(int tile, bool f16, int nterms, int maxord) {
-  return tile == 64 ? grouped_kernel_t<64>(f16, nterms, maxord)
-                    : grouped_kernel_t<kST>(f16, nterms, maxord);
+  return tile == 64 ? grouped_kernel_t<1>(f16, nterms, maxord)
+                    : grouped_kernel_t<4>(f16, nterms, maxord);
 }
 }  // namespace
 
@@ -1804,16 +1855,14 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
              "mv_herk_grouped: workspace too small (%zu < %lld)", ws_bytes,
              (long long)g.total);
   const bool f16 = form == MV_FORM_SPLIT_F16;
-  const int side = split ? tile : panel_side(form, max_m);
+  const int side = split ? kSP : panel_side(form, max_m);
   const void *kernel =
       split ? grouped_kernel(tile, f16, nterms, maxord)
       : form == MV_FORM_C128
           ? (const void *)&herk_plain_grouped_kernel<double, 32>
       : side == 64 ? (const void *)&herk_plain_grouped_kernel<float, 64>
                    : (const void *)&herk_plain_grouped_kernel<float, 32>;
-  const int threads = !split ? 256
-                      : tile == 64 ? SplitShape<64>::kThreads
-                                   : SplitShape<kST>::kThreads;
+  const int threads = split && tile == 64 ? 64 : 256;
   const int slots = kernel_slots(kernel, threads);
   if (slots <= 0) {
     set_error(MV_ERR_HIP, "mv_herk_grouped: occupancy query failed");
@@ -1827,18 +1876,19 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
   // slices of a problem: split forms bound the FP32 chain (form_cmax);
   // plain forms take slices of 64 K tiles (1024 columns) for parallelism
   herk_group_plan_kernel<<<1, 256, 0, st>>>(
-      problems_dev, nprob, side, split ? 0 : 1, split ? kSK : kPK,
+      problems_dev, nprob, side, split && tile == 64 ? 0 : 1,
+      split ? kSK : kPK,
       split ? form_cmax(form) : 64, part_bytes(form), split ? 1 : 0, probs,
       ws + g.parts, plan);
   if (int e = check_launch("mv_herk_grouped/plan")) return e;
   const int grid = (int)(max_items < slots ? max_items : slots);
+  // the reduce runs over panel pairs, of which there are more than tiles
+  int64_t pairs = 0;
+  for (int i = 0; i < nprob; ++i) {
+    const int64_t n = cdiv((int64_t)problems_host[i].m, (int64_t)side);
+    pairs += n * (n + 1) / 2;
+  }
   if (!split) {
-    // the reduce runs over panel pairs, of which there are more than tiles
-    int64_t pairs = 0;
-    for (int i = 0; i < nprob; ++i) {
-      const int64_t n = cdiv((int64_t)problems_host[i].m, (int64_t)side);
-      pairs += n * (n + 1) / 2;
-    }
     if (form == MV_FORM_C128)
       herk_plain_grouped_kernel<double, 32><<<grid, 256, 0, st>>>(probs, nprob,
                                                                   plan);
@@ -1861,7 +1911,7 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
   }
 #define MV_GROUP_LAUNCH(NT, MO, F, T)                                        \
   herk_split_grouped_kernel<NT, MO, F, T>                                    \
-      <<<grid, SplitShape<T>::kThreads, 0, st>>>(probs, nprob, plan)
+      <<<grid, threads, 0, st>>>(probs, nprob, plan)
 #define MV_GROUP_TILE(T)                                                     \
   if (nterms == 2 && maxord == 1) {                                          \
     if (f16) MV_GROUP_LAUNCH(2, 1, true, T);                                 \
@@ -1874,16 +1924,16 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
     else MV_GROUP_LAUNCH(3, 2, false, T);                                    \
   }
   if (tile == 64) {
-    MV_GROUP_TILE(64)
+    MV_GROUP_TILE(1)
   } else {
-    MV_GROUP_TILE(kST)
+    MV_GROUP_TILE(4)
   }
 #undef MV_GROUP_TILE
 #undef MV_GROUP_LAUNCH
   if (int e = check_launch("mv_herk_grouped/split")) return e;
   herk_group_reduce_kernel<float>
-      <<<reduce_grid<float>(tile, total_tiles), 256, 0, st>>>(probs, nprob,
-                                                             tile, plan);
+      <<<reduce_grid<float>(side, pairs), 256, 0, st>>>(probs, nprob, side,
+                                                        plan);
   return check_launch("mv_herk_grouped/reduce");
 }
 

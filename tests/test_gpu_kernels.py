@@ -509,6 +509,30 @@ def test_herk_split_accuracy(form, nterms, nprod, bound, m, k):
     assert err < bound
 
 
+@pytest.mark.parametrize("nterms,nprod,bound", [(2, 3, 6e-6), (3, 6, 1e-6)])
+@pytest.mark.parametrize("m", [1, 64, 65, 128, 129, 193, 257, 321, 385, 513,
+                               577, 641])
+def test_herk_split_panel_edges(m, nterms, nprod, bound):
+    """Every panel grouping from 1 to 11 panels and the row norms of each
+    panel (summed in FP64, so the diagonal has the terms' own error only: the
+    form's bound for two, one FP32 rounding of each square's factors, 2 x
+    2^-24, for three)."""
+    rng = np.random.default_rng(m)
+    k = 150
+    z = ((0.5 + rng.uniform(size=(m, k)))
+         * np.exp(2j * np.pi * rng.uniform(size=(m, k)))).astype(np.complex64)
+    ts, ncols = _split_terms(z, FORM_SPLIT_BF16, nterms)
+    h, v = _run_herk(FORM_SPLIT_BF16, ts, m, m, 1, ncols, k, nterms, nprod,
+                     nslices=4)
+    got = _vis_full(h, v, m)
+    want = z.astype(np.complex128).conj() @ z.astype(np.complex128).T
+    d = np.sqrt(np.diag(want).real)
+    err = (np.abs(got - want) / (d[:, None] * d[None])).max()
+    assert err < bound, err
+    diag = np.abs(np.diag(got) / np.diag(want) - 1).max()
+    assert diag < (6e-6 if nterms == 2 else 1.2e-7), diag
+
+
 @pytest.mark.parametrize("nfeed", [1, 2])
 @pytest.mark.parametrize("antpairs", [True, False])
 @pytest.mark.parametrize("precision", [1, 2])
