@@ -247,6 +247,23 @@ int mv_zmat_fused(const double *antpos, int nant, double freq,
                   double scale, void *z0, void *z1, void *z2, int64_t ldz,
                   int64_t seg_stride, mv_stream_t stream);
 
+/* mv_zmat_fused for nfreq frequencies of one time in one launch: freqs and
+ * scales (NULL: all 1) are device arrays of nfreq doubles; frequency f reads
+ * flux + f*ld_flux and beam + f*beam_stride (elements; 0: shared) and writes
+ * z0..z2 + f*z_stride (complex elements, or 32-bit words of a split term).
+ * Small instances share one launch instead of each leaving the GPU idle.
+ * No reference counterpart: it runs one frequency at a time. */
+int mv_zmat_fused_batch(const double *antpos, int nant, const double *freqs,
+                        int nfreq, const double *crd, int64_t ld_crd,
+                        const double *flux, int64_t ld_flux,
+                        const int32_t *idx, const void *beam, int beam_is_f64,
+                        int64_t ld_beam, int64_t beam_stride, int nbeam,
+                        const int32_t *beam_idx, int nfeed, int nax,
+                        int64_t count, const int32_t *n_dev, int form,
+                        int nterms, const double *scales, void *z0, void *z1,
+                        void *z2, int64_t ldz, int64_t seg_stride,
+                        int64_t z_stride, mv_stream_t stream);
+
 /* Split a complex matrix (c128 or c64, layout as mv_zmat_fused output) into
  * nterms 16-bit terms of `form` (SPLIT_BF16 / SPLIT_F16), after multiplying
  * by `scale`, in the K-tile-major term layout of mv_zmat_fused (ldt rows a
@@ -317,6 +334,23 @@ int mv_herk(int form, int nterms, int nprod, const void *z0, const void *z1,
             int64_t seg_len, const int32_t *seg_len_dev, int nslices,
             double scale, double *vacc, int64_t ldv, int accumulate,
             void *workspace, size_t ws_bytes, mv_stream_t stream);
+
+/* nbatch HERKs of one shape in one launch and one reduce: instance b has Z
+ * z0..z2 + b*z_stride (complex elements, or 32-bit words of a split term;
+ * split: a multiple of 4), the accumulator vacc + b*vacc_stride (complex
+ * elements, >= ldv*ldv), the scale scales[b] (device; NULL: 1) and its share
+ * of the workspace, which holds nbatch times mv_herk_workspace_bytes.  All
+ * read the same column count.  phases: 1 the MFMA kernel, 2 the reduce, 3
+ * both.  The slice count is mv_herk's for one instance, and each result has
+ * the same bits.  No reference counterpart (one cuBLAS call per frequency
+ * there). */
+int mv_herk_batch(int phases, int form, int nterms, int nprod, const void *z0,
+                  const void *z1, const void *z2, int64_t z_stride, int nbatch,
+                  int m, int64_t ldz, int nseg, int64_t seg_stride,
+                  int64_t seg_len, const int32_t *seg_len_dev, int nslices,
+                  const double *scales, double *vacc, int64_t ldv,
+                  int64_t vacc_stride, int accumulate, void *workspace,
+                  size_t ws_bytes, mv_stream_t stream);
 
 /* mv_herk with no workspace argument and no allocation: the split-K
  * partials go to a 128 MiB device array that the library holds from load
@@ -416,6 +450,15 @@ int mv_vacc_sum(const double *src, int nsrc_v, int64_t stride, double *dst,
 int mv_vis_expand(const double *vacc, int64_t ldv, int tile, int nant,
                   int nfeed, const int32_t *pairs, int64_t npairs, void *out,
                   int out_is_f64, mv_stream_t stream);
+
+/* mv_vis_expand of nbatch accumulators in one launch: instance b reads vacc +
+ * b*vacc_stride (complex elements) and writes out + b*out_stride (complex
+ * elements). */
+int mv_vis_expand_batch(const double *vacc, int64_t ldv, int64_t vacc_stride,
+                        int nbatch, int tile, int nant, int nfeed,
+                        const int32_t *pairs, int64_t npairs, void *out,
+                        int out_is_f64, int64_t out_stride,
+                        mv_stream_t stream);
 
 #ifdef __cplusplus
 }

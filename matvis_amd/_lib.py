@@ -56,6 +56,9 @@ SIGNATURES: dict[str, list] = {
     "mv_zmat_parts": [_P, _P, _P, _I, _P, _I, _I, _I, _L, _P, _I, _P],
     "mv_zmat_fused": [_P, _I, _D, _P, _L, _P, _P, _P, _I, _L, _I, _P, _I,
                       _I, _L, _P, _I, _I, _D, _P, _P, _P, _L, _L, _P],
+    "mv_zmat_fused_batch": [_P, _I, _P, _I, _P, _L, _P, _L, _P, _P, _I, _L,
+                            _L, _I, _P, _I, _I, _L, _P, _I, _I, _P, _P, _P,
+                            _P, _L, _L, _L, _P],
     "mv_split_z": [_P, _I, _L, _I, _L, _L, _L, _I, _I, _D, _P, _P, _P, _L,
                    _L, _P],
     "mv_herk_tile": [_I],
@@ -64,6 +67,8 @@ SIGNATURES: dict[str, list] = {
     "mv_herk_slices": [_I, _I, _I, _I, _I, _L, _I],
     "mv_herk": [_I, _I, _I, _P, _P, _P, _I, _L, _I, _L, _L, _P, _I, _D, _P,
                 _L, _I, _P, _S, _P],
+    "mv_herk_batch": [_I, _I, _I, _I, _P, _P, _P, _L, _I, _I, _L, _I, _L, _L,
+                      _P, _I, _P, _P, _L, _L, _I, _P, _S, _P],
     "mv_herk_noalloc": [_I, _I, _I, _P, _P, _P, _I, _L, _I, _L, _L, _P, _D,
                         _P, _L, _I, _P],
     "mv_herk_compute": [_I, _I, _I, _P, _P, _P, _I, _L, _I, _L, _L, _P, _I,
@@ -75,6 +80,8 @@ SIGNATURES: dict[str, list] = {
     "mv_herk_grouped": [_I, _I, _I, _I, _P, _P, _I, _P, _S, _P],
     "mv_vacc_sum": [_P, _I, _L, _P, _L, _P],
     "mv_vis_expand": [_P, _L, _I, _I, _I, _P, _L, _P, _I, _P],
+    "mv_vis_expand_batch": [_P, _L, _L, _I, _I, _I, _I, _P, _L, _P, _I, _L,
+                            _P],
 }
 
 _RESTYPES = {

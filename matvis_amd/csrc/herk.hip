@@ -47,6 +47,17 @@ __device__ __forceinline__ void tile_coords(int t, int nb, int &bi, int &bj) {
   bj = i + t;
 }
 
+// HERKs of one shape in one launch (the frequencies of a time): instance b's
+// Z starts b z_stride elements (complex, or 32-bit words of a split term)
+// after the first, its partials b ws_stride bytes, its accumulator
+// b vacc_stride complex elements.  The slice count is that of one instance, so
+// that each result has the same bits alone and in any batch.
+struct HerkBatch {
+  int n;
+  int64_t z_stride, ws_stride, vacc_stride;
+  const double *scales;  // device, one an instance, or null: the one scale
+};
+
 struct SliceCfg {
   int max_slices;  // partial slots per tile in the workspace
   int slots;       // workgroups resident at once (multiple of kXcd)
@@ -505,16 +516,21 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
 
 template <typename T, int P>
 __global__ __launch_bounds__(256, 2) void herk_plain_kernel(
-    PlainProblem<T> Q, int nseg, int64_t seg_len_host,
-    const int32_t *__restrict__ seg_len_dev, SliceCfg cfg) {
+    const PlainProblem<T> Q0, int nseg, int64_t seg_len_host,
+    const int32_t *__restrict__ seg_len_dev, SliceCfg cfg, HerkBatch hb) {
   __shared__ PlainStage<T, P> L0, L1;
   const int64_t seg_len = seg_columns(seg_len_host, seg_len_dev);
   const int kps = (int)cdiv(seg_len, (int64_t)kPK);  // K tiles per segment
   const int ktiles = kps * nseg;
-  const int ns = active_slices_wave(ktiles, Q.ngroups, cfg);
-  for_items((int64_t)Q.ngroups * ns, [&](int64_t it) {
-    plain_item<T, P>(Q, seg_len, (int)(it / Q.ngroups), (int)(it % Q.ngroups), ns,
-                     ktiles, kps, L0, L1);
+  const int ns = active_slices_wave(ktiles, Q0.ngroups, cfg);
+  const int64_t per = (int64_t)Q0.ngroups * ns;
+  for_items(per * hb.n, [&](int64_t it) {
+    const int64_t b = it / per, i = it - b * per;
+    PlainProblem<T> Q = Q0;
+    Q.z += b * hb.z_stride;
+    Q.part = (cplx<T> *)((char *)Q.part + b * hb.ws_stride);
+    plain_item<T, P>(Q, seg_len, (int)(i / Q.ngroups), (int)(i % Q.ngroups),
+                     ns, ktiles, kps, L0, L1);
   });
 }
 
@@ -939,18 +955,25 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
 }
 
 // One split HERK: K tiles and the slice count from the device column count,
-// items (group, slice) swept per XCD.
+// items (instance, slice, group) swept per XCD.
 template <int NT, int MAXORD, bool F16>
 __global__ __launch_bounds__(256, NT == 2 ? 2 : 1) void herk_split_kernel(
-    SplitProblem P, SliceCfg cfg) {
+    const SplitProblem P0, SliceCfg cfg, HerkBatch hb) {
   __shared__ SplitStage<NT, 4> L0, L1;
+  SplitProblem P = P0;
   const int64_t seg_len = seg_columns(P.seg_len_host, P.seg_len_dev);
   const int kps = (int)cdiv(seg_len, (int64_t)kSK);  // K tiles per segment
   const int ktiles = kps * P.nseg;
   const int ns = active_slices_wave(ktiles, P.ngroups, cfg);
-  for_items((int64_t)P.ngroups * ns, [&](int64_t it) {
-    split_item<NT, MAXORD, F16, 4>(P, (int)(it / P.ngroups),
-                                   (int)(it % P.ngroups), ns, ktiles, kps, L0,
+  const int64_t per = (int64_t)P.ngroups * ns;
+  for_items(per * hb.n, [&](int64_t it) {
+    const int64_t b = it / per, i = it - b * per;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) P.t[t] = P0.t[t] + b * hb.z_stride;
+    P.part = (cplx<float> *)((char *)P0.part + b * hb.ws_stride);
+    P.dpart = (double *)((char *)P0.dpart + b * hb.ws_stride);
+    split_item<NT, MAXORD, F16, 4>(P, (int)(i / P.ngroups),
+                                   (int)(i % P.ngroups), ns, ktiles, kps, L0,
                                    L1);
   });
 }
@@ -1219,19 +1242,21 @@ __device__ __forceinline__ void reduce_elems(
 
 // Blocks of 256 threads (128 element groups), per tile (looped past the
 // grid's 65535).
-template <typename TP> dim3 reduce_grid(int ts, int64_t ntiles) {
+template <typename TP>
+dim3 reduce_grid(int ts, int64_t ntiles, int nbatch = 1) {
   return dim3((unsigned)cdiv((int64_t)ts * ts,
                              (int64_t)128 * kReduceEpt<TP>),
-              (unsigned)(ntiles < 65535 ? ntiles : 65535));
+              (unsigned)(ntiles < 65535 ? ntiles : 65535), (unsigned)nbatch);
 }
 
-// grid reduce_grid<TP>(ts, ntiles); the slice count is found once per block
+// grid reduce_grid<TP>(ts, ntiles, instances); the slice count is found once
+// per block
 template <typename TP>
 __global__ __launch_bounds__(256) void herk_reduce_kernel(
     const cplx<TP> *__restrict__ part, const double *__restrict__ dpart,
     int ntiles, int ngroups, int nb, int ts, int64_t seg_len_host,
     const int32_t *__restrict__ seg_len_dev, int nseg, int kc, SliceCfg cfg,
-    double scale, cplx<double> *__restrict__ vacc, int64_t ldv,
+    HerkBatch hb, double scale, cplx<double> *__restrict__ vacc, int64_t ldv,
     int accumulate) {
   __shared__ int ns_shared;
   if (threadIdx.x < 64) {
@@ -1244,6 +1269,11 @@ __global__ __launch_bounds__(256) void herk_reduce_kernel(
   int h;
   const int64_t e = reduce_group<TP>(h);
   if (e >= (int64_t)ts * ts) return;
+  const int64_t b = blockIdx.z;
+  part = (const cplx<TP> *)((const char *)part + b * hb.ws_stride);
+  if (dpart) dpart = (const double *)((const char *)dpart + b * hb.ws_stride);
+  vacc += b * hb.vacc_stride;
+  if (hb.scales) scale = hb.scales[b];
   for (int tile = blockIdx.y; tile < ntiles; tile += gridDim.y)
     reduce_elems(part, dpart, ntiles, nb, ts, tile, e, h, ns_shared, scale,
                  vacc, ldv, accumulate);
@@ -1281,12 +1311,14 @@ __global__ __launch_bounds__(256) void vacc_sum_kernel(
 }
 
 // out[p, a, b] = V[i nf + b, j nf + a] from the r <= c half of the
-// accumulator, V[r, c] = conj(V[c, r]) for the other half.
+// accumulator, V[r, c] = conj(V[c, r]) for the other half; grid.y instances.
 template <typename TO>
 __global__ __launch_bounds__(256) void expand_kernel(
     const cplx<double> *__restrict__ vacc, int64_t ldv, int nant, int nf,
     const int32_t *__restrict__ pairs, int64_t npairs,
-    cplx<TO> *__restrict__ out) {
+    cplx<TO> *__restrict__ out, int64_t vacc_stride, int64_t out_stride) {
+  vacc += blockIdx.y * vacc_stride;
+  out += blockIdx.y * out_stride;
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int per = nf * nf;
   if (idx >= npairs * per) return;
@@ -1454,7 +1486,7 @@ const void *grouped_kernel_t(bool f16, int nterms, int maxord) {
 }
 
 int plan_herk(int form, int nterms, int maxord, int m, int nslices,
-              HerkPlan &p) {
+              int nbatch, HerkPlan &p) {
   const bool plain = form == MV_FORM_C128 || form == MV_FORM_C64;
   p.ts = plain ? panel_side(form, m) : kSP;
   p.nb = (int)cdiv((int64_t)m, (int64_t)p.ts);
@@ -1464,7 +1496,7 @@ int plan_herk(int form, int nterms, int maxord, int m, int nslices,
   const int slots = kernel_slots(herk_kernel(form, nterms, maxord, p.ts));
   if (slots <= 0) return -1;
   p.cfg = SliceCfg{nslices, slots, form_cmax(form), plain ? 2 : 4};
-  const int64_t items = (int64_t)p.ngroups * nslices;
+  const int64_t items = (int64_t)p.ngroups * nslices * nbatch;
   p.grid = (int)(items < slots ? items : slots);
   return 0;
 }
@@ -1478,7 +1510,7 @@ extern "C" int mv_herk_slices(int form, int nterms, int nprod, int m,
       seg_len < 0 || nslices < 1)
     return MV_ERR_ARG;
   HerkPlan p;
-  if (plan_herk(form, nterms, maxord, m, nslices, p))
+  if (plan_herk(form, nterms, maxord, m, nslices, 1, p))
     return MV_ERR_HIP;
   const int ktiles = (int)(cdiv(seg_len, (int64_t)p.kc) * nseg);
   return active_slices(ktiles, p.ngroups, p.cfg);
@@ -1501,6 +1533,7 @@ struct PlainLaunch {
   void *workspace;
   int phases;
   hipStream_t st;
+  HerkBatch hb;
 };
 
 template <typename T, int P>
@@ -1514,17 +1547,20 @@ int plain_run(const HerkPlan &p, const PlainLaunch &L) {
   Q.n = p.nb;
   Q.ngroups = p.ngroups;
   Q.npairs = p.ntiles;
-  Q.wide = plain_wide(Q, L.nseg);
+  Q.wide = plain_wide(Q, L.nseg) &&
+           L.hb.z_stride * 2 * (int64_t)sizeof(T) % 16 == 0;
   if (L.phases & kPhaseCompute) {
     herk_plain_kernel<T, P>
-        <<<p.grid, 256, 0, L.st>>>(Q, L.nseg, L.seg_len, L.seg_len_dev, p.cfg);
+        <<<p.grid, 256, 0, L.st>>>(Q, L.nseg, L.seg_len, L.seg_len_dev, p.cfg,
+                                   L.hb);
     if (int e = check_launch("mv_herk/plain")) return e;
   }
   if (!(L.phases & kPhaseReduce)) return MV_OK;
-  herk_reduce_kernel<T><<<reduce_grid<T>(p.ts, p.ntiles), 256, 0, L.st>>>(
-      (const cplx<T> *)L.workspace, nullptr, p.ntiles, p.ngroups, p.nb, p.ts,
-      L.seg_len, L.seg_len_dev, L.nseg, p.kc, p.cfg, L.scale,
-      (cplx<double> *)L.vacc, L.ldv, L.accumulate);
+  herk_reduce_kernel<T>
+      <<<reduce_grid<T>(p.ts, p.ntiles, L.hb.n), 256, 0, L.st>>>(
+          (const cplx<T> *)L.workspace, nullptr, p.ntiles, p.ngroups, p.nb,
+          p.ts, L.seg_len, L.seg_len_dev, L.nseg, p.kc, p.cfg, L.hb, L.scale,
+          (cplx<double> *)L.vacc, L.ldv, L.accumulate);
   return check_launch("mv_herk/reduce");
 }
 
@@ -1535,7 +1571,7 @@ int herk_run(int phases, int form, int nterms, int nprod, const void *z0,
              int64_t seg_stride, int64_t seg_len, const int32_t *seg_len_dev,
              int nslices, double scale, double *vacc, int64_t ldv,
              int accumulate, void *workspace, size_t ws_bytes,
-             mv_stream_t stream) {
+             mv_stream_t stream, HerkBatch hb = {1, 0, 0, 0, nullptr}) {
   const int ts = mv_herk_tile(form);
   MV_REQUIRE(ts > 0, "mv_herk: unknown form %d", form);
   MV_REQUIRE(z0 && vacc && workspace, "mv_herk: null pointer");
@@ -1555,11 +1591,13 @@ int herk_run(int phases, int form, int nterms, int nprod, const void *z0,
   const int64_t ntiles = nb * (nb + 1) / 2;
   MV_REQUIRE(ldv >= nb * ts, "mv_herk: ldv %lld < %lld (tile-padded m)",
              (long long)ldv, (long long)(nb * ts));
-  MV_REQUIRE(ntiles * nslices < (int64_t)INT32_MAX / 2,
+  MV_REQUIRE(ntiles * nslices * hb.n < (int64_t)INT32_MAX / 2,
              "mv_herk: too many work items");
-  MV_REQUIRE(ws_bytes >= mv_herk_workspace_bytes(form, m, nslices),
-             "mv_herk: workspace too small (%zu < %zu)", ws_bytes,
-             mv_herk_workspace_bytes(form, m, nslices));
+  const size_t ws_one = mv_herk_workspace_bytes(form, m, nslices);
+  MV_REQUIRE(ws_bytes / hb.n >= ws_one,
+             "mv_herk: workspace too small (%zu < %d x %zu)", ws_bytes, hb.n,
+             ws_one);
+  hb.ws_stride = (int64_t)ws_one;
   const bool plain = form == MV_FORM_C128 || form == MV_FORM_C64;
   const int maxord = plain ? 0 : split_maxord(nterms, nprod);
   if (plain)
@@ -1569,7 +1607,7 @@ int herk_run(int phases, int form, int nterms, int nprod, const void *z0,
              "(2,3) (2,4) (3,6)",
              nterms, nprod);
   HerkPlan p;
-  if (plan_herk(form, nterms, maxord, m, nslices, p)) {
+  if (plan_herk(form, nterms, maxord, m, nslices, hb.n, p)) {
     set_error(MV_ERR_HIP, "mv_herk: occupancy query failed");
     return MV_ERR_HIP;
   }
@@ -1577,7 +1615,7 @@ int herk_run(int phases, int form, int nterms, int nprod, const void *z0,
   if (plain) {
     const PlainLaunch L = {z0,      m,      ldz,  nseg, seg_stride, seg_len,
                            seg_len_dev, scale, vacc, ldv,  accumulate,
-                           workspace, phases, st};
+                           workspace, phases, st, hb};
     if (form == MV_FORM_C128) return plain_run<double, 32>(p, L);
     return p.ts == 64 ? plain_run<float, 64>(p, L) : plain_run<float, 32>(p, L);
   }
@@ -1612,7 +1650,7 @@ int herk_run(int phases, int form, int nterms, int nprod, const void *z0,
   P.ngroups = p.ngroups;
   P.accumulate = accumulate;
 #define MV_SPLIT_LAUNCH(NT, MO, F)                                           \
-  herk_split_kernel<NT, MO, F><<<p.grid, 256, 0, st>>>(P, p.cfg)
+  herk_split_kernel<NT, MO, F><<<p.grid, 256, 0, st>>>(P, p.cfg, hb)
   if (phases & kPhaseCompute) {
     if (nterms == 2 && maxord == 1) {
       if (f16) MV_SPLIT_LAUNCH(2, 1, true);
@@ -1628,10 +1666,11 @@ int herk_run(int phases, int form, int nterms, int nprod, const void *z0,
   }
 #undef MV_SPLIT_LAUNCH
   if (!(phases & kPhaseReduce)) return MV_OK;
-  herk_reduce_kernel<float><<<reduce_grid<float>(p.ts, p.ntiles), 256, 0, st>>>(
-      (const cplx<float> *)workspace, dpart, p.ntiles, p.ngroups, p.nb, p.ts,
-      seg_len, seg_len_dev, nseg, p.kc, p.cfg, scale, (cplx<double> *)vacc,
-      ldv, accumulate);
+  herk_reduce_kernel<float>
+      <<<reduce_grid<float>(p.ts, p.ntiles, hb.n), 256, 0, st>>>(
+          (const cplx<float> *)workspace, dpart, p.ntiles, p.ngroups, p.nb,
+          p.ts, seg_len, seg_len_dev, nseg, p.kc, p.cfg, hb, scale,
+          (cplx<double> *)vacc, ldv, accumulate);
   return check_launch("mv_herk/reduce");
 }
 
@@ -1659,6 +1698,28 @@ extern "C" int mv_herk_reduce(MV_HERK_ARGS) {
 }
 #undef MV_HERK_ARGS
 #undef MV_HERK_PASS
+
+extern "C" int mv_herk_batch(int phases, int form, int nterms, int nprod,
+                             const void *z0, const void *z1, const void *z2,
+                             int64_t z_stride, int nbatch, int m, int64_t ldz,
+                             int nseg, int64_t seg_stride, int64_t seg_len,
+                             const int32_t *seg_len_dev, int nslices,
+                             const double *scales, double *vacc, int64_t ldv,
+                             int64_t vacc_stride, int accumulate,
+                             void *workspace, size_t ws_bytes,
+                             mv_stream_t stream) {
+  MV_REQUIRE(phases >= 1 && phases <= 3, "mv_herk_batch: phases 1, 2 or 3");
+  MV_REQUIRE(nbatch >= 1 && nbatch <= 65535 && z_stride >= 0,
+             "mv_herk_batch: bad batch");
+  MV_REQUIRE(form == MV_FORM_C128 || form == MV_FORM_C64 || z_stride % 4 == 0,
+             "mv_herk_batch: split terms must be 16-byte aligned");
+  MV_REQUIRE(nbatch == 1 || vacc_stride >= ldv * ldv,
+             "mv_herk_batch: accumulators overlap");
+  return herk_run(phases, form, nterms, nprod, z0, z1, z2, m, ldz, nseg,
+                  seg_stride, seg_len, seg_len_dev, nslices, 1.0, vacc, ldv,
+                  accumulate, workspace, ws_bytes, stream,
+                  HerkBatch{nbatch, z_stride, 0, vacc_stride, scales});
+}
 
 // ------------------------------------------------------------ no-alloc entry
 
@@ -1948,25 +2009,37 @@ extern "C" int mv_vacc_sum(const double *src, int nsrc_v, int64_t stride,
   return check_launch("mv_vacc_sum");
 }
 
-extern "C" int mv_vis_expand(const double *vacc, int64_t ldv, int tile,
-                             int nant, int nfeed, const int32_t *pairs,
-                             int64_t npairs, void *out, int out_is_f64,
-                             mv_stream_t stream) {
+extern "C" int mv_vis_expand_batch(const double *vacc, int64_t ldv,
+                                   int64_t vacc_stride, int nbatch, int tile,
+                                   int nant, int nfeed, const int32_t *pairs,
+                                   int64_t npairs, void *out, int out_is_f64,
+                                   int64_t out_stride, mv_stream_t stream) {
   MV_REQUIRE(vacc && out, "mv_vis_expand: null pointer");
   MV_REQUIRE(tile > 0 && nant >= 1 && (nfeed == 1 || nfeed == 2) &&
                  npairs >= 0 && ldv >= (int64_t)nant * nfeed,
              "mv_vis_expand: bad sizes");
+  MV_REQUIRE(nbatch >= 1 && nbatch <= 65535 && vacc_stride >= 0 &&
+                 (nbatch == 1 || out_stride >= npairs * nfeed * nfeed),
+             "mv_vis_expand: bad batch");
   const int64_t total = npairs * nfeed * nfeed;
   if (total == 0) return MV_OK;
-  dim3 g((unsigned)cdiv(total, (int64_t)256));
+  dim3 g((unsigned)cdiv(total, (int64_t)256), (unsigned)nbatch);
   hipStream_t st = as_stream(stream);
   if (out_is_f64)
-    expand_kernel<double><<<g, 256, 0, st>>>((const cplx<double> *)vacc, ldv,
-                                             nant, nfeed, pairs, npairs,
-                                             (cplx<double> *)out);
+    expand_kernel<double><<<g, 256, 0, st>>>(
+        (const cplx<double> *)vacc, ldv, nant, nfeed, pairs, npairs,
+        (cplx<double> *)out, vacc_stride, out_stride);
   else
-    expand_kernel<float><<<g, 256, 0, st>>>((const cplx<double> *)vacc, ldv,
-                                            nant, nfeed, pairs, npairs,
-                                            (cplx<float> *)out);
+    expand_kernel<float><<<g, 256, 0, st>>>(
+        (const cplx<double> *)vacc, ldv, nant, nfeed, pairs, npairs,
+        (cplx<float> *)out, vacc_stride, out_stride);
   return check_launch("mv_vis_expand");
+}
+
+extern "C" int mv_vis_expand(const double *vacc, int64_t ldv, int tile,
+                             int nant, int nfeed, const int32_t *pairs,
+                             int64_t npairs, void *out, int out_is_f64,
+                             mv_stream_t stream) {
+  return mv_vis_expand_batch(vacc, ldv, 0, 1, tile, nant, nfeed, pairs, npairs,
+                             out, out_is_f64, 0, stream);
 }

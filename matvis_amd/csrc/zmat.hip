@@ -205,18 +205,37 @@ struct ZOut {
   void *z[3];
 };
 
-// One thread per source, ants_per_block antennas per block (grid.y).
-// POL: nfeed = nax = 2 (polarized) or 1.
+// The frequencies of one launch (grid.z): frequency, flux row, beam values,
+// scale and Z of each.  Without arrays, one frequency.
+struct FreqBatch {
+  const double *freqs, *scales;  // device, or null: freq, scale
+  double freq, scale;
+  int64_t ld_flux, beam_stride, z_stride;  // elements between frequencies
+  int n;
+};
+
+// One thread per source, ants_per_block antennas per block (grid.y), one
+// frequency per grid.z.  POL: nfeed = nax = 2 (polarized) or 1.
 template <int FORM, int NT, bool POL>
 __global__ __launch_bounds__(kThreads) void zmat_fused_kernel(
-    const double *__restrict__ antpos, int nant, double fc,
+    const double *__restrict__ antpos, int nant, FreqBatch fb,
     const double *__restrict__ crd, int64_t ld_crd,
     const double *__restrict__ flux, const int32_t *__restrict__ idx,
     const cplx<typename ZWriter<FORM, NT>::T> *__restrict__ beam,
     int64_t ld_beam, int nbeam, const int32_t *__restrict__ beam_idx,
-    int64_t count, const int32_t *__restrict__ n_dev, double scale,
+    int64_t count, const int32_t *__restrict__ n_dev,
     ZOut zo, int64_t ldz, int64_t seg_stride, int ants_per_block) {
   typedef typename ZWriter<FORM, NT>::T T;
+  constexpr bool plain = FORM == MV_FORM_C128 || FORM == MV_FORM_C64;
+  const int f = blockIdx.z;
+  const double fc = (fb.freqs ? fb.freqs[f] : fb.freq) / kC;
+  const double scale = fb.scales ? fb.scales[f] : fb.scale;
+  flux += f * fb.ld_flux;
+  beam += f * fb.beam_stride;
+#pragma unroll
+  for (int k = 0; k < NT; ++k)
+    zo.z[k] = (char *)zo.z[k] +
+              f * fb.z_stride * (int64_t)(plain ? sizeof(cplx<T>) : 4);
   constexpr int nf = POL ? 2 : 1;
   constexpr int na = POL ? 2 : 1;
   const int64_t s = (int64_t)blockIdx.x * kThreads + threadIdx.x;
@@ -291,24 +310,21 @@ __global__ __launch_bounds__(kThreads) void split_kernel(
 
 template <int FORM, int NT>
 int launch_fused(dim3 g, hipStream_t st, const double *antpos, int nant,
-                 double fc, const double *crd, int64_t ld_crd,
+                 const FreqBatch &fb, const double *crd, int64_t ld_crd,
                  const double *flux, const int32_t *idx, const void *beam,
                  int64_t ld_beam,
-                 int nbeam, const int32_t *beam_idx, int nf, int na,
-                 int64_t count, const int32_t *n_dev, double scale, ZOut zo,
+                 int nbeam, const int32_t *beam_idx, int nf,
+                 int64_t count, const int32_t *n_dev, ZOut zo,
                  int64_t ldz, int64_t seg_stride, int apb) {
   typedef typename ZWriter<FORM, NT>::T T;
-  (void)na;
   if (nf == 2)
     zmat_fused_kernel<FORM, NT, true><<<g, kThreads, 0, st>>>(
-        antpos, nant, fc, crd, ld_crd, flux, idx, (const cplx<T> *)beam,
-        ld_beam, nbeam, beam_idx, count, n_dev, scale, zo, ldz, seg_stride,
-        apb);
+        antpos, nant, fb, crd, ld_crd, flux, idx, (const cplx<T> *)beam,
+        ld_beam, nbeam, beam_idx, count, n_dev, zo, ldz, seg_stride, apb);
   else
     zmat_fused_kernel<FORM, NT, false><<<g, kThreads, 0, st>>>(
-        antpos, nant, fc, crd, ld_crd, flux, idx, (const cplx<T> *)beam,
-        ld_beam, nbeam, beam_idx, count, n_dev, scale, zo, ldz, seg_stride,
-        apb);
+        antpos, nant, fb, crd, ld_crd, flux, idx, (const cplx<T> *)beam,
+        ld_beam, nbeam, beam_idx, count, n_dev, zo, ldz, seg_stride, apb);
   return check_launch("mv_zmat_fused");
 }
 
@@ -367,16 +383,14 @@ extern "C" int mv_zmat_parts(const void *sqrt_flux, const void *beam,
   return check_launch("mv_zmat_parts");
 }
 
-extern "C" int mv_zmat_fused(const double *antpos, int nant, double freq,
-                             const double *crd, int64_t ld_crd,
-                             const double *flux, const int32_t *idx,
-                             const void *beam, int beam_is_f64,
-                             int64_t ld_beam, int nbeam,
-                             const int32_t *beam_idx, int nfeed, int nax,
-                             int64_t count, const int32_t *n_dev, int form,
-                             int nterms, double scale, void *z0, void *z1,
-                             void *z2, int64_t ldz, int64_t seg_stride,
-                             mv_stream_t stream) {
+namespace {
+int zmat_run(const double *antpos, int nant, const FreqBatch &fb,
+             const double *crd, int64_t ld_crd, const double *flux,
+             const int32_t *idx, const void *beam, int beam_is_f64,
+             int64_t ld_beam, int nbeam, const int32_t *beam_idx, int nfeed,
+             int nax, int64_t count, const int32_t *n_dev, int form,
+             int nterms, void *z0, void *z1, void *z2, int64_t ldz,
+             int64_t seg_stride, mv_stream_t stream) {
   MV_REQUIRE(antpos && crd && flux && beam && z0,
              "mv_zmat_fused: null pointer");
   MV_REQUIRE(nant >= 1 && nbeam >= 1 && count >= 0 && ld_crd >= count &&
@@ -408,21 +422,24 @@ extern "C" int mv_zmat_fused(const double *antpos, int nant, double freq,
   MV_REQUIRE(nterms < 2 || z1, "mv_zmat_fused: missing term array 1");
   MV_REQUIRE(nterms < 3 || z2, "mv_zmat_fused: missing term array 2");
   if (count == 0) return MV_OK;
-  const int apb = 16;
+  // 16 antennas a block share its sources' inputs; fewer where the launch
+  // would leave most of the 256 CUs' eight blocks each empty (32 antennas x
+  // 1,800 sources up, one frequency: 16 blocks of work for 256 CUs)
+  const int64_t xblocks = cdiv(cdiv(count, kZPad) * kZPad, kThreads);
+  int apb = 16;
+  while (apb > 2 && xblocks * cdiv(nant, apb) * fb.n < 2048) apb /= 2;
   // blocks go to the 8 XCDs round-robin by linear index x + y gx: with gx a
   // multiple of 8, the antenna blocks of one source range share an XCD and
   // its L2, which then serves their re-reads of the per-source inputs (the
   // blocks past the column count return at once)
-  dim3 g((unsigned)(cdiv(cdiv(cdiv(count, kZPad) * kZPad, kThreads),
-                         (int64_t)8) * 8),
-         (unsigned)cdiv(nant, apb));
+  dim3 g((unsigned)(cdiv(xblocks, (int64_t)8) * 8), (unsigned)cdiv(nant, apb),
+         (unsigned)fb.n);
   hipStream_t st = as_stream(stream);
-  const double fc = freq / kC;
   ZOut zo = {{z0, z1, z2}};
 #define MV_FUSED(F, NT)                                                      \
-  return launch_fused<F, NT>(g, st, antpos, nant, fc, crd, ld_crd, flux,     \
-                             idx, beam, ld_beam, nbeam, beam_idx, nfeed, nax,\
-                             count, n_dev, scale, zo, ldz, seg_stride, apb)
+  return launch_fused<F, NT>(g, st, antpos, nant, fb, crd, ld_crd, flux,     \
+                             idx, beam, ld_beam, nbeam, beam_idx, nfeed,     \
+                             count, n_dev, zo, ldz, seg_stride, apb)
   switch (form) {
     case MV_FORM_C128: MV_FUSED(MV_FORM_C128, 1);
     case MV_FORM_C64: MV_FUSED(MV_FORM_C64, 1);
@@ -434,6 +451,43 @@ extern "C" int mv_zmat_fused(const double *antpos, int nant, double freq,
       MV_FUSED(MV_FORM_SPLIT_F16, 3);
   }
 #undef MV_FUSED
+}
+}  // namespace
+
+extern "C" int mv_zmat_fused(const double *antpos, int nant, double freq,
+                             const double *crd, int64_t ld_crd,
+                             const double *flux, const int32_t *idx,
+                             const void *beam, int beam_is_f64,
+                             int64_t ld_beam, int nbeam,
+                             const int32_t *beam_idx, int nfeed, int nax,
+                             int64_t count, const int32_t *n_dev, int form,
+                             int nterms, double scale, void *z0, void *z1,
+                             void *z2, int64_t ldz, int64_t seg_stride,
+                             mv_stream_t stream) {
+  const FreqBatch fb = {nullptr, nullptr, freq, scale, 0, 0, 0, 1};
+  return zmat_run(antpos, nant, fb, crd, ld_crd, flux, idx, beam, beam_is_f64,
+                  ld_beam, nbeam, beam_idx, nfeed, nax, count, n_dev, form,
+                  nterms, z0, z1, z2, ldz, seg_stride, stream);
+}
+
+extern "C" int mv_zmat_fused_batch(
+    const double *antpos, int nant, const double *freqs, int nfreq,
+    const double *crd, int64_t ld_crd, const double *flux, int64_t ld_flux,
+    const int32_t *idx, const void *beam, int beam_is_f64, int64_t ld_beam,
+    int64_t beam_stride, int nbeam, const int32_t *beam_idx, int nfeed,
+    int nax, int64_t count, const int32_t *n_dev, int form, int nterms,
+    const double *scales, void *z0, void *z1, void *z2, int64_t ldz,
+    int64_t seg_stride, int64_t z_stride, mv_stream_t stream) {
+  MV_REQUIRE(freqs && nfreq >= 1 && nfreq <= 65535,
+             "mv_zmat_fused_batch: needs 1..65535 frequencies");
+  MV_REQUIRE(ld_flux >= 0 && beam_stride >= 0 &&
+                 (nfreq == 1 || z_stride >= 1),
+             "mv_zmat_fused_batch: bad strides");
+  const FreqBatch fb = {freqs,   scales,      0.0,      1.0,
+                        ld_flux, beam_stride, z_stride, nfreq};
+  return zmat_run(antpos, nant, fb, crd, ld_crd, flux, idx, beam, beam_is_f64,
+                  ld_beam, nbeam, beam_idx, nfeed, nax, count, n_dev, form,
+                  nterms, z0, z1, z2, ldz, seg_stride, stream);
 }
 
 extern "C" int mv_split_z(const void *z, int z_is_f64, int64_t rows, int nseg,

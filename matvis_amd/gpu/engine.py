@@ -3,7 +3,8 @@
 For each time: one rotation + cull + compaction per source chunk (shared by
 every frequency); then for each frequency and chunk the beam evaluation, the
 fused phase/Z kernel (Z written once) and the HERK into an FP64 accumulator;
-then the expansion into the API layout.  Everything is enqueued on the current
+then the expansion into the API layout.  Frequencies whose Z is small share
+these launches (:func:`freq_batch`).  Everything is enqueued on the current
 stream without host synchronization; results go to the host through pinned
 buffers on a second stream, double-buffered so the copy of time t overlaps the
 compute of time t+1.
@@ -30,21 +31,46 @@ from .._lib import FORM_C128, FORM_SPLIT_F16, call, lib
 from .._utils import log_progress
 from .._utils import logger as _progress_log
 from .beams import DeviceBeamSet
-from .herk import Herk, cdiv, expand, is_split, split_terms_alloc
+from .herk import (Herk, cdiv, expand, expand_batch, is_split,
+                   split_terms_alloc)
 from .matprod import f16_scale
 
 Z_PAD = 32  # mv_zmat_fused pads Z columns to a multiple of this
+
+
+#: device bytes the per-frequency buffers of one launch may take together
+#: (Z, split-K partials, accumulator): twice the 256 MB Infinity Cache.  Above
+#: it one frequency fills the GPU by itself (350 antennas x 100k sources: 0.7
+#: to 1.3 GB of Z, 1,000 HERK items for 512 workgroup slots).  Measured, a
+#: time with one launch per frequency and with this: 32 frequencies of 32
+#: antennas x 3k sources (one launch) 1.09 -> 0.058 ms, 16 of 128 antennas x
+#: 50k sources (two of 8) 1.08 -> 0.38 ms, 6 of 61 antennas x 20k sources in
+#: FP64 (two of 3) 0.49 -> 0.35 ms.
+BATCH_BYTES = 512 << 20
+
+
+def freq_batch(*, form: int, nterms: int, nprod: int, m: int, nax: int,
+               nfreq: int, nsrc_alloc: int) -> int:
+    """Frequencies per launch: as many as BATCH_BYTES holds, in even parts."""
+    seg = max(Z_PAD, cdiv(nsrc_alloc, Z_PAD) * Z_PAD)
+    herk = Herk(form, m, nterms, nprod)
+    esz = 4 * nterms if is_split(form) else 16 if form == FORM_C128 else 8
+    each = m * nax * seg * esz + herk.ldv * herk.ldv * 16 + int(
+        lib().mv_herk_workspace_bytes(form, m, herk.nslices(nax * nsrc_alloc)))
+    fit = max(1, min(nfreq, BATCH_BYTES // each))
+    return cdiv(nfreq, cdiv(nfreq, fit))
 
 
 def device_bytes(*, form: int, nterms: int, nprod: int, nant: int,
                  polarized: bool, nfreq: int, nsrc: int, nchunks: int,
                  chunk_size: int, nsrc_alloc: int, nbeam: int,
                  beam_pixels: int, beam_sets: int, npairs: int,
-                 precision: int) -> dict:
+                 precision: int, batch: int | None = None) -> dict:
     """Device bytes an engine and its rotation plugin hold, term by term, as
     their ``setup`` and ``run`` allocate them (beam_pixels: grid points of
     one beam plane, 0 for analytic beams; beam_sets: 1, or nfreq when the
-    beam tables differ by frequency).  ``total`` is their sum."""
+    beam tables differ by frequency; batch: frequencies per launch, the
+    engine's default when None).  ``total`` is their sum."""
     nf = 2 if polarized else 1
     m = nf * nant
     seg = max(Z_PAD, cdiv(nsrc_alloc, Z_PAD) * Z_PAD)
@@ -52,6 +78,8 @@ def device_bytes(*, form: int, nterms: int, nprod: int, nant: int,
     esz = 16 if form == FORM_C128 else 8  # beam values, plain Z elements
     herk = Herk(form, m, nterms, nprod)
     cull_ws = int(lib().mv_rotate_cull_workspace_bytes(chunk_size))
+    nb = batch or freq_batch(form=form, nterms=nterms, nprod=nprod, m=m,
+                             nax=nf, nfreq=nfreq, nsrc_alloc=nsrc_alloc)
     terms = {
         # rotation plugin: ECI, topocentric (and FP64 / BCRS copies), the
         # kept coordinates, fluxes, indices and its cull workspace
@@ -60,11 +88,11 @@ def device_bytes(*, form: int, nterms: int, nprod: int, nant: int,
         "antpos_flux": nant * 24 + nfreq * nsrc * 8,
         "chunk_coords": nchunks * seg * (24 + 4) + cull_ws,
         "beam_tables": beam_sets * nbeam * nf * nf * beam_pixels * esz,
-        "beam_values": (nchunks if beam_sets == 1 else 1) * nbeam * nf * nf
+        "beam_values": (nchunks if beam_sets == 1 else nb) * nbeam * nf * nf
         * seg * esz,
-        "z": m * nf * seg * (4 * nterms if is_split(form) else esz),
-        "vacc": herk.ldv * herk.ldv * 16,
-        "herk_workspace": int(lib().mv_herk_workspace_bytes(
+        "z": nb * m * nf * seg * (4 * nterms if is_split(form) else esz),
+        "vacc": nb * herk.ldv * herk.ldv * 16,
+        "herk_workspace": nb * int(lib().mv_herk_workspace_bytes(
             form, m, herk.nslices(nf * nsrc_alloc))),
         "output": 2 * nfreq * npairs * nf * nf * 2 * rsz,
     }
@@ -77,14 +105,15 @@ class VisibilityEngine:
 
     Parameters mirror ``gpu.simulate``: ``coords`` is a set-up
     :class:`~matvis_amd.core.coords.CoordinateRotation`; ``fluxes`` is
-    (nsrc, nfreq) Stokes I; ``form`` / ``nterms`` / ``nprod`` select the HERK.
+    (nsrc, nfreq) Stokes I; ``form`` / ``nterms`` / ``nprod`` select the HERK;
+    ``batch``: frequencies per launch (default: :func:`freq_batch`).
     """
 
     def __init__(self, *, antpos, freqs, coords, fluxes, beam_list, beam_idx,
                  polarized: bool, precision: int, form: int, nterms: int = 1,
                  nprod: int = 1, order: int = 1, nchunks: int, chunk_size: int,
                  nsrc_alloc: int, antpairs=None, beam_cache: dict | None = None,
-                 beam_src=None):
+                 beam_src=None, batch: int | None = None):
         self.antpos_h = np.asarray(antpos, dtype=np.float64)
         self.nant = self.antpos_h.shape[0]
         self.freqs = np.atleast_1d(np.asarray(freqs, dtype=np.float64))
@@ -121,6 +150,9 @@ class VisibilityEngine:
         #: cache), keyed by the caller's beam objects ``beam_src``
         self.beam_cache = beam_cache
         self.beam_src = list(beam_src) if beam_src is not None else None
+        self.batch = batch or freq_batch(
+            form=form, nterms=nterms, nprod=nprod, m=self.m, nax=self.nax,
+            nfreq=self.nfreq, nsrc_alloc=nsrc_alloc)
         self._ready = False
         #: optional (before, after) callables taking the stream, run around
         #: every HERK compute kernel (event timing of the dominant kernel;
@@ -133,6 +165,8 @@ class VisibilityEngine:
         seg, nalloc = self.seg, self.nsrc_alloc
         self.antpos = D.to_dev(self.antpos_h, np.float64)
         self.sqrt_flux = D.to_dev(self.sqrt_flux_h, np.float64)
+        F = self.batch
+        self.freqs_dev = D.to_dev(self.freqs, np.float64) if F > 1 else None
         self.beam_idx_dev = (None if self.beam_idx is None
                              else D.as_dev(self.beam_idx, np.int32))
         self.pairs_dev = (None if self.pairs_h is None
@@ -148,23 +182,27 @@ class VisibilityEngine:
         self.beam_sets = self._make_beam_sets()
         self.nbeam = self.beam_sets[0].nbeam
         shared = len(self.beam_sets) == 1
-        nA = nb if shared else 1
-        self.A = [D.zeros((self.nbeam, self.nfeed, self.nax, seg),
-                          self.beam_ctype) for _ in range(nA)]
+        nA = nb if shared else F
+        self.A = list(D.zeros((nA, self.nbeam, self.nfeed, self.nax, seg),
+                              self.beam_ctype))
         # Z: (m, nax, seg) complex (ldz the row stride), or nterms arrays of
         # 16-bit terms, K-tile-major (ldz the rows of a 16-column K tile;
         # 32 bits a complex element, 16-byte chunks of 4 columns: re x 4,
         # im x 4)
         if is_split(self.form):
             self.ldz = self.m
-            self.z = split_terms_alloc(self.nterms, self.m, self.nax * seg)
+            self.z = split_terms_alloc(self.nterms, self.m,
+                                       F * self.nax * seg)
         else:
             self.ldz = self.nax * seg
-            self.z = [D.zeros((self.m, self.ldz), self.beam_ctype)]
+            self.z = [D.zeros((F * self.m, self.ldz), self.beam_ctype)]
+        # elements (split: words) between the Z of a launch's frequencies
+        self.z_stride = self.m * self.nax * seg
         self.herk = Herk(self.form, self.m, self.nterms, self.nprod)
-        self.vacc = self.herk.new_vacc()
+        self.vaccs = D.zeros((F, self.herk.ldv, self.herk.ldv), np.complex128)
+        self.vacc = self.vaccs[0]
         self.nslices = self.herk.nslices(self.nax * nalloc)
-        self.herk.workspace(self.nslices)
+        self.herk.workspace(self.nslices, F)
         # per-(chunk, freq) power-of-two scales for the fp16 split
         self.scales = np.ones((nb, self.nfreq))
         if self.form == FORM_SPLIT_F16:
@@ -175,6 +213,10 @@ class VisibilityEngine:
                 for f in range(self.nfreq):
                     mx = float(part[f].max()) if part.shape[1] else 0.0
                     self.scales[c, f] = f16_scale(mx * bmax)
+        # Z's scales and the HERK's 1 / scale^2 on the device
+        self.scales_dev = (D.to_dev(np.stack([self.scales,
+                                              1.0 / self.scales ** 2]))
+                           if F > 1 and self.form == FORM_SPLIT_F16 else None)
         self._ready = True
 
     def _make_beam_sets(self):
@@ -282,10 +324,53 @@ class VisibilityEngine:
         expand(self.vacc, self.herk.ldv, self.herk.tile, self.nant,
                self.nfeed, self.pairs_dev, self.npairs, out_dev[fi], stream)
 
+    def compute_batch(self, f0: int, n: int, out_dev, stream=None):
+        """Frequencies f0 .. f0 + n - 1 of the staged time, each stage one
+        launch for all of them (per chunk), into out_dev[f0 : f0 + n]."""
+        shared = len(self.beam_sets) == 1
+        sp = D.stream_ptr(stream)
+        zp = [D.ptr(z) for z in self.z] + [None] * (3 - len(self.z))
+        for c in range(self.nchunks):
+            n_dev = self.n_up[self._parity][c:c + 1]
+            if not shared:
+                for k in range(n):
+                    self.beam_sets[f0 + k].eval(
+                        self.crd[c], self.seg, self.nsrc_alloc, self.A[k],
+                        self.seg, n_dev, stream)
+            a = self.A[c] if shared else self.A[0]
+            zs = hs = None
+            if self.scales_dev is not None:
+                zs, hs = self.scales_dev[0, c, f0:], self.scales_dev[1, c, f0:]
+            call("mv_zmat_fused_batch", D.ptr(self.antpos), self.nant,
+                 D.ptr(self.freqs_dev[f0:]), n, D.ptr(self.crd[c]), self.seg,
+                 D.ptr(self.sqrt_flux[f0]), self.nsrc, D.ptr(self.idx[c]),
+                 D.ptr(a), int(self.beam_ctype == np.complex128), self.seg,
+                 0 if shared else a.numel(), self.nbeam,
+                 D.ptr(self.beam_idx_dev), self.nfeed, self.nax,
+                 self.nsrc_alloc, D.ptr(n_dev), self.form, self.nterms,
+                 D.ptr(zs), zp[0], zp[1], zp[2], self.ldz, self.seg,
+                 self.z_stride, sp)
+            if self.herk_hooks:
+                self.herk_hooks[0](stream)
+            self.herk.run_batch(
+                self.z, self.z_stride, n, ldz=self.ldz, nseg=self.nax,
+                seg_stride=self.seg, seg_len=self.nsrc_alloc,
+                seg_len_dev=n_dev, vacc=self.vaccs, accumulate=c > 0,
+                nslices=self.nslices, scales=hs, stream=stream,
+                between=self.herk_hooks[1] if self.herk_hooks else None)
+        expand_batch(self.vaccs, self.herk.ldv, self.herk.tile, self.nant,
+                     self.nfeed, self.pairs_dev, self.npairs,
+                     out_dev[f0:f0 + n], stream)
+
     def compute_time(self, t: int, out_dev, parity: int = 0, stream=None):
         """Enqueue the whole of time index t; results land in out_dev
         (nfreq, npairs, nfeed, nfeed) and the chunk counts in n_up[parity]."""
         self.stage_time(t, parity, stream)
+        if self.batch > 1:
+            for f0 in range(0, self.nfreq, self.batch):
+                self.compute_batch(f0, min(self.batch, self.nfreq - f0),
+                                   out_dev, stream)
+            return out_dev
         for fi in range(self.nfreq):
             for c in range(self.nchunks):
                 prob = self.stage_z(fi, c, stream)

@@ -20,7 +20,7 @@ from ..core.coords import CoordinateRotation
 from . import coords as _coords  # noqa: F401  (registers rotation methods)
 from . import matprod as mp
 from .beams import spline_order
-from .engine import VisibilityEngine
+from .engine import VisibilityEngine, freq_batch
 from .herk import products_for
 
 logger = logging.getLogger(__name__)
@@ -65,11 +65,14 @@ def build_engine(
     split_terms: int | None = None,
     split_products: int | None = None,
     beam_cache: dict | None = None,
+    batch: int | None = None,
 ):
     """The set-up :class:`VisibilityEngine` of a simulation and its number
     of times; arguments as :func:`simulate_multi`.  ``beam_cache``: a dict
     shared between engines so that device beam tables of the same beam
-    objects are built once (see ``VisibilityEngine``)."""
+    objects are built once (see ``VisibilityEngine``); ``batch``: at most
+    this many frequencies per launch (a caller that steps the frequencies
+    itself passes 1)."""
     if not 0 < source_buffer <= 1:
         raise ValueError("source_buffer must satisfy 0 < source_buffer <= 1")
     if not 0 < memory_buffer <= 1:
@@ -93,13 +96,20 @@ def build_engine(
     )
     beams, _, beam_idx = _wrangle_beams(beam_idx, beam_list, polarized, nant,
                                         float(freqs[0]))
-    nchunks, npixc = fit_chunks(
-        freemem * memory_buffer, nchunks, form=form, nterms=nterms,
-        nprod=nprod, nant=nant, polarized=polarized, nfreq=freqs.size,
-        nsrc=nsrc, source_buffer=source_buffer, beams=beams,
-        npairs=nant * nant if antpairs is None else len(antpairs),
-        precision=precision)
+    sizes = dict(form=form, nterms=nterms, nprod=nprod, nant=nant,
+                 polarized=polarized, nfreq=freqs.size, nsrc=nsrc,
+                 source_buffer=source_buffer, beams=beams,
+                 npairs=nant * nant if antpairs is None else len(antpairs),
+                 precision=precision)
+    nchunks, npixc = fit_chunks(freemem * memory_buffer, nchunks, **sizes)
+    need = footprint(**sizes)
     nsrc_alloc = int(npixc * source_buffer)
+    # frequencies per launch, as many as fit beside the rest
+    F = batch or freq_batch(form=form, nterms=nterms, nprod=nprod,
+                            m=nfeed * nant, nax=nax, nfreq=freqs.size,
+                            nsrc_alloc=nsrc_alloc)
+    while F > 1 and need(nchunks, F) > freemem * memory_buffer:
+        F //= 2
     coord_cls = CoordinateRotation._methods[coord_method]
     coords = coord_cls(
         flux=np.sqrt(0.5 * fluxes[:, 0]), times=times,
@@ -114,23 +124,19 @@ def build_engine(
         precision=precision, form=form, nterms=nterms, nprod=nprod,
         order=spline_order(beam_spline_opts), nchunks=nchunks,
         chunk_size=npixc, nsrc_alloc=nsrc_alloc, antpairs=antpairs,
-        beam_cache=beam_cache, beam_src=beam_list,
+        beam_cache=beam_cache, beam_src=beam_list, batch=F,
     )
     logger.info(f"Running with {nchunks} chunks, form {form}")
     engine.setup()
     return engine, ntimes
 
 
-def fit_chunks(budget: float, nchunks: int, *, form, nterms, nprod, nant,
-               polarized, nfreq, nsrc, source_buffer, beams, npairs,
-               precision) -> tuple[int, int]:
-    """(nchunks, sources per chunk): the reference's chunk count
-    (get_desired_chunks, which sizes the reference's own buffers), raised
-    until this build's device footprint (engine.device_bytes: Z terms,
-    split-K workspace, FP64 accumulator, beam tables and values, output
-    buffers, the rotation plugin's arrays) fits the budget
-    (min(max_memory, free memory) x memory_buffer).  If even min(nsrc, 1000)
-    chunks do not fit, that count is used and a warning logged."""
+def footprint(*, form, nterms, nprod, nant, polarized, nfreq, nsrc,
+              source_buffer, beams, npairs, precision):
+    """A function of (nchunks, frequencies per launch): this build's device
+    bytes (engine.device_bytes: Z terms, split-K workspace, FP64
+    accumulator, beam tables and values, output buffers, the rotation
+    plugin's arrays)."""
     from ..beams import is_grid_beam, unwrap
     from .engine import device_bytes
 
@@ -140,7 +146,7 @@ def fit_chunks(budget: float, nchunks: int, *, form, nterms, nprod, nant,
     per_freq = nfreq > 1 and any(np.asarray(g.freq_array).size > 1
                                  for g in grid)
 
-    def need(ch):
+    def need(ch, batch=1):
         npc = int(np.ceil(nsrc / ch))
         return device_bytes(
             form=form, nterms=nterms, nprod=nprod, nant=nant,
@@ -148,8 +154,20 @@ def fit_chunks(budget: float, nchunks: int, *, form, nterms, nprod, nant,
             chunk_size=npc, nsrc_alloc=int(npc * source_buffer),
             nbeam=len(beams), beam_pixels=pixels,
             beam_sets=nfreq if per_freq else 1, npairs=npairs,
-            precision=precision)["total"]
+            precision=precision, batch=batch)["total"]
 
+    return need
+
+
+def fit_chunks(budget: float, nchunks: int, *, nsrc, **sizes
+               ) -> tuple[int, int]:
+    """(nchunks, sources per chunk): the reference's chunk count
+    (get_desired_chunks, which sizes the reference's own buffers), raised
+    until this build's device footprint with one frequency per launch
+    (:func:`footprint`, whose keywords this takes) fits the budget
+    (min(max_memory, free memory) x memory_buffer).  If even min(nsrc, 1000)
+    chunks do not fit, that count is used and a warning logged."""
+    need = footprint(nsrc=nsrc, **sizes)
     limit = max(nchunks, min(nsrc, 1000))
     ch = nchunks
     while ch < limit and need(ch) > budget:

@@ -91,8 +91,9 @@ class Herk:
                  nseg, int(seg_len), nslices)
         return int(n)
 
-    def workspace(self, nslices: int):
-        need = lib().mv_herk_workspace_bytes(self.form, self.m, nslices)
+    def workspace(self, nslices: int, batch: int = 1):
+        need = batch * lib().mv_herk_workspace_bytes(self.form, self.m,
+                                                     nslices)
         if self._ws is None or self._ws.numel() < need:
             self._ws = D.empty((max(need, 256),), np.uint8)
         return self._ws
@@ -122,10 +123,44 @@ class Herk:
         return vacc
 
 
+    def run_batch(self, z_terms, z_stride: int, batch: int, ldz: int,
+                  nseg: int, seg_stride: int, seg_len: int, vacc,
+                  accumulate: bool, nslices: int, seg_len_dev=None,
+                  scales=None, stream=None, between=None):
+        """`batch` instances of one shape in one launch (``mv_herk_batch``):
+        Z z_stride elements apart, accumulators vacc (batch, ldv, ldv),
+        ``scales`` a device array or None; ``between`` as :meth:`run`."""
+        ws = self.workspace(nslices, batch)
+        zp = [D.ptr(t) for t in z_terms] + [None] * (3 - len(z_terms))
+        args = (self.form, self.nterms, self.nprod, zp[0], zp[1], zp[2],
+                z_stride, batch, self.m, ldz, nseg, seg_stride, seg_len,
+                D.ptr(seg_len_dev), nslices, D.ptr(scales), D.ptr(vacc),
+                self.ldv, self.ldv * self.ldv, int(bool(accumulate)),
+                D.ptr(ws), ws.numel(), D.stream_ptr(stream))
+        if between is None:
+            call("mv_herk_batch", 3, *args)
+        else:
+            call("mv_herk_batch", 1, *args)
+            between(stream)
+            call("mv_herk_batch", 2, *args)
+        return vacc
+
+
 def expand(vacc, ldv: int, tile: int, nant: int, nfeed: int, pairs_dev,
            npairs: int, out, stream=None):
     """API layout (npairs, nfeed, nfeed) from the FP64 accumulator."""
     call("mv_vis_expand", D.ptr(vacc), ldv, tile, nant, nfeed,
          D.ptr(pairs_dev), npairs, D.ptr(out),
          int(out.dtype == D.tdtype(np.complex128)), D.stream_ptr(stream))
+    return out
+
+
+def expand_batch(vacc, ldv: int, tile: int, nant: int, nfeed: int, pairs_dev,
+                 npairs: int, out, stream=None):
+    """API layout (batch, npairs, nfeed, nfeed) from the accumulators
+    vacc (batch, ldv, ldv) in one launch."""
+    call("mv_vis_expand_batch", D.ptr(vacc), ldv, ldv * ldv, out.shape[0],
+         tile, nant, nfeed, D.ptr(pairs_dev), npairs, D.ptr(out),
+         int(out.dtype == D.tdtype(np.complex128)), npairs * nfeed * nfeed,
+         D.stream_ptr(stream))
     return out

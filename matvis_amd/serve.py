@@ -325,7 +325,7 @@ class VisibilityServer:
                 req = self.queue.pop(i)
             try:
                 engine, ntimes = build_engine(**req.kwargs,
-                                              beam_cache=self._beams)
+                                              beam_cache=self._beams, batch=1)
             except Exception as exc:  # reported on the request
                 req.error = exc
                 req.t_done = time.perf_counter()

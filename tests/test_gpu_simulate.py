@@ -647,3 +647,41 @@ def test_max_memory_bounds_device_allocation():
     torch.cuda.empty_cache()
     one = simulate_multi(**kw)
     assert nerr(v[0], one[0], nant, True)[0] < 1e-12
+
+
+@pytest.mark.parametrize("method,precision", [
+    ("GPUMatMul", 2), ("GPUMatMul", 1), ("GPUMatMulSplitBF16", 1),
+    ("GPUMatMulSplitF16", 2)])
+@pytest.mark.parametrize("nant,polarized,per_freq,chunks,pairs", [
+    (1, False, False, 1, False), (33, False, True, 2, True),
+    (9, True, False, 3, False), (40, True, True, 1, True)])
+def test_frequencies_per_launch(method, precision, nant, polarized, per_freq,
+                                chunks, pairs):
+    """Five frequencies in one launch, and as launches of 2, 2 and 1, against
+    one each: the same bits, with beam values shared or per frequency,
+    chunked, all or listed pairs."""
+    from matvis_amd.gpu.gpu import build_engine
+
+    p = small_problem(nant=nant, nsrc=1501, ntimes=1, polarized=polarized)
+    freqs = np.linspace(120e6, 180e6, 5)
+    rng = np.random.default_rng(3)
+    beam = GaussianBeam(sigma=0.2)
+    if per_freq:  # a beam that changes with frequency: one table each
+        beam = GaussianBeam(diameter=14.0)
+    kw = dict(antpos=p["antpos"], freqs=freqs, times=p["times"],
+              skycoords=astro.SkyCoord(p["ra"], p["dec"]),
+              telescope_loc=p["loc"],
+              fluxes=p["I_sky"][:, None] * rng.uniform(0.5, 2, (1501, 5)),
+              beam_list=[beam], polarized=polarized, precision=precision,
+              min_chunks=chunks, matprod_method=method,
+              antpairs=[(0, nant - 1), (nant // 2, 0)] if pairs else None,
+              coord_method="CoordinateRotationMatrix",
+              coord_method_params={"rotations": p["rotations"]})
+    want = None
+    for batch in (1, 2, None):
+        eng, nt = build_engine(batch=batch, **kw)
+        assert eng.batch == (batch or 5)
+        v = eng.run(nt)
+        if want is None:
+            want = v
+        assert np.isfinite(v).all() and np.array_equal(v, want), batch
