@@ -97,6 +97,90 @@ __global__ __launch_bounds__(kThreads) void prefilter_kernel(
   }
 }
 
+// The same filter as its impulse response: the coefficients of a cubic
+// B-spline through f with mirrored ends are c[i] = sum_k sqrt(3) z^|k|
+// f[mirror(i + k)], z = sqrt(3) - 2 the pole (sqrt(3) = -6 z / (1 - z^2)).
+// Truncated at |k| = 30 it is exact to 2 |z|^31 sqrt(3) = 6e-18 of max|f|.
+// A workgroup holds `width` lines in LDS and every element is a sum of its
+// own, where the recursion is a chain of 3 n dependent steps a line with one
+// line a thread (1,500 threads for a polarized 360 x 91 beam): 225 us a pass
+// there, 16 us here (15.2-16.6 in either precision).
+// A line that is not finite gives NaN throughout, as the recursion does.
+constexpr int kFirReach = 30;
+constexpr int kFirLds = 60 * 1024;  // bytes of lines a workgroup
+constexpr int kFirLines = 8;        // columns a workgroup: 64-128 B a row
+
+__device__ __forceinline__ int mirror(int i, int n);
+
+// axis 1: lines along az, `width` consecutive rows a workgroup; axis 0: lines
+// along za, `width` adjacent columns of one plane.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void prefilter_fir_kernel(
+    cplx<T> *planes, int64_t nplanes, int nza, int naz, int axis, int width) {
+  __shared__ __align__(16) char lds[kFirLds];
+  __shared__ int bad[2][kFirLines];
+  cplx<T> *x = (cplx<T> *)lds;
+  const int n = axis == 1 ? naz : nza;
+  int64_t base;
+  int lines;
+  if (axis == 1) {
+    const int64_t l0 = (int64_t)blockIdx.x * width;
+    base = l0 * naz;
+    lines = (int)min((int64_t)width, nplanes * nza - l0);
+  } else {
+    const int nb = (int)cdiv(naz, (int64_t)width);
+    const int c0 = (int)(blockIdx.x % nb) * width;
+    base = (int64_t)(blockIdx.x / nb) * nza * naz + c0;
+    lines = min(width, naz - c0);
+  }
+  // element e of the block's lines: line w, position i
+  auto split = [&](int e, int &w, int &i) {
+    if (axis == 1) {
+      w = e / n;
+      i = e - w * n;
+    } else {
+      i = e / lines;
+      w = e - i * lines;
+    }
+  };
+  auto addr = [&](int w, int i) {
+    return planes + base + (axis == 1 ? (int64_t)w * naz + i
+                                      : (int64_t)i * naz + w);
+  };
+  for (int w = threadIdx.x; w < lines; w += kThreads) bad[0][w] = bad[1][w] = 0;
+  __syncthreads();
+  const int total = lines * n;
+  for (int e = threadIdx.x; e < total; e += kThreads) {
+    int w, i;
+    split(e, w, i);
+    const cplx<T> v = *addr(w, i);
+    x[w * n + i] = v;
+    if (!(v.re - v.re == (T)0)) bad[0][w] = 1;
+    if (!(v.im - v.im == (T)0)) bad[1][w] = 1;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < total; e += kThreads) {
+    int w, i;
+    split(e, w, i);
+    const cplx<T> *f = x + w * n;
+    double h = 1.7320508075688772, sr = h * (double)f[i].re,
+           si = h * (double)f[i].im;
+    for (int k = 1; k <= kFirReach; ++k) {
+      h *= kPole;
+      int lo = i - k, hi = i + k;
+      if (lo < 0 || hi >= n) {
+        lo = mirror(lo, n);
+        hi = mirror(hi, n);
+      }
+      sr += h * ((double)f[lo].re + (double)f[hi].re);
+      si += h * ((double)f[lo].im + (double)f[hi].im);
+    }
+    if (bad[0][w]) sr = NAN;
+    if (bad[1][w]) si = NAN;
+    *addr(w, i) = cplx<T>{(T)sr, (T)si};
+  }
+}
+
 // ---------------------------------------------------------------- geometry
 
 // (tx, ty) -> (az, za), uvbeam orientation, az in [0, 2 pi)
@@ -432,6 +516,26 @@ extern "C" int mv_beam_prefilter(void *planes, int is_f64, int64_t nplanes,
   for (int axis = 1; axis >= 0; --axis) {
     int64_t lines = nplanes * (axis == 1 ? nza : naz);
     if (lines == 0) continue;
+    // lines a workgroup holds: a row of its own, or adjacent columns so that
+    // its reads are whole segments; lines longer than LDS (3,840 complex128)
+    // run the recursion
+    const int64_t line_bytes =
+        (int64_t)(axis == 1 ? naz : nza) * (is_f64 ? 16 : 8);
+    int64_t width = axis == 1 ? 1 : kFirLines;
+    if (width > kFirLds / line_bytes) width = kFirLds / line_bytes;
+    const int64_t blocks = width < 1    ? 0
+                           : axis == 1 ? cdiv(lines, width)
+                                       : nplanes * cdiv((int64_t)naz, width);
+    if (blocks >= 1 && blocks < INT32_MAX) {
+      if (is_f64)
+        prefilter_fir_kernel<double><<<(unsigned)blocks, kThreads, 0, s>>>(
+            (cplx<double> *)planes, nplanes, nza, naz, axis, (int)width);
+      else
+        prefilter_fir_kernel<float><<<(unsigned)blocks, kThreads, 0, s>>>(
+            (cplx<float> *)planes, nplanes, nza, naz, axis, (int)width);
+      if (int e = check_launch("mv_beam_prefilter")) return e;
+      continue;
+    }
     dim3 g((unsigned)cdiv(lines, kThreads));
     if (is_f64)
       prefilter_kernel<double><<<g, kThreads, 0, s>>>(

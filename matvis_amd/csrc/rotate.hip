@@ -1,9 +1,10 @@
 // (a) Rotation of ECI source vectors into the topocentric ENU frame, fused
 // with the horizon cull and a stable (ascending-index) stream compaction.
 //
-// Compaction runs as count -> scan -> scatter.  Each block owns a fixed run of
-// kItemsPerBlock sources and re-derives the same horizon flags in both the
-// count and the scatter pass, so the output order equals the reference's
+// Compaction runs as count -> scatter, each scatter block summing the counts
+// before its own (count -> scan -> scatter beyond kScanBlocks blocks).  Each
+// block owns a fixed run of kItemsPerBlock sources and re-derives the same
+// horizon flags in both the count and the scatter pass, so the output order equals the reference's
 // `xp.where(topo[2] > 0)` order (src/matvis/core/coords.py:115) for any grid.
 #include "common.h"
 
@@ -13,6 +14,10 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kRounds = 8;
 constexpr int kItemsPerBlock = kThreads * kRounds;  // 2048 sources per block
+// Up to this many blocks (4.2M sources) a scatter block reads all counts, 8 a
+// thread from L2, instead of a launch of its own for the scan: 3-4.5 us of a
+// cull's 13-17.
+constexpr int kScanBlocks = 2048;
 
 struct Mat3 {
   double m[9];
@@ -71,7 +76,8 @@ __global__ __launch_bounds__(kThreads) void cull_count_kernel(
   }
 }
 
-// Pass 2: exclusive scan of block counts (single workgroup); total -> n_up.
+// Pass 2 of a large chunk: exclusive scan of block counts (single workgroup);
+// total -> n_up.
 __global__ __launch_bounds__(1024) void cull_scan_kernel(
     int32_t *__restrict__ counts, int64_t nblocks,
     int32_t *__restrict__ n_up) {
@@ -100,22 +106,51 @@ __global__ __launch_bounds__(1024) void cull_scan_kernel(
   if (threadIdx.x == 0) *n_up = carry;
 }
 
-// Pass 3: recompute flags, place each kept source at its block offset plus its
+// Last pass: recompute flags, place each kept source at its block offset (the
+// scanned count, or the sum of the counts before it) plus its
 // rank inside the block, then zero-fill positions [n_up, nalloc).
 template <typename T>
 __global__ __launch_bounds__(kThreads) void cull_scatter_kernel(
     const double *__restrict__ eci, int64_t ld_eci, Mat3 R,
     const double *__restrict__ flux_in, int64_t chunk0, int64_t chunk_len,
-    int64_t nalloc, const int32_t *__restrict__ offsets,
-    const int32_t *__restrict__ n_up_dev, T *__restrict__ crd, int64_t ld_crd,
+    int64_t nalloc, const int32_t *__restrict__ offsets, int scanned,
+    int32_t *__restrict__ n_up_dev, T *__restrict__ crd, int64_t ld_crd,
     T *__restrict__ flux_out, int32_t *__restrict__ idx_out,
     int64_t nblocks_real) {
   __shared__ int wave_cnt[kThreads / 64];
+  __shared__ int wave_sum[2][kThreads / 64];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
+  // where this block's sources start, and the total count
+  int64_t start = 0, n_up = 0;
+  if (scanned) {
+    if ((int64_t)blockIdx.x < nblocks_real) start = offsets[blockIdx.x];
+    n_up = *n_up_dev;
+  } else {
+    int before = 0, all = 0;
+    for (int i = threadIdx.x; i < nblocks_real; i += kThreads) {
+      const int v = offsets[i];
+      all += v;
+      if (i < (int)blockIdx.x) before += v;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      before += __shfl_down(before, off, 64);
+      all += __shfl_down(all, off, 64);
+    }
+    if (lane == 0) {
+      wave_sum[0][wave] = before;
+      wave_sum[1][wave] = all;
+    }
+    __syncthreads();
+    for (int w = 0; w < kThreads / 64; ++w) {
+      start += wave_sum[0][w];
+      n_up += wave_sum[1][w];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) *n_up_dev = (int32_t)n_up;
+  }
   if ((int64_t)blockIdx.x < nblocks_real) {
     const int64_t base = (int64_t)blockIdx.x * kItemsPerBlock;
-    int64_t run = offsets[blockIdx.x];
+    int64_t run = start;
     for (int r = 0; r < kRounds; ++r) {
       int64_t p = base + r * kThreads + threadIdx.x;
       int64_t g = chunk0 + p;
@@ -152,7 +187,6 @@ __global__ __launch_bounds__(kThreads) void cull_scatter_kernel(
     }
   }
   // zero-fill the tail [n_up, nalloc)
-  const int64_t n_up = *n_up_dev;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
   for (int64_t q = n_up + (int64_t)blockIdx.x * kThreads + threadIdx.x;
        q < nalloc; q += stride) {
@@ -309,17 +343,20 @@ extern "C" int mv_rotate_cull(const double *eci, int64_t ld_eci,
                                                         chunk_len, counts);
     if (int e = check_launch("mv_rotate_cull/count")) return e;
   }
-  cull_scan_kernel<<<1, 1024, 0, s>>>(counts, nb, n_up_dev);
-  if (int e = check_launch("mv_rotate_cull/scan")) return e;
+  const int scanned = nb > kScanBlocks;
+  if (scanned) {
+    cull_scan_kernel<<<1, 1024, 0, s>>>(counts, nb, n_up_dev);
+    if (int e = check_launch("mv_rotate_cull/scan")) return e;
+  }
   int64_t grid = nb > 0 ? nb : 1;
   if (out_is_f64)
     cull_scatter_kernel<double><<<(unsigned)grid, kThreads, 0, s>>>(
-        eci, ld_eci, R, flux_in, chunk0, chunk_len, nalloc, counts, n_up_dev,
-        (double *)crd_out, ld_crd, (double *)flux_out, idx_out, nb);
+        eci, ld_eci, R, flux_in, chunk0, chunk_len, nalloc, counts, scanned,
+        n_up_dev, (double *)crd_out, ld_crd, (double *)flux_out, idx_out, nb);
   else
     cull_scatter_kernel<float><<<(unsigned)grid, kThreads, 0, s>>>(
-        eci, ld_eci, R, flux_in, chunk0, chunk_len, nalloc, counts, n_up_dev,
-        (float *)crd_out, ld_crd, (float *)flux_out, idx_out, nb);
+        eci, ld_eci, R, flux_in, chunk0, chunk_len, nalloc, counts, scanned,
+        n_up_dev, (float *)crd_out, ld_crd, (float *)flux_out, idx_out, nb);
   return check_launch("mv_rotate_cull/scatter");
 }
 

@@ -626,3 +626,85 @@ def test_herk_phases_match_single_call(form, nterms, nprod):
           accumulate=False, nslices=cap, between=lambda s: marks.append(s))
     assert len(marks) == 1
     np.testing.assert_array_equal(_vis_full(h, v1, m), _vis_full(h, v2, m))
+
+
+# ------------------------------------------------- spline, cull, phase edges
+
+
+@pytest.mark.parametrize("nza,naz,is_f64", [(2, 2, True), (3, 31, True),
+                                            (30, 61, False), (91, 366, True),
+                                            (9, 3841, True), (3841, 9, True),
+                                            (9, 7681, False)])
+def test_prefilter_sizes(nza, naz, is_f64):
+    """B-spline coefficients against scipy's spline_filter (mirrored ends)
+    where lines are shorter than the filter's reach, about as long, and too
+    long for LDS (the recursion); a NaN spoils its plane and no other.
+    Bounds: FP64 rounding of sums of magnitude <= 3 per axis; FP32 storage
+    between the two passes."""
+    from scipy.ndimage import spline_filter
+
+    rng = np.random.default_rng(nza * naz)
+    ct = np.complex128 if is_f64 else np.complex64
+    f = (rng.normal(size=(3, nza, naz)) + 1j * rng.normal(size=(3, nza, naz))
+         ).astype(ct)
+    f[2, nza // 2, naz // 2] = np.nan
+    d = _dev(f)
+    call("mv_beam_prefilter", D.ptr(d), int(is_f64), 3, nza, naz,
+         D.stream_ptr())
+    got = D.to_host(d)
+    for p in range(2):
+        want = (spline_filter(f[p].real.astype(np.float64), 3, mode="mirror")
+                + 1j * spline_filter(f[p].imag.astype(np.float64), 3,
+                                     mode="mirror"))
+        err = np.abs(got[p] - want).max() / np.abs(want).max()
+        assert err < (1e-14 if is_f64 else 5e-7), (p, err)
+    assert np.isnan(got[2].real).all() and np.isfinite(got[:2]).all()
+
+
+@pytest.mark.parametrize("nsrc", [2048 * 2048, 2048 * 2048 + 1])
+def test_cull_at_the_scan_boundary(nsrc):
+    """The largest chunk whose scatter blocks sum the counts themselves and
+    the smallest that runs the scan: count, order and coordinates."""
+    rng = np.random.default_rng(5)
+    eci = rng.normal(size=(3, nsrc))
+    rot = np.ascontiguousarray(np.linalg.qr(rng.normal(size=(3, 3)))[0])
+    z = rot[2, 0] * eci[0] + rot[2, 1] * eci[1] + rot[2, 2] * eci[2]
+    want = np.flatnonzero(z > 0).astype(np.int32)
+    src, crd = _dev(eci), D.empty((3, nsrc), np.float64)
+    idx, nup = D.empty((nsrc,), np.int32), D.zeros((1,), np.int32)
+    ws = D.empty((lib().mv_rotate_cull_workspace_bytes(nsrc),), np.uint8)
+    call("mv_rotate_cull", D.ptr(src), nsrc, rot.ctypes.data, None, 0, nsrc,
+         nsrc, D.ptr(crd), nsrc, None, 1, D.ptr(idx), D.ptr(nup), D.ptr(ws),
+         ws.numel(), D.stream_ptr())
+    n = int(D.to_host(nup)[0])
+    got = D.to_host(idx)
+    assert n == want.size
+    assert np.array_equal(got[:n], want) and (got[n:] == -1).all()
+    assert np.array_equal(D.to_host(crd)[2, :n], z[want])
+
+
+@pytest.mark.parametrize("is_f64", [True, False])
+def test_phase_in_every_quadrant(is_f64):
+    """exp(2 pi i b.s nu / c) at multiples of 1/8 turn and around them, up to
+    +-8 turns, against extended precision: FP64 within the rounding of the
+    phase itself (32 quarter turns x 4 roundings x 1.1e-16 x pi / 2 = 2.2e-14)
+    and FP32 within the rounding of the remainder and the polynomials (3e-8 +
+    6.6e-8 + 4.6e-8 together); a non-finite position gives NaN."""
+    t = np.concatenate([np.arange(-64, 65) / 8 + d
+                        for d in (0.0, 1e-9, -1e-9, 0.013, -0.06)])
+    n = t.size
+    crd = np.zeros((3, n + 1))
+    crd[0, :n] = t / 8
+    crd[0, n] = np.inf
+    freq = 299792458.0
+    ant = _dev(np.array([[8.0, 0.0, 0.0]]))
+    ct = np.complex128 if is_f64 else np.complex64
+    dev, out = _dev(crd), D.zeros((1, n + 1), ct)
+    call("mv_exptau", D.ptr(ant), 1, freq, D.ptr(dev), 1, n + 1, n + 1,
+         D.ptr(out), int(is_f64), n + 1, D.stream_ptr())
+    got = D.to_host(out)[0]
+    ph = np.longdouble(2) * np.arccos(np.longdouble(-1)) * (
+        np.longdouble(8) * crd[0, :n].astype(np.longdouble))
+    err = np.abs(got[:n] - (np.cos(ph) + 1j * np.sin(ph))).max()
+    assert err < (2.2e-14 if is_f64 else 1.4e-7), err
+    assert np.isnan(got[n].real) and np.isnan(got[n].imag)
