@@ -1,10 +1,11 @@
 // (c) Geometric phase and the Z matrix.
 //
-// Phase: cycles = (b . s) * (freq / c) in FP64, reduced to [-1/2, 1/2] turns
-// before sincos, so the sincos argument is small whatever the baseline length
-// (the reference forms exp(i * 2 pi freq (b . s) / c) directly,
-// src/matvis/core/tau.py:30-31,65-66).  FP64 forms take an FP64 sincospi of
-// the reduced phase; FP32 and split forms take the FP32 sincospi.
+// Phase: quarter turns 4 (b . s) (freq / c) in FP64, reduced to the nearest
+// whole one and a remainder in [-1/2, 1/2] before sincos, so the sincos
+// argument is small whatever the baseline length (the reference forms
+// exp(i * 2 pi freq (b . s) / c) directly, src/matvis/core/tau.py:30-31,65-66).
+// FP64 forms evaluate sine and cosine of the remainder in FP64; FP32 and split
+// forms round it to FP32 first.
 #include "common.h"
 
 namespace mv {
@@ -16,28 +17,69 @@ constexpr int kZPad = 32;  // Z columns are zero-padded to a multiple of this
 // 32-bit index
 constexpr int64_t kMaxRow = int64_t(1) << 30;
 
-__device__ __forceinline__ double reduced_turns(const double *__restrict__ ap,
-                                                double fc, double sx,
-                                                double sy, double sz) {
-  double cyc = (ap[0] * sx + ap[1] * sy + ap[2] * sz) * fc;
-  return cyc - rint(cyc);
+// cos and sin of the angle x, |x| <= pi / 4: Taylor polynomials in FP64
+// (through x^16 and x^17: 2e-18 and 1e-19 left), in FP32 minimax fits of the
+// same form (1e-10 and 4e-9 of x left; with rounding 6.6e-8 and 4.6e-8).
+__device__ __forceinline__ void cos_sin(double x, double &c, double &s) {
+  const double u = x * x;
+  double p = 1.0 / 355687428096000.0;  // 1 / 17!
+  p = fma(p, u, -1.0 / 1307674368000.0);
+  p = fma(p, u, 1.0 / 6227020800.0);
+  p = fma(p, u, -1.0 / 39916800.0);
+  p = fma(p, u, 1.0 / 362880.0);
+  p = fma(p, u, -1.0 / 5040.0);
+  p = fma(p, u, 1.0 / 120.0);
+  p = fma(p, u, -1.0 / 6.0);
+  s = fma(x * u, p, x);
+  double q = 1.0 / 20922789888000.0;  // 1 / 16!
+  q = fma(q, u, -1.0 / 87178291200.0);
+  q = fma(q, u, 1.0 / 479001600.0);
+  q = fma(q, u, -1.0 / 3628800.0);
+  q = fma(q, u, 1.0 / 40320.0);
+  q = fma(q, u, -1.0 / 720.0);
+  q = fma(q, u, 1.0 / 24.0);
+  q = fma(q, u, -0.5);
+  c = fma(q, u, 1.0);
+}
+__device__ __forceinline__ void cos_sin(float x, float &c, float &s) {
+  const float u = x * x;
+  float p = fmaf(-0.00019517266f, u, 0.0083321779f);
+  p = fmaf(p, u, -0.16666655f);
+  s = fmaf(x * u, p, x);
+  float q = fmaf(2.4438415e-05f, u, -0.0013887367f);
+  q = fmaf(q, u, 0.041666647f);
+  q = fmaf(q, u, -0.5f);
+  c = fmaf(q, u, 1.0f);
 }
 
-template <typename TO> struct Phasor;
-template <> struct Phasor<double> {
-  __device__ static cplx<double> eval(double turns) {
-    double s, c;
-    sincospi(2.0 * turns, &s, &c);
-    return {c, s};
-  }
-};
-template <> struct Phasor<float> {
-  __device__ static cplx<float> eval(double turns) {
-    float s, c;
-    sincospif((float)(2.0 * turns), &s, &c);
-    return {c, s};
-  }
-};
+__device__ __forceinline__ double flip_sign(double x, uint32_t bit31) {
+  return __builtin_bit_cast(
+      double, __builtin_bit_cast(uint64_t, x) ^ ((uint64_t)bit31 << 32));
+}
+__device__ __forceinline__ float flip_sign(float x, uint32_t bit31) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) ^ bit31);
+}
+
+// exp(i phase) of the antenna at ap for the direction (sx, sy, sz) = s times
+// 4 freq / c: y = ap . s quarter turns are k whole ones, folded by exchanges
+// and signs, and a remainder.  Adding 1.5 2^52 rounds y to the whole number
+// that then stands in the sum's low bits (|y| < 2^51).  A phase that is not
+// finite gives NaN.
+// The general sincospi this replaces reduced the phase once more and made the
+// kernel compute-bound for one feed, where every element has its own phase:
+// 8 frequencies of 128 antennas x 30k sources, split to bf16, 70.4 us.
+template <typename T>
+__device__ __forceinline__ cplx<T> phasor(const double *__restrict__ ap,
+                                          double sx, double sy, double sz) {
+  const double y = fma(ap[0], sx, fma(ap[1], sy, ap[2] * sz));
+  const double t = y + 0x1.8p52;
+  const uint32_t q = (uint32_t)__builtin_bit_cast(uint64_t, t);
+  T c, s;
+  cos_sin((T)((y - (t - 0x1.8p52)) * (0.5 * kPi)), c, s);
+  const bool odd = q & 1u;                           // quarter turn
+  const uint32_t half = (q << 30) & 0x80000000u;     // half turn
+  return {flip_sign(odd ? -s : c, half), flip_sign(odd ? c : s, half)};
+}
 
 template <typename TC, typename TO>
 __global__ __launch_bounds__(kThreads) void exptau_kernel(
@@ -47,9 +89,10 @@ __global__ __launch_bounds__(kThreads) void exptau_kernel(
   int64_t s = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   int a = blockIdx.y;
   if (s >= nsrc) return;
-  double t = reduced_turns(antpos + 3 * a, fc, (double)crd[s],
-                           (double)crd[ld_crd + s], (double)crd[2 * ld_crd + s]);
-  out[(int64_t)a * ld_out + s] = Phasor<TO>::eval(t);
+  const double w = 4.0 * fc;
+  out[(int64_t)a * ld_out + s] =
+      phasor<TO>(antpos + 3 * a, w * (double)crd[s],
+                 w * (double)crd[ld_crd + s], w * (double)crd[2 * ld_crd + s]);
 }
 
 template <typename T>
@@ -250,9 +293,9 @@ __global__ __launch_bounds__(kThreads) void zmat_fused_kernel(
   double sx = 0.0, sy = 0.0, sz = 0.0;
   T amp = (T)0;
   if (valid) {
-    sx = crd[s];
-    sy = crd[ld_crd + s];
-    sz = crd[2 * ld_crd + s];
+    sx = 4.0 * fc * crd[s];
+    sy = 4.0 * fc * crd[ld_crd + s];
+    sz = 4.0 * fc * crd[2 * ld_crd + s];
     amp = (T)(flux[idx ? (int64_t)idx[s] : s] * scale);
   }
   int cached = -1;
@@ -268,15 +311,16 @@ __global__ __launch_bounds__(kThreads) void zmat_fused_kernel(
         // out-of-range read
         const bool ok = (unsigned)b < (unsigned)nbeam;
 #pragma unroll
-        for (int q = 0; q < nf * na; ++q)
+        for (int q = 0; q < nf * na; ++q) {
+          // the source's amplitude goes in once a beam, not once an antenna
           A[q] = ok ? beam[((int64_t)b * nf * na + q) * ld_beam + s]
                     : cplx<T>{(T)NAN, (T)NAN};
+          A[q].re *= amp;
+          A[q].im *= amp;
+        }
         cached = b;
       }
-      cplx<T> e =
-          Phasor<T>::eval(reduced_turns(antpos + 3 * a, fc, sx, sy, sz));
-      e.re *= amp;
-      e.im *= amp;
+      const cplx<T> e = phasor<T>(antpos + 3 * a, sx, sy, sz);
 #pragma unroll
       for (int q = 0; q < nf * na; ++q) out[q] = cmul(A[q], e);
     }
