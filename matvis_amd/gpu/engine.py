@@ -39,14 +39,14 @@ Z_PAD = 32  # mv_zmat_fused pads Z columns to a multiple of this
 
 
 #: device bytes the per-frequency buffers of one launch may take together
-#: (Z, split-K partials, accumulator): twice the 256 MB Infinity Cache.  Above
-#: it one frequency fills the GPU by itself (350 antennas x 100k sources: 0.7
-#: to 1.3 GB of Z, 1,000 HERK items for 512 workgroup slots).  Measured, a
+#: (Z, split-K partials, accumulator).  Near it one frequency fills the GPU by
+#: itself (350 antennas x 100k sources: 0.7 to 1.3 GB of Z, 1,000 HERK items
+#: for 512 workgroup slots).  Measured, a
 #: time with one launch per frequency and with this: 32 frequencies of 32
-#: antennas x 3k sources (one launch) 1.09 -> 0.058 ms, 16 of 128 antennas x
-#: 50k sources (two of 8) 1.08 -> 0.38 ms, 6 of 61 antennas x 20k sources in
-#: FP64 (two of 3) 0.49 -> 0.35 ms.
-BATCH_BYTES = 512 << 20
+#: antennas x 3k sources 1.09 -> 0.058 ms, 16 of 128 antennas x 50k sources
+#: 1.08 -> 0.32 ms (half the bytes, two launches of 8: 0.37), 6 of 61 antennas
+#: x 20k sources in FP64 0.49 -> 0.29 ms (two of 3: 0.35).
+BATCH_BYTES = 1 << 30
 
 
 def freq_batch(*, form: int, nterms: int, nprod: int, m: int, nax: int,
