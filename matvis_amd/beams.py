@@ -168,8 +168,10 @@ def _interp_freq(data: np.ndarray, freqs: np.ndarray, freq: float):
     return spline(data)
 
 
-def grid_planes(beam, freq: float, polarized: bool, beam_type=None):
-    """Planes of a grid beam as the device kernels take them.
+def grid_planes(beam, freq: float, polarized: bool, beam_type=None,
+                keep_precision: bool = False):
+    """Planes of a grid beam as the device kernels take them (complex128, or
+    with ``keep_precision`` as stored where nothing is computed from them).
 
     Returns ``(planes, daz, dza, azmin, is_power)`` with ``planes`` shaped
     ``(nax, nfeed, nza, naz')`` -- the ``(nbeam, nax, nfeed, nza, naz)`` layout
@@ -205,7 +207,9 @@ def grid_planes(beam, freq: float, polarized: bool, beam_type=None):
     if polarized:
         if bt != "efield" or stored != "efield":
             raise ValueError("beam type must be efield if using polarized=True")
-        planes = _interp_freq(data[:2, :2], freqs, freq).astype(np.complex128)
+        planes = _interp_freq(data[:2, :2], freqs, freq)
+        if not (keep_precision and np.iscomplexobj(planes)):
+            planes = planes.astype(np.complex128)
         is_power = False
     else:
         if stored == "efield":

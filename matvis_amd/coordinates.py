@@ -13,9 +13,9 @@ def point_source_crd_eq(ra, dec):
     """ECI unit vectors, shape (3, nsrc) (coordinates.py:174-200)."""
     ra = np.asarray(ra, dtype=np.float64)
     dec = np.asarray(dec, dtype=np.float64)
-    return np.asarray(
-        [np.cos(ra) * np.cos(dec), np.cos(dec) * np.sin(ra), np.sin(dec)]
-    )
+    cos_dec = np.cos(dec)
+    return np.asarray([np.cos(ra) * cos_dec, cos_dec * np.sin(ra),
+                       np.sin(dec)])
 
 
 def enu_to_az_za(enu_e, enu_n, orientation="astropy", periodic_azimuth=True):

@@ -31,8 +31,7 @@ from .._lib import FORM_C128, FORM_SPLIT_F16, call, lib
 from .._utils import log_progress
 from .._utils import logger as _progress_log
 from .beams import DeviceBeamSet
-from .herk import (Herk, cdiv, expand, expand_batch, is_split,
-                   split_terms_alloc)
+from .herk import Herk, cdiv, expand, expand_batch, is_split
 from .matprod import f16_scale
 
 Z_PAD = 32  # mv_zmat_fused pads Z columns to a multiple of this
@@ -47,6 +46,10 @@ Z_PAD = 32  # mv_zmat_fused pads Z columns to a multiple of this
 #: 1.08 -> 0.32 ms (half the bytes, two launches of 8: 0.37), 6 of 61 antennas
 #: x 20k sources in FP64 0.49 -> 0.29 ms (two of 3: 0.35).
 BATCH_BYTES = 1 << 30
+
+
+#: a time's output that one host thread copies
+HOST_COPY_BYTES = 4 << 20
 
 
 def freq_batch(*, form: int, nterms: int, nprod: int, m: int, nax: int,
@@ -123,7 +126,7 @@ class VisibilityEngine:
         fl = np.asarray(fluxes, dtype=np.float64).reshape(self.nsrc, -1)
         if fl.shape[1] != self.nfreq:
             raise ValueError("fluxes must have shape (NSRCS, NFREQS)")
-        self.sqrt_flux_h = np.sqrt(0.5 * fl.T)  # (nfreq, nsrc)
+        self.flux_h = fl
         self.beam_list = beam_list
         self.beam_idx = beam_idx
         self.polarized = polarized
@@ -159,12 +162,20 @@ class VisibilityEngine:
         #: the FP64 reduce that follows it is outside the pair)
         self.herk_hooks = None
 
+    @property
+    def sqrt_flux_h(self):
+        """sqrt(I / 2), (nfreq, nsrc), on the host."""
+        return np.sqrt(0.5 * self.flux_h.T)
+
     # ---------------------------------------------------------------- setup
 
     def setup(self):
         seg, nalloc = self.seg, self.nsrc_alloc
         self.antpos = D.to_dev(self.antpos_h, np.float64)
-        self.sqrt_flux = D.to_dev(self.sqrt_flux_h, np.float64)
+        # sqrt(I / 2) frequency-major: the square root (rounded to nearest,
+        # as numpy's) and the transpose on the device
+        self.sqrt_flux = torch.sqrt(
+            0.5 * D.to_dev(self.flux_h, np.float64).t()).contiguous()
         F = self.batch
         self.freqs_dev = D.to_dev(self.freqs, np.float64) if F > 1 else None
         self.beam_idx_dev = (None if self.beam_idx is None
@@ -172,8 +183,9 @@ class VisibilityEngine:
         self.pairs_dev = (None if self.pairs_h is None
                           else D.to_dev(self.pairs_h, np.int32))
         nb = self.nchunks
-        self.crd = [D.zeros((3, seg), np.float64) for _ in range(nb)]
-        self.idx = [D.zeros((seg,), np.int32) for _ in range(nb)]
+        # no buffer needs clearing: every kernel writes what later ones read
+        self.crd = list(D.empty((nb, 3, seg), np.float64))
+        self.idx = list(D.empty((nb, seg), np.int32))
         self.n_up = D.zeros((2, nb), np.int32)
         ws = lib().mv_rotate_cull_workspace_bytes(self.chunk_size)
         self.rot_ws = D.empty((ws,), np.uint8)
@@ -183,7 +195,7 @@ class VisibilityEngine:
         self.nbeam = self.beam_sets[0].nbeam
         shared = len(self.beam_sets) == 1
         nA = nb if shared else F
-        self.A = list(D.zeros((nA, self.nbeam, self.nfeed, self.nax, seg),
+        self.A = list(D.empty((nA, self.nbeam, self.nfeed, self.nax, seg),
                               self.beam_ctype))
         # Z: (m, nax, seg) complex (ldz the row stride), or nterms arrays of
         # 16-bit terms, K-tile-major (ldz the rows of a 16-column K tile;
@@ -191,15 +203,15 @@ class VisibilityEngine:
         # im x 4)
         if is_split(self.form):
             self.ldz = self.m
-            self.z = split_terms_alloc(self.nterms, self.m,
-                                       F * self.nax * seg)
+            self.z = [D.empty((F * self.nax * seg // 16, self.m, 16), np.int32)
+                      for _ in range(self.nterms)]
         else:
             self.ldz = self.nax * seg
-            self.z = [D.zeros((F * self.m, self.ldz), self.beam_ctype)]
+            self.z = [D.empty((F * self.m, self.ldz), self.beam_ctype)]
         # elements (split: words) between the Z of a launch's frequencies
         self.z_stride = self.m * self.nax * seg
         self.herk = Herk(self.form, self.m, self.nterms, self.nprod)
-        self.vaccs = D.zeros((F, self.herk.ldv, self.herk.ldv), np.complex128)
+        self.vaccs = D.empty((F, self.herk.ldv, self.herk.ldv), np.complex128)
         self.vacc = self.vaccs[0]
         self.nslices = self.herk.nslices(self.nax * nalloc)
         self.herk.workspace(self.nslices, F)
@@ -207,12 +219,14 @@ class VisibilityEngine:
         self.scales = np.ones((nb, self.nfreq))
         if self.form == FORM_SPLIT_F16:
             bmax = max(b.max_abs for b in self.beam_sets) * 1.5
+            cs = self.chunk_size
+            top = torch.stack([
+                self.sqrt_flux[:, c * cs:(c + 1) * cs].amax(1)
+                if c * cs < self.nsrc else self.sqrt_flux.new_zeros(self.nfreq)
+                for c in range(nb)]).cpu().numpy()
             for c in range(nb):
-                sl = slice(c * self.chunk_size, (c + 1) * self.chunk_size)
-                part = self.sqrt_flux_h[:, sl]
                 for f in range(self.nfreq):
-                    mx = float(part[f].max()) if part.shape[1] else 0.0
-                    self.scales[c, f] = f16_scale(mx * bmax)
+                    self.scales[c, f] = f16_scale(float(top[c, f]) * bmax)
         # Z's scales and the HERK's 1 / scale^2 on the device
         self.scales_dev = (D.to_dev(np.stack([self.scales,
                                               1.0 / self.scales ** 2]))
@@ -401,7 +415,8 @@ class VisibilityEngine:
             out = np.zeros((self.nfreq, ntimes, self.npairs, self.nfeed,
                             self.nfeed), dtype=self.ctype)
         comp = torch.cuda.current_stream()
-        copy = torch.cuda.Stream()
+        # one time has nothing to overlap its copy with
+        copy = torch.cuda.Stream() if ntimes > 1 else comp
         dev = [self.new_output(), self.new_output()]
         pin = [torch.empty(tuple(dev[0].shape), dtype=dev[0].dtype,
                            pin_memory=True) for _ in range(2)]
@@ -414,8 +429,11 @@ class VisibilityEngine:
         # the pinned -> caller copy of a time (nfreq x npairs x nfeed^2
         # elements, 157 MB at 350 antennas x 20 frequencies) in frequency
         # blocks on several host threads: one thread copies ~6 GB/s, slower
-        # than the GPU produces a time
-        nthr = max(1, min(self.nfreq, 8, os.cpu_count() or 1))
+        # than the GPU produces a time.  Up to HOST_COPY_BYTES the threads'
+        # hand-over takes longer than the copy (1.2 ms a call of 4 times of
+        # 0.35 MB)
+        nthr = (max(1, min(self.nfreq, 8, os.cpu_count() or 1))
+                if pin[0].nbytes > HOST_COPY_BYTES else 1)
         blocks = np.array_split(np.arange(self.nfreq), nthr)
         pool = ThreadPoolExecutor(nthr) if nthr > 1 else None
 
