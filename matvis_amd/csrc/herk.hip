@@ -645,9 +645,15 @@ struct SplitProblem {
   int ngroups;  // work items a slice (panel groups, or pairs)
 };
 
-// Workgroups of the split kernels: four waves on a panel group (a launch's
-// large problems), or one wave on one panel pair (small ones, tile 64).
+// Workgroups of the split kernels: four or eight waves on a panel group (a
+// launch's large problems), or one wave on one panel pair (small ones, tile
+// 64).  Three terms' stages fill the LDS with one workgroup a CU, which with
+// four waves leaves each SIMD a single one whose every wait shows: eight waves
+// then share the four pairs, each taking half the columns of a K tile, and
+// add their sums up through LDS (m = 700, 2 x 9.8k columns: 230 -> 196 us; 2 x
+// 59.7k: 1,267 -> 1,167 us; 12 chunks of a sky, 2 frequencies: 6.6 -> 5.9 ms).
 constexpr int kSP = 64;  // rows of a panel
+template <int NT> constexpr int kGroupWaves = NT == 3 ? 8 : 4;
 
 // LDS position of word w (a multiple of 4) of row r in a K-tile panel of
 // 16 words a row: the row's 16-byte chunk c is stored at chunk c ^ swz(r).
@@ -666,7 +672,7 @@ __device__ __forceinline__ int lds_word(int r, int w) {
 // kernel are separate __shared__ objects, so that the compiler sees that
 // loads in flight into one do not alias reads from the other.
 template <int NT, int WAVES> struct alignas(16) SplitStage {
-  uint32_t x[WAVES == 4 ? 4 : 2][NT][kSP * kSK];
+  uint32_t x[WAVES == 1 ? 2 : 4][NT][kSP * kSK];
 };
 
 // [x lanes 0-31 | y lanes 0-31] and [x lanes 32-63 | y lanes 32-63] of each
@@ -715,12 +721,13 @@ __device__ __forceinline__ u32x4 halves_hi(u32x4 x, u32x4 y) {
 // Measured at m = 700, 2 x 59.7k columns, 2 terms, 3 products: on panel
 // groups instead of square 128-row tiles (17 items a slice, not 21; 68 panel
 // copies, not 72) and with the row norms spread over the groups, 20
-// frequencies of the 350-antenna sky take 16.2 ms (17.6), 16 of 128
-// antennas, unpolarized, 1.08 ms (1.21); three terms on a chunked sky 6.6 ms
-// (7.3).  Norms left with their diagonal pairs: 16.4, 1.09, 7.25 ms.  Taking
-// parts out of that 680 us launch: copies and barriers alone 283 us, no
-// copies 478, neither copies nor norms 465, no norms 635; it ran 1.30M cycles
-// at 2.0 GHz, 56% of them MFMA-busy.
+// frequencies of the 350-antenna sky took 16.2 ms (17.6), three terms on a
+// chunked sky 6.6 ms (7.3); norms left with their diagonal pairs 16.4 and
+// 7.25 ms.  What bounds it now is power: 627 us, 1.17M cycles at 1.88 GHz,
+// 63% of them MFMA-busy.  Without the copies 480 us (2.10 GHz), without the
+// norms 590 (1.83), without either 456 (2.05), copies from L2 alone 610: a
+// stall taken out (operand reads a step ahead, copies spread between the
+// MFMAs, three stages) comes back as a lower clock.
 template <int NT, int MAXORD, bool F16, int WAVES>
 __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
                                            int group, int ns, int ktiles,
@@ -728,15 +735,17 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
                                            SplitStage<NT, WAVES> &L0,
                                            SplitStage<NT, WAVES> &L1) {
   typedef SplitStage<NT, WAVES> Stage;
-  constexpr int kRuns = kSP / 16;  // 16-row runs of a panel
+  constexpr int kHalves = WAVES == 8 ? 2 : 1;  // waves a pair
+  constexpr int kRuns = kSP / 16 / kHalves;    // 16-row runs a wave copies
   // the wave's index in a scalar register: what it does is uniform over it
-  const int wave =
-      WAVES == 4 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
+  const int windex =
+      WAVES > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
+  const int wave = windex & 3, half = windex >> 2;
   const int lane = threadIdx.x & 63;
   const int lr = lane & 31, lh = lane >> 5;
   WavePair wp;
   int second = -1;  // one wave stages its pair's other panel too
-  if constexpr (WAVES == 4) {
+  if constexpr (WAVES > 1) {
     wp = group_wave(group, P.nb, wave);
   } else {
     tile_coords(group, P.nb, wp.i, wp.j);
@@ -748,46 +757,45 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
   }
   const int kt0 = (int)((int64_t)slice * ktiles / ns);
   const int kt1 = (int)((int64_t)(slice + 1) * ktiles / ns);
-  // copy lanes: run u covers rows 16 u .. 16 u + 15 of the panel; lane l
-  // fills LDS chunk l % 4 of row 16 u + l / 4, i.e. logical chunk
-  // (l % 4) ^ swz(row) of that row
-  uint32_t coff[WAVES == 4 ? 1 : 2][kRuns];
+  // copy lanes: run u covers rows 16 u .. 16 u + 15 of the wave's part of the
+  // panel; lane l fills LDS chunk l % 4 of row 16 u + l / 4, i.e. logical
+  // chunk (l % 4) ^ swz(row) of that row
+  constexpr int kPanels = WAVES == 1 ? 2 : 1;  // panels a wave copies
+  const int row0 = half * kRuns * 16;
+  uint32_t coff[kPanels][kRuns];
 #pragma unroll
-  for (int q = 0; q < (WAVES == 4 ? 1 : 2); ++q)
+  for (int q = 0; q < kPanels; ++q)
 #pragma unroll
     for (int u = 0; u < kRuns; ++u) {
-      const int r = u * 16 + (lane >> 2);
+      const int r = row0 + u * 16 + (lane >> 2);
       const int row = (q ? second : wp.load) * kSP + r;
       const int c = (lane & 3) ^ swz(r);
       coff[q][u] = (uint32_t)((row < P.m ? row : P.m - 1) * kSK + 4 * c);
     }
-  // the panels whose row norms this group sums (slots, -1: none)
-  int dslot[WAVES];
-  double dsum[WAVES];
+  // the panels whose row norms this group sums (slots, -1: none); with eight
+  // waves every other of them a half
+  constexpr int kNorms = WAVES == 1 ? 1 : 4;
+  int dslot[kNorms];
+  double dsum[kNorms];
   bool any_diag = false;
 #pragma unroll
-  for (int w = 0; w < WAVES; ++w) {
-    const WavePair q = WAVES == 4 ? group_wave(group, P.nb, w) : wp;
-    dslot[w] = q.norm;
+  for (int w = 0; w < kNorms; ++w) {
+    const WavePair q = WAVES > 1 ? group_wave(group, P.nb, w) : wp;
+    dslot[w] = kHalves == 1 || (w & 1) == half ? q.norm : -1;
     any_diag = any_diag || dslot[w] >= 0;
     dsum[w] = 0.0;
   }
   double dsum1[4] = {0.0, 0.0, 0.0, 0.0};  // the one wave's
+  const int nrow = (int)(threadIdx.x & 255) >> 2;  // the row it norms
 
-  // Three terms keep their two small products in accumulators of their own
-  // (set 1): only one product a column step rounds at the size of the sum.
-  // (One workgroup a CU fits by LDS, which leaves the registers for it.)
-  constexpr int kSets = NT == 3 ? 2 : 1;
-  v16f acc_re[kSets][2][2], acc_im[kSets][2][2];
+  v16f acc_re[2][2], acc_im[2][2];
 #pragma unroll
-  for (int q = 0; q < kSets; ++q)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        acc_re[q][i][j] = v16f{};
-        acc_im[q][i][j] = v16f{};
-      }
+    for (int j = 0; j < 2; ++j) {
+      acc_re[i][j] = v16f{};
+      acc_im[i][j] = v16f{};
+    }
 
   // position of the K tile to copy next: segment sg, tile kc within it;
   // whole K tiles: columns [seg_len, round_up(seg_len, 16)) of every
@@ -800,12 +808,11 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int u = 0; u < kRuns; ++u) {
+        const int run = (row0 + u * 16) * kSK;
         if (WAVES == 1 || wp.load >= 0)
-          copy16_to_lds(P.t[t] + k0 + coff[0][u],
-                        &D.x[wave][t][u * 16 * kSK]);
+          copy16_to_lds(P.t[t] + k0 + coff[0][u], &D.x[wave][t][run]);
         if (WAVES == 1 && second >= 0)
-          copy16_to_lds(P.t[t] + k0 + coff[WAVES == 1][u],
-                        &D.x[1][t][u * 16 * kSK]);
+          copy16_to_lds(P.t[t] + k0 + coff[kPanels - 1][u], &D.x[1][t][run]);
       }
     if (++kc == kps) {
       kc = 0;
@@ -816,16 +823,16 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
   // rows 16, 32, 48 further on
   auto diag_sums = [&](const Stage &D) {
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
+    for (int w = 0; w < kNorms; ++w) {
       if (dslot[w] < 0) continue;
 #pragma unroll
-      for (int q = 0; q < 4 / WAVES; ++q) {
-        const int row = q * 16 + ((int)threadIdx.x >> 2);
+      for (int q = 0; q < (WAVES == 1 ? 4 : 1); ++q) {
+        const int row = q * 16 + nrow;
         u32x4 r[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t)
           r[t] = *(const u32x4 *)&D.x[dslot[w]][t][lds_word(row, (lane & 3) * 4)];
-        if constexpr (WAVES == 4) dsum[w] += row_norm2<NT, F16>(r);
+        if constexpr (WAVES > 1) dsum[w] += row_norm2<NT, F16>(r);
         else dsum1[q] += row_norm2<NT, F16>(r);
       }
     }
@@ -849,23 +856,16 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
       for (int j = 0; j < 2; ++j)
         b[j] = *(const u32x4 *)&base[lds_word(j * 32 + lr, w)];
     };
-    auto mma_into = [&](const u32x4 (&a)[2], const u32x4 (&b)[2],
-                        v16f (&re)[2][2], v16f (&im)[2][2]) {
+    auto mma = [&](const u32x4 (&a)[2], const u32x4 (&b)[2]) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const u32x4 y = swap_negate4(b[j]);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-          re[i][j] = SplitMfma<F16>::op(a[i], b[j], re[i][j]);
-          im[i][j] = SplitMfma<F16>::op(a[i], y, im[i][j]);
+          acc_re[i][j] = SplitMfma<F16>::op(a[i], b[j], acc_re[i][j]);
+          acc_im[i][j] = SplitMfma<F16>::op(a[i], y, acc_im[i][j]);
         }
       }
-    };
-    auto mma = [&](const u32x4 (&a)[2], const u32x4 (&b)[2]) {
-      mma_into(a, b, acc_re[0], acc_im[0]);
-    };
-    auto mma_small = [&](const u32x4 (&a)[2], const u32x4 (&b)[2]) {
-      mma_into(a, b, acc_re[kSets - 1], acc_im[kSets - 1]);
     };
     u32x4 a[2], b[2];
     if constexpr (NT == 2 && MAXORD == 1) {
@@ -897,18 +897,18 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
         mma(a, b);
       }
     } else {
+      // the wave's columns: all 16, or 8 half .. 8 half + 7
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        ld_a(0, 1, 4 * q, 4 * q, a);
-        ld_b(0, 1, 4 * q, 4 * q, b);
+      for (int p = 0; p < 4 / kHalves; ++p) {
+        const int w = 4 * (p + half * (4 / kHalves));
+        ld_a(0, 1, w, w, a);
+        ld_b(0, 1, w, w, b);
         mma(a, b);
-        ld_b(1, 0, 4 * q, 4 * q, b);
-        mma_small(a, b);
-        ld_a(0, 2, 4 * q, 4 * q, a);
-        ld_b(2, 0, 4 * q, 4 * q, b);
-        mma_small(a, b);
-        // operand reads stay in their step: hoisted they would spill
-        __builtin_amdgcn_sched_barrier(0);
+        ld_b(1, 0, w, w, b);
+        mma(a, b);
+        ld_a(0, 2, w, w, a);
+        ld_b(2, 0, w, w, b);
+        mma(a, b);
       }
     }
   };
@@ -943,19 +943,42 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
       if ((lane & 3) == 0)
         P.dpart[((int64_t)slice * P.nb + panel) * kSP + row] = s;
     };
-    if constexpr (WAVES == 4) {
+    if constexpr (WAVES > 1) {
 #pragma unroll
-      for (int w = 0; w < WAVES; ++w)
+      for (int w = 0; w < kNorms; ++w)
         if (dslot[w] >= 0)
-          store(group_wave(group, P.nb, dslot[w]).load,
-                (int)threadIdx.x >> 2, dsum[w]);
+          store(group_wave(group, P.nb, dslot[w]).load, nrow, dsum[w]);
     } else {
 #pragma unroll
       for (int q = 0; q < 4; ++q) store(wp.i, q * 16 + (lane >> 2), dsum1[q]);
     }
   }
 
-  if (WAVES == 4 && wp.i < 0) return;  // no pair, no partials
+  if constexpr (kHalves == 2) {
+    // the second halves' sums go to the first through LDS, real parts and
+    // then imaginary parts: 16 KB a wave, two waves' in each stage's memory
+    static_assert(sizeof(Stage) >= 2 * 64 * 64 * 4, "two waves' sums a stage");
+    float *sums = (wave & 2 ? (float *)&L1 : (float *)&L0) +
+                  (wave & 1) * 64 * 64 + lane;
+    auto fold = [&](v16f(&acc)[2][2]) {
+      if (half == 1) {
+#pragma unroll
+        for (int e = 0; e < 64; ++e)
+          sums[e * 64] = acc[e >> 5][(e >> 4) & 1][e & 15];
+      }
+      lds_barrier();
+      if (half == 0) {
+#pragma unroll
+        for (int e = 0; e < 64; ++e)
+          acc[e >> 5][(e >> 4) & 1][e & 15] += sums[e * 64];
+      }
+      lds_barrier();
+    };
+    fold(acc_re);
+    fold(acc_im);
+    if (half == 1) return;
+  }
+  if (WAVES > 1 && wp.i < 0) return;  // no pair, no partials
   // 32x32 accumulator layout: lane l, register r ->
   //   row 8*(r/4) + 4*(l/32) + r%4, col l%32.
   // The thread's base offset is opaque to the optimizer so that the store
@@ -973,21 +996,18 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = i * 32 + 8 * (r >> 2) + (r & 3);
-        float re = acc_re[0][i][j][r], im = acc_im[0][i][j][r];
-        if constexpr (kSets == 2) {
-          re += acc_re[1][i][j][r];
-          im += acc_im[1][i][j][r];
-        }
-        out[row * kSP + j * 32] = cplx<float>{re, im};
+        out[row * kSP + j * 32] =
+            cplx<float>{acc_re[i][j][r], acc_im[i][j][r]};
       }
 }
 
 // One split HERK: K tiles and the slice count from the device column count,
 // items (instance, slice, group) swept per XCD.
 template <int NT, int MAXORD, bool F16>
-__global__ __launch_bounds__(256, NT == 2 ? 2 : 1) void herk_split_kernel(
+__global__ __launch_bounds__(64 * kGroupWaves<NT>, 2) void herk_split_kernel(
     const SplitProblem P0, SliceCfg cfg, HerkBatch hb) {
-  __shared__ SplitStage<NT, 4> L0, L1;
+  constexpr int W = kGroupWaves<NT>;
+  __shared__ SplitStage<NT, W> L0, L1;
   SplitProblem P = P0;
   const int64_t seg_len = seg_columns(P.seg_len_host, P.seg_len_dev);
   const int kps = (int)cdiv(seg_len, (int64_t)kSK);  // K tiles per segment
@@ -1000,7 +1020,7 @@ __global__ __launch_bounds__(256, NT == 2 ? 2 : 1) void herk_split_kernel(
     for (int t = 0; t < NT; ++t) P.t[t] = P0.t[t] + b * hb.z_stride;
     P.part = (cplx<float> *)((char *)P0.part + b * hb.ws_stride);
     P.dpart = (double *)((char *)P0.dpart + b * hb.ws_stride);
-    split_item<NT, MAXORD, F16, 4>(P, (int)(i / P.ngroups),
+    split_item<NT, MAXORD, F16, W>(P, (int)(i / P.ngroups),
                                    (int)(i % P.ngroups), ns, ktiles, kps, L0,
                                    L1);
   });
@@ -1091,7 +1111,7 @@ __device__ __forceinline__ int find_segment(const T *off, int n, T x) {
 // All problems' items in one persistent launch, problem-major then
 // slice-major, swept per XCD as in the single-problem kernel.
 template <int NT, int MAXORD, bool F16, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, NT == 2 ? 2 : 1) void
+__global__ __launch_bounds__(64 * WAVES, NT == 2 || WAVES == 8 ? 2 : 1) void
 herk_split_grouped_kernel(
     const SplitProblem *__restrict__ probs, int nprob, GroupPlan plan) {
   __shared__ SplitStage<NT, WAVES> L0, L1;
@@ -1397,7 +1417,7 @@ int form_cmax(int form) {
 
 // Resident workgroups of `kernel` on the current device (CUs x blocks per
 // CU), rounded down to a multiple of the XCD count; cached per device.
-template <class K> int kernel_slots(K kernel, int block = 256) {
+template <class K> int kernel_slots(K kernel, int block) {
   static std::mutex mu;
   static std::map<std::pair<const void *, int>, int> cache;
   int dev = 0;
@@ -1421,7 +1441,7 @@ template <class K> int kernel_slots(K kernel, int block = 256) {
 // ts: side of the partial tiles (plain: of the panels), nb of them a side,
 // ntiles partial tiles and ngroups work items a slice
 struct HerkPlan {
-  int ts, nb, ntiles, ngroups, kc;
+  int ts, nb, ntiles, ngroups, kc, threads;
   SliceCfg cfg;
   int grid;
 };
@@ -1499,18 +1519,19 @@ const void *herk_kernel(int form, int nterms, int maxord, int panel) {
              : (const void *)&herk_split_kernel<3, 2, false>;
 }
 
-// The grouped kernel instantiation for (form, nterms, maxord), `WAVES`
-// waves a workgroup.
-template <int WAVES>
+// The grouped kernel instantiation for (form, nterms, maxord): panel groups,
+// or one wave a pair.
+template <bool GROUP>
 const void *grouped_kernel_t(bool f16, int nterms, int maxord) {
+  constexpr int W2 = GROUP ? kGroupWaves<2> : 1, W3 = GROUP ? kGroupWaves<3> : 1;
   if (nterms == 2 && maxord == 1)
-    return f16 ? (const void *)&herk_split_grouped_kernel<2, 1, true, WAVES>
-               : (const void *)&herk_split_grouped_kernel<2, 1, false, WAVES>;
+    return f16 ? (const void *)&herk_split_grouped_kernel<2, 1, true, W2>
+               : (const void *)&herk_split_grouped_kernel<2, 1, false, W2>;
   if (nterms == 2)
-    return f16 ? (const void *)&herk_split_grouped_kernel<2, 2, true, WAVES>
-               : (const void *)&herk_split_grouped_kernel<2, 2, false, WAVES>;
-  return f16 ? (const void *)&herk_split_grouped_kernel<3, 2, true, WAVES>
-             : (const void *)&herk_split_grouped_kernel<3, 2, false, WAVES>;
+    return f16 ? (const void *)&herk_split_grouped_kernel<2, 2, true, W2>
+               : (const void *)&herk_split_grouped_kernel<2, 2, false, W2>;
+  return f16 ? (const void *)&herk_split_grouped_kernel<3, 2, true, W3>
+             : (const void *)&herk_split_grouped_kernel<3, 2, false, W3>;
 }
 
 int plan_herk(int form, int nterms, int maxord, int m, int nslices,
@@ -1521,7 +1542,9 @@ int plan_herk(int form, int nterms, int maxord, int m, int nslices,
   p.ntiles = p.nb * (p.nb + 1) / 2;
   p.ngroups = panel_groups(p.nb);
   p.kc = plain ? kPK : kSK;
-  const int slots = kernel_slots(herk_kernel(form, nterms, maxord, p.ts));
+  p.threads = plain ? 256 : 64 * (nterms == 3 ? kGroupWaves<3> : kGroupWaves<2>);
+  const int slots =
+      kernel_slots(herk_kernel(form, nterms, maxord, p.ts), p.threads);
   if (slots <= 0) return -1;
   p.cfg = SliceCfg{nslices, slots, form_cmax(form), plain ? 2 : 4};
   const int64_t items = (int64_t)p.ngroups * nslices * nbatch;
@@ -1678,7 +1701,7 @@ int herk_run(int phases, int form, int nterms, int nprod, const void *z0,
   P.ngroups = p.ngroups;
   P.accumulate = accumulate;
 #define MV_SPLIT_LAUNCH(NT, MO, F)                                           \
-  herk_split_kernel<NT, MO, F><<<p.grid, 256, 0, st>>>(P, p.cfg, hb)
+  herk_split_kernel<NT, MO, F><<<p.grid, p.threads, 0, st>>>(P, p.cfg, hb)
   if (phases & kPhaseCompute) {
     if (nterms == 2 && maxord == 1) {
       if (f16) MV_SPLIT_LAUNCH(2, 1, true);
@@ -1860,8 +1883,8 @@ GroupLayout group_layout(int form, int ts, const mv_herk_problem *q,
 }
 
 const void *grouped_kernel(int tile, bool f16, int nterms, int maxord) {
-  return tile == 64 ? grouped_kernel_t<1>(f16, nterms, maxord)
-                    : grouped_kernel_t<4>(f16, nterms, maxord);
+  return tile == 64 ? grouped_kernel_t<false>(f16, nterms, maxord)
+                    : grouped_kernel_t<true>(f16, nterms, maxord);
 }
 }  // namespace
 
@@ -1951,7 +1974,10 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
           ? (const void *)&herk_plain_grouped_kernel<double, 32>
       : side == 64 ? (const void *)&herk_plain_grouped_kernel<float, 64>
                    : (const void *)&herk_plain_grouped_kernel<float, 32>;
-  const int threads = split && tile == 64 ? 64 : 256;
+  const int threads =
+      !split       ? 256
+      : tile == 64 ? 64
+                   : 64 * (nterms == 3 ? kGroupWaves<3> : kGroupWaves<2>);
   const int slots = kernel_slots(kernel, threads);
   if (slots <= 0) {
     set_error(MV_ERR_HIP, "mv_herk_grouped: occupancy query failed");
@@ -1998,24 +2024,24 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
                                                             plan);
     return check_launch("mv_herk_grouped/reduce");
   }
-#define MV_GROUP_LAUNCH(NT, MO, F, T)                                        \
-  herk_split_grouped_kernel<NT, MO, F, T>                                    \
+#define MV_GROUP_LAUNCH(NT, MO, F, GW)                                       \
+  herk_split_grouped_kernel<NT, MO, F, GW ? kGroupWaves<NT> : 1>             \
       <<<grid, threads, 0, st>>>(probs, nprob, plan)
-#define MV_GROUP_TILE(T)                                                     \
+#define MV_GROUP_TILE(GW)                                                    \
   if (nterms == 2 && maxord == 1) {                                          \
-    if (f16) MV_GROUP_LAUNCH(2, 1, true, T);                                 \
-    else MV_GROUP_LAUNCH(2, 1, false, T);                                    \
+    if (f16) MV_GROUP_LAUNCH(2, 1, true, GW);                                \
+    else MV_GROUP_LAUNCH(2, 1, false, GW);                                   \
   } else if (nterms == 2) {                                                  \
-    if (f16) MV_GROUP_LAUNCH(2, 2, true, T);                                 \
-    else MV_GROUP_LAUNCH(2, 2, false, T);                                    \
+    if (f16) MV_GROUP_LAUNCH(2, 2, true, GW);                                \
+    else MV_GROUP_LAUNCH(2, 2, false, GW);                                   \
   } else {                                                                   \
-    if (f16) MV_GROUP_LAUNCH(3, 2, true, T);                                 \
-    else MV_GROUP_LAUNCH(3, 2, false, T);                                    \
+    if (f16) MV_GROUP_LAUNCH(3, 2, true, GW);                                \
+    else MV_GROUP_LAUNCH(3, 2, false, GW);                                   \
   }
   if (tile == 64) {
-    MV_GROUP_TILE(1)
+    MV_GROUP_TILE(false)
   } else {
-    MV_GROUP_TILE(4)
+    MV_GROUP_TILE(true)
   }
 #undef MV_GROUP_TILE
 #undef MV_GROUP_LAUNCH
