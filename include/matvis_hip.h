@@ -395,8 +395,8 @@ int mv_herk_reduce(int form, int nterms, int nprod, const void *z0,
  * int32 column count or 0, vacc = device complex128 (ldv x ldv), scale,
  * accumulate; nslices = slice capacity given to this problem's share of the
  * workspace (mv_herk_max_slices, or more); kchain = the longest K-slice in
- * K tiles (0: the form's cap, 192 tiles for the split forms and 64 for the
- * plain ones; larger values are clamped to it): the problem runs
+ * K tiles (0: 96 tiles for the split forms and 64 for the plain ones; at most
+ * 192 and 64, larger values are clamped): the problem runs
  * ceil(K tiles / kchain) slices, at most nslices (shorter slices give a
  * small batch more work items to spread over the GPU, at the cost of more
  * partials to reduce); reserved = 0. */

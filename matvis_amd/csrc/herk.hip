@@ -1040,59 +1040,86 @@ struct GroupPlan {
 // panel grid of side ts, partial
 // areas carved from `parts` in problem order: cap x ntiles x ts^2 partial
 // elements of part_bytes each, then, with row_norms, cap x ntiles x ts FP64
-// row norms), its slice count (enough slices that no chain exceeds cmax K
-// tiles, at most its capacity: a function of the problem alone) and the
-// prefix offsets.
+// row norms), its slice count (enough slices that no chain exceeds its kchain
+// and cmax K tiles, chain0 where it names none, at most its capacity: a
+// function of the problem alone) and the prefix offsets.
 __global__ __launch_bounds__(256) void herk_group_plan_kernel(
     const mv_herk_problem *__restrict__ pub, int nprob, int ts, int panels,
-    int kc, int cmax, int part_bytes, int row_norms,
+    int kc, int cmax, int chain0, int part_bytes, int row_norms,
     SplitProblem *__restrict__ probs, char *__restrict__ parts,
     GroupPlan plan) {
-  for (int p = threadIdx.x; p < nprob; p += blockDim.x) {
-    const mv_herk_problem &q = pub[p];
+  // Prefix sums of items, partial tiles and partial bytes over the problems,
+  // 256 at a time: each thread forms its problem's in registers and the block
+  // scans them in LDS (one thread walking the descriptors took 9 us for 24
+  // problems).
+  __shared__ int64_t items_s[256], bytes_s[256];
+  __shared__ int32_t tiles_s[256];
+  int64_t items0 = 0, bytes0 = 0;
+  int32_t tiles0 = 0;
+  const int t = threadIdx.x;
+  for (int p0 = 0; p0 < nprob; p0 += 256) {
+    const int p = p0 + t;
     SplitProblem P;
-    for (int t = 0; t < 3; ++t) P.t[t] = (const uint32_t *)q.z[t];
-    P.ldz = q.ldz;
-    P.seg_stride = q.seg_stride;
-    P.seg_len_host = q.seg_len;
-    P.seg_len_dev = (const int32_t *)q.seg_len_dev;
-    P.vacc = (cplx<double> *)q.vacc;
-    P.ldv = q.ldv;
-    P.scale = q.scale;
-    P.m = q.m;
-    P.nseg = q.nseg;
-    P.accumulate = q.accumulate;
-    P.nb = icdiv(q.m, ts);
-    P.ntiles = P.nb * (P.nb + 1) / 2;
-    P.ngroups = panels ? panel_groups(P.nb) : P.ntiles;
-    P.part = nullptr;
-    P.dpart = nullptr;
-    probs[p] = P;
-    const int64_t seg_len = seg_columns(q.seg_len, P.seg_len_dev);
-    const int ktiles = (int)(cdiv(seg_len, (int64_t)kc) * q.nseg);
-    const int chain = q.kchain > 0 && q.kchain < cmax ? q.kchain : cmax;
-    int ns = ktiles > 0 ? icdiv(ktiles, chain) : 1;
-    ns = ns < 1 ? 1 : (ns > q.nslices ? q.nslices : ns);
-    plan.ns[p] = ns;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int64_t items = 0, bytes = 0;
+    int64_t items = 0, bytes = 0, own = 0;
     int32_t tiles = 0;
-    for (int p = 0; p < nprob; ++p) {
-      SplitProblem &P = probs[p];
-      const int64_t cap = pub[p].nslices;
-      P.part = (cplx<float> *)(parts + bytes);
-      bytes += cap * P.ntiles * (int64_t)ts * ts * part_bytes;
-      P.dpart = row_norms ? (double *)(parts + bytes) : nullptr;
-      if (row_norms) bytes += cap * P.nb * (int64_t)ts * 8;
-      plan.item_off[p] = items;
-      plan.tile_off[p] = tiles;
-      items += (int64_t)P.ngroups * plan.ns[p];
-      tiles += P.ntiles;
+    if (p < nprob) {
+      const mv_herk_problem &q = pub[p];
+      for (int k = 0; k < 3; ++k) P.t[k] = (const uint32_t *)q.z[k];
+      P.ldz = q.ldz;
+      P.seg_stride = q.seg_stride;
+      P.seg_len_host = q.seg_len;
+      P.seg_len_dev = (const int32_t *)q.seg_len_dev;
+      P.vacc = (cplx<double> *)q.vacc;
+      P.ldv = q.ldv;
+      P.scale = q.scale;
+      P.m = q.m;
+      P.nseg = q.nseg;
+      P.accumulate = q.accumulate;
+      P.nb = icdiv(q.m, ts);
+      P.ntiles = P.nb * (P.nb + 1) / 2;
+      P.ngroups = panels ? panel_groups(P.nb) : P.ntiles;
+      const int64_t seg_len = seg_columns(q.seg_len, P.seg_len_dev);
+      const int ktiles = (int)(cdiv(seg_len, (int64_t)kc) * q.nseg);
+      const int chain = q.kchain > 0 ? (q.kchain < cmax ? q.kchain : cmax)
+                                     : chain0;
+      int ns = ktiles > 0 ? icdiv(ktiles, chain) : 1;
+      ns = ns < 1 ? 1 : (ns > q.nslices ? q.nslices : ns);
+      plan.ns[p] = ns;
+      own = (int64_t)q.nslices * P.ntiles * ts * ts * part_bytes;
+      bytes = own + (row_norms ? (int64_t)q.nslices * P.nb * ts * 8 : 0);
+      items = (int64_t)P.ngroups * ns;
+      tiles = P.ntiles;
     }
-    plan.item_off[nprob] = items;
-    plan.tile_off[nprob] = tiles;
+    items_s[t] = items;
+    bytes_s[t] = bytes;
+    tiles_s[t] = tiles;
+    __syncthreads();
+    for (int off = 1; off < 256; off <<= 1) {
+      const int64_t i = t >= off ? items_s[t - off] : 0;
+      const int64_t b = t >= off ? bytes_s[t - off] : 0;
+      const int32_t n = t >= off ? tiles_s[t - off] : 0;
+      __syncthreads();
+      items_s[t] += i;
+      bytes_s[t] += b;
+      tiles_s[t] += n;
+      __syncthreads();
+    }
+    if (p < nprob) {
+      char *at = parts + bytes0 + bytes_s[t] - bytes;
+      P.part = (cplx<float> *)at;
+      P.dpart = row_norms ? (double *)(at + own) : nullptr;
+      probs[p] = P;
+      plan.item_off[p] = items0 + items_s[t] - items;
+      plan.tile_off[p] = tiles0 + tiles_s[t] - tiles;
+    }
+    items0 += items_s[255];
+    bytes0 += bytes_s[255];
+    tiles0 += tiles_s[255];
+    __syncthreads();
+  }
+  if (t == 0) {
+    plan.item_off[nprob] = items0;
+    plan.tile_off[nprob] = tiles0;
   }
 }
 
@@ -1414,6 +1441,13 @@ int form_cmax(int form) {
     default: return 192;
   }
 }
+
+// Longest K-slice, in K tiles, of a grouped split problem that asks for none:
+// half the accuracy limit.  Measured at 192, 96 and 64 K tiles: 24 instances
+// of 64-350 antennas 628, 408 and 391 us, two of 350 antennas 274, 229 and
+// 189, 256 that fill the GPU by themselves 20.99, 21.22 and 21.98 ms (the
+// partials of more slices).
+constexpr int kGroupChain = 96;
 
 // Resident workgroups of `kernel` on the current device (CUs x blocks per
 // CU), rounded down to a multiple of the XCD count; cached per device.
@@ -1988,13 +2022,13 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
   GroupPlan plan{(int32_t *)(ws + g.ns), (int64_t *)(ws + g.item_off),
                  (int32_t *)(ws + g.tile_off)};
   hipStream_t st = as_stream(stream);
-  // slices of a problem: split forms bound the FP32 chain (form_cmax);
-  // plain forms take slices of 64 K tiles (1024 columns) for parallelism
+  // slices of a problem that names no chain: kGroupChain K tiles; plain forms
+  // take slices of 64 K tiles (1024 columns) for parallelism
   herk_group_plan_kernel<<<1, 256, 0, st>>>(
       problems_dev, nprob, side, split && tile == 64 ? 0 : 1,
       split ? kSK : kPK,
-      split ? form_cmax(form) : 64, part_bytes(form), split ? 1 : 0, probs,
-      ws + g.parts, plan);
+      split ? form_cmax(form) : 64, split ? kGroupChain : 64,
+      part_bytes(form), split ? 1 : 0, probs, ws + g.parts, plan);
   if (int e = check_launch("mv_herk_grouped/plan")) return e;
   const int grid = (int)(max_items < slots ? max_items : slots);
   // the reduce runs over panel pairs, of which there are more than tiles

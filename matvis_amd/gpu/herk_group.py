@@ -65,6 +65,28 @@ def _addr(t) -> int:
     return 0 if t is None else int(t.data_ptr())
 
 
+def merge_tiles(form: int, nterms: int, problems: list, tiles: list) -> list:
+    """The tiles a batch runs with: its 64-row problems join the 128-row
+    launch (four-wave panel groups) when that idles few waves.  Two launches
+    one after the other each end in a tail of their own, which costs a batch
+    more than the up to three idle waves of a problem of one or two panels:
+    24 instances of 64-350 antennas 408 -> 380 us, 256 of them unchanged (20.9
+    ms).  The line lies where the idle waves' share reaches a tenth; the bits
+    of two-term results are the same in either launch, three-term ones (whose
+    group kernel halves the columns) keep the tiles asked for."""
+    tiles = [int(t) for t in tiles]
+    if not is_split(form) or nterms != 2 or len(set(tiles)) == 1:
+        return tiles
+    idle = work = 0
+    for p, t in zip(problems, tiles):
+        n = -(-p["m"] // 64)
+        pairs, cols = n * (n + 1) // 2, p["nseg"] * p["seg_len"]
+        if t == 64:  # 1 pair in a group of its own, 3 in one
+            idle += (-pairs % 4) * cols
+        work += pairs * cols
+    return [128] * len(tiles) if 10 * idle <= work else tiles
+
+
 class HerkGroup:
     """One grouped launch over problems sharing a form and a tile.
 
@@ -136,12 +158,12 @@ class HerkGroup:
 
 
 class GroupedBatch:
-    """A batch of HERK problems of one form, one grouped launch per tile class;
-    ``capture()`` records the launches in a HIP graph for ``replay()``."""
+    """A batch of HERK problems of one form, one grouped launch per tile class
+    (:func:`merge_tiles`); ``capture()`` records the launches in a HIP graph for ``replay()``."""
 
     def __init__(self, form: int, nterms: int, nprod: int, problems: list,
                  tiles: list[int], kchains: list[int] | None = None):
-        self.tiles = [int(t) for t in tiles]
+        self.tiles = merge_tiles(form, nterms, problems, tiles)
         self.kchains = ([int(k) for k in kchains] if kchains is not None
                         else None)
         classes: dict[int, list] = {}
