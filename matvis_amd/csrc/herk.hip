@@ -308,26 +308,31 @@ template <> struct PlainMfma<float> {
 };
 
 constexpr int kPT = 64;  // side the accumulator of the plain forms is padded to
-constexpr int kPK = 16;  // complex columns per LDS stage (one K tile)
+constexpr int kPK = 16;  // complex columns of a K tile as slices count them
+// Complex columns per LDS stage: 128 bytes a row.  FP64 stages of 8 columns
+// make 32 KB a workgroup, so that three share a CU (160 KB, 168 registers)
+// and the matrix cores have work while two wait for copies or operands:
+// m = 700, 29.9k sources, 16 columns and two workgroups 1.49 ms, 8 and two
+// 1.52, 8 and three 1.44 (1.27 at the rate a large FP64 product reaches).
+template <typename T> constexpr int kPStageK = sizeof(T) == 8 ? 8 : 16;
 
-// Bytes of a panel row in LDS (one K tile) and the 16-byte chunks it has.
-template <typename T> constexpr int kPRowBytes = kPK * 2 * (int)sizeof(T);
+// Bytes of a panel row in LDS (one stage) and the 16-byte chunks it has.
+template <typename T> constexpr int kPRowBytes =
+    kPStageK<T> * 2 * (int)sizeof(T);
 
 // Where column c of row r of a panel sits in LDS: rows are not padded; the
-// row's 16-byte chunks are permuted by an XOR with bits of the row, so that
-// the 16 rows (times the columns of a lane group) one operand read touches
-// fall in distinct banks: 16 chunks of one complex128 against r % 16, 8
-// chunks of two complex64 against (r / 2) % 8 (rows 2q and 2q + 1 are the two
-// halves of the 64 banks).
-template <typename T> __device__ __forceinline__ int plain_swz(int r) {
-  return sizeof(T) == 8 ? (r & 15) : ((r >> 1) & 7);
-}
+// row's eight 16-byte chunks are permuted by an XOR with (r / 2) % 8, so that
+// the rows (times the columns of a lane group) one operand read touches fall
+// in distinct banks: rows 2q and 2q + 1 are the two halves of the 64 banks.
+// A 16-byte read serves 16 lanes at a time, 8 rows of one lane group and the
+// other 8 of the next, whose chunk differs in its lowest bit (complex128).
+__device__ __forceinline__ int plain_swz(int r) { return (r >> 1) & 7; }
 template <typename T> __device__ __forceinline__ int plain_pos(int r, int c) {
   const int b = c * 2 * (int)sizeof(T);  // byte within the row
-  return r * kPRowBytes<T> + (((b >> 4) ^ plain_swz<T>(r)) << 4) + (b & 15);
+  return r * kPRowBytes<T> + (((b >> 4) ^ plain_swz(r)) << 4) + (b & 15);
 }
 
-// One K tile of a group's four panels; the two stages of a kernel are
+// One stage of a group's four panels; the two stages of a kernel are
 // separate __shared__ objects (see the split forms' stages).
 template <typename T, int P> struct alignas(16) PlainStage {
   char x[4][P * kPRowBytes<T>];
@@ -391,6 +396,7 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
                                            PlainStage<T, P> &L1) {
   typedef typename PlainMfma<T>::acc acc_t;
   typedef T vec2 __attribute__((ext_vector_type(2)));
+  constexpr int PK = kPStageK<T>;
   constexpr int RB = kPRowBytes<T>, CH = RB / 16;  // row bytes, chunks a row
   constexpr int NB = P / 16;                       // 16-row blocks a panel
   constexpr int NI = P * RB / 1024;                // 1 KB copies a panel
@@ -411,16 +417,16 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
     for (int u = 0; u < NI; ++u) {
       const int r = u * (1024 / RB) + lane / CH;
       const int gr = prow0 + r < Q.m ? prow0 + r : Q.m - 1;
-      const int c = (lane % CH) ^ plain_swz<T>(r);
+      const int c = (lane % CH) ^ plain_swz(r);
       off[u] = (uint32_t)((int64_t)gr * Q.ldz * (2 * (int)sizeof(T)) / 16) + c;
     }
   }
   int sg = kt0 / (kps > 0 ? kps : 1), kc = kt0 - sg * kps;
   auto copy = [&](PlainStage<T, P> &D) {
-    const int64_t c0 = (int64_t)kc * kPK;
+    const int64_t c0 = (int64_t)kc * PK;
     if (wp.load >= 0) {
       const cplx<T> *src = Q.z + sg * Q.seg_stride + c0;
-      if (c0 + kPK <= seg_len) {
+      if (c0 + PK <= seg_len) {
         if (Q.wide) {
 #pragma unroll
           for (int u = 0; u < NI; ++u)
@@ -434,16 +440,16 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
             const int gr = prow0 + r < Q.m ? prow0 + r : Q.m - 1;
             const char *row = (const char *)(src + (int64_t)gr * Q.ldz);
             __builtin_amdgcn_global_load_lds(
-                (const uint32_t *)(row + (((x >> 4) ^ plain_swz<T>(r)) << 4) +
+                (const uint32_t *)(row + (((x >> 4) ^ plain_swz(r)) << 4) +
                                    (x & 15)),
                 (uint32_t *)&D.x[wave][u * 256], 4, 0, 0);
           }
         }
       } else {
-        const int valid = (int)(seg_len - c0);  // 1 .. kPK - 1 columns
+        const int valid = (int)(seg_len - c0);  // 1 .. PK - 1 columns
 #pragma unroll 1
-        for (int e = lane; e < P * kPK; e += 64) {
-          const int r = e / kPK, c = e % kPK;
+        for (int e = lane; e < P * PK; e += 64) {
+          const int r = e / PK, c = e % PK;
           const int gr = prow0 + r < Q.m ? prow0 + r : Q.m - 1;
           const cplx<T> v = src[(int64_t)gr * Q.ldz + (c < valid ? c : 0)];
           *(vec2 *)&D.x[wave][plain_pos<T>(r, c)] =
@@ -470,7 +476,7 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
   auto compute = [&](const PlainStage<T, P> &D) {
     const char *A = D.x[wp.si], *B = D.x[wp.sj];
 #pragma unroll
-    for (int ks = 0; ks < kPK / 4; ++ks) {
+    for (int ks = 0; ks < PK / 4; ++ks) {
       const int pos = plain_pos<T>(rl, 4 * ks + g);
       vec2 a[NB], b[NB];
 #pragma unroll
@@ -538,15 +544,19 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
       }
 }
 
+// Workgroups a CU holds (kPStageK).
+template <typename T> constexpr int kPlainWgs = sizeof(T) == 8 ? 3 : 2;
+
 template <typename T, int P>
-__global__ __launch_bounds__(256, 2) void herk_plain_kernel(
+__global__ __launch_bounds__(256, kPlainWgs<T>) void herk_plain_kernel(
     const PlainProblem<T> Q0, int nseg, int64_t seg_len_host,
     const int32_t *__restrict__ seg_len_dev, SliceCfg cfg, HerkBatch hb) {
   __shared__ PlainStage<T, P> L0, L1;
   const int64_t seg_len = seg_columns(seg_len_host, seg_len_dev);
-  const int kps = (int)cdiv(seg_len, (int64_t)kPK);  // K tiles per segment
-  const int ktiles = kps * nseg;
-  const int ns = active_slices_wave(ktiles, Q0.ngroups, cfg);
+  const int ns = active_slices_wave((int)cdiv(seg_len, (int64_t)kPK) * nseg,
+                                    Q0.ngroups, cfg);
+  // stages per segment
+  const int kps = (int)cdiv(seg_len, (int64_t)kPStageK<T>);
   const int64_t per = (int64_t)Q0.ngroups * ns;
   for_items(per * hb.n, [&](int64_t it) {
     const int64_t b = it / per, i = it - b * per;
@@ -554,7 +564,7 @@ __global__ __launch_bounds__(256, 2) void herk_plain_kernel(
     Q.z += b * hb.z_stride;
     Q.part = (cplx<T> *)((char *)Q.part + b * hb.ws_stride);
     plain_item<T, P>(Q, seg_len, (int)(i / Q.ngroups), (int)(i % Q.ngroups),
-                     ns, ktiles, kps, L0, L1);
+                     ns, kps * nseg, kps, L0, L1);
   });
 }
 
@@ -1159,7 +1169,7 @@ herk_split_grouped_kernel(
 // Grouped plain HERK: the items of all problems, as the grouped split
 // kernel; each problem's Z is its term pointer 0.
 template <typename T, int P>
-__global__ __launch_bounds__(256, 2) void herk_plain_grouped_kernel(
+__global__ __launch_bounds__(256, kPlainWgs<T>) void herk_plain_grouped_kernel(
     const SplitProblem *__restrict__ probs, int nprob, GroupPlan plan) {
   __shared__ PlainStage<T, P> L0, L1;
   const int64_t items = plan.item_off[nprob];
@@ -1179,7 +1189,7 @@ __global__ __launch_bounds__(256, 2) void herk_plain_grouped_kernel(
     Q.wide = plain_wide(Q, S.nseg);
     const int ns = plan.ns[p];
     const int64_t local = it - plan.item_off[p];
-    const int kps = (int)cdiv(seg_len, (int64_t)kPK);
+    const int kps = (int)cdiv(seg_len, (int64_t)kPStageK<T>);
     plain_item<T, P>(Q, seg_len, (int)(local / Q.ngroups), (int)(local % Q.ngroups), ns,
                      kps * S.nseg, kps, L0, L1);
   });
