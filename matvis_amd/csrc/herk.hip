@@ -25,6 +25,7 @@
 // products are the same sums, and Y is a register reorder of X.)
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 #include "common.h"
@@ -196,21 +197,29 @@ __device__ __forceinline__ void wait_global_loads() {
 // ------------------------------------------------------------ panel groups
 
 // The upper triangle of the n x n grid of P-row panels is cut into groups of
-// at most four panel pairs (i, j), i <= j, that touch at most four panels: a
-// workgroup stages the group's panels and each of its four waves computes one
-// pair.  Every pair is in exactly one group and only the last group of a run
-// of diagonal pairs holds fewer than four, where square tiles of 2 x 2 pairs
-// leave a wave idle on every diagonal tile and two on every tile of a
-// half-empty last column (11 panels: 17 groups instead of 21 tiles).
-//   Off the diagonal: blocks I < J of two panels, all four pairs.
-//   n even, diagonal: the pairs (2I, 2I), (2I, 2I + 1), (2I + 1, 2I + 1) of
-//     I = 0, 1, ... in sequence, four a group (at most four adjacent panels).
+// panel pairs (i, j), i <= j, that touch at most four panels: a workgroup
+// stages the group's panels and its four waves compute the pairs, a pair a
+// wave or, where there are fewer than four, parts of pairs.  A wave of a
+// diagonal pair leaves out the blocks below the diagonal, and what a group
+// takes is its longest wave (a whole pair 4 quadrants, a diagonal one 3):
+//   Off the diagonal: blocks I < J of two panels, all four pairs; 4.
+//   n even, diagonal: of whole fours of blocks the pairs (2I, 2I),
+//     (2I, 2I + 1), (2I + 1, 2I + 1) in sequence, four a group (at most four
+//     adjacent panels), 4; of the last one to three blocks each block by
+//     itself, (2I, 2I + 1) as two halves, 3.
 //   n odd, last panel L = n - 1: per block (2I, 2I), (2I, 2I + 1), (2I, L),
-//     (2I + 1, L); then the pairs (2I + 1, 2I + 1) and (L, L), four a group.
+//     (2I + 1, L), 4; then the pairs (2I + 1, 2I + 1) and (L, L), four a
+//     group, 3, or the last two as halves, 2, or the last one as quadrants, 1.
+// Square tiles of 2 x 2 pairs leave a wave idle on every diagonal tile and
+// two on every tile of a half-empty last column (11 panels: 21 tiles).
+// Measured against whole pairs, four a group in sequence: m = 128 split, 2 x
+// 15k columns, 47 -> 42 us; m = 32 complex64, 3.6k columns, 9.6 -> 7.0; 6
+// frequencies of 61 antennas (m = 122) FP64, a time 283 -> 258; 24 grouped
+// instances of 64-350 antennas 458 -> 417; m = 700 1% less.
 __host__ __device__ inline int panel_groups(int n) {
   const int h = n / 2;
   const int off = h * (h - 1) / 2;
-  return (n & 1) ? off + h + icdiv(h + 1, 4) : off + icdiv(3 * h, 4);
+  return off + (n & 1 ? h + icdiv(h + 1, 4) : icdiv(3 * h, 4));
 }
 
 // Row-major index of pair (i, j), i <= j, in the upper triangle of n panels.
@@ -218,16 +227,27 @@ __host__ __device__ inline int pair_index(int i, int j, int n) {
   return i * n - i * (i - 1) / 2 + (j - i);
 }
 
+// The part of a panel pair's blocks that a wave computes, in quadrants
+// (half a panel's rows by half a panel's columns).
+enum PairPart : int {
+  kWhole,    // all four
+  kDiagonal, // a diagonal pair's: all but the one below the diagonal, and in
+             // the others no block below the diagonal
+  kTop,      // the first panel's first half
+  kBottom,   // the first panel's second half
+  kQuad00, kQuad01, kQuad11,  // one quadrant
+};
+
 // What wave w of group g does: it stages panel `load` into slot w (none if
-// negative) and computes the pair of panels (i, j), held in slots si and sj
-// (none if i is negative).
+// negative) and computes `part` of the pair of panels (i, j), held in slots
+// si and sj (none if i is negative).
 // norm: the slot of a panel whose row norms (the split forms' exact diagonal)
 // the group sums as its w-th, -1 if none.  Each panel's are summed once, by a
 // group that stages it: the work would otherwise gather in the last groups.
 // Blocks I, I + 1 off the diagonal take the odd panel of I; the even panels
 // and the last odd one stay with the group of their diagonal pair.
 struct WavePair {
-  int load, i, j, si, sj, norm;
+  int load, i, j, si, sj, norm, part;
 };
 __host__ __device__ inline WavePair group_wave(int g, int n, int w) {
   const int h = n / 2;
@@ -246,43 +266,74 @@ __host__ __device__ inline WavePair group_wave(int g, int n, int w) {
     p.j = 2 * J + (w & 1);
     p.load = w < 2 ? 2 * I + w : 2 * J + w - 2;
     p.norm = w == 1 && J == I + 1 ? 1 : -1;
+    p.part = kWhole;
     return p;
   }
   g -= off;
-  if (n & 1) {
-    const int L = n - 1;
-    if (g < h) {
-      // slots: 0 = 2g, 1 = 2g + 1, 2 = L
-      p.load = w < 2 ? 2 * g + w : (w == 2 ? L : -1);
-      p.si = w == 3 ? 1 : 0;
-      p.sj = w < 2 ? w : 2;
-      p.i = 2 * g + p.si;
-      p.j = w < 2 ? 2 * g + w : L;
-      p.norm = w == 0 ? 0 : -1;
+  if (!(n & 1)) {
+    const int fours = 3 * (h / 4);  // groups of the whole fours of blocks
+    if (g < fours) {
+      // pair s of the sequence: block s / 3, entry s % 3
+      const int s0 = 4 * g, s = s0 + w;
+      const int first = 2 * (s0 / 3) + (s0 % 3 == 2);  // row panel of pair s0
+      p.load = first + w < n ? first + w : -1;
+      p.i = 2 * (s / 3) + (s % 3 == 2);
+      p.j = 2 * (s / 3) + (s % 3 != 0);
+      p.si = p.i - first;
+      p.sj = p.j - first;
+      p.norm = s % 3 == 0 || s == 3 * h - 1 ? p.si : -1;
+      p.part = s % 3 == 1 ? kWhole : kDiagonal;
       return p;
     }
-    const int e = 4 * (g - h) + w;  // (2e + 1, 2e + 1), the last one (L, L)
-    p.load = e < h ? 2 * e + 1 : (e == h ? L : -1);
-    p.i = p.j = p.load;
-    p.si = p.sj = w;
-    p.norm = e == h - 1 || e == h ? w : -1;
+    const int I = h / 4 * 4 + g - fours;
+    p.load = w < 2 ? 2 * I + w : -1;
+    p.si = w == 1 ? 1 : 0;
+    p.sj = w == 0 ? 0 : 1;
+    p.i = 2 * I + p.si;
+    p.j = 2 * I + p.sj;
+    p.norm = w == 0 ? 0 : (w == 1 && I == h - 1 ? 1 : -1);
+    p.part = w < 2 ? kDiagonal : (w == 2 ? kTop : kBottom);
     return p;
   }
-  // pair s of the sequence: block s / 3, entry s % 3
-  const int s0 = 4 * g, s = s0 + w;
-  const int first = 2 * (s0 / 3) + (s0 % 3 == 2);  // row panel of pair s0
-  p.load = first + w < n ? first + w : -1;
-  if (s >= 3 * h) {
-    p.i = p.j = p.norm = -1;
+  const int L = n - 1;
+  if (g < h) {
+    // slots: 0 = 2g, 1 = 2g + 1, 2 = L
+    p.load = w < 2 ? 2 * g + w : (w == 2 ? L : -1);
+    p.si = w == 3 ? 1 : 0;
+    p.sj = w < 2 ? w : 2;
+    p.i = 2 * g + p.si;
+    p.j = w < 2 ? 2 * g + w : L;
+    p.norm = w == 0 ? 0 : -1;
+    p.part = w == 0 ? kDiagonal : kWhole;
+    return p;
+  }
+  // pairs e0 .. e0 + count - 1 of (2e + 1, 2e + 1), the last one (L, L)
+  const int e0 = 4 * (g - h);
+  const int count = h + 1 - e0 < 4 ? h + 1 - e0 : 4;
+  const int s = count > 2 ? w : (count == 2 ? w >> 1 : 0);  // the wave's pair
+  p.load = w < count ? (e0 + w < h ? 2 * (e0 + w) + 1 : L) : -1;
+  p.norm = w < count && e0 + w >= h - 1 ? w : -1;
+  p.si = p.sj = s;
+  p.i = e0 + s < h ? 2 * (e0 + s) + 1 : L;
+  p.part = count > 2 ? kDiagonal
+           : count == 2 ? (w & 1 ? kQuad11 : kTop)
+                        : (w == 0 ? kQuad00 : (w == 1 ? kQuad01 : kQuad11));
+  if (s >= count || (count == 1 && w == 3)) {
+    p.i = -1;
     p.si = p.sj = 0;
-    return p;
+    p.part = kQuad11;
   }
-  p.i = 2 * (s / 3) + (s % 3 == 2);
-  p.j = 2 * (s / 3) + (s % 3 != 0);
-  p.si = p.i - first;
-  p.sj = p.j - first;
-  p.norm = p.i == p.j && (s % 3 == 0 || s == 3 * h - 1) ? p.si : -1;
+  p.j = p.i;
   return p;
+}
+template <int V> using Int = std::integral_constant<int, V>;
+
+// First row and column quadrant of a part.
+__host__ __device__ inline int part_row(int part) {
+  return part == kBottom || part == kQuad11 ? 1 : 0;
+}
+__host__ __device__ inline int part_col(int part) {
+  return part >= kQuad01 ? 1 : 0;
 }
 
 // ------------------------------------------------------------ plain forms
@@ -463,85 +514,105 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
     }
   };
 
-  constexpr int kSets = sizeof(T) == 4 && P == 32 ? 2 : 1;
-  acc_t t1[kSets][NB][NB], t2[kSets][NB][NB], t3[kSets][NB][NB];
+  // The K loop of a wave that computes NI rows and NJ columns of blocks from
+  // (oi, oj), without those below the diagonal where DIAG.  A loop for each
+  // part: the waves of a group run different ones, with the same barriers.
+  // (Branches around the parts' MFMAs within one loop spill accumulators.)
+  auto run = [&](auto ni_, auto nj_, auto diag_, int oi, int oj) {
+    constexpr int NI = decltype(ni_)::value, NJ = decltype(nj_)::value;
+    constexpr bool DIAG = decltype(diag_)::value;
+    constexpr int kSets = sizeof(T) == 4 && P == 32 ? 2 : 1;
+    acc_t t1[kSets][NI][NJ], t2[kSets][NI][NJ], t3[kSets][NI][NJ];
 #pragma unroll
-  for (int q = 0; q < kSets; ++q)
+    for (int q = 0; q < kSets; ++q)
 #pragma unroll
-    for (int i = 0; i < NB; ++i)
+      for (int i = 0; i < NI; ++i)
 #pragma unroll
-      for (int j = 0; j < NB; ++j)
-        t1[q][i][j] = t2[q][i][j] = t3[q][i][j] = acc_t{};
+        for (int j = 0; j < NJ; ++j)
+          t1[q][i][j] = t2[q][i][j] = t3[q][i][j] = acc_t{};
 
-  auto compute = [&](const PlainStage<T, P> &D) {
-    const char *A = D.x[wp.si], *B = D.x[wp.sj];
+    auto compute = [&](const PlainStage<T, P> &D) {
+      const char *A = D.x[wp.si] + oi * 16 * RB, *B = D.x[wp.sj] + oj * 16 * RB;
 #pragma unroll
-    for (int ks = 0; ks < PK / 4; ++ks) {
-      const int pos = plain_pos<T>(rl, 4 * ks + g);
-      vec2 a[NB], b[NB];
+      for (int ks = 0; ks < PK / 4; ++ks) {
+        const int pos = plain_pos<T>(rl, 4 * ks + g);
+        vec2 a[NI], b[NJ];
 #pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        a[i] = *(const vec2 *)&A[i * 16 * RB + pos];
-        b[i] = *(const vec2 *)&B[i * 16 * RB + pos];
+        for (int i = 0; i < NI; ++i)
+          a[i] = *(const vec2 *)&A[i * 16 * RB + pos];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+          b[j] = *(const vec2 *)&B[j * 16 * RB + pos];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int i = 0; i < NI; ++i) {
+            if (DIAG && i > j) continue;
+            constexpr int S = kSets - 1;
+            acc_t &x = t1[ks & S][i][j], &y = t2[ks & S][i][j],
+                  &z = t3[ks & S][i][j];
+            x = PlainMfma<T>::op(a[i][0], b[j][0], x);
+            y = PlainMfma<T>::op(a[i][1], b[j][1], y);
+            z = PlainMfma<T>::op(a[i][0] - a[i][1], b[j][0] + b[j][1], z);
+          }
+        // operand reads stay in their step: hoisted over the unrolled steps
+        // they would spill (the other waves of the SIMD cover their latency)
+        __builtin_amdgcn_sched_barrier(0);
       }
-#pragma unroll
-      for (int j = 0; j < NB; ++j)
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-          constexpr int S = kSets - 1;
-          acc_t &x = t1[ks & S][i][j], &y = t2[ks & S][i][j],
-                &z = t3[ks & S][i][j];
-          x = PlainMfma<T>::op(a[i][0], b[j][0], x);
-          y = PlainMfma<T>::op(a[i][1], b[j][1], y);
-          z = PlainMfma<T>::op(a[i][0] - a[i][1], b[j][0] + b[j][1], z);
-        }
-      // operand reads stay in their step: hoisted over the unrolled steps
-      // they would spill (the other wave of the SIMD covers their latency)
-      __builtin_amdgcn_sched_barrier(0);
+    };
+    // one stage computed from C while the next is copied into N
+    auto step = [&](PlainStage<T, P> &C, PlainStage<T, P> &N, int kt) {
+      if (kt + 1 < kt1) copy(N);
+      if (wp.i >= 0) compute(C);
+      wait_global_loads();  // this wave's copies into N
+      lds_barrier();
+    };
+    for (int kt = kt0; kt < kt1; kt += 2) {
+      step(L0, L1, kt);
+      if (kt + 1 < kt1) step(L1, L0, kt + 1);
     }
-  };
-  // one K tile computed from stage C while the next is copied into N
-  auto step = [&](PlainStage<T, P> &C, PlainStage<T, P> &N, int kt) {
-    if (kt + 1 < kt1) copy(N);
-    if (wp.i >= 0) compute(C);
-    wait_global_loads();  // this wave's copies into N
-    lds_barrier();
+    // every wave is past the last barrier: LDS is free for the next item
+
+    if (wp.i < 0) return;
+    // 16x16 accumulator: lane l = 16 g + rl, register r -> row
+    // PlainMfma<T>::row(g, r), column rl
+    // (the base is opaque so that the store addresses are formed here)
+    cplx<T> *out = Q.part + ((int64_t)slice * Q.npairs +
+                             pair_index(wp.i, wp.j, Q.n)) * P * P;
+    int obase =
+        (PlainMfma<T>::row(g, 0) + oi * 16) * P + rl + oj * 16;
+    asm volatile("" : "+v"(obase));
+    out += obase;
+    constexpr int rstep = PlainMfma<T>::kRowStep * P;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        if (DIAG && i > j) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          T x = t1[0][i][j][r], y = t2[0][i][j][r], w = t3[0][i][j][r];
+          if constexpr (kSets == 2) {
+            x += t1[1][i][j][r];
+            y += t2[1][i][j][r];
+            w += t3[1][i][j][r];
+          }
+          out[i * 16 * P + r * rstep + j * 16] = cplx<T>{x + y, (w - x) + y};
+        }
+      }
   };
 
   if (kt0 < kt1) copy(L0);
   wait_global_loads();
   lds_barrier();
-  for (int kt = kt0; kt < kt1; kt += 2) {
-    step(L0, L1, kt);
-    if (kt + 1 < kt1) step(L1, L0, kt + 1);
-  }
-  // every wave is past the last barrier: LDS is free for the next item
-
-  if (wp.i < 0) return;
-  // 16x16 accumulator: lane l = 16 g + rl, register r -> row
-  // PlainMfma<T>::row(g, r), column rl
-  // (the base is opaque so that the store addresses are formed here)
-  cplx<T> *out = Q.part +
-                 ((int64_t)slice * Q.npairs + pair_index(wp.i, wp.j, Q.n)) * P * P;
-  int obase = PlainMfma<T>::row(g, 0) * P + rl;
-  asm volatile("" : "+v"(obase));
-  out += obase;
-  constexpr int rstep = PlainMfma<T>::kRowStep * P;
-#pragma unroll
-  for (int i = 0; i < NB; ++i)
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        T x = t1[0][i][j][r], y = t2[0][i][j][r], w = t3[0][i][j][r];
-        if constexpr (kSets == 2) {
-          x += t1[1][i][j][r];
-          y += t2[1][i][j][r];
-          w += t3[1][i][j][r];
-        }
-        out[i * 16 * P + r * rstep + j * 16] =
-            cplx<T>{x + y, (w - x) + y};
-      }
+  constexpr int HB = NB / 2;  // blocks a quadrant's side
+  constexpr Int<NB> whole{};
+  constexpr Int<HB> half{};
+  const int oi = part_row(wp.part) * HB, oj = part_col(wp.part) * HB;
+  if (wp.part == kWhole) run(whole, whole, Int<0>{}, 0, 0);
+  else if (wp.part == kDiagonal) run(whole, whole, Int<1>{}, 0, 0);
+  else if (wp.part <= kBottom) run(half, whole, Int<0>{}, oi, 0);
+  else run(half, half, Int<0>{}, oi, oj);
 }
 
 // Workgroups a CU holds (kPStageK).
@@ -763,6 +834,7 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
     wp.si = 0;
     wp.sj = wp.i == wp.j ? 0 : 1;
     wp.norm = wp.i == wp.j ? 0 : -1;
+    wp.part = wp.i == wp.j ? kDiagonal : kWhole;
     if (wp.i != wp.j) second = wp.j;
   }
   const int kt0 = (int)((int64_t)slice * ktiles / ns);
@@ -797,15 +869,6 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
   }
   double dsum1[4] = {0.0, 0.0, 0.0, 0.0};  // the one wave's
   const int nrow = (int)(threadIdx.x & 255) >> 2;  // the row it norms
-
-  v16f acc_re[2][2], acc_im[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      acc_re[i][j] = v16f{};
-      acc_im[i][j] = v16f{};
-    }
 
   // position of the K tile to copy next: segment sg, tile kc within it;
   // whole K tiles: columns [seg_len, round_up(seg_len, 16)) of every
@@ -847,105 +910,7 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
       }
     }
   };
-  // the MFMAs of one K tile from stage D
-  auto compute = [&](const Stage &D) {
-    const uint32_t(*Ax)[kSP * kSK] = D.x[wp.si];
-    const uint32_t(*Bx)[kSP * kSK] = D.x[wp.sj];
-    // lane half lh reads term t_lh at word offset w_lh of its row
-    auto ld_a = [&](int t0, int t1, int w0, int w1, u32x4 (&a)[2]) {
-      const uint32_t *base = Ax[lh ? t1 : t0];
-      const int w = lh ? w1 : w0;
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        a[i] = *(const u32x4 *)&base[lds_word(i * 32 + lr, w)];
-    };
-    auto ld_b = [&](int t0, int t1, int w0, int w1, u32x4 (&b)[2]) {
-      const uint32_t *base = Bx[lh ? t1 : t0];
-      const int w = lh ? w1 : w0;
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        b[j] = *(const u32x4 *)&base[lds_word(j * 32 + lr, w)];
-    };
-    auto mma = [&](const u32x4 (&a)[2], const u32x4 (&b)[2]) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const u32x4 y = swap_negate4(b[j]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          acc_re[i][j] = SplitMfma<F16>::op(a[i], b[j], acc_re[i][j]);
-          acc_im[i][j] = SplitMfma<F16>::op(a[i], y, acc_im[i][j]);
-        }
-      }
-    };
-    u32x4 a[2], b[2];
-    if constexpr (NT == 2 && MAXORD == 1) {
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        u32x4 a1[2], b1[2];
-        ld_a(0, 1, 8 * ks, 8 * ks, a);  // [hi|lo] of columns 8ks..8ks+3
-        ld_b(1, 0, 8 * ks, 8 * ks, b);  // [lo|hi]
-        mma(a, b);
-        ld_a(0, 1, 8 * ks + 4, 8 * ks + 4, a1);
-        ld_b(1, 0, 8 * ks + 4, 8 * ks + 4, b1);
-        mma(a1, b1);
-        // hi of columns 8ks..8ks+3 in lanes 0-31 and of 8ks+4..8ks+7 in
-        // lanes 32-63, for A and B alike
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          a[i] = halves_lo(a[i], a1[i]);
-          b[i] = halves_hi(b[i], b1[i]);
-        }
-        mma(a, b);
-      }
-    } else if constexpr (NT == 2) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        ld_a(0, 1, 4 * q, 4 * q, a);
-        ld_b(0, 1, 4 * q, 4 * q, b);
-        mma(a, b);
-        ld_b(1, 0, 4 * q, 4 * q, b);
-        mma(a, b);
-      }
-    } else {
-      // the wave's columns: all 16, or 8 half .. 8 half + 7
-#pragma unroll
-      for (int p = 0; p < 4 / kHalves; ++p) {
-        const int w = 4 * (p + half * (4 / kHalves));
-        ld_a(0, 1, w, w, a);
-        ld_b(0, 1, w, w, b);
-        mma(a, b);
-        ld_b(1, 0, w, w, b);
-        mma(a, b);
-        ld_a(0, 2, w, w, a);
-        ld_b(2, 0, w, w, b);
-        mma(a, b);
-      }
-    }
-  };
-  // one K tile computed from stage C while the next is copied into N
-  auto step = [&](Stage &C, Stage &N, int kt) {
-    if (kt + 1 < kt1) copy(N);
-    if (any_diag) diag_sums(C);
-    if (WAVES == 1 || wp.i >= 0) {
-      // issue priority to waves in their MFMA phase over waves copying or
-      // waiting at the barrier
-      __builtin_amdgcn_s_setprio(1);
-      compute(C);
-      __builtin_amdgcn_s_setprio(0);
-    }
-    wait_global_loads();  // this wave's copies into N
-    lds_barrier();
-  };
-
-  if (kt0 < kt1) copy(L0);
-  wait_global_loads();
-  lds_barrier();
-  for (int kt = kt0; kt < kt1; kt += 2) {
-    step(L0, L1, kt);
-    if (kt + 1 < kt1) step(L1, L0, kt + 1);
-  }
-  // every wave is past the last barrier: LDS is free for the next item
-  if (any_diag) {
+  auto store_norms = [&]() {
     // the four threads of a row are lanes 4 q .. 4 q + 3
     auto store = [&](int panel, int row, double s) {
       s += __shfl_xor(s, 1, 64);
@@ -962,53 +927,179 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
 #pragma unroll
       for (int q = 0; q < 4; ++q) store(wp.i, q * 16 + (lane >> 2), dsum1[q]);
     }
-  }
+  };
+  // The K loop of a wave that computes NI x NJ blocks from block (oi, oj),
+  // without the one below the diagonal where DIAG.  A loop for each part: the
+  // waves of a group run different ones, with the same barriers.  (Branches
+  // around the parts' MFMAs within one loop spill accumulators.)
+  auto run = [&](auto ni_, auto nj_, auto diag_, int oi, int oj) {
+    constexpr int NI = decltype(ni_)::value, NJ = decltype(nj_)::value;
+    constexpr bool DIAG = decltype(diag_)::value;
+    v16f acc_re[NI][NJ], acc_im[NI][NJ];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        acc_re[i][j] = v16f{};
+        acc_im[i][j] = v16f{};
+      }
 
-  if constexpr (kHalves == 2) {
-    // the second halves' sums go to the first through LDS, real parts and
-    // then imaginary parts: 16 KB a wave, two waves' in each stage's memory
-    static_assert(sizeof(Stage) >= 2 * 64 * 64 * 4, "two waves' sums a stage");
-    float *sums = (wave & 2 ? (float *)&L1 : (float *)&L0) +
-                  (wave & 1) * 64 * 64 + lane;
-    auto fold = [&](v16f(&acc)[2][2]) {
-      if (half == 1) {
+    // the MFMAs of one K tile from stage D
+    auto compute = [&](const Stage &D) {
+      const uint32_t(*Ax)[kSP * kSK] = D.x[wp.si];
+      const uint32_t(*Bx)[kSP * kSK] = D.x[wp.sj];
+      // lane half lh reads term t_lh at word offset w_lh of its row
+      auto ld_a = [&](int t0, int t1, int w0, int w1, u32x4 (&a)[NI]) {
+        const uint32_t *base = Ax[lh ? t1 : t0] + oi * 32 * kSK;
+        const int w = lh ? w1 : w0;
 #pragma unroll
-        for (int e = 0; e < 64; ++e)
-          sums[e * 64] = acc[e >> 5][(e >> 4) & 1][e & 15];
-      }
-      lds_barrier();
-      if (half == 0) {
+        for (int i = 0; i < NI; ++i)
+          a[i] = *(const u32x4 *)&base[lds_word(i * 32 + lr, w)];
+      };
+      auto ld_b = [&](int t0, int t1, int w0, int w1, u32x4 (&b)[NJ]) {
+        const uint32_t *base = Bx[lh ? t1 : t0] + oj * 32 * kSK;
+        const int w = lh ? w1 : w0;
 #pragma unroll
-        for (int e = 0; e < 64; ++e)
-          acc[e >> 5][(e >> 4) & 1][e & 15] += sums[e * 64];
+        for (int j = 0; j < NJ; ++j)
+          b[j] = *(const u32x4 *)&base[lds_word(j * 32 + lr, w)];
+      };
+      auto mma = [&](const u32x4 (&a)[NI], const u32x4 (&b)[NJ]) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const u32x4 y = swap_negate4(b[j]);
+#pragma unroll
+          for (int i = 0; i < NI; ++i) {
+            if (DIAG && i > j) continue;
+            acc_re[i][j] = SplitMfma<F16>::op(a[i], b[j], acc_re[i][j]);
+            acc_im[i][j] = SplitMfma<F16>::op(a[i], y, acc_im[i][j]);
+          }
+        }
+      };
+      u32x4 a[NI], b[NJ];
+      if constexpr (NT == 2 && MAXORD == 1) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          u32x4 a1[NI], b1[NJ];
+          ld_a(0, 1, 8 * ks, 8 * ks, a);  // [hi|lo] of columns 8ks..8ks+3
+          ld_b(1, 0, 8 * ks, 8 * ks, b);  // [lo|hi]
+          mma(a, b);
+          ld_a(0, 1, 8 * ks + 4, 8 * ks + 4, a1);
+          ld_b(1, 0, 8 * ks + 4, 8 * ks + 4, b1);
+          mma(a1, b1);
+          // hi of columns 8ks..8ks+3 in lanes 0-31 and of 8ks+4..8ks+7 in
+          // lanes 32-63, for A and B alike
+#pragma unroll
+          for (int i = 0; i < NI; ++i) a[i] = halves_lo(a[i], a1[i]);
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) b[j] = halves_hi(b[j], b1[j]);
+          mma(a, b);
+        }
+      } else if constexpr (NT == 2) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          ld_a(0, 1, 4 * q, 4 * q, a);
+          ld_b(0, 1, 4 * q, 4 * q, b);
+          mma(a, b);
+          ld_b(1, 0, 4 * q, 4 * q, b);
+          mma(a, b);
+        }
+      } else {
+        // the wave's columns: all 16, or 8 half .. 8 half + 7
+#pragma unroll
+        for (int p = 0; p < 4 / kHalves; ++p) {
+          const int w = 4 * (p + half * (4 / kHalves));
+          ld_a(0, 1, w, w, a);
+          ld_b(0, 1, w, w, b);
+          mma(a, b);
+          ld_b(1, 0, w, w, b);
+          mma(a, b);
+          ld_a(0, 2, w, w, a);
+          ld_b(2, 0, w, w, b);
+          mma(a, b);
+        }
       }
+    };
+    // one K tile computed from stage C while the next is copied into N
+    auto step = [&](Stage &C, Stage &N, int kt) {
+      if (kt + 1 < kt1) copy(N);
+      if (any_diag) diag_sums(C);
+      if (WAVES == 1 || wp.i >= 0) {
+        // issue priority to waves in their MFMA phase over waves copying or
+        // waiting at the barrier
+        __builtin_amdgcn_s_setprio(1);
+        compute(C);
+        __builtin_amdgcn_s_setprio(0);
+      }
+      wait_global_loads();  // this wave's copies into N
       lds_barrier();
     };
-    fold(acc_re);
-    fold(acc_im);
-    if (half == 1) return;
-  }
-  if (WAVES > 1 && wp.i < 0) return;  // no pair, no partials
-  // 32x32 accumulator layout: lane l, register r ->
-  //   row 8*(r/4) + 4*(l/32) + r%4, col l%32.
-  // The thread's base offset is opaque to the optimizer so that the store
-  // addresses are formed here rather than kept live across the K loop.
-  cplx<float> *out =
-      P.part + ((int64_t)slice * P.ntiles + pair_index(wp.i, wp.j, P.nb)) *
-                   kSP * kSP;
-  int obase = 4 * lh * kSP + lr;
-  asm volatile("" : "+v"(obase));
-  out += obase;
+
+    for (int kt = kt0; kt < kt1; kt += 2) {
+      step(L0, L1, kt);
+      if (kt + 1 < kt1) step(L1, L0, kt + 1);
+    }
+    // every wave is past the last barrier: LDS is free for the next item
+    if (any_diag) store_norms();
+
+    if constexpr (kHalves == 2) {
+      // the second halves' sums go to the first through LDS, real parts and
+      // then imaginary parts: 16 KB a wave, two waves' in each stage's memory
+      static_assert(sizeof(Stage) >= 2 * 64 * 64 * 4, "two waves' sums a stage");
+      float *sums = (wave & 2 ? (float *)&L1 : (float *)&L0) +
+                    (wave & 1) * 64 * 64 + lane;
+      auto fold = [&](v16f(&acc)[NI][NJ]) {
+        if (half == 1) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+          for (int e = 0; e < NI * NJ * 16; ++e)
+            sums[e * 64] = acc[(e >> 4) / NJ][(e >> 4) % NJ][e & 15];
+        }
+        lds_barrier();
+        if (half == 0) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+          for (int e = 0; e < NI * NJ * 16; ++e)
+            acc[(e >> 4) / NJ][(e >> 4) % NJ][e & 15] += sums[e * 64];
+        }
+        lds_barrier();
+      };
+      fold(acc_re);
+      fold(acc_im);
+      if (half == 1) return;
+    }
+    if (WAVES > 1 && wp.i < 0) return;  // no pair, no partials
+    // 32x32 accumulator layout: lane l, register r ->
+    //   row 8*(r/4) + 4*(l/32) + r%4, col l%32.
+    // The thread's base offset is opaque to the optimizer so that the store
+    // addresses are formed here rather than kept live across the K loop.
+    cplx<float> *out =
+        P.part + ((int64_t)slice * P.ntiles + pair_index(wp.i, wp.j, P.nb)) *
+                     kSP * kSP;
+    int obase = (4 * lh + oi * 32) * kSP + lr + oj * 32;
+    asm volatile("" : "+v"(obase));
+    out += obase;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = i * 32 + 8 * (r >> 2) + (r & 3);
-        out[row * kSP + j * 32] =
-            cplx<float>{acc_re[i][j][r], acc_im[i][j][r]};
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        if (DIAG && i > j) continue;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int row = i * 32 + 8 * (r >> 2) + (r & 3);
+          out[row * kSP + j * 32] =
+              cplx<float>{acc_re[i][j][r], acc_im[i][j][r]};
+        }
       }
+  };
+
+  if (kt0 < kt1) copy(L0);
+  wait_global_loads();
+  lds_barrier();
+  const int oi = part_row(wp.part), oj = part_col(wp.part);
+  if (wp.part == kWhole) run(Int<2>{}, Int<2>{}, Int<0>{}, 0, 0);
+  else if (wp.part == kDiagonal) run(Int<2>{}, Int<2>{}, Int<1>{}, 0, 0);
+  else if constexpr (WAVES > 1) {
+    if (wp.part <= kBottom) run(Int<1>{}, Int<2>{}, Int<0>{}, oi, 0);
+    else run(Int<1>{}, Int<1>{}, Int<0>{}, oi, oj);
+  }
 }
 
 // One split HERK: K tiles and the slice count from the device column count,
@@ -1209,6 +1300,8 @@ __global__ __launch_bounds__(256, kPlainWgs<T>) void herk_plain_grouped_kernel(
 // group.  The chains combine in a fixed order, ((c0 + c1) + (c2 + c3)) +
 // ((c4 + c5) + (c6 + c7)); lane half h then stores element h of the group.
 // (Four elements a lane halve the grid and measured slower.)
+// Below the diagonal of a diagonal tile nothing is read (the compute kernels
+// leave its blocks out): what is above it is stored there too, conjugated.
 template <typename TP> constexpr int kReduceEpt = 2;
 
 // The first element of the calling lane's group and its lane half.
@@ -1230,6 +1323,17 @@ __device__ __forceinline__ void reduce_elems_t(
   static_assert(E == 2, "lane half h stores element h of its group");
   const int64_t tsz = (int64_t)ts * ts;
   const int64_t r = e / ts, c = e % ts;
+  if (bi == bj && r > c + 1) return;  // both lane halves
+  // what is accumulated onto is loaded before the sums, not waited for after
+  cplx<double> *tile0 = vacc + (int64_t)bi * ts * ldv + (int64_t)bj * ts;
+  cplx<double> *dst = tile0 + r * ldv + c + h;
+  cplx<double> *mirror = tile0 + (c + h) * ldv + r;
+  const bool above = bi != bj || r <= c + h, mirrored = bi == bj && r < c + h;
+  cplx<double> old = {0.0, 0.0}, old_m = {0.0, 0.0};
+  if (accumulate) {
+    if (above) old = *dst;
+    if (mirrored) old_m = *mirror;
+  }
   const cplx<TP> *src = part + (int64_t)tile * tsz + e;
   const int64_t step = (int64_t)ntiles * tsz;
   // diagonal tiles (DTILE) also sum the row norms of the group's row, in the
@@ -1299,13 +1403,14 @@ __device__ __forceinline__ void reduce_elems_t(
   } else if (bi == bj && r == c + h) {
     vi -= vi;  // the diagonal is real: 0, or NaN where it is not finite
   }
-  cplx<double> *dst =
-      vacc + ((int64_t)bi * ts + r) * ldv + (int64_t)bj * ts + c + h;
+  vr *= scale;
+  vi *= scale;
   if (accumulate) {
-    dst->re += vr * scale;
-    dst->im += vi * scale;
+    if (above) *dst = cplx<double>{old.re + vr, old.im + vi};
+    if (mirrored) *mirror = cplx<double>{old_m.re + vr, old_m.im - vi};
   } else {
-    *dst = cplx<double>{vr * scale, vi * scale};
+    if (above) *dst = cplx<double>{vr, vi};
+    if (mirrored) *mirror = cplx<double>{vr, -vi};
   }
 }
 

@@ -533,6 +533,38 @@ def test_herk_split_panel_edges(m, nterms, nprod, bound):
     assert diag < (6e-6 if nterms == 2 else 1.2e-7), diag
 
 
+@pytest.mark.parametrize("form,nterms,nprod", [
+    (FORM_C128, 1, 1), (FORM_C64, 1, 1), (FORM_SPLIT_BF16, 2, 3),
+    (FORM_SPLIT_BF16, 3, 6)])
+@pytest.mark.parametrize("m", [17, 33, 65, 97, 129, 257, 449, 577])
+def test_herk_diagonal_tiles_are_hermitian(m, form, nterms, nprod):
+    """Each way a group's waves share its panel pairs (whole, diagonal, halves,
+    quadrants: 1 to 19 panels): the accumulator's diagonal 32-row blocks hold
+    the conjugates below the diagonal, bit for bit, and accumulating the same
+    product again doubles every element, exactly."""
+    from matvis_amd.gpu.herk import Herk
+    k = 90
+    z = _herk_case(m, k, np.complex128 if form == FORM_C128 else np.complex64,
+                   seed=m)
+    if nterms == 1:
+        zs, ldz, cols = [_dev(z)], k, k
+    else:
+        zs, cols = _split_terms(z, form, nterms)
+        ldz = m
+    h = Herk(form, m, nterms, nprod)
+    v = h.new_vacc()
+    got = []
+    for accumulate in (False, True):
+        h.run(zs, ldz=ldz, nseg=1, seg_stride=cols, seg_len=k, vacc=v,
+              accumulate=accumulate, nslices=3)
+        got.append(D.to_host(v)[:m, :m].copy())
+    upper = np.triu(np.ones((m, m), bool))
+    np.testing.assert_array_equal(got[1][upper], 2 * got[0][upper])
+    for b in range(0, m, 32):
+        blk = got[1][b:b + 32, b:b + 32]
+        np.testing.assert_array_equal(blk, blk.conj().T)
+
+
 @pytest.mark.parametrize("nfeed", [1, 2])
 @pytest.mark.parametrize("antpairs", [True, False])
 @pytest.mark.parametrize("precision", [1, 2])
