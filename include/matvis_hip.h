@@ -422,10 +422,11 @@ size_t mv_herk_grouped_workspace_bytes(int form, int tile,
  * a plan and a reduce launch): every problem's (tile, K-slice) items,
  * problem-major, are swept by one workgroup per resident slot, so small
  * problems share the GPU instead of each launch idling most of it.  Split
- * forms: `tile` = 128 or 64 (rows per workgroup tile; 64 suits m <= 128);
- * plain forms (MV_FORM_C128, MV_FORM_C64, nterms = 1, z[0] the complex Z):
- * `tile` = 64.  A problem's slice count depends on that problem alone, so
- * its result is the same in any group.  problems_host is read
+ * forms: `tile` = 128 or 64 (ldv covers m rounded up to it; two terms run
+ * the same kernel at either, three-term problems of up to 64 rows are faster
+ * at 64); plain forms (MV_FORM_C128, MV_FORM_C64, nterms = 1, z[0] the
+ * complex Z): `tile` = 64.  A problem's slice count depends on that problem
+ * alone, so its result is the same in any group.  problems_host is read
  * for validation and launch geometry, problems_dev (the same array in device
  * memory) by the kernels, so a captured graph replays with whatever the
  * device array holds.  No reference counterpart: the reference runs one

@@ -727,8 +727,8 @@ struct SplitProblem {
 };
 
 // Workgroups of the split kernels: four or eight waves on a panel group (a
-// launch's large problems), or one wave on one panel pair (small ones, tile
-// 64).  Three terms' stages fill the LDS with one workgroup a CU, which with
+// launch's problems, and grouped ones), or one wave on one panel pair (grouped
+// three-term problems of tile 64, wave_pairs).  Three terms' stages fill the LDS with one workgroup a CU, which with
 // four waves leaves each SIMD a single one whose every wait shows: eight waves
 // then share the four pairs, each taking half the columns of a K tile, and
 // add their sums up through LDS (m = 700, 2 x 9.8k columns: 230 -> 196 us; 2 x
@@ -1668,17 +1668,27 @@ const void *herk_kernel(int form, int nterms, int maxord, int panel) {
              : (const void *)&herk_split_kernel<3, 2, false>;
 }
 
-// The grouped kernel instantiation for (form, nterms, maxord): panel groups,
-// or one wave a pair.
-template <bool GROUP>
-const void *grouped_kernel_t(bool f16, int nterms, int maxord) {
-  constexpr int W2 = GROUP ? kGroupWaves<2> : 1, W3 = GROUP ? kGroupWaves<3> : 1;
+// Whether a grouped split launch gives a wave a panel pair instead of a
+// workgroup a panel group: three terms at tile 64.  Two terms take panel
+// groups at either tile since a group's waves share single panels' pairs: 64
+// instances of m = 64, 5k-40k columns (one feed), 341 us a pair a wave, 304 in
+// groups; 400 of them 2,325 and 1,833; 64 of m = 128, 928 and 638; 8 of m =
+// 64, 136 and 83.  Three terms, in groups of eight waves: m = 64, 64 instances
+// 481 and 528, 400 instances 2,965 and 3,146 (m = 128: 1,450 and 1,148).
+bool wave_pairs(int nterms, int tile) { return nterms == 3 && tile == 64; }
+
+// The grouped split kernel for (form, nterms, maxord, wave_pairs).
+const void *grouped_kernel(bool f16, int nterms, int maxord, bool pairs) {
+  constexpr int W2 = kGroupWaves<2>, W3 = kGroupWaves<3>;
   if (nterms == 2 && maxord == 1)
     return f16 ? (const void *)&herk_split_grouped_kernel<2, 1, true, W2>
                : (const void *)&herk_split_grouped_kernel<2, 1, false, W2>;
   if (nterms == 2)
     return f16 ? (const void *)&herk_split_grouped_kernel<2, 2, true, W2>
                : (const void *)&herk_split_grouped_kernel<2, 2, false, W2>;
+  if (pairs)
+    return f16 ? (const void *)&herk_split_grouped_kernel<3, 2, true, 1>
+               : (const void *)&herk_split_grouped_kernel<3, 2, false, 1>;
   return f16 ? (const void *)&herk_split_grouped_kernel<3, 2, true, W3>
              : (const void *)&herk_split_grouped_kernel<3, 2, false, W3>;
 }
@@ -2030,11 +2040,6 @@ GroupLayout group_layout(int form, int ts, const mv_herk_problem *q,
   g.total = g.parts + bytes;
   return g;
 }
-
-const void *grouped_kernel(int tile, bool f16, int nterms, int maxord) {
-  return tile == 64 ? grouped_kernel_t<false>(f16, nterms, maxord)
-                    : grouped_kernel_t<true>(f16, nterms, maxord);
-}
 }  // namespace
 
 extern "C" size_t mv_herk_problem_bytes(void) {
@@ -2117,15 +2122,16 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
              (long long)g.total);
   const bool f16 = form == MV_FORM_SPLIT_F16;
   const int side = split ? kSP : panel_side(form, max_m);
+  const bool by_wave = split && wave_pairs(nterms, tile);
   const void *kernel =
-      split ? grouped_kernel(tile, f16, nterms, maxord)
+      split ? grouped_kernel(f16, nterms, maxord, by_wave)
       : form == MV_FORM_C128
           ? (const void *)&herk_plain_grouped_kernel<double, 32>
       : side == 64 ? (const void *)&herk_plain_grouped_kernel<float, 64>
                    : (const void *)&herk_plain_grouped_kernel<float, 32>;
   const int threads =
       !split       ? 256
-      : tile == 64 ? 64
+      : by_wave    ? 64
                    : 64 * (nterms == 3 ? kGroupWaves<3> : kGroupWaves<2>);
   const int slots = kernel_slots(kernel, threads);
   if (slots <= 0) {
@@ -2140,7 +2146,7 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
   // slices of a problem that names no chain: kGroupChain K tiles; plain forms
   // take slices of 64 K tiles (1024 columns) for parallelism
   herk_group_plan_kernel<<<1, 256, 0, st>>>(
-      problems_dev, nprob, side, split && tile == 64 ? 0 : 1,
+      problems_dev, nprob, side, by_wave ? 0 : 1,
       split ? kSK : kPK,
       split ? form_cmax(form) : 64, split ? kGroupChain : 64,
       part_bytes(form), split ? 1 : 0, probs, ws + g.parts, plan);
@@ -2173,26 +2179,19 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
                                                             plan);
     return check_launch("mv_herk_grouped/reduce");
   }
-#define MV_GROUP_LAUNCH(NT, MO, F, GW)                                       \
-  herk_split_grouped_kernel<NT, MO, F, GW ? kGroupWaves<NT> : 1>             \
-      <<<grid, threads, 0, st>>>(probs, nprob, plan)
-#define MV_GROUP_TILE(GW)                                                    \
-  if (nterms == 2 && maxord == 1) {                                          \
-    if (f16) MV_GROUP_LAUNCH(2, 1, true, GW);                                \
-    else MV_GROUP_LAUNCH(2, 1, false, GW);                                   \
-  } else if (nterms == 2) {                                                  \
-    if (f16) MV_GROUP_LAUNCH(2, 2, true, GW);                                \
-    else MV_GROUP_LAUNCH(2, 2, false, GW);                                   \
-  } else {                                                                   \
-    if (f16) MV_GROUP_LAUNCH(3, 2, true, GW);                                \
-    else MV_GROUP_LAUNCH(3, 2, false, GW);                                   \
-  }
-  if (tile == 64) {
-    MV_GROUP_TILE(false)
-  } else {
-    MV_GROUP_TILE(true)
-  }
-#undef MV_GROUP_TILE
+#define MV_GROUP_LAUNCH(NT, MO, W)                                           \
+  do {                                                                       \
+    if (f16)                                                                 \
+      herk_split_grouped_kernel<NT, MO, true, W>                             \
+          <<<grid, threads, 0, st>>>(probs, nprob, plan);                    \
+    else                                                                     \
+      herk_split_grouped_kernel<NT, MO, false, W>                            \
+          <<<grid, threads, 0, st>>>(probs, nprob, plan);                    \
+  } while (0)
+  if (nterms == 2 && maxord == 1) MV_GROUP_LAUNCH(2, 1, kGroupWaves<2>);
+  else if (nterms == 2) MV_GROUP_LAUNCH(2, 2, kGroupWaves<2>);
+  else if (by_wave) MV_GROUP_LAUNCH(3, 2, 1);
+  else MV_GROUP_LAUNCH(3, 2, kGroupWaves<3>);
 #undef MV_GROUP_LAUNCH
   if (int e = check_launch("mv_herk_grouped/split")) return e;
   herk_group_reduce_kernel<float>

@@ -3,13 +3,10 @@
 The knobs, chosen per class of problems (m rounded up to a power of two,
 K = nseg x seg_len rounded up to a power of four):
 
-* tile side (split forms): 64 rows (one wave per workgroup tile, up to
-  eight workgroups per CU) or 128 rows (four waves of 64 x 64, two
-  workgroups per CU).  Waves per tile go with the side.  Small problems
-  waste most of a 128-row tile (m = 64 keeps one of its four waves busy);
-  large ones lose operand reuse on 64-row tiles.  A 256-row tile would need
-  256 x 256 complex FP32 accumulators (512 KB, a CU's whole register file),
-  so it is not a candidate.  The plain forms have one tile (64 rows).
+* tile side (split forms): 64 or 128 rows.  Three-term problems of up to 64
+  rows run one wave a panel pair at 64 and eight waves a panel group at 128;
+  all others run panel groups at either (herk_group.launch_tiles).  The plain
+  forms have one tile (64 rows).
 * kchain, the longest K-slice in K tiles (split forms 192, 96 or 48; plain
   forms 64, 32 or 16): shorter slices give a batch that does not fill the
   GPU more work items, at the cost of more partial tiles to write and

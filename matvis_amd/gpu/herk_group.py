@@ -65,26 +65,26 @@ def _addr(t) -> int:
     return 0 if t is None else int(t.data_ptr())
 
 
-def merge_tiles(form: int, nterms: int, problems: list, tiles: list) -> list:
-    """The tiles a batch runs with: its 64-row problems join the 128-row
-    launch (four-wave panel groups) when that idles few waves.  Two launches
-    one after the other each end in a tail of their own, which costs a batch
-    more than the up to three idle waves of a problem of one or two panels:
-    24 instances of 64-350 antennas 408 -> 380 us, 256 of them unchanged (20.9
-    ms).  The line lies where the idle waves' share reaches a tenth; the bits
-    of two-term results are the same in either launch, three-term ones (whose
-    group kernel halves the columns) keep the tiles asked for."""
+def launch_tiles(form: int, nterms: int, problems: list, tiles: list) -> list:
+    """The tiles a batch of split problems runs with: 128 rather than 64, one
+    launch instead of two one after the other, except for
+
+    * three-term problems of one panel: the 64-row launch gives a wave a panel
+      pair, and groups of eight waves are faster from two panels up (64
+      instances of m = 128: 1,450 -> 1,148 us; of m = 64: 481 and 528).  Two
+      terms run the same kernel at either tile, with the same bits;
+    * problems whose accumulator is padded to 64 rows only;
+    * batches that would not fit a launch together (its limit of tiles)."""
     tiles = [int(t) for t in tiles]
-    if not is_split(form) or nterms != 2 or len(set(tiles)) == 1:
+    if not is_split(form):
         return tiles
-    idle = work = 0
-    for p, t in zip(problems, tiles):
-        n = -(-p["m"] // 64)
-        pairs, cols = n * (n + 1) // 2, p["nseg"] * p["seg_len"]
-        if t == 64:  # 1 pair in a group of its own, 3 in one
-            idle += (-pairs % 4) * cols
-        work += pairs * cols
-    return [128] * len(tiles) if 10 * idle <= work else tiles
+    keep = [t == 64 and (p["ldv"] < -(-p["m"] // 128) * 128
+                         or (nterms == 3 and p["m"] <= 64))
+            for p, t in zip(problems, tiles)]
+    side = [-(-p["m"] // 128) for p in problems]
+    if sum(n * (n + 1) // 2 for n in side) >= 65536:
+        return tiles
+    return [64 if k else 128 for k in keep]
 
 
 class HerkGroup:
@@ -159,11 +159,12 @@ class HerkGroup:
 
 class GroupedBatch:
     """A batch of HERK problems of one form, one grouped launch per tile class
-    (:func:`merge_tiles`); ``capture()`` records the launches in a HIP graph for ``replay()``."""
+    (:func:`launch_tiles`); ``capture()`` records the launches in a HIP graph
+    for ``replay()``."""
 
     def __init__(self, form: int, nterms: int, nprod: int, problems: list,
                  tiles: list[int], kchains: list[int] | None = None):
-        self.tiles = merge_tiles(form, nterms, problems, tiles)
+        self.tiles = launch_tiles(form, nterms, problems, tiles)
         self.kchains = ([int(k) for k in kchains] if kchains is not None
                         else None)
         classes: dict[int, list] = {}

@@ -324,3 +324,57 @@ def test_autotuner_shortens_slices_of_an_underfilled_batch():
         assert e < 1e-6, e
     again = autotune.tune(FORM_SPLIT_BF16, 2, 3, probs, budget_s=5.0)
     assert again.cached and again.config == plan.config
+
+
+def _noise_problem(m, cols, seed, ldv):
+    """A two-term problem of m rows and cols (a multiple of 16) columns."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    terms = [torch.randn((cols // 16 * m * 32,), device="cuda", generator=g)
+             .mul_(2.0 ** (-8 * k)).to(torch.bfloat16).view(torch.int32)
+             .view(cols // 16, m, 16) for k in range(2)]
+    return dict(terms=terms, m=m, ldz=m, nseg=1, seg_stride=cols,
+                seg_len=cols, vacc=D.zeros((ldv, ldv), np.complex128),
+                ldv=ldv, scale=1.0, accumulate=False)
+
+
+@pytest.mark.parametrize("nprob", [255, 256, 257, 513])
+def test_grouped_plan_block_edges(nprob):
+    """The plan scans 256 problems at a time: problems of 1 to 3 panels and
+    uneven slice counts at the edges of a block have the bits they have in a
+    launch by themselves."""
+    from matvis_amd.gpu.herk_group import HerkGroup
+    rng = np.random.default_rng(nprob)
+    shapes = [(int(rng.choice([5, 64, 65, 130])),
+               16 * int(rng.integers(1, 250))) for _ in range(nprob)]
+    probs = [_noise_problem(m, c, i, -(-m // 128) * 128)
+             for i, (m, c) in enumerate(shapes)]
+    HerkGroup(FORM_SPLIT_BF16, 2, 3, 128, probs).run()
+    for i in sorted({0, 1, 254, min(255, nprob - 1), min(256, nprob - 1),
+                     nprob - 1}):
+        alone = dict(probs[i], vacc=D.zeros(tuple(probs[i]["vacc"].shape),
+                                            np.complex128))
+        HerkGroup(FORM_SPLIT_BF16, 2, 3, 128, [alone]).run()
+        np.testing.assert_array_equal(D.to_host(probs[i]["vacc"]),
+                                      D.to_host(alone["vacc"]))
+
+
+def test_grouped_batch_tiles():
+    """Accumulators padded to 64 rows keep the 64-row launch, whose bits are
+    the 128-row launch's for two terms."""
+    from matvis_amd.gpu.herk_group import GroupedBatch, launch_tiles
+    ms = (64, 40, 100, 300)
+    tight = [_noise_problem(m, 480, m, -(-m // 64) * 64) for m in ms[:2]]
+    wide = [_noise_problem(m, 480, m, -(-m // 128) * 128) for m in ms]
+    tiles = [64, 64, 64, 128]
+    assert launch_tiles(FORM_SPLIT_BF16, 2, wide, tiles) == [128] * 4
+    assert launch_tiles(FORM_SPLIT_BF16, 3, wide, tiles) == [64, 64, 128, 128]
+    assert launch_tiles(FORM_SPLIT_BF16, 2, tight + wide[2:], tiles) == [
+        64, 64, 128, 128]
+    GroupedBatch(FORM_SPLIT_BF16, 2, 3, wide, tiles).run()
+    GroupedBatch(FORM_SPLIT_BF16, 2, 3, tight + wide[3:], [64, 64, 128]).run()
+    for t, w in zip(tight, wide):
+        n = t["ldv"]
+        np.testing.assert_array_equal(D.to_host(t["vacc"]),
+                                      D.to_host(w["vacc"])[:n, :n])
