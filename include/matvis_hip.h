@@ -93,6 +93,19 @@ int mv_rotate_cull(const double *eci, int64_t ld_eci, const double *rot9,
                    int32_t *n_up_dev, void *workspace, size_t ws_bytes,
                    mv_stream_t stream);
 
+/* The chunks of chunk_size sources each of [chunk0, chunk0 + nsrc) (nsrc <=
+ * nchunks chunk_size; the last ones short or empty) in the launches of
+ * one mv_rotate_cull without fluxes: chunk c's outputs are crd_out + c 3
+ * ld_crd, idx_out + c ld_idx and n_up_dev[c].  workspace: nchunks times
+ * mv_rotate_cull_workspace_bytes(chunk_size).  Replaces the chunk loop over
+ * select_chunk (src/matvis/core/coords.py:99-150). */
+int mv_rotate_cull_chunks(const double *eci, int64_t ld_eci,
+                          const double *rot9, int64_t chunk0, int64_t nsrc,
+                          int64_t chunk_size, int nchunks, int64_t nalloc,
+                          double *crd_out, int64_t ld_crd, int32_t *idx_out,
+                          int64_t ld_idx, int32_t *n_up_dev, void *workspace,
+                          size_t ws_bytes, mv_stream_t stream);
+
 /* BCRS corrections of ICRS unit vectors, the per-source part of the ERFA
  * rotation: light deflection by the Sun (limiter dlim, 1e-6 in the
  * reference), aberration and the bias-precession-nutation matrix, giving CIRS
@@ -196,6 +209,24 @@ int mv_beam_gaussian(const double *sigma, int nbeam, int polarized,
                      const void *crd, int crd_is_f64, int64_t ld_crd,
                      int64_t count, const int32_t *n_dev, void *out,
                      int out_is_f64, int64_t ld_out, mv_stream_t stream);
+
+/* mv_beam_interp and mv_beam_gaussian over nchunks (up to 65535) chunks of
+ * sources in one launch: chunk c's coordinates start c crd_stride elements
+ * and its output c out_stride complex elements after the first's, and its
+ * count is n_dev[c] (n_dev nullable: `count` each). */
+int mv_beam_interp_chunks(const void *planes, int is_f64, int nbeam,
+                          int nfeed, int nax, int nza, int naz,
+                          const double *grid, int order, int is_power,
+                          const void *crd, int crd_is_f64, int64_t ld_crd,
+                          int64_t crd_stride, int64_t count, int nchunks,
+                          const int32_t *n_dev, void *out, int64_t ld_out,
+                          int64_t out_stride, mv_stream_t stream);
+int mv_beam_gaussian_chunks(const double *sigma, int nbeam, int polarized,
+                            const void *crd, int crd_is_f64, int64_t ld_crd,
+                            int64_t crd_stride, int64_t count, int nchunks,
+                            const int32_t *n_dev, void *out, int out_is_f64,
+                            int64_t ld_out, int64_t out_stride,
+                            mv_stream_t stream);
 
 /* ---------------------------------------------------------------- (c) ---- */
 

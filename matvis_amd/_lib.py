@@ -40,18 +40,24 @@ SIGNATURES: dict[str, list] = {
     "mv_rotate_cull_workspace_bytes": [_L],
     "mv_rotate_cull": [_P, _L, _P, _P, _L, _L, _L, _P, _L, _P, _I, _P, _P,
                        _P, _S, _P],
+    "mv_rotate_cull_chunks": [_P, _L, _P, _L, _L, _L, _I, _L, _P, _L, _P, _L,
+                              _P, _P, _S, _P],
     "mv_bcrs_update": [_P, _L, _L, _P, _D, _P, _L, _P],
     "mv_coherency_rotate": [_P, _P, _L, _P, _P, _L, _I, _P, _L, _P, _P, _L,
                             _I, _I, _P, _P],
     "mv_beam_prefilter": [_P, _I, _L, _I, _I, _P],
     "mv_beam_interp": [_P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _P, _I, _L,
                        _L, _P, _P, _L, _P],
+    "mv_beam_interp_chunks": [_P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _P, _I,
+                              _L, _L, _L, _I, _P, _P, _L, _L, _P],
     "mv_beam_interp_azza": [_P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _P, _P,
                             _L, _P, _L, _P],
     "mv_beam_interp_banded_workspace_bytes": [_I, _I, _I, _L],
     "mv_beam_interp_banded": [_P, _I, _I, _I, _I, _I, _I, _P, _I, _I, _P, _I,
                               _L, _L, _P, _P, _L, _P, _S, _P],
     "mv_beam_gaussian": [_P, _I, _I, _P, _I, _L, _L, _P, _P, _I, _L, _P],
+    "mv_beam_gaussian_chunks": [_P, _I, _I, _P, _I, _L, _L, _L, _I, _P, _P,
+                                _I, _L, _L, _P],
     "mv_exptau": [_P, _I, _D, _P, _I, _L, _L, _P, _I, _L, _P],
     "mv_zmat_parts": [_P, _P, _P, _I, _P, _I, _I, _I, _L, _P, _I, _P],
     "mv_zmat_fused": [_P, _I, _D, _P, _L, _P, _P, _P, _I, _L, _I, _P, _I,

@@ -290,6 +290,12 @@ __device__ __forceinline__ cplx<T> interp_value(double az, double za,
 // sources that is what keeps the tap gathers' latency covered; the planes,
 // about 1 MB for one polarized 360 x 91 complex64 beam, stay in L2).
 // AZZA: positions come as (az, za) arrays instead of topocentric vectors.
+// Elements between the coordinates and the outputs of a launch's chunks
+// (grid.z here, grid.y of gaussian_kernel); their counts are adjacent.
+struct ChunkStrides {
+  int64_t crd, out;
+};
+
 template <typename T, typename TC, int ORDER, bool AZZA = false>
 __global__ __launch_bounds__(kThreads) void interp_kernel(
     const cplx<T> *__restrict__ planes, int nbeam, int nfeed, int nax, int nza,
@@ -297,9 +303,12 @@ __global__ __launch_bounds__(kThreads) void interp_kernel(
     const TC *__restrict__ crd, int64_t ld_crd, int64_t count,
     const int32_t *__restrict__ n_dev, cplx<T> *__restrict__ out,
     int64_t ld_out, const double *__restrict__ az_in,
-    const double *__restrict__ za_in) {
+    const double *__restrict__ za_in, ChunkStrides cs) {
   const int64_t p = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (p >= count) return;
+  if (!AZZA) crd += blockIdx.z * cs.crd;
+  out += blockIdx.z * cs.out;
+  if (n_dev) n_dev += blockIdx.z;
   // output plane (b, fd, ax) and its input plane (b, ax, fd)
   const int q = blockIdx.y;
   const int ax = q % nax, fd = (q / nax) % nfeed, b = q / (nax * nfeed);
@@ -481,9 +490,12 @@ __global__ __launch_bounds__(kThreads) void gaussian_kernel(
     const double *__restrict__ sigma, int nbeam, int polarized,
     const TC *__restrict__ crd, int64_t ld_crd, int64_t count,
     const int32_t *__restrict__ n_dev, cplx<T> *__restrict__ out,
-    int64_t ld_out) {
+    int64_t ld_out, ChunkStrides cs) {
   int64_t p = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (p >= count) return;
+  crd += blockIdx.y * cs.crd;
+  out += blockIdx.y * cs.out;
+  if (n_dev) n_dev += blockIdx.y;
   const int64_t n = n_dev ? min((int64_t)*n_dev, count) : count;
   const int nplane = polarized ? 4 : 1;
   double az, za;
@@ -553,17 +565,17 @@ static void launch_interp(int order, dim3 g, hipStream_t s, const void *planes,
                           int nbeam, int nfeed, int nax, int nza, int naz,
                           const double *grid, int is_power, const void *crd,
                           int64_t ld_crd, int64_t count, const int32_t *n_dev,
-                          void *out, int64_t ld_out) {
+                          void *out, int64_t ld_out, ChunkStrides cs) {
   if (order == 1)
     interp_kernel<T, TC, 1><<<g, kThreads, 0, s>>>(
         (const cplx<T> *)planes, nbeam, nfeed, nax, nza, naz, grid, is_power,
         (const TC *)crd, ld_crd, count, n_dev, (cplx<T> *)out, ld_out,
-        nullptr, nullptr);
+        nullptr, nullptr, cs);
   else
     interp_kernel<T, TC, 3><<<g, kThreads, 0, s>>>(
         (const cplx<T> *)planes, nbeam, nfeed, nax, nza, naz, grid, is_power,
         (const TC *)crd, ld_crd, count, n_dev, (cplx<T> *)out, ld_out,
-        nullptr, nullptr);
+        nullptr, nullptr, cs);
 }
 
 extern "C" int mv_beam_interp(const void *planes, int is_f64, int nbeam,
@@ -572,36 +584,44 @@ extern "C" int mv_beam_interp(const void *planes, int is_f64, int nbeam,
                               const void *crd, int crd_is_f64, int64_t ld_crd,
                               int64_t count, const int32_t *n_dev, void *out,
                               int64_t ld_out, mv_stream_t stream) {
+  return mv_beam_interp_chunks(planes, is_f64, nbeam, nfeed, nax, nza, naz,
+                               grid, order, is_power, crd, crd_is_f64, ld_crd,
+                               0, count, 1, n_dev, out, ld_out, 0, stream);
+}
+
+extern "C" int mv_beam_interp_chunks(
+    const void *planes, int is_f64, int nbeam, int nfeed, int nax, int nza,
+    int naz, const double *grid, int order, int is_power, const void *crd,
+    int crd_is_f64, int64_t ld_crd, int64_t crd_stride, int64_t count,
+    int nchunks, const int32_t *n_dev, void *out, int64_t ld_out,
+    int64_t out_stride, mv_stream_t stream) {
   MV_REQUIRE(planes && grid && crd && out, "mv_beam_interp: null pointer");
   MV_REQUIRE(order == 1 || order == 3,
              "mv_beam_interp: order must be 1 or 3 (got %d)", order);
   MV_REQUIRE(nbeam >= 1 && nfeed >= 1 && nax >= 1 && nza >= 1 && naz >= 1 &&
-                 count >= 0 && ld_crd >= count && ld_out >= count,
+                 count >= 0 && ld_crd >= count && ld_out >= count &&
+                 nchunks >= 1 && nchunks <= 65535 && crd_stride >= 0 &&
+                 out_stride >= 0,
              "mv_beam_interp: bad sizes");
   MV_REQUIRE((int64_t)nbeam * nfeed * nax <= 65535,
              "mv_beam_interp: too many planes");
   if (count == 0) return MV_OK;
-  dim3 g((unsigned)cdiv(count, kThreads), (unsigned)(nbeam * nfeed * nax));
+  dim3 g((unsigned)cdiv(count, kThreads), (unsigned)(nbeam * nfeed * nax),
+         (unsigned)nchunks);
   hipStream_t s = as_stream(stream);
+  const ChunkStrides cs = {crd_stride, out_stride};
+#define MV_INTERP(T, TC)                                                     \
+  launch_interp<T, TC>(order, g, s, planes, nbeam, nfeed, nax, nza, naz,     \
+                       grid, is_power, crd, ld_crd, count, n_dev, out,       \
+                       ld_out, cs)
   if (is_f64) {
-    if (crd_is_f64)
-      launch_interp<double, double>(order, g, s, planes, nbeam, nfeed, nax,
-                                    nza, naz, grid, is_power, crd, ld_crd,
-                                    count, n_dev, out, ld_out);
-    else
-      launch_interp<double, float>(order, g, s, planes, nbeam, nfeed, nax,
-                                   nza, naz, grid, is_power, crd, ld_crd,
-                                   count, n_dev, out, ld_out);
+    if (crd_is_f64) MV_INTERP(double, double);
+    else MV_INTERP(double, float);
   } else {
-    if (crd_is_f64)
-      launch_interp<float, double>(order, g, s, planes, nbeam, nfeed, nax, nza,
-                                   naz, grid, is_power, crd, ld_crd, count,
-                                   n_dev, out, ld_out);
-    else
-      launch_interp<float, float>(order, g, s, planes, nbeam, nfeed, nax, nza,
-                                  naz, grid, is_power, crd, ld_crd, count,
-                                  n_dev, out, ld_out);
+    if (crd_is_f64) MV_INTERP(float, double);
+    else MV_INTERP(float, float);
   }
+#undef MV_INTERP
   return check_launch("mv_beam_interp");
 }
 
@@ -741,7 +761,8 @@ extern "C" int mv_beam_interp_azza(const void *planes, int is_f64, int nbeam,
 #define MV_AZZA(T, O)                                                        \
   interp_kernel<T, double, O, true><<<g, kThreads, 0, s>>>(                  \
       (const cplx<T> *)planes, nbeam, nfeed, nax, nza, naz, grid, is_power,  \
-      nullptr, 0, count, nullptr, (cplx<T> *)out, ld_out, az, za)
+      nullptr, 0, count, nullptr, (cplx<T> *)out, ld_out, az, za,            \
+      ChunkStrides{0, 0})
   if (is_f64) {
     if (order == 1) MV_AZZA(double, 1);
     else MV_AZZA(double, 3);
@@ -759,16 +780,29 @@ extern "C" int mv_beam_gaussian(const double *sigma, int nbeam, int polarized,
                                 const int32_t *n_dev, void *out,
                                 int out_is_f64, int64_t ld_out,
                                 mv_stream_t stream) {
+  return mv_beam_gaussian_chunks(sigma, nbeam, polarized, crd, crd_is_f64,
+                                 ld_crd, 0, count, 1, n_dev, out, out_is_f64,
+                                 ld_out, 0, stream);
+}
+
+extern "C" int mv_beam_gaussian_chunks(
+    const double *sigma, int nbeam, int polarized, const void *crd,
+    int crd_is_f64, int64_t ld_crd, int64_t crd_stride, int64_t count,
+    int nchunks, const int32_t *n_dev, void *out, int out_is_f64,
+    int64_t ld_out, int64_t out_stride, mv_stream_t stream) {
   MV_REQUIRE(sigma && crd && out, "mv_beam_gaussian: null pointer");
-  MV_REQUIRE(nbeam >= 1 && count >= 0 && ld_crd >= count && ld_out >= count,
+  MV_REQUIRE(nbeam >= 1 && count >= 0 && ld_crd >= count && ld_out >= count &&
+                 nchunks >= 1 && nchunks <= 65535 && crd_stride >= 0 &&
+                 out_stride >= 0,
              "mv_beam_gaussian: bad sizes");
   if (count == 0) return MV_OK;
-  dim3 g((unsigned)cdiv(count, kThreads));
+  dim3 g((unsigned)cdiv(count, kThreads), (unsigned)nchunks);
   hipStream_t s = as_stream(stream);
+  const ChunkStrides cs = {crd_stride, out_stride};
 #define MV_GAUSS(T, TC)                                                    \
   gaussian_kernel<T, TC><<<g, kThreads, 0, s>>>(                           \
       sigma, nbeam, polarized, (const TC *)crd, ld_crd, count, n_dev,      \
-      (cplx<T> *)out, ld_out)
+      (cplx<T> *)out, ld_out, cs)
   if (out_is_f64) {
     if (crd_is_f64) MV_GAUSS(double, double);
     else MV_GAUSS(double, float);

@@ -2,22 +2,41 @@
 // with the horizon cull and a stable (ascending-index) stream compaction.
 //
 // Compaction runs as count -> scatter, each scatter block summing the counts
-// before its own (count -> scan -> scatter beyond kScanBlocks blocks).  Each
-// block owns a fixed run of kItemsPerBlock sources and re-derives the same
-// horizon flags in both the count and the scatter pass, so the output order equals the reference's
+// before its own; as count -> scan -> scatter beyond kScanBlocks blocks; and
+// as one launch up to kOneBlocks blocks, each counting the sources before its
+// own run by itself.  Each block owns a fixed run of kItemsPerBlock sources
+// and every pass derives the same horizon flags, so the output order equals the reference's
 // `xp.where(topo[2] > 0)` order (src/matvis/core/coords.py:115) for any grid.
+// All chunks of a time share the launches (grid.y).
 #include "common.h"
 
 namespace mv {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kRounds = 8;
-constexpr int kItemsPerBlock = kThreads * kRounds;  // 2048 sources per block
+constexpr int kItemsPerBlock = 2048;  // sources a block places
 // Up to this many blocks (4.2M sources) a scatter block reads all counts, 8 a
 // thread from L2, instead of a launch of its own for the scan: 3-4.5 us of a
 // cull's 13-17.
 constexpr int kScanBlocks = 2048;
+// Up to this many blocks (8,192 sources) the last one counts the sources
+// before it about as fast as a count launch would: 1 to 4 blocks 3.0, 4.2, 6.5
+// and 8 us, 6 and 8 of them 10.0 and 12.0, against 3.8 + 6.0 and the gap
+// between two launches.
+constexpr int kOneBlocks = 4;
+
+// One time's sources in chunks: chunk y holds sources [chunk0 + y size,
+// chunk0 + min((y + 1) size, total)) and its outputs start y *_stride
+// elements after the first chunk's.
+struct CullChunks {
+  int64_t chunk0, size, total, nalloc;
+  int64_t crd_stride, idx_stride;
+  int nblocks;  // of a chunk
+};
+__device__ __forceinline__ int64_t chunk_len(const CullChunks &K, int y) {
+  const int64_t left = K.total - y * K.size;
+  return left < 0 ? 0 : (left < K.size ? left : K.size);
+}
 
 struct Mat3 {
   double m[9];
@@ -53,34 +72,51 @@ __device__ __forceinline__ bool above_horizon(const double *__restrict__ eci,
   return rot_row(R, 2, x, y, z) > 0.0;
 }
 
-// Pass 1: number of above-horizon sources in each block's run.
-__global__ __launch_bounds__(kThreads) void cull_count_kernel(
-    const double *__restrict__ eci, int64_t ld_eci, Mat3 R, int64_t chunk0,
-    int64_t chunk_len, int32_t *__restrict__ counts) {
-  __shared__ int wave_sum[kThreads / 64];
-  const int64_t base = (int64_t)blockIdx.x * kItemsPerBlock;
-  int local = 0;
-#pragma unroll
-  for (int r = 0; r < kRounds; ++r) {
-    int64_t p = base + r * kThreads + threadIdx.x;
-    if (p < chunk_len && above_horizon(eci, ld_eci, R, chunk0 + p)) ++local;
+// Sums of a and b over the workgroup of WAVES waves, in every thread.
+template <int WAVES>
+__device__ __forceinline__ void block_sums(int &a, int &b) {
+  __shared__ int sums[2][WAVES];
+  for (int off = 32; off > 0; off >>= 1) {
+    a += __shfl_xor(a, off, 64);
+    b += __shfl_xor(b, off, 64);
   }
-  // wave reduction
-  for (int off = 32; off > 0; off >>= 1) local += __shfl_down(local, off, 64);
-  if ((threadIdx.x & 63) == 0) wave_sum[threadIdx.x >> 6] = local;
+  if ((threadIdx.x & 63) == 0) {
+    sums[0][threadIdx.x >> 6] = a;
+    sums[1][threadIdx.x >> 6] = b;
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int s = 0;
-    for (int w = 0; w < kThreads / 64; ++w) s += wave_sum[w];
-    counts[blockIdx.x] = s;
+  a = b = 0;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    a += sums[0][w];
+    b += sums[1][w];
   }
 }
 
-// Pass 2 of a large chunk: exclusive scan of block counts (single workgroup);
+// Pass 1: number of above-horizon sources in each block's run.
+__global__ __launch_bounds__(kThreads) void cull_count_kernel(
+    const double *__restrict__ eci, int64_t ld_eci, Mat3 R, CullChunks K,
+    int32_t *__restrict__ counts) {
+  const int64_t len = chunk_len(K, blockIdx.y);
+  const int64_t base = (int64_t)blockIdx.x * kItemsPerBlock + threadIdx.x;
+  const int64_t g0 = K.chunk0 + blockIdx.y * K.size;
+  int local = 0, none = 0;
+#pragma unroll
+  for (int r = 0; r < kItemsPerBlock / kThreads; ++r) {
+    const int64_t p = base + r * kThreads;
+    if (p < len && above_horizon(eci, ld_eci, R, g0 + p)) ++local;
+  }
+  block_sums<kThreads / 64>(local, none);
+  if (threadIdx.x == 0)
+    counts[(int64_t)blockIdx.y * K.nblocks + blockIdx.x] = local;
+}
+
+// Pass 2 of a large chunk: exclusive scan of block counts;
 // total -> n_up.
 __global__ __launch_bounds__(1024) void cull_scan_kernel(
     int32_t *__restrict__ counts, int64_t nblocks,
     int32_t *__restrict__ n_up) {
+  counts += blockIdx.x * nblocks;  // one workgroup a chunk
   __shared__ int buf[1024];
   __shared__ int carry;
   if (threadIdx.x == 0) carry = 0;
@@ -103,93 +139,117 @@ __global__ __launch_bounds__(1024) void cull_scan_kernel(
     if (threadIdx.x == 1023) carry += incl;
     __syncthreads();
   }
-  if (threadIdx.x == 0) *n_up = carry;
+  if (threadIdx.x == 0) n_up[blockIdx.x] = carry;
 }
 
-// Last pass: recompute flags, place each kept source at its block offset (the
-// scanned count, or the sum of the counts before it) plus its
-// rank inside the block, then zero-fill positions [n_up, nalloc).
-template <typename T>
-__global__ __launch_bounds__(kThreads) void cull_scatter_kernel(
+// How a scatter block finds where its sources start.
+enum CullStart { kCounts, kScanned, kOwn };
+
+// Last (or only) pass: recompute flags, place each kept source at its block's
+// start (the sum of the counts before it, the scanned count, or its own count
+// of the sources before it) plus its rank inside the block, and zero-fill
+// positions [n_up, nalloc).
+// A block's sources are loaded at once and ranked with one exchange of wave
+// counts: 6.0 us, where loads and an exchange for every 256 sources took 7.1-8.5.
+template <typename T, int THREADS, CullStart START>
+__global__ __launch_bounds__(THREADS) void cull_scatter_kernel(
     const double *__restrict__ eci, int64_t ld_eci, Mat3 R,
-    const double *__restrict__ flux_in, int64_t chunk0, int64_t chunk_len,
-    int64_t nalloc, const int32_t *__restrict__ offsets, int scanned,
-    int32_t *__restrict__ n_up_dev, T *__restrict__ crd, int64_t ld_crd,
-    T *__restrict__ flux_out, int32_t *__restrict__ idx_out,
-    int64_t nblocks_real) {
-  __shared__ int wave_cnt[kThreads / 64];
-  __shared__ int wave_sum[2][kThreads / 64];
+    const double *__restrict__ flux_in, CullChunks K,
+    const int32_t *__restrict__ offsets, int32_t *__restrict__ n_up_dev,
+    T *__restrict__ crd, int64_t ld_crd, T *__restrict__ flux_out,
+    int32_t *__restrict__ idx_out) {
+  constexpr int kWaves = THREADS / 64, kRounds = kItemsPerBlock / THREADS;
+  __shared__ int wave_cnt[kRounds][kWaves];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  // where this block's sources start, and the total count
+  const int64_t len = chunk_len(K, blockIdx.y);
+  const int64_t g0 = K.chunk0 + blockIdx.y * K.size;
+  offsets += (int64_t)blockIdx.y * K.nblocks;
+  n_up_dev += blockIdx.y;
+  crd += blockIdx.y * K.crd_stride;
+  if (idx_out) idx_out += blockIdx.y * K.idx_stride;
+  // this thread's sources: THREADS apart, so that a round's are adjacent
+  const int64_t base = (int64_t)blockIdx.x * kItemsPerBlock + threadIdx.x;
+  double x[kRounds], y[kRounds], z[kRounds];
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int64_t p = base + r * THREADS;
+    x[r] = y[r] = z[r] = 0.0;
+    if (p < len) {
+      x[r] = eci[g0 + p];
+      y[r] = eci[ld_eci + g0 + p];
+      z[r] = eci[2 * ld_eci + g0 + p];
+    }
+  }
+  // sources kept before this block's and, from counts, in all
   int64_t start = 0, n_up = 0;
-  if (scanned) {
-    if ((int64_t)blockIdx.x < nblocks_real) start = offsets[blockIdx.x];
+  if constexpr (START == kScanned) {
+    start = offsets[blockIdx.x];
     n_up = *n_up_dev;
   } else {
     int before = 0, all = 0;
-    for (int i = threadIdx.x; i < nblocks_real; i += kThreads) {
-      const int v = offsets[i];
-      all += v;
-      if (i < (int)blockIdx.x) before += v;
+    if constexpr (START == kCounts) {
+      for (int i = threadIdx.x; i < K.nblocks; i += THREADS) {
+        const int v = offsets[i];
+        all += v;
+        if (i < (int)blockIdx.x) before += v;
+      }
+    } else {
+      const int64_t own = (int64_t)blockIdx.x * kItemsPerBlock;
+      const int64_t end = own < len ? own : len;
+#pragma unroll 4
+      for (int64_t p = threadIdx.x; p < end; p += THREADS)
+        before += above_horizon(eci, ld_eci, R, g0 + p);
     }
-    for (int off = 32; off > 0; off >>= 1) {
-      before += __shfl_down(before, off, 64);
-      all += __shfl_down(all, off, 64);
-    }
-    if (lane == 0) {
-      wave_sum[0][wave] = before;
-      wave_sum[1][wave] = all;
-    }
-    __syncthreads();
-    for (int w = 0; w < kThreads / 64; ++w) {
-      start += wave_sum[0][w];
-      n_up += wave_sum[1][w];
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) *n_up_dev = (int32_t)n_up;
+    block_sums<kWaves>(before, all);
+    start = before;
+    n_up = all;
   }
-  if ((int64_t)blockIdx.x < nblocks_real) {
-    const int64_t base = (int64_t)blockIdx.x * kItemsPerBlock;
-    int64_t run = start;
-    for (int r = 0; r < kRounds; ++r) {
-      int64_t p = base + r * kThreads + threadIdx.x;
-      int64_t g = chunk0 + p;
-      bool keep = false;
-      double x = 0, y = 0, z = 0;
-      if (p < chunk_len) {
-        x = eci[g];
-        y = eci[ld_eci + g];
-        z = eci[2 * ld_eci + g];
-        keep = rot_row(R, 2, x, y, z) > 0.0;
-      }
-      uint64_t mask = __ballot(keep);
-      int rank = __popcll(mask & ((1ull << lane) - 1ull));
-      if (lane == 0) wave_cnt[wave] = __popcll(mask);
-      __syncthreads();
-      int before = 0, total = 0;
+  uint64_t mask[kRounds];
 #pragma unroll
-      for (int w = 0; w < kThreads / 64; ++w) {
-        before += (w < wave) ? wave_cnt[w] : 0;
-        total += wave_cnt[w];
-      }
-      if (keep) {
-        int64_t dst = run + before + rank;
-        if (dst >= 0 && dst < nalloc) {
-          crd[dst] = (T)rot_row(R, 0, x, y, z);
-          crd[ld_crd + dst] = (T)rot_row(R, 1, x, y, z);
-          crd[2 * ld_crd + dst] = (T)rot_row(R, 2, x, y, z);
-          if (flux_out) flux_out[dst] = (T)flux_in[g];
-          if (idx_out) idx_out[dst] = (int32_t)g;
-        }
-      }
-      run += total;
-      __syncthreads();
+  for (int r = 0; r < kRounds; ++r) {
+    const bool keep = base + r * THREADS < len &&
+                      rot_row(R, 2, x[r], y[r], z[r]) > 0.0;
+    mask[r] = __ballot(keep);
+    if (lane == 0) wave_cnt[r][wave] = __popcll(mask[r]);
+  }
+  __syncthreads();
+  int64_t run = start;
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    int before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      before += (w < wave) ? wave_cnt[r][w] : 0;
+      total += wave_cnt[r][w];
     }
+    if (mask[r] >> lane & 1) {
+      const int64_t dst = run + before + __popcll(mask[r] & ((1ull << lane) - 1));
+      const int64_t g = g0 + base + r * THREADS;
+      if (dst < K.nalloc) {
+        crd[dst] = (T)rot_row(R, 0, x[r], y[r], z[r]);
+        crd[ld_crd + dst] = (T)rot_row(R, 1, x[r], y[r], z[r]);
+        crd[2 * ld_crd + dst] = (T)rot_row(R, 2, x[r], y[r], z[r]);
+        if (flux_out) flux_out[dst] = (T)flux_in[g];
+        if (idx_out) idx_out[dst] = (int32_t)g;
+      }
+    }
+    run += total;
+  }
+  int64_t stride = (int64_t)gridDim.x * THREADS;
+  int64_t first = (int64_t)blockIdx.x * THREADS + threadIdx.x;
+  if constexpr (START == kOwn) {
+    // the last block knows the count, and fills the tail
+    if (blockIdx.x + 1 < gridDim.x) return;
+    n_up = run;
+    stride = THREADS;
+    first = threadIdx.x;
+  }
+  if constexpr (START != kScanned) {
+    if (first == 0) *n_up_dev = (int32_t)n_up;
   }
   // zero-fill the tail [n_up, nalloc)
-  const int64_t stride = (int64_t)gridDim.x * kThreads;
-  for (int64_t q = n_up + (int64_t)blockIdx.x * kThreads + threadIdx.x;
-       q < nalloc; q += stride) {
+  for (int64_t q = n_up + first; q < K.nalloc; q += stride) {
     crd[q] = (T)0;
     crd[ld_crd + q] = (T)0;
     crd[2 * ld_crd + q] = (T)0;
@@ -312,6 +372,38 @@ extern "C" size_t mv_rotate_cull_workspace_bytes(int64_t chunk_len) {
   return (size_t)(cdiv(nb * 4, 256) * 256);
 }
 
+namespace mv {
+namespace {
+template <typename T>
+int run_cull(const double *eci, int64_t ld_eci, const Mat3 &R,
+             const double *flux_in, const CullChunks &K, int nchunks,
+             int32_t *counts, int32_t *n_up, void *crd, int64_t ld_crd,
+             void *flux_out, int32_t *idx, hipStream_t s) {
+  const dim3 g((unsigned)K.nblocks, (unsigned)nchunks);
+#define MV_SCATTER(THREADS, START)                                           \
+  cull_scatter_kernel<T, THREADS, START><<<g, THREADS, 0, s>>>(              \
+      eci, ld_eci, R, flux_in, K, counts, n_up, (T *)crd, ld_crd,            \
+      (T *)flux_out, idx)
+  if (K.nblocks <= kOneBlocks) {
+    MV_SCATTER(1024, kOwn);
+    return check_launch("mv_rotate_cull");
+  }
+  cull_count_kernel<<<g, kThreads, 0, s>>>(eci, ld_eci, R, K, counts);
+  if (int e = check_launch("mv_rotate_cull/count")) return e;
+  if (K.nblocks > kScanBlocks) {
+    cull_scan_kernel<<<(unsigned)nchunks, 1024, 0, s>>>(counts, K.nblocks,
+                                                        n_up);
+    if (int e = check_launch("mv_rotate_cull/scan")) return e;
+    MV_SCATTER(kThreads, kScanned);
+  } else {
+    MV_SCATTER(kThreads, kCounts);
+  }
+#undef MV_SCATTER
+  return check_launch("mv_rotate_cull/scatter");
+}
+}  // namespace
+}  // namespace mv
+
 extern "C" int mv_rotate_cull(const double *eci, int64_t ld_eci,
                               const double *rot9, const double *flux_in,
                               int64_t chunk0, int64_t chunk_len,
@@ -334,30 +426,45 @@ extern "C" int mv_rotate_cull(const double *eci, int64_t ld_eci,
   MV_REQUIRE(ws_bytes >= mv_rotate_cull_workspace_bytes(chunk_len),
              "mv_rotate_cull: workspace too small (%zu < %zu)", ws_bytes,
              mv_rotate_cull_workspace_bytes(chunk_len));
-  hipStream_t s = as_stream(stream);
-  Mat3 R = load_mat(rot9);
-  int32_t *counts = (int32_t *)workspace;
-  int64_t nb = cdiv(chunk_len, kItemsPerBlock);
-  if (nb > 0) {
-    cull_count_kernel<<<(unsigned)nb, kThreads, 0, s>>>(eci, ld_eci, R, chunk0,
-                                                        chunk_len, counts);
-    if (int e = check_launch("mv_rotate_cull/count")) return e;
-  }
-  const int scanned = nb > kScanBlocks;
-  if (scanned) {
-    cull_scan_kernel<<<1, 1024, 0, s>>>(counts, nb, n_up_dev);
-    if (int e = check_launch("mv_rotate_cull/scan")) return e;
-  }
-  int64_t grid = nb > 0 ? nb : 1;
-  if (out_is_f64)
-    cull_scatter_kernel<double><<<(unsigned)grid, kThreads, 0, s>>>(
-        eci, ld_eci, R, flux_in, chunk0, chunk_len, nalloc, counts, scanned,
-        n_up_dev, (double *)crd_out, ld_crd, (double *)flux_out, idx_out, nb);
-  else
-    cull_scatter_kernel<float><<<(unsigned)grid, kThreads, 0, s>>>(
-        eci, ld_eci, R, flux_in, chunk0, chunk_len, nalloc, counts, scanned,
-        n_up_dev, (float *)crd_out, ld_crd, (float *)flux_out, idx_out, nb);
-  return check_launch("mv_rotate_cull/scatter");
+  const int64_t nb = chunk_len > 0 ? cdiv(chunk_len, kItemsPerBlock) : 1;
+  const CullChunks K = {chunk0, chunk_len, chunk_len, nalloc, 0, 0, (int)nb};
+  return (out_is_f64 ? run_cull<double> : run_cull<float>)(
+      eci, ld_eci, load_mat(rot9), flux_in, K, 1, (int32_t *)workspace,
+      n_up_dev, crd_out, ld_crd, flux_out, idx_out, as_stream(stream));
+}
+
+extern "C" int mv_rotate_cull_chunks(
+    const double *eci, int64_t ld_eci, const double *rot9, int64_t chunk0,
+    int64_t nsrc, int64_t chunk_size, int nchunks, int64_t nalloc,
+    double *crd_out, int64_t ld_crd, int32_t *idx_out, int64_t ld_idx,
+    int32_t *n_up_dev, void *workspace, size_t ws_bytes,
+    mv_stream_t stream) {
+  MV_REQUIRE(eci && rot9 && crd_out && idx_out && n_up_dev && workspace,
+             "mv_rotate_cull_chunks: null pointer");
+  MV_REQUIRE(chunk0 >= 0 && nsrc >= 0 && chunk_size >= 1 && nchunks >= 1 &&
+                 nchunks <= 65535 && nalloc >= 0 && ld_crd >= nalloc &&
+                 ld_idx >= nalloc && chunk0 + nsrc <= ld_eci &&
+                 nsrc <= chunk_size * nchunks,
+             "mv_rotate_cull_chunks: bad sizes chunk0=%lld nsrc=%lld "
+             "chunk_size=%lld nchunks=%d nalloc=%lld ld_crd=%lld ld_idx=%lld "
+             "ld_eci=%lld",
+             (long long)chunk0, (long long)nsrc, (long long)chunk_size,
+             nchunks,
+             (long long)nalloc, (long long)ld_crd, (long long)ld_idx,
+             (long long)ld_eci);
+  MV_REQUIRE(chunk0 + nsrc < (int64_t)INT32_MAX &&
+                 chunk_size < (int64_t)INT32_MAX,
+             "mv_rotate_cull_chunks: source index exceeds int32");
+  const size_t need =
+      (size_t)nchunks * mv_rotate_cull_workspace_bytes(chunk_size);
+  MV_REQUIRE(ws_bytes >= need,
+             "mv_rotate_cull_chunks: workspace too small (%zu < %zu)",
+             ws_bytes, need);
+  const CullChunks K = {chunk0, chunk_size, nsrc, nalloc, 3 * ld_crd, ld_idx,
+                        (int)cdiv(chunk_size, kItemsPerBlock)};
+  return run_cull<double>(eci, ld_eci, load_mat(rot9), nullptr, K, nchunks,
+                          (int32_t *)workspace, n_up_dev, crd_out, ld_crd,
+                          nullptr, idx_out, as_stream(stream));
 }
 
 // ------------------------------------------------- coherency (polarized sky)

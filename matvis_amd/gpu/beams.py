@@ -102,10 +102,13 @@ class DeviceBeamSet:
         return np.sqrt(amax) if self.is_power else amax
 
     def eval(self, crd, ld_crd: int, count: int, out, ld_out: int,
-             n_dev=None, stream=None):
-        """A (nbeam, nfeed, nax, ld_out) at topocentric vectors crd (3, ld)."""
+             n_dev=None, stream=None, nchunks: int = 1, crd_stride: int = 0,
+             out_stride: int = 0):
+        """A (nbeam, nfeed, nax, ld_out) at topocentric vectors crd (3, ld),
+        of nchunks chunks (their counts n_dev, the arrays *_stride elements
+        apart) in one launch; the za bands take one chunk."""
         crd_is_f64 = int(crd.dtype == torch.float64)
-        if self.use_interp and self.banded:
+        if self.use_interp and self.banded and nchunks == 1:
             need = lib().mv_beam_interp_banded_workspace_bytes(
                 int(self.is_f64), self.nza, self.naz, count)
             if self._band_ws is None or self._band_ws.numel() < need:
@@ -117,16 +120,17 @@ class DeviceBeamSet:
                  D.ptr(out), ld_out, D.ptr(self._band_ws),
                  self._band_ws.numel(), D.stream_ptr(stream))
         elif self.use_interp:
-            call("mv_beam_interp", D.ptr(self.planes), int(self.is_f64),
-                 self.nbeam, self.nfeed, self.nax, self.nza, self.naz,
-                 D.ptr(self.grid), self.order, int(self.is_power), D.ptr(crd),
-                 crd_is_f64, ld_crd, count, D.ptr(n_dev), D.ptr(out), ld_out,
+            call("mv_beam_interp_chunks", D.ptr(self.planes),
+                 int(self.is_f64), self.nbeam, self.nfeed, self.nax, self.nza,
+                 self.naz, D.ptr(self.grid), self.order, int(self.is_power),
+                 D.ptr(crd), crd_is_f64, ld_crd, crd_stride, count, nchunks,
+                 D.ptr(n_dev), D.ptr(out), ld_out, out_stride,
                  D.stream_ptr(stream))
         else:
-            call("mv_beam_gaussian", D.ptr(self.sigma), self.nbeam,
-                 int(self.polarized), D.ptr(crd), crd_is_f64, ld_crd, count,
-                 D.ptr(n_dev), D.ptr(out), int(self.is_f64), ld_out,
-                 D.stream_ptr(stream))
+            call("mv_beam_gaussian_chunks", D.ptr(self.sigma), self.nbeam,
+                 int(self.polarized), D.ptr(crd), crd_is_f64, ld_crd,
+                 crd_stride, count, nchunks, D.ptr(n_dev), D.ptr(out),
+                 int(self.is_f64), ld_out, out_stride, D.stream_ptr(stream))
         return out
 
 

@@ -48,6 +48,9 @@ Z_PAD = 32  # mv_zmat_fused pads Z columns to a multiple of this
 BATCH_BYTES = 1 << 30
 
 
+#: chunks a launch takes (a grid dimension)
+MAX_GRID = 65535
+
 #: a time's output that one host thread copies
 HOST_COPY_BYTES = 4 << 20
 
@@ -89,7 +92,7 @@ def device_bytes(*, form: int, nterms: int, nprod: int, nant: int,
         "coords": nsrc * (24 + 3 * rsz + 24 + 24 + 16 + 8)
         + nsrc_alloc * (3 * rsz + 4 * 16 + 4) + cull_ws,
         "antpos_flux": nant * 24 + nfreq * nsrc * 8,
-        "chunk_coords": nchunks * seg * (24 + 4) + cull_ws,
+        "chunk_coords": nchunks * (seg * (24 + 4) + cull_ws),
         "beam_tables": beam_sets * nbeam * nf * nf * beam_pixels * esz,
         "beam_values": (nchunks if beam_sets == 1 else nb) * nbeam * nf * nf
         * seg * esz,
@@ -187,7 +190,8 @@ class VisibilityEngine:
         self.crd = list(D.empty((nb, 3, seg), np.float64))
         self.idx = list(D.empty((nb, seg), np.int32))
         self.n_up = D.zeros((2, nb), np.int32)
-        ws = lib().mv_rotate_cull_workspace_bytes(self.chunk_size)
+        ws = (min(nb, MAX_GRID)
+              * lib().mv_rotate_cull_workspace_bytes(self.chunk_size))
         self.rot_ws = D.empty((ws,), np.uint8)
         # beams: one table set per distinct frequency response
         self.beam_ctype = np.complex128 if self.form == FORM_C128 else np.complex64
@@ -285,17 +289,20 @@ class VisibilityEngine:
         sp = D.stream_ptr(stream)
         nup = self.n_up[parity]
         shared = len(self.beam_sets) == 1
-        for c in range(self.nchunks):
+        for c in range(0, self.nchunks, MAX_GRID):
+            n = min(self.nchunks - c, MAX_GRID)
             chunk0 = min(c * self.chunk_size, self.nsrc)
-            clen = max(0, min(self.chunk_size, self.nsrc - chunk0))
-            call("mv_rotate_cull", D.ptr(src), self.nsrc, rot.ctypes.data,
-                 None, chunk0, clen, self.nsrc_alloc, D.ptr(self.crd[c]),
-                 self.seg, None, 1, D.ptr(self.idx[c]), D.ptr(nup[c:c + 1]),
+            clen = min(n * self.chunk_size, self.nsrc - chunk0)
+            call("mv_rotate_cull_chunks", D.ptr(src), self.nsrc,
+                 rot.ctypes.data, chunk0, clen, max(1, self.chunk_size), n,
+                 self.nsrc_alloc, D.ptr(self.crd[c]), self.seg,
+                 D.ptr(self.idx[c]), self.seg, D.ptr(nup[c:c + 1]),
                  D.ptr(self.rot_ws), self.rot_ws.numel(), sp)
             if shared:
-                self.beam_sets[0].eval(self.crd[c], self.seg, self.nsrc_alloc,
-                                       self.A[c], self.seg, nup[c:c + 1],
-                                       stream)
+                self.beam_sets[0].eval(
+                    self.crd[c], self.seg, self.nsrc_alloc, self.A[c],
+                    self.seg, nup[c:c + 1], stream, n, 3 * self.seg,
+                    self.A[c].numel())
         self._parity = parity
 
     def stage_z(self, fi: int, c: int, stream=None):

@@ -715,6 +715,53 @@ def test_cull_at_the_scan_boundary(nsrc):
     assert np.array_equal(D.to_host(crd)[2, :n], z[want])
 
 
+@pytest.mark.parametrize("size,nchunks,nsrc", [
+    (1, 3, 2), (255, 4, 1000), (2048, 3, 4097), (2049, 2, 4098),
+    (8192, 3, 20000), (8193, 3, 20000), (4096, 2, 100)])
+def test_cull_chunks(size, nchunks, nsrc):
+    """Chunks in one launch (a block to many a chunk, each side of the single
+    launch's limit, short and empty last chunks): the counts, order,
+    coordinates and zeroed tails of each; and their beams in one launch, with
+    the bits of a launch a chunk."""
+    from matvis_amd.beams import GaussianBeam
+    from matvis_amd.gpu.beams import DeviceBeamSet
+    rng = np.random.default_rng(size)
+    first = 7
+    eci = rng.normal(size=(3, first + nsrc))
+    eci /= np.linalg.norm(eci, axis=0)
+    rot = np.ascontiguousarray(np.linalg.qr(rng.normal(size=(3, 3)))[0])
+    topo = O.rotate(rot, eci)
+    src, ld = _dev(eci), size + 3
+    crd = D.zeros((nchunks, 3, ld), np.float64) - 7.0
+    idx, nup = D.zeros((nchunks, ld), np.int32) - 7, D.zeros((nchunks,), np.int32)
+    ws = D.empty((nchunks * lib().mv_rotate_cull_workspace_bytes(size),),
+                 np.uint8)
+    call("mv_rotate_cull_chunks", D.ptr(src), first + nsrc, rot.ctypes.data,
+         first, nsrc, size, nchunks, size, D.ptr(crd), ld, D.ptr(idx), ld,
+         D.ptr(nup), D.ptr(ws), ws.numel(), D.stream_ptr())
+    c, i, n = D.to_host(crd), D.to_host(idx), D.to_host(nup)
+    for k in range(nchunks):
+        lo, hi = first + k * size, first + min(nsrc, (k + 1) * size)
+        want = lo + np.flatnonzero(topo[2, lo:max(lo, hi)] > 0)
+        assert n[k] == want.size
+        assert np.array_equal(i[k, :n[k]], want)
+        assert (i[k, n[k]:size] == -1).all() and (i[k, size:] == -7).all()
+        assert np.array_equal(c[k, :, :n[k]], topo[:, want])
+        assert (c[k, :, n[k]:size] == 0).all() and (c[k, :, size:] == -7).all()
+    for beams in ([synth.harmonic_efield_beam(seed=1, naz=36, nza=10,
+                                              polarized=True,
+                                              dtype=np.complex128)],
+                  [GaussianBeam(diameter=14.0)]):
+        t = DeviceBeamSet(beams, 1.5e8, True, np.complex64, 3)
+        one = D.zeros((nchunks, t.nbeam, 2, 2, ld), np.complex64)
+        many = D.zeros((nchunks, t.nbeam, 2, 2, ld), np.complex64)
+        for k in range(nchunks):
+            t.eval(crd[k], ld, size, one[k], ld, nup[k:k + 1])
+        t.eval(crd, ld, size, many, ld, nup, None, nchunks, 3 * ld,
+               one[0].numel())
+        assert np.array_equal(D.to_host(one), D.to_host(many))
+
+
 @pytest.mark.parametrize("is_f64", [True, False])
 def test_phase_in_every_quadrant(is_f64):
     """exp(2 pi i b.s nu / c) at multiples of 1/8 turn and around them, up to
