@@ -328,17 +328,6 @@ __host__ __device__ inline WavePair group_wave(int g, int n, int w) {
 }
 template <int V> using Int = std::integral_constant<int, V>;
 
-// K tiles a stage holds.  The only group of n = 1 or 2 panels would leave three
-// or two of a stage's four panel slots empty: they hold the same panels of the
-// next K tiles instead, so that every wave copies and as much is in flight as
-// for four panels: these groups wait for copies more than for MFMAs (30% busy
-// before).  Panel p of a stage's q-th K tile is in slot q n + p.
-// Measured, 16 frequencies of 128 antennas x 30k sources, two terms: HERK 160
-// -> 145 us, a time 321 -> 306; m = 32 complex64, 3.5 K tiles a slice: the same.
-__host__ __device__ inline int stage_tiles(int n) {
-  return n == 1 ? 4 : n == 2 ? 2 : 1;
-}
-
 // First row and column quadrant of a part.
 __host__ __device__ inline int part_row(int part) {
   return part == kBottom || part == kQuad11 ? 1 : 0;
@@ -466,14 +455,9 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, rl = lane & 15;
-  WavePair wp = group_wave(group, Q.n, wave);
+  const WavePair wp = group_wave(group, Q.n, wave);
   const int kt0 = (int)((int64_t)slice * ktiles / ns);
   const int kt1 = (int)((int64_t)(slice + 1) * ktiles / ns);
-  // K tiles a stage, and which of them this wave copies (64-row panels are
-  // three or more)
-  const int tps = P == 32 ? stage_tiles(Q.n) : 1;
-  const int mine = tps > 1 ? wave / Q.n : 0;
-  if (tps > 1) wp.load = wave - mine * Q.n;
 
   // this lane's part of copy u: row u 1024 / RB + lane / CH of the panel,
   // LDS chunk lane % CH, i.e. logical chunk (lane % CH) ^ swz(row)
@@ -488,11 +472,10 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
       off[u] = (uint32_t)((int64_t)gr * Q.ldz * (2 * (int)sizeof(T)) / 16) + c;
     }
   }
-  int sg = (kt0 + mine) / (kps > 0 ? kps : 1), kc = kt0 + mine - sg * kps;
-  // the stage of K tiles kt .. kt + tps - 1
-  auto copy = [&](PlainStage<T, P> &D, int kt) {
+  int sg = kt0 / (kps > 0 ? kps : 1), kc = kt0 - sg * kps;
+  auto copy = [&](PlainStage<T, P> &D) {
     const int64_t c0 = (int64_t)kc * PK;
-    if (wp.load >= 0 && kt + mine < kt1) {
+    if (wp.load >= 0) {
       const cplx<T> *src = Q.z + sg * Q.seg_stride + c0;
       if (c0 + PK <= seg_len) {
         if (Q.wide) {
@@ -525,19 +508,19 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
         }
       }
     }
-    for (kc += tps; kc >= kps; kc -= kps) ++sg;
+    if (++kc == kps) {
+      kc = 0;
+      ++sg;
+    }
   };
 
   // The K loop of a wave that computes NI rows and NJ columns of blocks from
-  // (oi, oj), without those below the diagonal where DIAG; MULTI: of stages of
-  // several K tiles.  A loop for each
+  // (oi, oj), without those below the diagonal where DIAG.  A loop for each
   // part: the waves of a group run different ones, with the same barriers.
   // (Branches around the parts' MFMAs within one loop spill accumulators.)
-  auto run = [&](auto ni_, auto nj_, auto diag_, auto multi_, int oi, int oj) {
+  auto run = [&](auto ni_, auto nj_, auto diag_, int oi, int oj) {
     constexpr int NI = decltype(ni_)::value, NJ = decltype(nj_)::value;
     constexpr bool DIAG = decltype(diag_)::value;
-    constexpr bool MULTI = decltype(multi_)::value;
-    const int step_tiles = MULTI ? tps : 1;
     constexpr int kSets = sizeof(T) == 4 && P == 32 ? 2 : 1;
     acc_t t1[kSets][NI][NJ], t2[kSets][NI][NJ], t3[kSets][NI][NJ];
 #pragma unroll
@@ -548,9 +531,8 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
         for (int j = 0; j < NJ; ++j)
           t1[q][i][j] = t2[q][i][j] = t3[q][i][j] = acc_t{};
 
-    auto compute = [&](const PlainStage<T, P> &D, int slot0) {
-      const char *A = D.x[slot0 + wp.si] + oi * 16 * RB,
-                 *B = D.x[slot0 + wp.sj] + oj * 16 * RB;
+    auto compute = [&](const PlainStage<T, P> &D) {
+      const char *A = D.x[wp.si] + oi * 16 * RB, *B = D.x[wp.sj] + oj * 16 * RB;
 #pragma unroll
       for (int ks = 0; ks < PK / 4; ++ks) {
         const int pos = plain_pos<T>(rl, 4 * ks + g);
@@ -580,22 +562,14 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
     };
     // one stage computed from C while the next is copied into N
     auto step = [&](PlainStage<T, P> &C, PlainStage<T, P> &N, int kt) {
-      if (kt + step_tiles < kt1) copy(N, kt + step_tiles);
-      if (wp.i >= 0) {
-        if constexpr (MULTI) {
-          const int left = kt1 - kt, tiles = left < tps ? left : tps;
-#pragma unroll 1
-          for (int q = 0; q < tiles; ++q) compute(C, q * Q.n);
-        } else {
-          compute(C, 0);
-        }
-      }
+      if (kt + 1 < kt1) copy(N);
+      if (wp.i >= 0) compute(C);
       wait_global_loads();  // this wave's copies into N
       lds_barrier();
     };
-    for (int kt = kt0; kt < kt1; kt += 2 * step_tiles) {
+    for (int kt = kt0; kt < kt1; kt += 2) {
       step(L0, L1, kt);
-      if (kt + step_tiles < kt1) step(L1, L0, kt + step_tiles);
+      if (kt + 1 < kt1) step(L1, L0, kt + 1);
     }
     // every wave is past the last barrier: LDS is free for the next item
 
@@ -628,21 +602,17 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
       }
   };
 
-  if (kt0 < kt1) copy(L0, kt0);
+  if (kt0 < kt1) copy(L0);
   wait_global_loads();
   lds_barrier();
   constexpr int HB = NB / 2;  // blocks a quadrant's side
   constexpr Int<NB> whole{};
   constexpr Int<HB> half{};
   const int oi = part_row(wp.part) * HB, oj = part_col(wp.part) * HB;
-  auto parts = [&](auto multi) {
-    if (wp.part == kDiagonal) run(whole, whole, Int<1>{}, multi, 0, 0);
-    else if (wp.part <= kBottom) run(half, whole, Int<0>{}, multi, oi, 0);
-    else run(half, half, Int<0>{}, multi, oi, oj);
-  };
-  if (wp.part == kWhole) run(whole, whole, Int<0>{}, Int<0>{}, 0, 0);
-  else if (tps == 1) parts(Int<0>{});
-  else if constexpr (P == 32) parts(Int<1>{});
+  if (wp.part == kWhole) run(whole, whole, Int<0>{}, 0, 0);
+  else if (wp.part == kDiagonal) run(whole, whole, Int<1>{}, 0, 0);
+  else if (wp.part <= kBottom) run(half, whole, Int<0>{}, oi, 0);
+  else run(half, half, Int<0>{}, oi, oj);
 }
 
 // Workgroups a CU holds (kPStageK).
@@ -869,10 +839,6 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
   }
   const int kt0 = (int)((int64_t)slice * ktiles / ns);
   const int kt1 = (int)((int64_t)(slice + 1) * ktiles / ns);
-  // K tiles a stage, and which of them this wave copies
-  const int tps = WAVES > 1 ? stage_tiles(P.nb) : 1;
-  const int mine = tps > 1 ? wave / P.nb : 0;
-  if (tps > 1) wp.load = wave - mine * P.nb;
   // copy lanes: run u covers rows 16 u .. 16 u + 15 of the wave's part of the
   // panel; lane l fills LDS chunk l % 4 of row 16 u + l / 4, i.e. logical
   // chunk (l % 4) ^ swz(row) of that row
@@ -907,26 +873,28 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
   // position of the K tile to copy next: segment sg, tile kc within it;
   // whole K tiles: columns [seg_len, round_up(seg_len, 16)) of every
   // segment are zero by contract
-  int sg = (kt0 + mine) / (kps > 0 ? kps : 1), kc = kt0 + mine - sg * kps;
+  int sg = kt0 / (kps > 0 ? kps : 1), kc = kt0 - sg * kps;
   const int64_t seg_tiles = P.seg_stride / kSK;
-  // the stage of K tiles kt .. kt + tps - 1
-  auto copy = [&](Stage &D, int kt) {
+  auto copy = [&](Stage &D) {
     const int64_t k0 = (sg * seg_tiles + kc) * P.ldz * kSK;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int u = 0; u < kRuns; ++u) {
         const int run = (row0 + u * 16) * kSK;
-        if (WAVES == 1 || (wp.load >= 0 && kt + mine < kt1))
+        if (WAVES == 1 || wp.load >= 0)
           copy16_to_lds(P.t[t] + k0 + coff[0][u], &D.x[wave][t][run]);
         if (WAVES == 1 && second >= 0)
           copy16_to_lds(P.t[t] + k0 + coff[kPanels - 1][u], &D.x[1][t][run]);
       }
-    for (kc += tps; kc >= kps; kc -= kps) ++sg;
+    if (++kc == kps) {
+      kc = 0;
+      ++sg;
+    }
   };
   // thread t: quarter t % 4 (4 columns) of row t / 4, and with one wave the
   // rows 16, 32, 48 further on
-  auto diag_sums = [&](const Stage &D, int slot0) {
+  auto diag_sums = [&](const Stage &D) {
 #pragma unroll
     for (int w = 0; w < kNorms; ++w) {
       if (dslot[w] < 0) continue;
@@ -936,7 +904,7 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
         u32x4 r[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t)
-          r[t] = *(const u32x4 *)&D.x[slot0 + dslot[w]][t][lds_word(row, (lane & 3) * 4)];
+          r[t] = *(const u32x4 *)&D.x[dslot[w]][t][lds_word(row, (lane & 3) * 4)];
         if constexpr (WAVES > 1) dsum[w] += row_norm2<NT, F16>(r);
         else dsum1[q] += row_norm2<NT, F16>(r);
       }
@@ -961,15 +929,12 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
     }
   };
   // The K loop of a wave that computes NI x NJ blocks from block (oi, oj),
-  // without the one below the diagonal where DIAG; MULTI: of stages of several
-  // K tiles.  A loop for each part: the
+  // without the one below the diagonal where DIAG.  A loop for each part: the
   // waves of a group run different ones, with the same barriers.  (Branches
   // around the parts' MFMAs within one loop spill accumulators.)
-  auto run = [&](auto ni_, auto nj_, auto diag_, auto multi_, int oi, int oj) {
+  auto run = [&](auto ni_, auto nj_, auto diag_, int oi, int oj) {
     constexpr int NI = decltype(ni_)::value, NJ = decltype(nj_)::value;
     constexpr bool DIAG = decltype(diag_)::value;
-    constexpr bool MULTI = decltype(multi_)::value;
-    const int step_tiles = MULTI ? tps : 1;
     v16f acc_re[NI][NJ], acc_im[NI][NJ];
 #pragma unroll
     for (int i = 0; i < NI; ++i)
@@ -980,9 +945,9 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
       }
 
     // the MFMAs of one K tile from stage D
-    auto compute = [&](const Stage &D, int slot0) {
-      const uint32_t(*Ax)[kSP * kSK] = D.x[slot0 + wp.si];
-      const uint32_t(*Bx)[kSP * kSK] = D.x[slot0 + wp.sj];
+    auto compute = [&](const Stage &D) {
+      const uint32_t(*Ax)[kSP * kSK] = D.x[wp.si];
+      const uint32_t(*Bx)[kSP * kSK] = D.x[wp.sj];
       // lane half lh reads term t_lh at word offset w_lh of its row
       auto ld_a = [&](int t0, int t1, int w0, int w1, u32x4 (&a)[NI]) {
         const uint32_t *base = Ax[lh ? t1 : t0] + oi * 32 * kSK;
@@ -1056,31 +1021,22 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
     };
     // one K tile computed from stage C while the next is copied into N
     auto step = [&](Stage &C, Stage &N, int kt) {
-      if (kt + step_tiles < kt1) copy(N, kt + step_tiles);
-      auto tile = [&](int slot0) {
-        if (any_diag) diag_sums(C, slot0);
-        if (WAVES == 1 || wp.i >= 0) {
-          // issue priority to waves in their MFMA phase over waves copying or
-          // waiting at the barrier
-          __builtin_amdgcn_s_setprio(1);
-          compute(C, slot0);
-          __builtin_amdgcn_s_setprio(0);
-        }
-      };
-      if constexpr (MULTI) {
-        const int left = kt1 - kt, tiles = left < tps ? left : tps;
-#pragma unroll 1
-        for (int q = 0; q < tiles; ++q) tile(q * P.nb);
-      } else {
-        tile(0);
+      if (kt + 1 < kt1) copy(N);
+      if (any_diag) diag_sums(C);
+      if (WAVES == 1 || wp.i >= 0) {
+        // issue priority to waves in their MFMA phase over waves copying or
+        // waiting at the barrier
+        __builtin_amdgcn_s_setprio(1);
+        compute(C);
+        __builtin_amdgcn_s_setprio(0);
       }
       wait_global_loads();  // this wave's copies into N
       lds_barrier();
     };
 
-    for (int kt = kt0; kt < kt1; kt += 2 * step_tiles) {
+    for (int kt = kt0; kt < kt1; kt += 2) {
       step(L0, L1, kt);
-      if (kt + step_tiles < kt1) step(L1, L0, kt + step_tiles);
+      if (kt + 1 < kt1) step(L1, L0, kt + 1);
     }
     // every wave is past the last barrier: LDS is free for the next item
     if (any_diag) store_norms();
@@ -1134,21 +1090,16 @@ __device__ __forceinline__ void split_item(const SplitProblem &P, int slice,
       }
   };
 
-  if (kt0 < kt1) copy(L0, kt0);
+  if (kt0 < kt1) copy(L0);
   wait_global_loads();
   lds_barrier();
   const int oi = part_row(wp.part), oj = part_col(wp.part);
-  auto parts = [&](auto multi) {
-    if (wp.part == kDiagonal) run(Int<2>{}, Int<2>{}, Int<1>{}, multi, 0, 0);
-    else if constexpr (WAVES > 1) {
-      if (wp.part <= kBottom) run(Int<1>{}, Int<2>{}, Int<0>{}, multi, oi, 0);
-      else run(Int<1>{}, Int<1>{}, Int<0>{}, multi, oi, oj);
-    }
-  };
-  if (wp.part == kWhole)
-    run(Int<2>{}, Int<2>{}, Int<0>{}, Int<0>{}, 0, 0);
-  else if (tps == 1) parts(Int<0>{});
-  else if constexpr (WAVES > 1) parts(Int<1>{});
+  if (wp.part == kWhole) run(Int<2>{}, Int<2>{}, Int<0>{}, 0, 0);
+  else if (wp.part == kDiagonal) run(Int<2>{}, Int<2>{}, Int<1>{}, 0, 0);
+  else if constexpr (WAVES > 1) {
+    if (wp.part <= kBottom) run(Int<1>{}, Int<2>{}, Int<0>{}, oi, 0);
+    else run(Int<1>{}, Int<1>{}, Int<0>{}, oi, oj);
+  }
 }
 
 // One split HERK: K tiles and the slice count from the device column count,

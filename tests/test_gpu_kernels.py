@@ -322,38 +322,6 @@ def test_herk_plain_panel_edges(m, form):
     assert err < (1e-13 if form == FORM_C128 else 2e-6), err
 
 
-@pytest.mark.parametrize("form,nterms,nprod,bound",
-                         [(FORM_C128, 1, 1, 1e-13), (FORM_C64, 1, 1, 2e-6),
-                          (FORM_SPLIT_BF16, 2, 3, 6e-6),
-                          (FORM_SPLIT_BF16, 3, 6, 1e-6)])
-@pytest.mark.parametrize("panels", [1, 2])
-def test_herk_stages_of_several_k_tiles(panels, form, nterms, nprod, bound):
-    """Groups of one or two panels take four or two K tiles a stage: slices
-    whose K tiles fill the last stage or not, over two segments that end
-    within a stage (bounds of the panel-edge tests)."""
-    split = nterms > 1
-    m = panels * (64 if split else 32) - 3
-    for n, nslices in ((9, 1), (16, 1), (55, 1), (55, 3), (77, 1), (150, 2),
-                       (203, 7)):
-        seg = -(-n // 16) * 16
-        rng = np.random.default_rng(n)
-        z = ((0.5 + rng.uniform(size=(m, 2 * seg)))
-             * np.exp(2j * np.pi * rng.uniform(size=(m, 2 * seg))))
-        z[:, n:seg] = z[:, seg + n:] = 0
-        z = z.astype(np.complex128 if form == FORM_C128 else np.complex64)
-        if split:
-            ts, ncols = _split_terms(z, form, nterms)
-            h, v = _run_herk(form, ts, m, m, 2, seg, n, nterms, nprod,
-                             nslices=nslices)
-        else:
-            h, v = _run_herk(form, [_dev(z)], m, 2 * seg, 2, seg, n,
-                             nslices=nslices)
-        want = z.astype(np.complex128).conj() @ z.astype(np.complex128).T
-        d = np.sqrt(np.diag(want).real)
-        err = (np.abs(_vis_full(h, v, m) - want) / (d[:, None] * d[None])).max()
-        assert err < bound, (n, nslices, err)
-
-
 def test_herk_segments_and_device_length():
     m, seg, n = 70, 48, 37
     z = _herk_case(m, 2 * seg, np.complex128, seed=9)
