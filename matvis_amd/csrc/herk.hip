@@ -418,17 +418,20 @@ __host__ __device__ inline int plain_wide(const PlainProblem<T> &Q, int nseg) {
 // the matrix cores bind this kernel, and the sums and differences are one
 // VALU instruction an operand.  The accumulators' chains are half as long as
 // four products' (K / 4 MFMAs, not K / 2), which offsets the third term of
-// Im.  FP32 chains are cut further: two accumulator sets over alternate
-// columns at P = 32 (kSets), half as many K tiles a slice (form_cmax).
+// Im.  Chains are cut further: in FP32 two accumulator sets over alternate
+// columns at P = 32 (kSets) and half as many K tiles a slice, in FP64 64 K
+// tiles a slice (form_cmax).
 // Errors |dV| / |V| (2-norms) of four products -> these: complex64 against
 // FP64, incoherent Z 0.9-2.8e-7 -> 0.8-2.3e-7, nearly coherent Z (phases
 // within 0.3 rad) 1.9-6.3e-8 -> 1.9-5.4e-8, a whole time of the 350-antenna
-// sky 8.4e-7 -> 3.8e-7; complex128 against extended precision, incoherent
-// 2.0-2.8e-16 -> 1.9-2.9e-16, nearly coherent 0.8-1.5e-16 -> 0.9-1.8e-16,
-// the whole time 9.9e-15 (its phases) in both.  The diagonal is exactly real.
+// sky 8.4e-7 -> 3.8e-7; complex128 against extended precision, off the
+// diagonal, incoherent Z, m = 700 and 12k, 30k, 60k columns 1.3, 1.7, 2.1e-15
+// -> 1.4, 1.3, 1.5e-15, m = 130, 60k 1.4e-15 in both, m = 64, 600 2.3e-16 ->
+// 2.6e-16; the whole time 9.9e-15 (its phases) in both.  The diagonal is
+// exactly real.
 //
 // Measured, m = 700 (350 antennas, polarized): FP64, 29.9k sources up, 2.47
-// -> 1.48 ms; FP32, 59.7k sources, 2.71 -> 1.51 ms: 80% of the rate of
+// -> 1.50 ms; FP32, 59.7k sources, 2.71 -> 1.51 ms: 80% of the rate of
 // three products at the peak (78.6 and 157 TFLOP/s), from 63% and 58% of four
 // products'.  Square tiles, copies through registers with a mask on every
 // element and half of each operand read thrown away made the difference.
