@@ -419,14 +419,14 @@ __host__ __device__ inline int plain_wide(const PlainProblem<T> &Q, int nseg) {
 // VALU instruction an operand.  The accumulators' chains are half as long as
 // four products' (K / 4 MFMAs, not K / 2), which offsets the third term of
 // Im.  Chains are cut further: in FP32 two accumulator sets over alternate
-// columns at P = 32 (kSets) and half as many K tiles a slice, in FP64 64 K
+// columns at P = 32 (kSets) and half as many K tiles a slice, in FP64 96 K
 // tiles a slice (form_cmax).
 // Errors |dV| / |V| (2-norms) of four products -> these: complex64 against
 // FP64, incoherent Z 0.9-2.8e-7 -> 0.8-2.3e-7, nearly coherent Z (phases
 // within 0.3 rad) 1.9-6.3e-8 -> 1.9-5.4e-8, a whole time of the 350-antenna
 // sky 8.4e-7 -> 3.8e-7; complex128 against extended precision, off the
 // diagonal, incoherent Z, m = 700 and 12k, 30k, 60k columns 1.3, 1.7, 2.1e-15
-// -> 1.4, 1.3, 1.5e-15, m = 130, 60k 1.4e-15 in both, m = 64, 600 2.3e-16 ->
+// -> 1.4, 1.6, 1.7e-15, m = 130, 60k 1.4e-15 in both, m = 64, 600 2.3e-16 ->
 // 2.6e-16; the whole time 9.9e-15 (its phases) in both.  The diagonal is
 // exactly real.
 //
@@ -1570,13 +1570,14 @@ int split_maxord(int nterms, int nprod) {
 // partial tiles written per launch stay small.
 int form_cmax(int form) {
   switch (form) {
-    // FP64 has no such limit; slices of 64 K tiles keep the three-product sums
-    // (longer terms than the four products') no less accurate than those were:
-    // incoherent Z off the diagonal, m = 700, 30k columns, one slice a slot
-    // 2.3e-15, 128 tiles 1.6e-15, 64 tiles 1.3e-15 (four products 1.7e-15), 60k
-    // 1.9, 1.5 (2.1); nearly coherent Z, 60k, 64 tiles 2.1e-16 (3.3e-16).  It
-    // takes 2% (350 antennas, 29.9k sources up, 3 frequencies 4.82 -> 4.92 ms).
-    case MV_FORM_C128: return 64;
+    // FP64 has no such limit; slices of 96 K tiles keep the three-product sums
+    // (longer terms than the four products') no less accurate than those were.
+    // Off the diagonal, m = 700, incoherent Z, 30k columns: one slice a slot
+    // 2.3e-15, 96 tiles 1.6e-15, 64 tiles 1.3e-15 (four products 1.7e-15); 60k
+    // 96 tiles 1.7, 64 tiles 1.5 (2.1); nearly coherent Z, 60k, 96 tiles
+    // 2.3e-16 (3.3e-16).  350 antennas, 29.9k sources up, 3 frequencies: one
+    // slice a slot 4.77 ms, 96 tiles 4.86, 64 tiles 4.91.
+    case MV_FORM_C128: return 96;
     case MV_FORM_C64: return 128;
     default: return 192;
   }
