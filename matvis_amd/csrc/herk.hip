@@ -64,6 +64,8 @@ struct SliceCfg {
   int slots;       // workgroups resident at once (multiple of kXcd)
   int cmax;        // at most this many K tiles per slice
   int ovh;         // per-item cost beyond its K tiles, in K-tile units
+  int spread;      // an instance that leaves slots idle: at most
+                   // sqrt(spread x K tiles) slices
 };
 
 // Active slice count for `ktiles` K tiles over `ntiles` items a slice (panel
@@ -73,16 +75,19 @@ struct SliceCfg {
 // slice + per-item overhead), the smallest count on ties.  Where they cannot
 // (small_slices), a power of two: an instance that leaves slots idle shares
 // its launch with others (frequencies, HerkBatch), and counts that divide the
-// slots leave no nearly empty last round, at most sqrt(30 ktiles): a slice
+// slots leave no nearly empty last round, at most sqrt(spread ktiles): a slice
 // more costs its share of the reduce, about a thirtieth of the time of a K
 // tile in a launch that leaves most slots idle (3.5 us, FP64), and shortens
-// every chain by ktiles / ns^2 of them.  Pure integer
-// function of its arguments: the compute and reduce kernels and the host
-// agree on it.
+// every chain by ktiles / ns^2 of them, so that 30 is the cheapest.  The plain
+// forms take 120: their chains round once or twice a column, with 30 more than
+// with one slice a K tile (32 antennas, 3k sources in complex64: 7.8e-8 of |V|
+// against 6.5e-8), and the time is the same (m = 32, 1.8k columns 13.1 us in
+// both).
+// Pure integer function of its arguments: the compute and reduce kernels and
+// the host agree on it.
 // Measured, HERK and reduce of a time: 16 frequencies of 128 antennas, 1,866
 // K tiles, 72 -> 64 slices (1,152 -> 1,024 items for 512 slots, and one launch
-// instead of two) 254 -> 214 us; 32 of 32 antennas, 113 K tiles, 57 -> 32
-// slices, 26.6 -> 26.9 us.
+// instead of two) 254 -> 214 us.
 __host__ __device__ inline void slice_range(int ktiles, const SliceCfg &c,
                                             int &lo, int &hi) {
   lo = icdiv(ktiles, c.cmax);
@@ -103,7 +108,8 @@ __host__ __device__ inline bool small_slices(int ktiles, int ntiles, int lo,
                                              int &ns) {
   if ((int64_t)ntiles * hi > c.slots) return false;
   ns = 1;
-  while (2 * ns <= hi && 4 * (int64_t)ns * ns <= 30 * (int64_t)ktiles) ns *= 2;
+  while (2 * ns <= hi && 4 * (int64_t)ns * ns <= (int64_t)c.spread * ktiles)
+    ns *= 2;
   if (ns < lo) ns = lo;
   return true;
 }
@@ -362,9 +368,9 @@ constexpr int kPT = 64;  // side the accumulator of the plain forms is padded to
 constexpr int kPK = 16;  // complex columns of a K tile as slices count them
 // Complex columns per LDS stage: 128 bytes a row.  FP64 stages of 8 columns
 // make 32 KB a workgroup, so that three share a CU (160 KB, 168 registers)
-// and the matrix cores have work while two wait for copies or operands:
-// m = 700, 29.9k sources, 16 columns and two workgroups 1.49 ms, 8 and two
-// 1.52, 8 and three 1.44 (1.27 at the rate a large FP64 product reaches).
+// and the matrix cores have work while two wait for copies or operands: m =
+// 700, 2 x 29.9k columns, 16 columns and two workgroups 1.49 ms, 8 and two 1.52,
+// 8 and three 1.44 (these with three real products a complex one).
 template <typename T> constexpr int kPStageK = sizeof(T) == 8 ? 8 : 16;
 
 // Bytes of a panel row in LDS (one stage) and the 16-byte chunks it has.
@@ -411,30 +417,29 @@ __host__ __device__ inline int plain_wide(const PlainProblem<T> &Q, int nseg) {
 // The P x P panel pairs of one (slice, group) item, each wave its own pair as
 // (P / 16)^2 blocks of 16x16.
 //
-// Three real products a complex one, conj(a + ib)(c + id):
-//   T1 = a c, T2 = b d, T3 = (a - b)(c + d): Re = T1 + T2, Im = T3 - T1 + T2,
-// one 16x16x4 MFMA each per 4 complex columns (lane group g = l / 16 supplies
-// column g), where the four products of the plain formula take four MFMAs:
-// the matrix cores bind this kernel, and the sums and differences are one
-// VALU instruction an operand.  The accumulators' chains are half as long as
-// four products' (K / 4 MFMAs, not K / 2), which offsets the third term of
-// Im.  Chains are cut further: in FP32 two accumulator sets over alternate
-// columns at P = 32 (kSets) and half as many K tiles a slice, in FP64 96 K
-// tiles a slice (form_cmax).
-// Errors |dV| / |V| (2-norms) of four products -> these: complex64 against
-// FP64, incoherent Z 0.9-2.8e-7 -> 0.8-2.3e-7, nearly coherent Z (phases
-// within 0.3 rad) 1.9-6.3e-8 -> 1.9-5.4e-8, a whole time of the 350-antenna
-// sky 8.4e-7 -> 3.8e-7; complex128 against extended precision, off the
-// diagonal, incoherent Z, m = 700 and 12k, 30k, 60k columns 1.3, 1.7, 2.1e-15
-// -> 1.4, 1.6, 1.7e-15, m = 130, 60k 1.4e-15 in both, m = 64, 600 2.3e-16 ->
-// 2.6e-16; the whole time 9.9e-15 (its phases) in both.  The diagonal is
-// exactly real.
+// Two real products over 2K reals, as the top of this file has them: one
+// 16x16x4 MFMA each per 2 complex columns, lane group g = l / 16 supplying part
+// g % 2 of column g / 2.  An imaginary part is thus a single chain whose terms
+// a d and -b c of a column follow one another: its partial sums, and with them
+// its rounding, stay as small as Im V is where the rows are nearly in phase
+// (short baselines, the feeds of one antenna).  Three real products a complex
+// one (Im as a difference of their sums) take a quarter fewer MFMAs, but round
+// Im at the size of |V|: phases within 0.01 rad, 60k columns, errors of Im /
+// |V| 2e-11 -> 8e-7 in complex64 and 5e-20 -> 1.4e-16 in complex128.  The
+// real part's chain, whose terms do add up, is cut into two over alternate
+// columns, and slices are short (form_cmax).
 //
-// Measured, m = 700 (350 antennas, polarized): FP64, 29.9k sources up, 2.47
-// -> 1.50 ms; FP32, 59.7k sources, 2.71 -> 1.51 ms: 80% of the rate of
-// three products at the peak (78.6 and 157 TFLOP/s), from 63% and 58% of four
-// products'.  Square tiles, copies through registers with a mask on every
-// element and half of each operand read thrown away made the difference.
+// Measured with the reduce, m = 700, 59.7k columns, against square tiles with
+// copies through registers, a mask on every element and half of each operand
+// read thrown away: FP64 2.39 -> 2.01 ms, FP32 1.34 -> 1.04 ms, 74% and 72% of
+// the peak (78.6 and 157 TFLOP/s); m = 64, 3.6k columns 26 -> 19 and 22 -> 16
+// us.  (Three products 1.50 and 0.78 ms.)
+// Errors against 64 bits (complex128: extended precision) over sqrt(V_ii
+// V_jj), m = 160, 60k columns, one chain a real part -> two and shorter slices:
+// Re, phases within 0.3 rad 6.6e-8 -> 3.7e-8 and 1.5e-16 -> 9.0e-17, incoherent
+// Z 2.1e-9 -> 1.6e-9 and 4.2e-18 -> 2.9e-18; Im as before (7e-10 and 1.4e-18,
+// incoherent 2e-9 and 4e-18).  A time of the 350-antenna sky in complex64
+// 9.6e-7 -> 3.7e-7 of |V|.  The diagonal is exactly real.
 //
 // Copies go straight from global memory into the other LDS stage
 // (global_load_lds: 16 bytes a lane where rows are 16-byte aligned, else 4),
@@ -524,39 +529,35 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
   auto run = [&](auto ni_, auto nj_, auto diag_, int oi, int oj) {
     constexpr int NI = decltype(ni_)::value, NJ = decltype(nj_)::value;
     constexpr bool DIAG = decltype(diag_)::value;
-    constexpr int kSets = sizeof(T) == 4 && P == 32 ? 2 : 1;
-    acc_t t1[kSets][NI][NJ], t2[kSets][NI][NJ], t3[kSets][NI][NJ];
+    acc_t re[2][NI][NJ], im[NI][NJ];
 #pragma unroll
-    for (int q = 0; q < kSets; ++q)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-          t1[q][i][j] = t2[q][i][j] = t3[q][i][j] = acc_t{};
+      for (int j = 0; j < NJ; ++j) re[0][i][j] = re[1][i][j] = im[i][j] = acc_t{};
 
     auto compute = [&](const PlainStage<T, P> &D) {
       const char *A = D.x[wp.si] + oi * 16 * RB, *B = D.x[wp.sj] + oj * 16 * RB;
 #pragma unroll
-      for (int ks = 0; ks < PK / 4; ++ks) {
-        const int pos = plain_pos<T>(rl, 4 * ks + g);
-        vec2 a[NI], b[NJ];
+      for (int ks = 0; ks < PK / 2; ++ks) {
+        const int pos = plain_pos<T>(rl, 2 * ks + (g >> 1));
+        T a[NI], bre[NJ], bim[NJ];
 #pragma unroll
         for (int i = 0; i < NI; ++i)
-          a[i] = *(const vec2 *)&A[i * 16 * RB + pos];
+          a[i] = ((const T *)&A[i * 16 * RB + pos])[g & 1];
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
-          b[j] = *(const vec2 *)&B[j * 16 * RB + pos];
+        for (int j = 0; j < NJ; ++j) {
+          const vec2 b = *(const vec2 *)&B[j * 16 * RB + pos];
+          bre[j] = g & 1 ? b[1] : b[0];
+          bim[j] = g & 1 ? -b[0] : b[1];
+        }
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
           for (int i = 0; i < NI; ++i) {
             if (DIAG && i > j) continue;
-            constexpr int S = kSets - 1;
-            acc_t &x = t1[ks & S][i][j], &y = t2[ks & S][i][j],
-                  &z = t3[ks & S][i][j];
-            x = PlainMfma<T>::op(a[i][0], b[j][0], x);
-            y = PlainMfma<T>::op(a[i][1], b[j][1], y);
-            z = PlainMfma<T>::op(a[i][0] - a[i][1], b[j][0] + b[j][1], z);
+            acc_t &x = re[ks & 1][i][j], &y = im[i][j];
+            x = PlainMfma<T>::op(a[i], bre[j], x);
+            y = PlainMfma<T>::op(a[i], bim[j], y);
           }
         // operand reads stay in their step: hoisted over the unrolled steps
         // they would spill (the other waves of the SIMD cover their latency)
@@ -593,15 +594,9 @@ __device__ __forceinline__ void plain_item(const PlainProblem<T> &Q,
       for (int j = 0; j < NJ; ++j) {
         if (DIAG && i > j) continue;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          T x = t1[0][i][j][r], y = t2[0][i][j][r], w = t3[0][i][j][r];
-          if constexpr (kSets == 2) {
-            x += t1[1][i][j][r];
-            y += t2[1][i][j][r];
-            w += t3[1][i][j][r];
-          }
-          out[i * 16 * P + r * rstep + j * 16] = cplx<T>{x + y, (w - x) + y};
-        }
+        for (int r = 0; r < 4; ++r)
+          out[i * 16 * P + r * rstep + j * 16] =
+              cplx<T>{re[0][i][j][r] + re[1][i][j][r], im[i][j][r]};
       }
   };
 
@@ -1563,22 +1558,19 @@ int split_maxord(int nterms, int nprod) {
   return -1;
 }
 
-// Longest FP32 accumulation chain per slice, in K tiles of 16 columns.  The
-// split forms' diagonal is summed exactly, and off the diagonal the FP32
+// Longest accumulation chain per slice, in K tiles of 16 columns, for m rows.
+// The split forms' diagonal is summed exactly, and off the diagonal the FP32
 // chain error stays near 1e-7 relative at 62 tiles and grows about as the
 // square root of the length; 192 tiles keeps it well under 1e-6 while the
-// partial tiles written per launch stay small.
-int form_cmax(int form) {
+// partial tiles written per launch stay small.  The plain forms' real parts grow
+// with the length in the same way, in FP64 too: with two chains of 96 K tiles
+// 9.0e-17 of sqrt(V_ii V_jj) where one slice a slot in one chain gave 1.5e-16
+// (m = 160, 60k columns, phases within 0.3 rad), and the workspace of 96 is what
+// long sums already take.  Problems of few rows write few partials: 64.
+int form_cmax(int form, int m) {
   switch (form) {
-    // FP64 has no such limit; slices of 96 K tiles keep the three-product sums
-    // (longer terms than the four products') no less accurate than those were.
-    // Off the diagonal, m = 700, incoherent Z, 30k columns: one slice a slot
-    // 2.3e-15, 96 tiles 1.6e-15, 64 tiles 1.3e-15 (four products 1.7e-15); 60k
-    // 96 tiles 1.7, 64 tiles 1.5 (2.1); nearly coherent Z, 60k, 96 tiles
-    // 2.3e-16 (3.3e-16).  350 antennas, 29.9k sources up, 3 frequencies: one
-    // slice a slot 4.77 ms, 96 tiles 4.86, 64 tiles 4.91.
     case MV_FORM_C128: return 96;
-    case MV_FORM_C64: return 128;
+    case MV_FORM_C64: return m > 128 ? 128 : 64;
     default: return 192;
   }
 }
@@ -1667,7 +1659,7 @@ extern "C" int mv_herk_max_slices(int form, int m, int64_t kmax) {
   if (ts == 0 || m <= 0 || kmax < 0) return 0;
   const int64_t ktiles = cdiv(kmax, (int64_t)16);
   if (ktiles == 0) return 1;
-  const int64_t lo = cdiv(ktiles, (int64_t)form_cmax(form));
+  const int64_t lo = cdiv(ktiles, (int64_t)form_cmax(form, m));
   const int64_t ns = lo + 64 < ktiles ? lo + 64 : ktiles;
   return (int)(ns < 1 ? 1 : ns);
 }
@@ -1731,7 +1723,8 @@ int plan_herk(int form, int nterms, int maxord, int m, int nslices,
   const int slots =
       kernel_slots(herk_kernel(form, nterms, maxord, p.ts), p.threads);
   if (slots <= 0) return -1;
-  p.cfg = SliceCfg{nslices, slots, form_cmax(form), plain ? 2 : 4};
+  p.cfg = SliceCfg{nslices, slots, form_cmax(form, m), plain ? 2 : 4,
+                   plain ? 120 : 30};
   const int64_t items = (int64_t)p.ngroups * nslices * nbatch;
   p.grid = (int)(items < slots ? items : slots);
   return 0;
@@ -1964,6 +1957,8 @@ namespace {
 // from load until the process ends, one copy on each device it runs on
 // (128 MiB: room for 48 slices of the 350-antenna polarized split form,
 // more than its accuracy cap of 192 K tiles a slice needs at 100k sources).
+// A sum that would take more slices than fit runs longer ones than form_cmax:
+// the 31 of complex128 at m = 700 hold 241 K tiles each of 2 x 59.7k columns.
 // Host code uses the per-device address from hipGetSymbolAddress, never the
 // array's name.  Every call on a device shares that device's copy and
 // leaves its partials in it; nothing in it needs clearing (each call's
@@ -2174,7 +2169,7 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
   herk_group_plan_kernel<<<1, 256, 0, st>>>(
       problems_dev, nprob, side, by_wave ? 0 : 1,
       split ? kSK : kPK,
-      split ? form_cmax(form) : 64, split ? kGroupChain : 64,
+      split ? form_cmax(form, max_m) : 64, split ? kGroupChain : 64,
       part_bytes(form), split ? 1 : 0, probs, ws + g.parts, plan);
   if (int e = check_launch("mv_herk_grouped/plan")) return e;
   const int grid = (int)(max_items < slots ? max_items : slots);

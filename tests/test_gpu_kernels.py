@@ -305,6 +305,29 @@ def test_herk_plain_vs_numpy(m, k, form):
 
 
 @pytest.mark.parametrize("form", [FORM_C128, FORM_C64])
+@pytest.mark.parametrize("m,k", [(24, 2048), (160, 2048), (160, 9000)])
+def test_herk_plain_imaginary_part(m, k, form):
+    """Rows nearly in phase (within 1e-4 rad): Im V = sum(a d - b c) is far
+    smaller than |V| = k, and its rounding is that of its own partial sums.
+    Every one of the 2 k adds of a chain rounds by at most eps times the
+    largest partial sum (from any column on: twice the largest prefix) and
+    the two products of a column."""
+    dtype = np.complex128 if form == FORM_C128 else np.complex64
+    rng = np.random.default_rng(m + k)
+    z = np.exp(1e-4j * rng.uniform(-1, 1, size=(m, k))).astype(dtype)
+    h, v = _run_herk(form, [_dev(z)], m, k, 1, k, k)
+    got = _vis_full(h, v, m).imag
+    eps = 2.0 ** (-53 if form == FORM_C128 else -24)
+    x, y = z.real.astype(np.longdouble), z.imag.astype(np.longdouble)
+    term = float(np.abs(x).max() * np.abs(y).max())
+    for i in range(0, m, 5):
+        steps = x[i] * y - y[i] * x
+        prefix = float(np.abs(np.cumsum(steps, 1)).max())
+        err = float(np.abs(got[i] - steps.sum(1)).max())
+        assert err <= 2 * k * eps * (2 * prefix + 2 * term), (i, err / k)
+
+
+@pytest.mark.parametrize("form", [FORM_C128, FORM_C64])
 @pytest.mark.parametrize("m", [31, 32, 33, 96, 97, 128, 129, 192, 193, 257,
                                320, 321, 385, 577])
 def test_herk_plain_panel_edges(m, form):
