@@ -64,25 +64,30 @@ struct SliceCfg {
   int slots;       // workgroups resident at once (multiple of kXcd)
   int cmax;        // at most this many K tiles per slice
   int ovh;         // per-item cost beyond its K tiles, in K-tile units
-  int spread;      // an instance that leaves slots idle: at most
-                   // sqrt(spread x K tiles) slices
+  int reach;       // counts from the least one on that are considered
+  int full;        // an instance that leaves slots idle keeps chains as
+                   // short as the fullest of 64 counts has them
 };
 
 // Active slice count for `ktiles` K tiles over `ntiles` items a slice (panel
 // groups): enough slices that no chain exceeds cmax K tiles; then, where the
-// next 63 counts (at most the capacity and ktiles) can fill the resident
-// slots, the one of them with the least cost = rounds of slots x (K tiles per
-// slice + per-item overhead), the smallest count on ties.  Where they cannot
-// (small_slices), a power of two: an instance that leaves slots idle shares
-// its launch with others (frequencies, HerkBatch), and counts that divide the
-// slots leave no nearly empty last round, at most sqrt(spread ktiles): a slice
-// more costs its share of the reduce, about a thirtieth of the time of a K
-// tile in a launch that leaves most slots idle (3.5 us, FP64), and shortens
-// every chain by ktiles / ns^2 of them, so that 30 is the cheapest.  The plain
-// forms take 120: their chains round once or twice a column, with 30 more than
-// with one slice a K tile (32 antennas, 3k sources in complex64: 7.8e-8 of |V|
-// against 6.5e-8), and the time is the same (m = 32, 1.8k columns 13.1 us in
-// both).
+// counts within reach (at most the capacity and ktiles) can fill the resident
+// slots, the one of the first 64 with the least cost = rounds of slots x (K
+// tiles per slice + per-item overhead), the smallest count on ties.  Where they
+// cannot (small_slices), a power of two: an instance that leaves slots idle
+// shares its launch with others (frequencies, HerkBatch), and counts that
+// divide the slots leave no nearly empty last round.  The largest of at most
+// sqrt(30 ktiles): a slice more costs its share of the reduce, about a thirtieth
+// of the time of a K tile in a launch that leaves most slots idle (3.5 us,
+// FP64), and shortens every chain by ktiles / ns^2 of them.
+// The plain forms and fp16 terms, whose error is that of the chains, go on to
+// the power of two whose chains are no longer than those of the fullest of 64
+// counts, and reach for 128.  (Without: errors over |V|, 2 x 18k columns, 256
+// rows of fp16 terms 64 slices 6.7e-8, 75 6.4e-8, 128 5.3e-8; 200 of complex64
+// 64 slices 9.9e-8, 128 7.0e-8; 32 of 1.8k complex64 columns 32 slices 7.8e-8, 64
+// 6.5e-8.  Times at 64 and 128 slices: m = 128, 20k columns, complex64 42 and 38
+// us, FP64 65 and 54.)  Two bf16 terms are coarser than any chain, and of three
+// each wave sums half the columns.
 // Pure integer function of its arguments: the compute and reduce kernels and
 // the host agree on it.
 // Measured, HERK and reduce of a time: 16 frequencies of 128 antennas, 1,866
@@ -92,7 +97,7 @@ __host__ __device__ inline void slice_range(int ktiles, const SliceCfg &c,
                                             int &lo, int &hi) {
   lo = icdiv(ktiles, c.cmax);
   lo = lo < 1 ? 1 : (lo > c.max_slices ? c.max_slices : lo);
-  hi = lo + 63;
+  hi = lo + c.reach - 1;
   if (hi > c.max_slices) hi = c.max_slices;
   if (hi > ktiles) hi = ktiles > lo ? ktiles : lo;
 }
@@ -108,7 +113,10 @@ __host__ __device__ inline bool small_slices(int ktiles, int ntiles, int lo,
                                              int &ns) {
   if ((int64_t)ntiles * hi > c.slots) return false;
   ns = 1;
-  while (2 * ns <= hi && 4 * (int64_t)ns * ns <= (int64_t)c.spread * ktiles)
+  const int most = hi < lo + 63 ? hi : lo + 63;
+  const int chain = c.full ? icdiv(ktiles, most) : ktiles;
+  while (2 * ns <= hi && (4 * (int64_t)ns * ns <= 30 * (int64_t)ktiles ||
+                          icdiv(ktiles, ns) > chain))
     ns *= 2;
   if (ns < lo) ns = lo;
   return true;
@@ -119,6 +127,7 @@ __host__ __device__ inline int active_slices(int ktiles, int ntiles,
   int lo, hi, ns;
   slice_range(ktiles, c, lo, hi);
   if (small_slices(ktiles, ntiles, lo, hi, c, ns)) return ns;
+  if (hi > lo + 63) hi = lo + 63;
   int best = lo;
   int64_t best_cost = INT64_MAX;
   for (ns = lo; ns <= hi; ++ns) {
@@ -1620,6 +1629,13 @@ int panel_side(int form, int m) {
   return form == MV_FORM_C64 && m > 128 ? 64 : 32;
 }
 
+// Slice counts beyond the least that an instance may take (slice_range): 128
+// where five panels or fewer leave slots idle with them (4 groups of 512 slots).
+int slice_reach(int form, int m) {
+  const int panel = form == MV_FORM_SPLIT_F16 ? 64 : panel_side(form, m);
+  return form != MV_FORM_SPLIT_BF16 && m <= 5 * panel ? 128 : 64;
+}
+
 }  // namespace
 }  // namespace mv
 
@@ -1660,7 +1676,8 @@ extern "C" int mv_herk_max_slices(int form, int m, int64_t kmax) {
   const int64_t ktiles = cdiv(kmax, (int64_t)16);
   if (ktiles == 0) return 1;
   const int64_t lo = cdiv(ktiles, (int64_t)form_cmax(form, m));
-  const int64_t ns = lo + 64 < ktiles ? lo + 64 : ktiles;
+  const int64_t most = lo + slice_reach(form, m);
+  const int64_t ns = most < ktiles ? most : ktiles;
   return (int)(ns < 1 ? 1 : ns);
 }
 
@@ -1724,7 +1741,7 @@ int plan_herk(int form, int nterms, int maxord, int m, int nslices,
       kernel_slots(herk_kernel(form, nterms, maxord, p.ts), p.threads);
   if (slots <= 0) return -1;
   p.cfg = SliceCfg{nslices, slots, form_cmax(form, m), plain ? 2 : 4,
-                   plain ? 120 : 30};
+                   slice_reach(form, m), form != MV_FORM_SPLIT_BF16};
   const int64_t items = (int64_t)p.ngroups * nslices * nbatch;
   p.grid = (int)(items < slots ? items : slots);
   return 0;

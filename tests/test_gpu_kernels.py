@@ -327,6 +327,22 @@ def test_herk_plain_imaginary_part(m, k, form):
         assert err <= 2 * k * eps * (2 * prefix + 2 * term), (i, err / k)
 
 
+@pytest.mark.parametrize("form,nterms,nprod", [
+    (FORM_C128, 1, 1), (FORM_C64, 1, 1), (FORM_SPLIT_F16, 2, 3)])
+@pytest.mark.parametrize("m", [12, 64, 122, 160, 256])
+def test_herk_small_instances_keep_short_chains(m, form, nterms, nprod):
+    """Instances that leave the GPU's slots idle run slices no longer than the
+    64 counts from one slice per 256 K tiles (complex128: one in all) on
+    allow."""
+    from matvis_amd.gpu.herk import Herk
+    h = Herk(form, m, nterms, nprod)
+    for ktiles in (64, 113, 225, 700, 1500, 2250):
+        ns = h.active_slices(1, 16 * ktiles, h.nslices(16 * ktiles))
+        least = 1 if form == FORM_C128 else -(-ktiles // 256)
+        most = min(ktiles, least + 63)
+        assert -(-ktiles // ns) <= -(-ktiles // most), (ktiles, ns)
+
+
 @pytest.mark.parametrize("form", [FORM_C128, FORM_C64])
 @pytest.mark.parametrize("m", [31, 32, 33, 96, 97, 128, 129, 192, 193, 257,
                                320, 321, 385, 577])
