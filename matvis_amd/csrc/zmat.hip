@@ -1,7 +1,7 @@
 // (c) Geometric phase and the Z matrix.
 //
-// Phase: quarter turns 4 (b . s) (freq / c) in FP64, reduced to the nearest
-// whole one and a remainder in [-1/2, 1/2] before sincos, so the sincos
+// Phase: turns (b . s) (freq / c) in FP64, reduced to the nearest quarter turn
+// and a remainder of at most half of one before sincos, so the sincos
 // argument is small whatever the baseline length (the reference forms
 // exp(i * 2 pi freq (b . s) / c) directly, src/matvis/core/tau.py:30-31,65-66).
 // FP64 forms evaluate sine and cosine of the remainder in FP64; FP32 and split
@@ -60,25 +60,28 @@ __device__ __forceinline__ float flip_sign(float x, uint32_t bit31) {
   return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) ^ bit31);
 }
 
-// exp(i phase) of the antenna at ap for the direction (sx, sy, sz), w =
-// 4 freq / c: y = (ap . s) w quarter turns are k whole ones, folded by
-// exchanges and signs, and a remainder.  (Directions scaled by w beforehand
-// save a product an element and round three times, not once: 4% more error of
-// an FP64 phase.)  Adding 1.5 2^52 rounds y to the whole number
-// that then stands in the sum's low bits (|y| < 2^51).  A phase that is not
-// finite gives NaN.
+// exp(i phase) of the antenna at ap for the direction (sx, sy, sz), fc = freq /
+// c: r = (ap . s) fc turns without the whole ones (exact at any size), of which
+// 4 r is k quarter turns, folded by exchanges and signs, and a remainder.
+// (Directions scaled by fc beforehand save a product an element and round three
+// times, not once: 4% more error of an FP64 phase.)  Adding 1.5 2^52 rounds 4 r
+// to the whole number that then stands in the sum's low bits.  A phase that is
+// not finite gives NaN.
 // The general sincospi this replaces reduced the phase once more and made the
 // kernel compute-bound for one feed, where every element has its own phase:
-// 8 frequencies of 128 antennas x 30k sources, split to bf16, 70.4 us.
+// 8 frequencies of 128 antennas x 30k sources, split to bf16, 70.4 -> 62.5 us;
+// taking the whole turns off first, which keeps phases of 2^49 turns and more
+// right, adds 4% (46.6 -> 48.7 us in launches back to back).
 template <typename T>
 __device__ __forceinline__ cplx<T> phasor(const double *__restrict__ ap,
-                                          double w, double sx, double sy,
+                                          double fc, double sx, double sy,
                                           double sz) {
-  const double y = (ap[0] * sx + ap[1] * sy + ap[2] * sz) * w;
-  const double t = y + 0x1.8p52;
+  const double cyc = (ap[0] * sx + ap[1] * sy + ap[2] * sz) * fc;
+  const double r = cyc - rint(cyc);
+  const double t = fma(4.0, r, 0x1.8p52);
   const uint32_t q = (uint32_t)__builtin_bit_cast(uint64_t, t);
   T c, s;
-  cos_sin((T)((y - (t - 0x1.8p52)) * (0.5 * kPi)), c, s);
+  cos_sin((T)(fma(4.0, r, -(t - 0x1.8p52)) * (0.5 * kPi)), c, s);
   const bool odd = q & 1u;                           // quarter turn
   const uint32_t half = (q << 30) & 0x80000000u;     // half turn
   return {flip_sign(odd ? -s : c, half), flip_sign(odd ? c : s, half)};
@@ -93,7 +96,7 @@ __global__ __launch_bounds__(kThreads) void exptau_kernel(
   int a = blockIdx.y;
   if (s >= nsrc) return;
   out[(int64_t)a * ld_out + s] =
-      phasor<TO>(antpos + 3 * a, 4.0 * fc, (double)crd[s],
+      phasor<TO>(antpos + 3 * a, fc, (double)crd[s],
                  (double)crd[ld_crd + s], (double)crd[2 * ld_crd + s]);
 }
 
@@ -318,7 +321,7 @@ __global__ __launch_bounds__(kThreads) void zmat_fused_kernel(
                     : cplx<T>{(T)NAN, (T)NAN};
         cached = b;
       }
-      cplx<T> e = phasor<T>(antpos + 3 * a, 4.0 * fc, sx, sy, sz);
+      cplx<T> e = phasor<T>(antpos + 3 * a, fc, sx, sy, sz);
       // an antenna at a time: a product of amplitude and beam shared by the
       // antennas would round the same way in all of them, and add up in V (6%
       // more error of a complex64 time of 32 antennas)

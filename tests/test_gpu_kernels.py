@@ -826,3 +826,23 @@ def test_phase_in_every_quadrant(is_f64):
     err = np.abs(got[:n] - (np.cos(ph) + 1j * np.sin(ph))).max()
     assert err < (2.2e-14 if is_f64 else 1.4e-7), err
     assert np.isnan(got[n].real) and np.isnan(got[n].imag)
+
+
+@pytest.mark.parametrize("is_f64", [True, False])
+def test_phase_of_many_turns(is_f64):
+    """Whole turns leave the phase exactly, however many there are: quarter
+    turns beside 2^e whole ones, which FP64 holds up to e = 50, are the four
+    directions themselves (FP32: cos(0) and sin(0) are exact too)."""
+    freq = 299792458.0  # one turn a metre
+    x = np.array([s * (2.0 ** e + q / 4) for e in range(10, 51)
+                  for q in range(4) for s in (1, -1)])
+    n = x.size
+    crd = np.zeros((3, n))
+    crd[0] = x
+    ct = np.complex128 if is_f64 else np.complex64
+    ant, dev, out = _dev(np.eye(1, 3)), _dev(crd), D.zeros((1, n), ct)
+    call("mv_exptau", D.ptr(ant), 1, freq, D.ptr(dev), 1, n, n,
+         D.ptr(out), int(is_f64), n, D.stream_ptr())
+    turn = np.array([1, 1j, -1, -1j])
+    want = turn[np.round(4 * np.fmod(x, 1.0)).astype(int) % 4]
+    np.testing.assert_array_equal(D.to_host(out)[0], want.astype(ct))
