@@ -208,7 +208,9 @@ def grid_planes(beam, freq: float, polarized: bool, beam_type=None,
         if bt != "efield" or stored != "efield":
             raise ValueError("beam type must be efield if using polarized=True")
         planes = _interp_freq(data[:2, :2], freqs, freq)
-        if not (keep_precision and np.iscomplexobj(planes)):
+        # (types of the other byte order or of extended precision convert)
+        if not (keep_precision and planes.dtype in (np.complex64,
+                                                    np.complex128)):
             planes = planes.astype(np.complex128)
         is_power = False
     else:

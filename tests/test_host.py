@@ -358,6 +358,25 @@ def test_chunks_fit_this_builds_footprint():
                       **kw)[0] == 1000
 
 
+@pytest.mark.parametrize("dtype", ["<c8", "<c16", ">c8", ">c16",
+                                   "clongdouble", "f4", ">f8"])
+@pytest.mark.parametrize("wrap", [True, False])
+def test_stored_beam_planes_have_types_the_device_takes(dtype, wrap):
+    """Planes kept as stored are complex64 or complex128 in native byte
+    order, whatever the beam's array is (a non-wrapping azimuth grid makes
+    no copy), with the values of the converted planes."""
+    beam = synth.harmonic_efield_beam(seed=4, naz=36, nza=10)
+    with np.errstate(all="ignore"):
+        data = beam.data_array if "c" in dtype else beam.data_array.real
+        beam.data_array = data.astype(dtype)
+    if not wrap:
+        beam.axis1_array = beam.axis1_array[:20]
+        beam.data_array = beam.data_array[..., :20]
+    kept = grid_planes(beam, 150e6, True, keep_precision=True)[0]
+    assert kept.dtype in (np.complex64, np.complex128) and kept.dtype.isnative
+    np.testing.assert_array_equal(kept, grid_planes(beam, 150e6, True)[0])
+
+
 def test_human_readable_size_and_ceildiv():
     """The reference's expected strings (tests/test_utils.py:20-38)."""
     from matvis_amd._utils import ceildiv, human_readable_size as h
