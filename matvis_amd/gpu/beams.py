@@ -33,15 +33,25 @@ def spline_order(spline_opts: dict | None) -> int:
     return order
 
 
+def _largest(planes) -> torch.Tensor:
+    """Largest |value| of a beam's planes, in FP64 on their device."""
+    if planes.numel() == 0:
+        return planes.new_ones((), dtype=torch.float64)
+    wide = torch.complex128 if planes.is_complex() else torch.float64
+    return planes.to(wide).abs().amax()
+
+
 class DeviceBeamSet:
     """Device-resident tables of a beam list at one frequency."""
 
     def __init__(self, beam_list, freq: float, polarized: bool, complex_dtype,
-                 order: int = 1, banded: bool = False):
+                 order: int = 1, banded: bool = False, with_max: bool = True):
         """``banded``: interpolate with the grid staged in LDS by za band
         (the same values as the default tap gathers, which measured faster
         on MI355X for every grid whose rows fit in LDS); the bands need
-        every beam to share beam 0's za spacing."""
+        every beam to share beam 0's za spacing.  ``with_max``: take
+        ``max_abs``, the tables' largest |response| (fp16 terms scale by it;
+        three launches a grid beam and a wait)."""
         self.nbeam = len(beam_list)
         self.nfeed = self.nax = 2 if polarized else 1
         self.polarized = polarized
@@ -67,15 +77,22 @@ class DeviceBeamSet:
             shapes = {p[0].shape for p in preps}
             if len(shapes) != 1:
                 raise ValueError("all grid beams must share one az/za grid shape")
-            self._host = [p[0] for p in preps]
-            shape = self._host[0].shape
+            shape = preps[0][0].shape
             self.is_power = bool(preps[0][4])
             self.nza, self.naz = shape[-2:]
             grid = np.array([[p[1], p[2], p[3]] for p in preps], np.float64)
             self.grid = D.to_dev(grid, np.float64)
             self.planes = D.empty((self.nbeam,) + shape, self.complex_dtype)
-            for k, p in enumerate(self._host):
-                self.planes[k].copy_(D.to_dev(p))
+            self.max_abs = None
+            tops = []
+            for k, p in enumerate(preps):
+                up = D.to_dev(p[0])
+                self.planes[k].copy_(up)
+                if with_max:
+                    tops.append(_largest(up))
+            if with_max:
+                amax = float(torch.stack(tops).amax())
+                self.max_abs = np.sqrt(amax) if self.is_power else amax
             if order == 3:
                 call("mv_beam_prefilter", D.ptr(self.planes), int(self.is_f64),
                      self.nbeam * self.nax * self.nfeed, self.nza, self.naz,
@@ -89,17 +106,8 @@ class DeviceBeamSet:
             sig = [unwrap(b)[0].get_sigma(freq) for b in beam_list]
             self.sigma = D.to_dev(np.asarray(sig, np.float64))
             self.is_power = False
-            self._host = None
+            self.max_abs = 1.0
             self.banded = False
-
-    @property
-    def max_abs(self) -> float:
-        """Largest |response| of the tables (1 for analytic beams)."""
-        if self._host is None:
-            return 1.0
-        amax = max((float(np.abs(p.astype(np.complex128)).max())
-                    for p in self._host if p.size), default=1.0)
-        return np.sqrt(amax) if self.is_power else amax
 
     def eval(self, crd, ld_crd: int, count: int, out, ld_out: int,
              n_dev=None, stream=None, nchunks: int = 1, crd_stride: int = 0,
@@ -161,7 +169,7 @@ class GPUBeamInterpolator(BeamInterpolator):
             self.beam_idx = D.as_dev(self.beam_idx, np.int32)
         self.tables = DeviceBeamSet(
             self.beam_list, self.freq, self.polarized, self.complex_dtype,
-            spline_order(self.spline_opts),
+            spline_order(self.spline_opts), with_max=False,
         )
 
     def interp(self, tx, ty, out):

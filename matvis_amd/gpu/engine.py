@@ -249,7 +249,8 @@ class VisibilityEngine:
         that their ids stay unique, and by everything the tables depend on)."""
         if self.beam_cache is None or self.beam_src is None:
             return DeviceBeamSet(self.beam_list, f, self.polarized,
-                                 self.beam_ctype, self.order)
+                                 self.beam_ctype, self.order,
+                                 with_max=self.form == FORM_SPLIT_F16)
         fkey = tuple(k[2:] if k[0] == "grid" else k for k in self._beam_key(f))
         key = (tuple(id(b) for b in self.beam_src), self.polarized,
                np.dtype(self.beam_ctype).str, self.order, fkey)

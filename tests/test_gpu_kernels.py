@@ -846,3 +846,26 @@ def test_phase_of_many_turns(is_f64):
     turn = np.array([1, 1j, -1, -1j])
     want = turn[np.round(4 * np.fmod(x, 1.0)).astype(int) % 4]
     np.testing.assert_array_equal(D.to_host(out)[0], want.astype(ct))
+
+
+@pytest.mark.parametrize("polarized", [True, False])
+def test_beam_tables_hold_their_own_maximum(polarized):
+    """The largest |response| is that of the tables as they went up, whatever
+    the caller does to the beam's array afterwards (without the azimuth wrap
+    the planes are a view of it), and a set keeps no planes on the host."""
+    from matvis_amd.beams import grid_planes
+    from matvis_amd.gpu.beams import DeviceBeamSet
+    beams = [synth.harmonic_efield_beam(seed=k, naz=36, nza=10) for k in (1, 2)]
+    for b in beams:
+        b.axis1_array = b.axis1_array[:20]
+        b.data_array = b.data_array[..., :20]
+    planes = [grid_planes(b, 1.5e8, polarized)[0] for b in beams]
+    want = max(np.abs(p).max() for p in planes)
+    want = want if polarized else np.sqrt(want)
+    t = DeviceBeamSet(beams, 1.5e8, polarized, np.complex64, 3)
+    for b in beams:
+        b.data_array *= 100.0
+    assert abs(t.max_abs / want - 1) < 1e-12
+    held = list(vars(t).values())
+    held += [x for v in held if isinstance(v, (list, tuple)) for x in v]
+    assert not [v for v in held if isinstance(v, np.ndarray)]
