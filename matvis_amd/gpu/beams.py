@@ -109,24 +109,33 @@ class DeviceBeamSet:
             self.max_abs = 1.0
             self.banded = False
 
+    def _eval_banded(self, crd, ld_crd, count, out, ld_out, n_dev, stream):
+        """One chunk by za band; crd, out and n_dev device addresses (crd with
+        its is_f64)."""
+        need = lib().mv_beam_interp_banded_workspace_bytes(
+            int(self.is_f64), self.nza, self.naz, count)
+        if self._band_ws is None or self._band_ws.numel() < need:
+            self._band_ws = D.empty((max(need, 256),), np.uint8)
+        call("mv_beam_interp_banded", D.ptr(self.planes), int(self.is_f64),
+             self.nbeam, self.nfeed, self.nax, self.nza, self.naz,
+             D.ptr(self.grid), self.order, int(self.is_power), crd[0],
+             crd[1], ld_crd, count, n_dev, out, ld_out, D.ptr(self._band_ws),
+             self._band_ws.numel(), D.stream_ptr(stream))
+
     def eval(self, crd, ld_crd: int, count: int, out, ld_out: int,
              n_dev=None, stream=None, nchunks: int = 1, crd_stride: int = 0,
              out_stride: int = 0):
         """A (nbeam, nfeed, nax, ld_out) at topocentric vectors crd (3, ld),
         of nchunks chunks (their counts n_dev, the arrays *_stride elements
-        apart) in one launch; the za bands take one chunk."""
+        apart) in one launch; by za band a launch a chunk."""
         crd_is_f64 = int(crd.dtype == torch.float64)
-        if self.use_interp and self.banded and nchunks == 1:
-            need = lib().mv_beam_interp_banded_workspace_bytes(
-                int(self.is_f64), self.nza, self.naz, count)
-            if self._band_ws is None or self._band_ws.numel() < need:
-                self._band_ws = D.empty((max(need, 1),), np.uint8)
-            call("mv_beam_interp_banded", D.ptr(self.planes),
-                 int(self.is_f64), self.nbeam, self.nfeed, self.nax, self.nza,
-                 self.naz, D.ptr(self.grid), self.order, int(self.is_power),
-                 D.ptr(crd), crd_is_f64, ld_crd, count, D.ptr(n_dev),
-                 D.ptr(out), ld_out, D.ptr(self._band_ws),
-                 self._band_ws.numel(), D.stream_ptr(stream))
+        if self.use_interp and self.banded:
+            for c in range(nchunks):
+                self._eval_banded(
+                    (D.ptr(crd) + c * crd_stride * crd.element_size(),
+                     crd_is_f64), ld_crd, count,
+                    D.ptr(out) + c * out_stride * out.element_size(), ld_out,
+                    None if n_dev is None else D.ptr(n_dev[c:c + 1]), stream)
         elif self.use_interp:
             call("mv_beam_interp_chunks", D.ptr(self.planes),
                  int(self.is_f64), self.nbeam, self.nfeed, self.nax, self.nza,

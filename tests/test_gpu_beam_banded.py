@@ -10,7 +10,7 @@ import torch
 import oracle as O
 from _problems import small_problem
 from matvis_amd import _device as D
-from matvis_amd import astro
+from matvis_amd import astro, synth
 from matvis_amd._lib import call, lib
 from matvis_amd.gpu.beams import DeviceBeamSet
 from matvis_amd.gpu.gpu import simulate
@@ -108,3 +108,22 @@ def test_large_beam_matches_oracle_and_bands_match_gathers():
         dbs.eval(crd, 3000, 3000, out, 3000)
     torch.cuda.synchronize()
     assert torch.equal(outs[0], outs[1])
+
+
+def test_banded_over_chunks():
+    """A set made with bands evaluates every chunk by them, with the bits of
+    the tap gathers over the same chunks."""
+    beam = synth.harmonic_efield_beam(seed=3, naz=36, nza=10)
+    count, ld = 700, 704
+    crd = D.zeros((3, 3, ld), np.float64)
+    for c in range(3):
+        crd[c, :, :count] = D.to_dev(_positions(count, c))
+    n = D.to_dev(np.array([700, 0, 333], np.int32))
+    out = []
+    for banded in (True, False):
+        t = DeviceBeamSet([beam], 1.5e8, True, np.complex64, 3, banded=banded)
+        a = D.zeros((3, 1, 2, 2, ld), np.complex64)
+        t.eval(crd, ld, count, a, ld, n, None, 3, 3 * ld, a[0].numel())
+        assert (t._band_ws is not None) == banded
+        out.append(D.to_host(a))
+    np.testing.assert_array_equal(out[0], out[1])
