@@ -51,6 +51,10 @@ BATCH_BYTES = 1 << 30
 #: chunks a launch takes (a grid dimension)
 MAX_GRID = 65535
 
+#: fluxes uploaded at a time (their rows; the whole table fits beside its
+#: square roots below this)
+FLUX_BLOCK_BYTES = 64 << 20
+
 #: a time's output that one host thread copies
 HOST_COPY_BYTES = 4 << 20
 
@@ -91,7 +95,9 @@ def device_bytes(*, form: int, nterms: int, nprod: int, nant: int,
         # kept coordinates, fluxes, indices and its cull workspace
         "coords": nsrc * (24 + 3 * rsz + 24 + 24 + 16 + 8)
         + nsrc_alloc * (3 * rsz + 4 * 16 + 4) + cull_ws,
-        "antpos_flux": nant * 24 + nfreq * nsrc * 8,
+        # the square roots, and the block of fluxes they are taken from
+        "antpos_flux": nant * 24 + nfreq * nsrc * 8
+        + min(nfreq * nsrc * 8, FLUX_BLOCK_BYTES),
         "chunk_coords": nchunks * (seg * (24 + 4) + cull_ws),
         "beam_tables": beam_sets * nbeam * nf * nf * beam_pixels * esz,
         "beam_values": (nchunks if beam_sets == 1 else nb) * nbeam * nf * nf
@@ -175,10 +181,14 @@ class VisibilityEngine:
     def setup(self):
         seg, nalloc = self.seg, self.nsrc_alloc
         self.antpos = D.to_dev(self.antpos_h, np.float64)
-        # sqrt(I / 2) frequency-major: the square root (rounded to nearest,
-        # as numpy's) and the transpose on the device
-        self.sqrt_flux = torch.sqrt(
-            0.5 * D.to_dev(self.flux_h, np.float64).t()).contiguous()
+        # sqrt(I / 2) frequency-major: the transpose and the square root
+        # (rounded to nearest, as numpy's) on the device, in place
+        self.sqrt_flux = D.empty((self.nfreq, self.nsrc), np.float64)
+        step = max(1, FLUX_BLOCK_BYTES // (8 * self.nfreq))
+        for k in range(0, self.nsrc, step):
+            self.sqrt_flux[:, k:k + step].copy_(
+                D.to_dev(self.flux_h[k:k + step], np.float64).t())
+        self.sqrt_flux.mul_(0.5).sqrt_()
         F = self.batch
         self.freqs_dev = D.to_dev(self.freqs, np.float64) if F > 1 else None
         self.beam_idx_dev = (None if self.beam_idx is None

@@ -685,3 +685,38 @@ def test_frequencies_per_launch(method, precision, nant, polarized, per_freq,
         if want is None:
             want = v
         assert np.isfinite(v).all() and np.array_equal(v, want), batch
+
+
+def test_flux_upload_stays_within_the_footprint():
+    """A flux table larger than the rest (200k sources x 64 frequencies, 98
+    MiB): setting the engine up holds it once, and a block of it, not the
+    products on the way to its square roots; the values are numpy's."""
+    import torch
+
+    from matvis_amd.gpu.engine import device_bytes
+    from matvis_amd.gpu.gpu import build_engine
+
+    nsrc, nfreq = 200_000, 64
+    p = small_problem(nant=2, nsrc=nsrc, ntimes=1, polarized=False)
+    rng = np.random.default_rng(1)
+    flux = rng.uniform(0.5, 2, (nsrc, nfreq))
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    eng, _ = build_engine(
+        antpos=p["antpos"], freqs=np.linspace(1e8, 2e8, nfreq),
+        times=p["times"], skycoords=astro.SkyCoord(p["ra"], p["dec"]),
+        telescope_loc=p["loc"], fluxes=flux, beam_list=[GaussianBeam(sigma=0.2)],
+        polarized=False, precision=1, source_buffer=0.55, batch=1,
+        coord_method="CoordinateRotationMatrix",
+        coord_method_params={"rotations": p["rotations"]})
+    peak = torch.cuda.max_memory_allocated() - base
+    model = device_bytes(
+        form=eng.form, nterms=1, nprod=1, nant=2, polarized=False,
+        nfreq=nfreq, nsrc=nsrc, nchunks=1, chunk_size=eng.chunk_size,
+        nsrc_alloc=eng.nsrc_alloc, nbeam=1, beam_pixels=0, beam_sets=1,
+        npairs=4, precision=1, batch=1)["total"]
+    assert peak <= model, (peak, model)
+    np.testing.assert_array_equal(eng.sqrt_flux.cpu().numpy(),
+                                  np.sqrt(0.5 * flux.T))
