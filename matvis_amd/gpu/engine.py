@@ -30,6 +30,7 @@ from .. import _device as D
 from .._lib import FORM_C128, FORM_SPLIT_F16, call, lib
 from .._utils import log_progress
 from .._utils import logger as _progress_log
+from ..beams import is_grid_beam, unwrap
 from .beams import DeviceBeamSet
 from .herk import Herk, cdiv, expand, expand_batch, is_split
 from .matprod import f16_scale
@@ -59,14 +60,38 @@ FLUX_BLOCK_BYTES = 64 << 20
 HOST_COPY_BYTES = 4 << 20
 
 
+def beam_key(beam_list, f) -> tuple:
+    """Frequency-response key: equal keys give identical beam tables."""
+    key = []
+    for b in beam_list:
+        inner, _ = unwrap(b)
+        if is_grid_beam(b):
+            key.append(("grid", id(inner)) if np.asarray(
+                inner.freq_array).size <= 1 else ("grid", id(inner), f))
+        else:
+            key.append(("gauss", inner.get_sigma(f)))
+    return tuple(key)
+
+
+def beams_by_frequency(beam_list, freqs) -> bool:
+    """Whether an engine keeps beam tables, and the values of a launch's
+    frequencies, for each frequency."""
+    freqs = np.atleast_1d(freqs)
+    first = beam_key(beam_list, freqs[0])
+    return any(beam_key(beam_list, f) != first for f in freqs[1:])
+
+
 def freq_batch(*, form: int, nterms: int, nprod: int, m: int, nax: int,
-               nfreq: int, nsrc_alloc: int) -> int:
-    """Frequencies per launch: as many as BATCH_BYTES holds, in even parts."""
+               nfreq: int, nsrc_alloc: int, nbeam: int = 0) -> int:
+    """Frequencies per launch: as many as BATCH_BYTES holds, in even parts.
+    nbeam: beams whose values each frequency has for itself (0: shared)."""
     seg = max(Z_PAD, cdiv(nsrc_alloc, Z_PAD) * Z_PAD)
     herk = Herk(form, m, nterms, nprod)
-    esz = 4 * nterms if is_split(form) else 16 if form == FORM_C128 else 8
-    each = m * nax * seg * esz + herk.ldv * herk.ldv * 16 + int(
-        lib().mv_herk_workspace_bytes(form, m, herk.nslices(nax * nsrc_alloc)))
+    bsz = 16 if form == FORM_C128 else 8
+    esz = 4 * nterms if is_split(form) else bsz
+    each = (m * esz + nbeam * nax * bsz) * nax * seg + (
+        herk.ldv * herk.ldv * 16 + int(lib().mv_herk_workspace_bytes(
+            form, m, herk.nslices(nax * nsrc_alloc))))
     fit = max(1, min(nfreq, BATCH_BYTES // each))
     return cdiv(nfreq, cdiv(nfreq, fit))
 
@@ -89,7 +114,8 @@ def device_bytes(*, form: int, nterms: int, nprod: int, nant: int,
     herk = Herk(form, m, nterms, nprod)
     cull_ws = int(lib().mv_rotate_cull_workspace_bytes(chunk_size))
     nb = batch or freq_batch(form=form, nterms=nterms, nprod=nprod, m=m,
-                             nax=nf, nfreq=nfreq, nsrc_alloc=nsrc_alloc)
+                             nax=nf, nfreq=nfreq, nsrc_alloc=nsrc_alloc,
+                             nbeam=nbeam if beam_sets > 1 else 0)
     terms = {
         # rotation plugin: ECI, topocentric (and FP64 / BCRS copies), the
         # kept coordinates, fluxes, indices and its cull workspace
@@ -164,7 +190,8 @@ class VisibilityEngine:
         self.beam_src = list(beam_src) if beam_src is not None else None
         self.batch = batch or freq_batch(
             form=form, nterms=nterms, nprod=nprod, m=self.m, nax=self.nax,
-            nfreq=self.nfreq, nsrc_alloc=nsrc_alloc)
+            nfreq=self.nfreq, nsrc_alloc=nsrc_alloc,
+            nbeam=len(beam_list) * beams_by_frequency(beam_list, self.freqs))
         self._ready = False
         #: optional (before, after) callables taking the stream, run around
         #: every HERK compute kernel (event timing of the dominant kernel;
@@ -248,8 +275,7 @@ class VisibilityEngine:
         self._ready = True
 
     def _make_beam_sets(self):
-        keys = [self._beam_key(f) for f in self.freqs]
-        if all(k == keys[0] for k in keys):
+        if not beams_by_frequency(self.beam_list, self.freqs):
             return [self._beam_set(self.freqs[0])]
         return [self._beam_set(f) for f in self.freqs]
 
@@ -261,7 +287,8 @@ class VisibilityEngine:
             return DeviceBeamSet(self.beam_list, f, self.polarized,
                                  self.beam_ctype, self.order,
                                  with_max=self.form == FORM_SPLIT_F16)
-        fkey = tuple(k[2:] if k[0] == "grid" else k for k in self._beam_key(f))
+        fkey = tuple(k[2:] if k[0] == "grid" else k
+                     for k in beam_key(self.beam_list, f))
         key = (tuple(id(b) for b in self.beam_src), self.polarized,
                np.dtype(self.beam_ctype).str, self.order, fkey)
         hit = self.beam_cache.get(key)
@@ -270,20 +297,6 @@ class VisibilityEngine:
                                  self.beam_ctype, self.order), self.beam_src)
             self.beam_cache[key] = hit
         return hit[0]
-
-    def _beam_key(self, f):
-        """Frequency-response key: equal keys give identical beam tables."""
-        from ..beams import is_grid_beam, unwrap
-
-        key = []
-        for b in self.beam_list:
-            inner, _ = unwrap(b)
-            if is_grid_beam(b):
-                key.append(("grid", id(inner)) if np.asarray(
-                    inner.freq_array).size <= 1 else ("grid", id(inner), f))
-            else:
-                key.append(("gauss", inner.get_sigma(f)))
-        return tuple(key)
 
     # ---------------------------------------------------------------- compute
 

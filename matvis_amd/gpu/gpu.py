@@ -20,7 +20,7 @@ from ..core.coords import CoordinateRotation
 from . import coords as _coords  # noqa: F401  (registers rotation methods)
 from . import matprod as mp
 from .beams import spline_order
-from .engine import VisibilityEngine, freq_batch
+from .engine import VisibilityEngine, beams_by_frequency, freq_batch
 from .herk import products_for
 
 logger = logging.getLogger(__name__)
@@ -100,14 +100,16 @@ def build_engine(
                  polarized=polarized, nfreq=freqs.size, nsrc=nsrc,
                  source_buffer=source_buffer, beams=beams,
                  npairs=nant * nant if antpairs is None else len(antpairs),
-                 precision=precision)
+                 precision=precision,
+                 per_freq=beams_by_frequency(beams, freqs))
     nchunks, npixc = fit_chunks(freemem * memory_buffer, nchunks, **sizes)
     need = footprint(**sizes)
     nsrc_alloc = int(npixc * source_buffer)
     # frequencies per launch, as many as fit beside the rest
     F = batch or freq_batch(form=form, nterms=nterms, nprod=nprod,
                             m=nfeed * nant, nax=nax, nfreq=freqs.size,
-                            nsrc_alloc=nsrc_alloc)
+                            nsrc_alloc=nsrc_alloc,
+                            nbeam=len(beams) * sizes["per_freq"])
     while F > 1 and need(nchunks, F) > freemem * memory_buffer:
         F //= 2
     coord_cls = CoordinateRotation._methods[coord_method]
@@ -132,19 +134,18 @@ def build_engine(
 
 
 def footprint(*, form, nterms, nprod, nant, polarized, nfreq, nsrc,
-              source_buffer, beams, npairs, precision):
+              source_buffer, beams, npairs, precision, per_freq=False):
     """A function of (nchunks, frequencies per launch): this build's device
     bytes (engine.device_bytes: Z terms, split-K workspace, FP64
     accumulator, beam tables and values, output buffers, the rotation
-    plugin's arrays)."""
+    plugin's arrays).  per_freq: the beams differ by frequency
+    (engine.beams_by_frequency)."""
     from ..beams import is_grid_beam, unwrap
     from .engine import device_bytes
 
     grid = [unwrap(b)[0] for b in beams if is_grid_beam(b)]
     pixels = max((int(np.prod(g.data_array.shape[-2:])) + 3
                   * int(g.data_array.shape[-2]) for g in grid), default=0)
-    per_freq = nfreq > 1 and any(np.asarray(g.freq_array).size > 1
-                                 for g in grid)
 
     def need(ch, batch=1):
         npc = int(np.ceil(nsrc / ch))

@@ -720,3 +720,48 @@ def test_flux_upload_stays_within_the_footprint():
     assert peak <= model, (peak, model)
     np.testing.assert_array_equal(eng.sqrt_flux.cpu().numpy(),
                                   np.sqrt(0.5 * flux.T))
+
+
+def test_max_memory_bounds_frequencies_per_launch():
+    """Gaussian beams whose width changes with frequency, one an antenna:
+    each frequency of a launch has beam values as large as its Z, which the
+    model counts, and as many of them share a launch as its share (0.9) of
+    max_memory holds; the allocations of a run stay within max_memory."""
+    import torch
+
+    from matvis_amd.gpu.engine import device_bytes
+    from matvis_amd.gpu.gpu import build_engine
+
+    nant, nsrc, nfreq, budget = 24, 6000, 8, 96 << 20
+    p = small_problem(nant=nant, nsrc=nsrc, ntimes=1)
+    rng = np.random.default_rng(2)
+    beams = [GaussianBeam(diameter=d) for d in rng.uniform(10, 15, nant)]
+    kw = dict(antpos=p["antpos"], freqs=np.linspace(1e8, 2e8, nfreq),
+              times=p["times"], skycoords=astro.SkyCoord(p["ra"], p["dec"]),
+              telescope_loc=p["loc"],
+              fluxes=rng.uniform(0.5, 2, (nsrc, nfreq)), beam_list=beams,
+              beam_idx=np.arange(nant), polarized=True, precision=2,
+              coord_method="CoordinateRotationMatrix",
+              coord_method_params={"rotations": p["rotations"]})
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    eng, nt = build_engine(max_memory=budget, **kw)
+    v = eng.run(nt)
+    torch.cuda.synchronize()
+    peak = torch.cuda.max_memory_allocated() - base
+    model = device_bytes(
+        form=eng.form, nterms=eng.nterms, nprod=eng.nprod, nant=nant,
+        polarized=True, nfreq=nfreq, nsrc=nsrc, nchunks=eng.nchunks,
+        chunk_size=eng.chunk_size, nsrc_alloc=eng.nsrc_alloc, nbeam=nant,
+        beam_pixels=0, beam_sets=nfreq, npairs=nant * nant, precision=2,
+        batch=eng.batch)
+    held = sum(a.numel() * a.element_size() for a in eng.A)
+    assert model["beam_values"] == held
+    model = model["total"]
+    print(f"  {eng.nchunks} chunks, {eng.batch} frequencies a launch, peak "
+          f"{peak / 2**20:.1f} MiB, model {model / 2**20:.1f}", flush=True)
+    assert eng.batch > 1 and model <= 0.9 * budget and peak <= budget
+    del eng
+    np.testing.assert_array_equal(v, simulate_multi(**kw))
