@@ -39,7 +39,7 @@ import numpy as np
 import torch
 
 from . import _device as D
-from ._lib import FORM_C64, FORM_C128
+from ._lib import lib
 from .gpu.herk import is_split
 
 _ids = itertools.count()
@@ -68,6 +68,8 @@ class SimRequest:
     visibilities: int = 0
     #: projected device work (set when the shortest-first policy needs it)
     work: float | None = None
+    #: projected device bytes (set when the request may be admitted)
+    nbytes: int | None = None
     result: np.ndarray | None = None
     error: Exception | None = None
     done: threading.Event = field(default_factory=threading.Event)
@@ -89,26 +91,38 @@ def projected_work(engine_kwargs: dict) -> float:
 
 
 def projected_bytes(engine_kwargs: dict) -> int:
-    """Device bytes a request will hold while resident: Z, accumulator,
-    HERK workspace, coordinates, beam values and the output of one time."""
+    """Device bytes a request will hold while resident: its engine's, one
+    frequency a launch (engine.device_bytes, with the slices each form's own
+    rule sizes the partials for), and its share of a grouped launch's
+    partials."""
+    from .gpu.gpu import _resolve_matprod, footprint
+    from .gpu.engine import beams_by_frequency
     from .gpu.herk import Herk
 
-    nant = len(engine_kwargs["antpos"])
-    nf = 2 if engine_kwargs.get("polarized") else 1
-    m = nant * nf
-    nsrc = np.asarray(engine_kwargs["fluxes"]).shape[0]
-    nfreq = np.atleast_1d(engine_kwargs["freqs"]).size
-    seg = -(-nsrc // 32) * 32
-    method = engine_kwargs.get("matprod_method", "GPUMatMul")
-    split = "Split" in method
-    zbytes = m * nf * seg * (8 if split else
-                             (16 if engine_kwargs.get("precision", 1) == 2
-                              else 8))
-    ldv = -(-m // 128) * 128
-    work = ldv * ldv * 16 * 64  # accumulator and a bound on the partials
-    out = nfreq * nant * nant * nf * nf * 16
-    return int(zbytes + work + 3 * seg * 12 + 4 * nf * nf * seg * 16 + out
-               + nsrc * nfreq * 8)
+    kw = engine_kwargs
+    nant = len(kw["antpos"])
+    nf = 2 if kw.get("polarized") else 1
+    nsrc = np.asarray(kw["fluxes"]).shape[0]
+    freqs = np.atleast_1d(np.asarray(kw["freqs"], dtype=np.float64))
+    precision = kw.get("precision", 1)
+    pairs = kw.get("antpairs")
+    form, nterms, nprod = _resolve_matprod(
+        kw.get("matprod_method", "GPUMatMul"), precision,
+        kw.get("split_terms"), kw.get("split_products"))
+    source_buffer = kw.get("source_buffer", 1.0)
+    nchunks = max(1, int(kw.get("min_chunks", 1)))
+    need = footprint(
+        form=form, nterms=nterms, nprod=nprod, nant=nant,
+        polarized=nf == 2, nfreq=freqs.size, nsrc=nsrc,
+        source_buffer=source_buffer, beams=kw["beam_list"],
+        npairs=nant * nant if pairs is None else len(pairs),
+        precision=precision,
+        per_freq=beams_by_frequency(kw["beam_list"], freqs))(nchunks)
+    herk = Herk(form, nf * nant, nterms, nprod)
+    seg = int(-(-nsrc // nchunks) * source_buffer)
+    group = lib().mv_herk_workspace_bytes(form, nf * nant,
+                                          herk.nslices(nf * seg))
+    return int(need + group)
 
 
 class _Active:
@@ -319,10 +333,16 @@ class VisibilityServer:
                 if not self.queue:
                     return
                 i = self._next_index()
-                need = projected_bytes(self.queue[i].kwargs)
+                req = self.queue[i]
+                if req.nbytes is None:
+                    try:
+                        req.nbytes = projected_bytes(req.kwargs)
+                    except Exception:  # build_engine reports what is wrong
+                        req.nbytes = 0
+                need = req.nbytes
                 if self.active and self.used + need > self.budget:
                     return
-                req = self.queue.pop(i)
+                self.queue.pop(i)
             try:
                 engine, ntimes = build_engine(**req.kwargs,
                                               beam_cache=self._beams, batch=1)

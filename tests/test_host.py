@@ -377,6 +377,36 @@ def test_stored_beam_planes_have_types_the_device_takes(dtype, wrap):
     np.testing.assert_array_equal(kept, grid_planes(beam, 150e6, True)[0])
 
 
+@pytest.mark.parametrize("method,precision,terms", [
+    ("GPUMatMul", 2, None), ("GPUMatMul", 1, None),
+    ("GPUMatMulSplitBF16", 1, 3), ("GPUMatMulSplitF16", 1, None)])
+@pytest.mark.parametrize("nant,polarized,nsrc", [
+    (350, True, 100_000), (350, True, 400_000), (1024, False, 200_000),
+    (24, True, 500)])
+def test_server_projection_covers_a_request(method, precision, terms, nant,
+                                            polarized, nsrc):
+    """The bytes a request is admitted with cover its engine's Z, accumulator
+    and split-K partials as their own rules size them, and its share of a
+    grouped launch's partials."""
+    from matvis_amd._lib import lib
+    from matvis_amd.gpu.gpu import _resolve_matprod
+    from matvis_amd.gpu.herk import Herk
+    from matvis_amd.serve import projected_bytes
+
+    kw = dict(antpos=np.zeros((nant, 3)), freqs=[1.5e8, 1.6e8],
+              fluxes=np.zeros((nsrc, 2)), beam_list=[GaussianBeam(sigma=0.2)],
+              polarized=polarized, precision=precision, matprod_method=method,
+              split_terms=terms)
+    nf = 2 if polarized else 1
+    m = nant * nf
+    form, nterms, nprod = _resolve_matprod(method, precision, terms, None)
+    h = Herk(form, m, nterms, nprod)
+    partials = lib().mv_herk_workspace_bytes(form, m, h.nslices(nf * nsrc))
+    z = m * nf * nsrc * (4 * nterms if "Split" in method else 8 * precision)
+    least = z + 16 * h.ldv ** 2 + 2 * partials
+    assert least <= projected_bytes(kw) <= 1.5 * least + 2e8
+
+
 def test_human_readable_size_and_ceildiv():
     """The reference's expected strings (tests/test_utils.py:20-38)."""
     from matvis_amd._utils import ceildiv, human_readable_size as h
