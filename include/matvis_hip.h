@@ -460,7 +460,8 @@ size_t mv_herk_grouped_workspace_bytes(int form, int tile,
  * alone, so its result is the same in any group.  problems_host is read
  * for validation and launch geometry, problems_dev (the same array in device
  * memory) by the kernels, so a captured graph replays with whatever the
- * device array holds.  No reference counterpart: the reference runs one
+ * device array holds, in shapes no larger than problems_host's (they size the
+ * workspace and the launches).  No reference counterpart: the reference runs one
  * cuBLAS call per (time, frequency, chunk). */
 int mv_herk_grouped(int form, int nterms, int nprod, int tile,
                     const mv_herk_problem *problems_host,

@@ -2059,8 +2059,16 @@ bool is_split_form(int form) {
 }
 int part_bytes(int form) { return form == MV_FORM_C128 ? 16 : 8; }
 
-GroupLayout group_layout(int form, int ts, const mv_herk_problem *q,
-                         int nprob) {
+// Panel side of a grouped launch.
+int group_side(int form, const mv_herk_problem *q, int nprob) {
+  int m = 0;
+  for (int i = 0; i < nprob; ++i) m = q[i].m > m ? q[i].m : m;
+  return is_split_form(form) ? kSP : panel_side(form, m);
+}
+
+// The partial areas are those of the plan kernel: slices of panel pairs.
+GroupLayout group_layout(int form, const mv_herk_problem *q, int nprob) {
+  const int ts = group_side(form, q, nprob);
   GroupLayout g;
   g.probs = 0;
   g.ns = align256((int64_t)nprob * sizeof(SplitProblem));
@@ -2070,10 +2078,10 @@ GroupLayout group_layout(int form, int ts, const mv_herk_problem *q,
   int64_t bytes = 0;
   for (int i = 0; i < nprob; ++i) {
     const int64_t nb = cdiv((int64_t)q[i].m, (int64_t)ts);
-    const int64_t ntiles = nb * (nb + 1) / 2;
-    bytes += (int64_t)q[i].nslices * ntiles *
-             ((int64_t)ts * ts * part_bytes(form) +
-              (is_split_form(form) ? (int64_t)ts * 8 : 0));
+    const int64_t pairs = nb * (nb + 1) / 2;
+    bytes += (int64_t)q[i].nslices *
+             (pairs * ts * ts * part_bytes(form) +
+              (is_split_form(form) ? nb * ts * 8 : 0));
   }
   g.total = g.parts + bytes;
   return g;
@@ -2095,7 +2103,7 @@ bool group_tile_ok(int form, int tile) {
 extern "C" size_t mv_herk_grouped_workspace_bytes(
     int form, int tile, const mv_herk_problem *problems, int nprob) {
   if (!group_tile_ok(form, tile) || !problems || nprob < 1) return 0;
-  return (size_t)group_layout(form, tile, problems, nprob).total;
+  return (size_t)group_layout(form, problems, nprob).total;
 }
 
 extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
@@ -2116,10 +2124,8 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
   MV_REQUIRE(problems_host && problems_dev && workspace && nprob >= 1,
              "mv_herk_grouped: null pointer or no problems");
   int64_t total_tiles = 0, max_items = 0;
-  int max_m = 0;
   for (int i = 0; i < nprob; ++i) {
     const mv_herk_problem &q = problems_host[i];
-    max_m = q.m > max_m ? q.m : max_m;
     MV_REQUIRE(q.m >= 1 && q.nseg >= 1 && q.seg_len >= 0 &&
                    q.nslices >= 1 && q.kchain >= 0,
                "mv_herk_grouped: problem %d: bad sizes m=%d nseg=%d "
@@ -2154,12 +2160,12 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
   MV_REQUIRE(total_tiles < 65536 && max_items < (int64_t)INT32_MAX / 2,
              "mv_herk_grouped: too many tiles (%lld) or items",
              (long long)total_tiles);
-  const GroupLayout g = group_layout(form, tile, problems_host, nprob);
+  const GroupLayout g = group_layout(form, problems_host, nprob);
   MV_REQUIRE(ws_bytes >= (size_t)g.total,
              "mv_herk_grouped: workspace too small (%zu < %lld)", ws_bytes,
              (long long)g.total);
   const bool f16 = form == MV_FORM_SPLIT_F16;
-  const int side = split ? kSP : panel_side(form, max_m);
+  const int side = group_side(form, problems_host, nprob);
   const bool by_wave = split && wave_pairs(nterms, tile);
   const void *kernel =
       split ? grouped_kernel(f16, nterms, maxord, by_wave)
@@ -2186,7 +2192,7 @@ extern "C" int mv_herk_grouped(int form, int nterms, int nprod, int tile,
   herk_group_plan_kernel<<<1, 256, 0, st>>>(
       problems_dev, nprob, side, by_wave ? 0 : 1,
       split ? kSK : kPK,
-      split ? form_cmax(form, max_m) : 64, split ? kGroupChain : 64,
+      split ? form_cmax(form, 0) : 64, split ? kGroupChain : 64,
       part_bytes(form), split ? 1 : 0, probs, ws + g.parts, plan);
   if (int e = check_launch("mv_herk_grouped/plan")) return e;
   const int grid = (int)(max_items < slots ? max_items : slots);

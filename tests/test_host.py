@@ -407,6 +407,37 @@ def test_server_projection_covers_a_request(method, precision, terms, nant,
     assert least <= projected_bytes(kw) <= 1.5 * least + 2e8
 
 
+@pytest.mark.parametrize("m", [1, 31, 64, 65, 128, 129, 350, 700])
+def test_grouped_workspace_is_that_of_the_panels(m):
+    """A grouped launch's workspace holds, beside its descriptors, the slices
+    of panel pairs its kernels write (and the split forms' row norms), whichever
+    tile the accumulators are padded to."""
+    from matvis_amd._lib import (FORM_C64, FORM_C128, FORM_SPLIT_BF16, lib)
+    from matvis_amd.gpu.herk_group import PROBLEM_DTYPE
+
+    p = np.zeros(3, PROBLEM_DTYPE)
+    p["m"], p["nslices"] = [m, 1, 1], [50, 1, 1]
+
+    def extra(form, tile):  # of 50 slices of m rows over one of a row
+        def total():
+            return lib().mv_herk_grouped_workspace_bytes(
+                form, tile, p.ctypes.data, 3)
+        p["nslices"][0] = 50
+        many = total()
+        p["nslices"][0] = 1
+        return many - total()
+
+    def pairs(side):
+        n = -(-m // side)
+        return n * (n + 1) // 2 * side * side, n * side
+
+    area, rows = pairs(64)
+    for tile in (64, 128):
+        assert extra(FORM_SPLIT_BF16, tile) == 49 * (area * 8 + rows * 8)
+    assert extra(FORM_C128, 64) == 49 * pairs(32)[0] * 16
+    assert extra(FORM_C64, 64) == 49 * pairs(64 if m > 128 else 32)[0] * 8
+
+
 def test_human_readable_size_and_ceildiv():
     """The reference's expected strings (tests/test_utils.py:20-38)."""
     from matvis_amd._utils import ceildiv, human_readable_size as h
