@@ -378,3 +378,28 @@ def test_grouped_batch_tiles():
         n = t["ldv"]
         np.testing.assert_array_equal(D.to_host(t["vacc"]),
                                       D.to_host(w["vacc"])[:n, :n])
+
+
+def test_grouped_complex64_bits_alone_and_in_a_group():
+    """complex64 problems of up to 128 rows run 32-row panels alone and 64-row
+    ones beside larger problems: the same bits."""
+    import torch
+    from matvis_amd._lib import FORM_C64
+    from matvis_amd.gpu.herk_group import HerkGroup
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    probs = []
+    for m, k in ((5, 77), (64, 3000), (100, 2049), (128, 5000), (200, 1500)):
+        z = torch.randn((m, k, 2), device="cuda", generator=g)
+        ldv = -(-m // 64) * 64
+        probs.append(dict(terms=[z], m=m, ldz=k, nseg=1, seg_stride=k,
+                          seg_len=k, vacc=D.zeros((ldv, ldv), np.complex128),
+                          ldv=ldv, scale=1.0, accumulate=False))
+    HerkGroup(FORM_C64, 1, 1, 64, probs).run()
+    for p in probs[:-1]:
+        alone = dict(p, vacc=D.zeros(tuple(p["vacc"].shape), np.complex128))
+        HerkGroup(FORM_C64, 1, 1, 64, [alone]).run()
+        m = p["m"]
+        up = np.triu_indices(m)
+        np.testing.assert_array_equal(D.to_host(p["vacc"])[:m, :m][up],
+                                      D.to_host(alone["vacc"])[:m, :m][up])
