@@ -3,21 +3,22 @@
 The knobs, chosen per class of problems (m rounded up to a power of two,
 K = nseg x seg_len rounded up to a power of four):
 
-* tile side (split forms): 64 or 128 rows.  Three-term problems of up to 64
-  rows run one wave a panel pair at 64 and eight waves a panel group at 128;
-  all others run panel groups at either (herk_group.launch_tiles).  The plain
+* tile side (split forms): 64 or 128 rows, where the two are different
+  launches (herk_group.launch_tiles): three-term problems of up to 64 rows run
+  one wave a panel pair at 64 and eight waves a panel group at 128; all others
+  run panel groups at either, and tiles are reported as they run.  The plain
   forms have one tile (64 rows).
 * kchain, the longest K-slice in K tiles (split forms 192, 96 or 48; plain
   forms 64, 32 or 16): shorter slices give a batch that does not fill the
   GPU more work items, at the cost of more partial tiles to write and
-  reduce.  The split forms' 192 is also their accuracy cap on an FP32
-  chain, so the tuner only shortens chains.
+  reduce.  The split forms' 192 is their accuracy cap on an FP32 chain.
 
-Search: coordinate descent from the default (64-row tiles for m <= 128,
-128 otherwise; the form's chain cap).  Classes are visited in order of
-descending work.  Each candidate changes one knob of one class and is timed
-as the whole batch's grouped launches (HIP events, the mean of `reps` runs
-after one warm run).  A change is kept when it is at least 1% faster.  The
+Search: coordinate descent from what an untuned launch runs (64-row tiles for
+m <= 128, 128 otherwise; chains of 96 K tiles in the split forms, 64 in the
+plain ones), whose time is the plan's default_ms.  Classes are visited in
+order of descending work.  Each candidate changes one knob of one class and is
+timed as the whole batch's grouped launches (HIP events, the mean of `reps`
+runs after one warm run).  A change is kept when it is at least 1% faster.  The
 search ends after a pass without a kept change or when the time budget is
 spent.  Results are cached per batch signature (form, terms, products and
 the multiset of classes) in memory and, if ``MATVIS_AMD_TUNE_CACHE`` names a
@@ -37,10 +38,12 @@ from dataclasses import dataclass, field
 import torch
 
 from .herk import is_split
-from .herk_group import GroupedBatch, tile_for
+from .herk_group import GroupedBatch, launch_tiles, tile_for
 
-#: K-slice lengths (K tiles) the search tries, longest (the default) first
+#: K-slice lengths (K tiles) the search tries, longest first
 CHAINS = {True: (192, 96, 48), False: (64, 32, 16)}
+#: those of a launch that names none (kGroupChain in csrc/herk.hip)
+UNTUNED_CHAIN = {True: 96, False: 64}
 #: tile sides of the grouped kernels
 TILES = {True: (64, 128), False: (64,)}
 #: a candidate must beat the incumbent by this fraction to be kept
@@ -67,8 +70,14 @@ def signature(form: int, nterms: int, nprod: int, problems: list) -> str:
 
 
 def default_config(form: int, cls: tuple[int, int]) -> tuple[int, int]:
+    """A class's default tile and longest chain."""
     split = is_split(form)
     return (tile_for(form, cls[0]), CHAINS[split][0])
+
+
+def untuned_config(form: int, cls: tuple[int, int]) -> tuple[int, int]:
+    """What a class runs with when nothing is tuned."""
+    return (default_config(form, cls)[0], UNTUNED_CHAIN[is_split(form)])
 
 
 @dataclass
@@ -93,6 +102,23 @@ class Plan:
 def assignment(config: dict, problems: list) -> tuple[list, list]:
     cls = [problem_class(p) for p in problems]
     return ([config[c][0] for c in cls], [config[c][1] for c in cls])
+
+
+def effective(form: int, nterms: int, config: dict, problems: list) -> tuple:
+    """(tiles, chains) the batch runs with under a configuration."""
+    tiles, chains = assignment(config, problems)
+    return launch_tiles(form, nterms, problems, tiles), chains
+
+
+def _as_run(form, nterms, config, problems) -> dict:
+    """The configuration with each class's tile as it runs, where its
+    problems share one."""
+    tiles, _ = effective(form, nterms, config, problems)
+    run: dict[tuple, set] = {}
+    for p, t in zip(problems, tiles):
+        run.setdefault(problem_class(p), set()).add(t)
+    return {c: (next(iter(run[c])) if len(run.get(c, ())) == 1 else t, k)
+            for c, (t, k) in config.items()}
 
 
 def time_assignment(form, nterms, nprod, problems, tiles, kchains,
@@ -148,15 +174,16 @@ def tune(form: int, nterms: int, nprod: int, problems: list,
     key = signature(form, nterms, nprod, problems)
     hit = _cached(key)
     if hit is not None:
-        tiles, chains = assignment(hit, problems)
-        return Plan(tiles, chains, dict(hit), cached=True)
+        tiles, chains = effective(form, nterms, hit, problems)
+        return Plan(tiles, chains, _as_run(form, nterms, hit, problems),
+                    cached=True)
     split = is_split(form)
     classes = sorted({problem_class(p) for p in problems})
     work = {c: 0.0 for c in classes}
     for p in problems:
         work[problem_class(p)] += float(p["m"]) ** 2 * p["nseg"] * p["seg_len"]
     order = sorted(classes, key=lambda c: -work[c])
-    config = {c: default_config(form, c) for c in classes}
+    config = {c: untuned_config(form, c) for c in classes}
 
     def measure(cfg):
         return time_assignment(form, nterms, nprod, problems,
@@ -177,13 +204,18 @@ def tune(form: int, nterms: int, nprod: int, problems: list,
                     break
                 trial = dict(config)
                 trial[c] = cand
+                if (effective(form, nterms, trial, problems)
+                        == effective(form, nterms, config, problems)):
+                    continue  # the same launch
                 ms = measure(trial)
                 trials += 1
                 if ms < best * (1.0 - GAIN):
                     best, config, improved = ms, trial, True
+    # kept as searched: accumulators of another batch of this signature may
+    # be padded otherwise
     with _lock:
         _cache[key] = dict(config)
     _store_file(key, config)
-    tiles, chains = assignment(config, problems)
-    return Plan(tiles, chains, config, default_ms=default, best_ms=best,
-                trials=trials)
+    tiles, chains = effective(form, nterms, config, problems)
+    return Plan(tiles, chains, _as_run(form, nterms, config, problems),
+                default_ms=default, best_ms=best, trials=trials)

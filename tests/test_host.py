@@ -499,3 +499,36 @@ def test_autotune_classes_signature_and_cache(tmp_path, monkeypatch):
     key = A.signature(FORM_SPLIT_BF16, 2, 4, ps)
     A._store_file(key, cfg)
     assert A._cached(key) == cfg
+
+
+@pytest.mark.parametrize("nterms,nprod", [(2, 3), (3, 6)])
+def test_autotune_tries_launches_that_differ(nterms, nprod, monkeypatch):
+    """The search starts from what an untuned launch runs (chains of 96 K
+    tiles), times no two configurations that are the same launch, and reports
+    the tiles that run: two terms take 128-row launches at either tile, three
+    of up to 64 rows have both."""
+    from matvis_amd._lib import FORM_SPLIT_BF16
+    from matvis_amd.gpu import autotune as A
+
+    probs = [dict(m=m, nseg=1, seg_len=k, ldv=-(-m // 128) * 128)
+             for m, k in ((50, 977), (100, 9000), (300, 20000))]
+    seen = []
+
+    def timed(form, nt, npd, problems, tiles, chains, reps=3):
+        run = A.launch_tiles(form, nt, problems, tiles)
+        seen.append((tuple(run), tuple(chains)))
+        return 1.0 + 0.1 * sum(c != 48 for c in chains)
+
+    monkeypatch.setattr(A, "time_assignment", timed)
+    monkeypatch.setattr(A, "_cache", {})
+    monkeypatch.delenv("MATVIS_AMD_TUNE_CACHE", raising=False)
+    plan = A.tune(FORM_SPLIT_BF16, nterms, nprod, probs)
+    first = 64 if nterms == 3 else 128
+    assert seen[0] == ((first, 128, 128), (96, 96, 96))
+    assert all(a != b for a, b in zip(seen, seen[1:]))
+    assert len({t for t, _ in seen}) == (2 if nterms == 3 else 1)
+    assert plan.kchains == [48] * 3 and plan.tiles == [first, 128, 128]
+    assert sorted(t for t, _ in plan.config.values()) == sorted(plan.tiles)
+    again = A.tune(FORM_SPLIT_BF16, nterms, nprod, probs)
+    assert again.cached and (again.tiles, again.config) == (plan.tiles,
+                                                            plan.config)
