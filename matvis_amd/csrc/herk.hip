@@ -445,14 +445,16 @@ __host__ __device__ inline int plain_wide(const PlainProblem<T> &Q, int nseg) {
 // the peak (78.6 and 157 TFLOP/s); m = 64, 3.6k columns 26 -> 19 and 22 -> 16
 // us.  (Three products 1.50 and 0.78 ms.)
 // Errors against 64 bits (complex128: extended precision) over sqrt(V_ii
-// V_jj), m = 160, 60k columns, one chain a real part -> two and shorter slices:
-// Re, phases within 0.3 rad 6.6e-8 -> 3.7e-8 and 1.5e-16 -> 9.0e-17, incoherent
-// Z 2.1e-9 -> 1.6e-9 and 4.2e-18 -> 2.9e-18; Im as before (7e-10 and 1.4e-18,
-// incoherent 2e-9 and 4e-18).  A time of the 350-antenna sky in complex64
-// 9.6e-7 -> 3.7e-7 of |V|.  The diagonal is exactly real.
+// V_jj), m = 160, 60k columns, one chain a real part and 64-78 slices -> two
+// and 128 (slice_reach): Re, phases within 0.3 rad 6.6e-8 -> 1.9e-8 and 1.5e-16
+// -> 7.2e-17, incoherent Z 2.1e-9 -> 1.1e-9 and 4.2e-18 -> 2.2e-18; Im 6.9e-10
+// -> 5.3e-10 and 1.4e-18 -> 1.0e-18, incoherent 2.0e-9 -> 1.5e-9 and 4.1e-18 ->
+// 3.0e-18.  A time of the 350-antenna sky in complex64 9.6e-7 -> 2.3e-7 of |V|.
+// The diagonal is exactly real.
 //
 // Copies go straight from global memory into the other LDS stage
-// (global_load_lds: 16 bytes a lane where rows are 16-byte aligned, else 4),
+// (global_load_lds: 16 bytes a lane where rows are 16-byte aligned, else 4:
+// complex64 rows of an odd length, m = 700, 59.7k columns 1.28 ms for 1.04),
 // each wave one panel, while the current K tile is computed; the last K tile
 // of a segment that is not whole goes through registers with a column mask.
 // Rows past m are read as row m - 1: they reach output rows and columns past
@@ -1573,14 +1575,15 @@ int split_maxord(int nterms, int nprod) {
 // chain error stays near 1e-7 relative at 62 tiles and grows about as the
 // square root of the length; 192 tiles keeps it well under 1e-6 while the
 // partial tiles written per launch stay small.  The plain forms' real parts grow
-// with the length in the same way, in FP64 too: with two chains of 96 K tiles
-// 9.0e-17 of sqrt(V_ii V_jj) where one slice a slot in one chain gave 1.5e-16
-// (m = 160, 60k columns, phases within 0.3 rad), and the workspace of 96 is what
-// long sums already take.  Problems of few rows write few partials: 64.
+// with the length in the same way, in FP64 too.  96 K tiles: 59.7k sources of 350
+// antennas in complex64 with 128 3.7e-7 of |V|, with 96 2.3e-7, in the same 8.69
+// ms for 4 frequencies; complex128, m = 160, 60k columns, 9.0e-17 of
+// sqrt(V_ii V_jj) where one slice a slot gave 1.5e-16.  Problems of few rows
+// write few partials: 64.
 int form_cmax(int form, int m) {
   switch (form) {
     case MV_FORM_C128: return 96;
-    case MV_FORM_C64: return m > 128 ? 128 : 64;
+    case MV_FORM_C64: return m > 128 ? 96 : 64;
     default: return 192;
   }
 }
