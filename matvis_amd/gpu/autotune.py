@@ -15,8 +15,8 @@ K = nseg x seg_len rounded up to a power of four):
 
 Search: coordinate descent from what an untuned launch runs (64-row tiles for
 m <= 128, 128 otherwise; chains of 96 K tiles in the split forms, 64 in the
-plain ones), whose time is the plan's default_ms.  Classes are visited in
-order of descending work.  Each candidate changes one knob of one class and is
+plain ones), whose time is the plan's default_ms, or from the longest chains in
+every class where those are faster.  Classes are visited in order of descending work.  Each candidate changes one knob of one class and is
 timed as the whole batch's grouped launches (HIP events, the mean of `reps`
 runs after one warm run).  A change is kept when it is at least 1% faster.  The
 search ends after a pass without a kept change or when the time budget is
@@ -192,6 +192,14 @@ def tune(form: int, nterms: int, nprod: int, problems: list,
     t_end = time.perf_counter() + budget_s
     best = default = measure(config)
     trials = 1
+    # the longest chains of all classes at once: a batch that fills the GPU
+    # gains a little of them in each class, less than GAIN by itself
+    longest = {c: default_config(form, c) for c in classes}
+    if longest != config:
+        ms = measure(longest)
+        trials += 1
+        if ms < best * (1.0 - GAIN):
+            best, config = ms, longest
     improved = True
     while improved and time.perf_counter() < t_end:
         improved = False
