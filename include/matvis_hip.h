@@ -327,9 +327,9 @@ int mv_herk_max_slices(int form, int m, int64_t kmax);
 
 /* The slice count mv_herk uses for seg_len columns per segment given a
  * capacity of nslices (the kernels choose it on the device from the device
- * column count by the same rule): enough slices that no FP32 accumulation
- * chain exceeds the form's limit, then the one that best fills the GPU's
- * resident workgroup slots.  Returns the count, or a negative status.  No
+ * column count by the same rule): enough slices that no accumulation chain
+ * exceeds the form's limit, then the one that best fills the GPU's resident
+ * workgroup slots, or a power of two where none can.  Returns the count, or a negative status.  No
  * reference counterpart (reporting and workspace planning). */
 int mv_herk_slices(int form, int nterms, int nprod, int m, int nseg,
                    int64_t seg_len, int nslices);
