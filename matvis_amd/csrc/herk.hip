@@ -229,8 +229,8 @@ __device__ __forceinline__ void wait_global_loads() {
 // two on every tile of a half-empty last column (11 panels: 21 tiles).
 // Measured against whole pairs, four a group in sequence: m = 128 split, 2 x
 // 15k columns, 47 -> 42 us; m = 32 complex64, 3.6k columns, 9.6 -> 7.0; 6
-// frequencies of 61 antennas (m = 122) FP64, a time 283 -> 258; 24 grouped
-// instances of 64-350 antennas 458 -> 417; m = 700 1% less.
+// frequencies of 61 antennas (m = 122) FP64 (three real products), a time 283 ->
+// 258; 24 grouped instances of 64-350 antennas 458 -> 417; m = 700 1% less.
 __host__ __device__ inline int panel_groups(int n) {
   const int h = n / 2;
   const int off = h * (h - 1) / 2;
